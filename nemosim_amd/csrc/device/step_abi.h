@@ -144,6 +144,16 @@ int nemo_dev_apply_stdp(uint32_t* syn, const uint32_t* rcm_fwd, int32_t* rcm_acc
 		const void* stdp_dev, int32_t fx_reward, void* stream);
 int nemo_dev_fill_u32(uint32_t* p, uint32_t value, size_t n, void* stream);
 int nemo_dev_fill_u64(uint64_t* p, uint64_t value, size_t n, void* stream);
+/* The raster of a run (rows of `words` 64-bit words, one per cycle) as fired
+ * counts and ids (csrc/device/raster_kernel.hip). counts, offs and out are
+ * host memory the device can reach (pinned). The ids of cycle t take the
+ * positions offs[t], offs[t]+1, ... of the run's list; those in [lo, hi) are
+ * written to out[position - lo], as ids[local index], or first + local index
+ * where ids is NULL. */
+int nemo_dev_raster_count(const uint64_t* raster, uint32_t words, uint32_t n, uint32_t cycles, uint32_t* counts,
+		void* stream);
+int nemo_dev_raster_ids(const uint64_t* raster, uint32_t words, uint32_t n, uint32_t cycles, const uint64_t* offs,
+		uint64_t lo, uint64_t hi, const uint32_t* ids, uint32_t first, uint32_t* out, void* stream);
 /* Evaluates the device math pieces on inputs in[] (for tests):
  * kind 0 = logf_glibc(in), 1 = sinf_rng(in), 2 = kuramoto_wrap(in), 3 = sinf_glibc(in) */
 int nemo_dev_eval_libm(int kind, const float* in_dev, float* out_dev, size_t n, void* stream);

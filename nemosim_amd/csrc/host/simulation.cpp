@@ -192,10 +192,12 @@ Simulation::Simulation(const NetworkImpl& net, const ConfigurationImpl& conf) :
 	if(m_n >= (1u << 26)) {
 		throw exception(NEMO_API_UNSUPPORTED, "the HIP backend supports up to 2^26 neurons per simulation");
 	}
+	m_affineIds = true;
 	if(m_n > 0) {
 		m_dense.assign(size_t(maxG - m_minG) + 1, 0u);
 		for(uint32_t l = 0; l < m_n; ++l) {
 			m_dense[m_localToGlobal[l] - m_minG] = l + 1;
+			m_affineIds = m_affineIds && m_localToGlobal[l] == m_minG + l;
 		}
 	} else {
 		m_minG = 0;
@@ -1511,30 +1513,118 @@ Simulation::run(unsigned nsteps, const nemo_schedule_t* schedule, unsigned long 
 	launch(nsteps, events);
 }
 
+/* Pinned staging of readFired, one block for the process: it is used only
+ * while the device lock is held, and never freed, so no HIP call runs at
+ * process exit. Counts and list positions of READ_CYCLES cycles at a time,
+ * and two windows of ids, so that the device fills one while the host copies
+ * the other into the caller's buffer. */
+namespace {
+const size_t READ_CYCLES = 16384;
+const size_t READ_WINDOW = size_t(1) << 18;   /* ids: 1 MB */
+
+struct ReadStaging {
+	uint64_t offs[READ_CYCLES];
+	uint32_t counts[READ_CYCLES];
+	uint32_t ids[2][READ_WINDOW];
+};
+
+ReadStaging*
+readStaging()
+{
+	static ReadStaging* st = nullptr;
+	if(!st) {
+		void* p = nullptr;
+		hipCheck(hipHostMalloc(&p, sizeof(ReadStaging), hipHostMallocPortable), "hipHostMalloc");
+		st = static_cast<ReadStaging*>(p);
+	}
+	return st;
+}
+} // namespace
+
+/* Rasters of up to 96 KB are copied and decoded here (62 KB: 35 us for the
+ * count and the list, 47 us by the kernels, whose launches and waits cost
+ * that much whatever the size; 125 KB: 50 us either way), larger ones by the
+ * kernels of csrc/device/raster_kernel.hip (250 KB: 73 us here, 48 us there;
+ * 25 MB: 26.8 against 0.5 ms). An ids buffer that is too small receives the
+ * cycles that fit in whole, and counts those and the one that did not. */
+static const size_t READ_HOST_WORDS = 96u * 1024u / 8u;
+
 void
 Simulation::readFired(unsigned counts[], unsigned ids[], size_t cap, size_t* total)
 {
 	std::lock_guard<DeviceMutex> devLock(deviceMutex());
 	requireOwnRaster();
-	size_t nw = size_t(m_lastRunSteps) * m_words;
-	m_rasterHost.resize(nw);
-	if(nw) {
-		hipCheck(hipMemcpy(m_rasterHost.data(), d_raster.ptr, nw * 8, hipMemcpyDeviceToHost), "D2H");
-	}
-	size_t k = 0;
-	std::vector<unsigned> one;
-	for(unsigned t = 0; t < m_lastRunSteps; ++t) {
-		decodeStep(m_rasterHost.data() + size_t(t) * m_words, one);
-		if(counts) counts[t] = unsigned(one.size());
-		if(ids) {
-			if(k + one.size() > cap) {
-				throw exception(NEMO_BUFFER_OVERFLOW, "fired-id buffer too small");
-			}
-			std::copy(one.begin(), one.end(), ids + k);
+	const size_t nw = size_t(m_lastRunSteps) * m_words;
+	if(nw <= READ_HOST_WORDS || m_n == 0) {
+		m_rasterHost.resize(nw);
+		if(nw) {
+			hipCheck(hipMemcpy(m_rasterHost.data(), d_raster.ptr, nw * 8, hipMemcpyDeviceToHost), "D2H");
 		}
-		k += one.size();
+		size_t k = 0;
+		std::vector<unsigned> one;
+		for(unsigned t = 0; t < m_lastRunSteps; ++t) {
+			decodeStep(m_rasterHost.data() + size_t(t) * m_words, one);
+			if(counts) counts[t] = unsigned(one.size());
+			if(ids) {
+				if(k + one.size() > cap) {
+					throw exception(NEMO_BUFFER_OVERFLOW, "fired-id buffer too small");
+				}
+				std::copy(one.begin(), one.end(), ids + k);
+			}
+			k += one.size();
+		}
+		if(total) *total = k;
+		return;
 	}
-	if(total) *total = k;
+	hipStream_t st = static_cast<hipStream_t>(m_stream);
+	hipCheck(hipSetDevice(m_device), "hipSetDevice");
+	if(ids && !m_affineIds && !d_ids.ptr) {
+		d_ids.upload(m_localToGlobal.data(), size_t(m_n) * 4);
+	}
+	ReadStaging* rs = readStaging();
+	const uint64_t* raster = d_raster.as<uint64_t>();
+	size_t done = 0;   /* ids of the earlier cycles */
+	for(size_t t0 = 0; t0 < m_lastRunSteps; t0 += READ_CYCLES) {
+		const size_t nt = std::min<size_t>(READ_CYCLES, m_lastRunSteps - t0);
+		const uint64_t* rows = raster + t0 * m_words;
+		hipCheck(nemo_dev_raster_count(rows, m_words, m_n, uint32_t(nt), rs->counts, st), "raster counts");
+		hipCheck(hipStreamSynchronize(st), "hipStreamSynchronize");
+		uint64_t here = 0;
+		size_t fit = 0;   /* cycles whose ids fit */
+		bool over = false;
+		for(; fit < nt && !over; ++fit) {
+			if(counts) counts[t0 + fit] = rs->counts[fit];
+			if(ids && done + here + rs->counts[fit] > cap) {
+				over = true;
+				break;
+			}
+			rs->offs[fit] = here;
+			here += rs->counts[fit];
+		}
+		if(ids && here > 0) {
+			/* window by window; a window's launch covers the cycles with ids in it */
+			auto list = [&](uint64_t lo) {
+				const uint64_t hi = std::min<uint64_t>(here, lo + READ_WINDOW);
+				const size_t c0 = size_t(std::upper_bound(rs->offs, rs->offs + fit, lo) - rs->offs) - 1;
+				const size_t c1 = size_t(std::lower_bound(rs->offs, rs->offs + fit, hi) - rs->offs);
+				hipCheck(nemo_dev_raster_ids(rows + c0 * m_words, m_words, m_n, uint32_t(c1 - c0), rs->offs + c0, lo, hi,
+							m_affineIds ? nullptr : d_ids.as<uint32_t>(), m_minG, rs->ids[(lo / READ_WINDOW) & 1u], st),
+						"raster ids");
+			};
+			list(0);
+			for(uint64_t lo = 0; lo < here; lo += READ_WINDOW) {
+				hipCheck(hipStreamSynchronize(st), "hipStreamSynchronize");
+				if(lo + READ_WINDOW < here) list(lo + READ_WINDOW);
+				std::memcpy(ids + done + lo, rs->ids[(lo / READ_WINDOW) & 1u],
+						size_t(std::min<uint64_t>(here - lo, READ_WINDOW)) * 4);
+			}
+		}
+		done += size_t(here);
+		if(over) {
+			throw exception(NEMO_BUFFER_OVERFLOW, "fired-id buffer too small");
+		}
+	}
+	if(total) *total = done;
 }
 
 void

@@ -194,6 +194,8 @@ class Simulation
 
 		/* index maps */
 		std::vector<unsigned> m_localToGlobal;
+		bool m_affineIds = true;               /* user index = m_minG + local index */
+		DevBuf d_ids;                          /* [n] user indices, where not affine (readFired) */
 		std::vector<uint32_t> m_dense;         /* gidx - m_minG -> local + 1 (0: none) */
 		unsigned m_minG = 0;
 		std::vector<uint8_t> m_model;
