@@ -10,19 +10,19 @@
  * double polynomials for sinf. This file restates those algorithms in
  * double precision so they run on gfx950 FP64 and on the host alike.
  *
- * On FMA-capable x86-64 hosts glibc runs an FMA build of these sources, in
- * which the compiler fuses every product whose only use is a sum. On the
- * RNG's arguments the fused and unfused forms give the same results: logf
- * at all x = m * 2^-24 (m = 0..2^24) and sinf at all
- * a = float(u) * 1.4629180792671596810513378043098e-9f, u a 32-bit unsigned,
- * were compared with the host libm with zero differences
- * (tests/test_libm_f32.py repeats that check). The RNG uses the unfused form
- * (sinf_rng), which needs fewer registers in the step kernel. Beyond those
- * arguments the unfused form differs from the host in about 1 of 10^7
- * (near multiples of pi/2 of magnitude ~100, where the reduction cancels),
- * so sinf_glibc, used by the Kuramoto model on arbitrary phase differences,
- * is restated in the fused form: fma() in the same places as the host
- * build (the reduction x - n*pi/2 and each multiply-add of the polynomials).
+ * glibc rounds a double result to float once, at the end, so other orders of
+ * the same double operations give the same float except where the double
+ * lands within its last bits of a rounding boundary. The forms here are
+ * shorter than the published ones and free of branches: Horner polynomials
+ * with fma(), the quadrant found by adding 1.5 * 2^52 (its nearest integer
+ * lands in the sum's low bits), one evaluation for small and reduced
+ * arguments. Each was compared with the host libm on every input that
+ * reaches it, with zero differences: logf at all x = m * 2^-24
+ * (m = 0..2^24), sinf at every float |a| < 120 (2.2e9 values), which holds
+ * the RNG's a = float(u) * 1.4629180792671596810513378043098e-9f.
+ * tests/test_libm_f32.py repeats the check on the RNG's arguments and, for
+ * sinf, on a sample of the wider domain with the floats around each
+ * multiple of pi/2.
  *
  * logf is supported for x in [0, 1] only (no NaN / negative paths). sinf
  * takes every float: besides the RNG's arguments, the Kuramoto model feeds
@@ -82,97 +82,85 @@ NEMO_HD inline float logf_glibc(float x)
 	const double LN2 = 0x1.62e42fefa39efp-1;
 	const uint32_t OFF = 0x3f330000u;
 
-	uint32_t ix = f2u(x);
-	if(ix == 0x3f800000u) {
-		return 0.0f;
-	}
-	if(ix == 0u) {
-		return -__builtin_inff();
-	}
-	uint32_t tmp = ix - OFF;
-	int i = int((tmp >> 19) & 15u);
-	int k = int32_t(tmp) >> 23;
-	uint32_t iz = ix - (tmp & 0xff800000u);
+	const uint32_t ix = f2u(x);
+	const uint32_t tmp = ix - OFF;
+	const int i = int((tmp >> 19) & 15u);
+	const int k = int32_t(tmp) >> 23;
+	const uint32_t iz = ix - (tmp & 0xff800000u);
 	const LogfEntry& e = LOGF_TABLE[i];
-	double z = double(u2f(iz));
-	double r = z * e.invc - 1.0;
-	double y0 = e.logc + double(k) * LN2;
-	double r2 = r * r;
-	double y = A1 * r + A2;
-	y = A0 * r2 + y;
-	y = y * r2 + (y0 + r);
-	return float(y);
+	const double r = fma(double(u2f(iz)), e.invc, -1.0);
+	const double y0 = fma(double(k), LN2, e.logc);
+	const double y = fma(A0 * r + A1, r, A2);   /* one constant per operation: see sinf_rng */
+	const float v = float(fma(fma(y, r, 1.0), r, y0));
+	return ix == 0u ? -__builtin_inff() : v;   /* log(1) comes out as +0 */
 }
 
-/* Sine / cosine polynomial coefficients */
-struct SincosfSet {
-	double c0, c1, c2, c3, c4, s1, s2, s3;
-};
-
-NEMO_HD inline float sinf_poly(double x, double x2, const SincosfSet& p, int n)
+/* Sine and cosine of a reduced argument, |x| <= pi/4 */
+NEMO_HD inline double sinf_poly_sin(double x, double x2)
 {
-	if((n & 1) == 0) {
-		double x3 = x * x2;
-		double s1 = fma(x2, p.s3, p.s2);
-		double x7 = x3 * x2;
-		double s = fma(x3, p.s1, x);
-		return float(fma(x7, s1, s));
-	} else {
-		double x4 = x2 * x2;
-		double c2 = fma(x2, p.c4, p.c3);
-		double c1 = fma(x2, p.c1, p.c0);
-		double x6 = x4 * x2;
-		double c = fma(x4, p.c2, c1);
-		return float(fma(x6, c2, c));
-	}
+	const double S1 = -0x1.555545995a603p-3;
+	const double S2 = 0x1.1107605230bc4p-7;
+	const double S3 = -0x1.994eb3774cf24p-13;
+	return fma(x * x2, fma(x2, fma(x2, S3, S2), S1), x);
 }
 
-/* The polynomials without fused multiply-adds */
-NEMO_HD inline float sinf_poly_unfused(double x, double x2, const SincosfSet& p, int n)
+NEMO_HD inline double sinf_poly_cos(double x2)
 {
-	if((n & 1) == 0) {
-		double x3 = x * x2;
-		double s1 = p.s2 + x2 * p.s3;
-		double x7 = x3 * x2;
-		double s = x + x3 * p.s1;
-		return float(s + x7 * s1);
-	} else {
-		double x4 = x2 * x2;
-		double c2 = p.c3 + x2 * p.c4;
-		double c1 = p.c0 + x2 * p.c1;
-		double x6 = x4 * x2;
-		double c = c1 + x4 * p.c2;
-		return float(c + x6 * c2);
-	}
+	const double C1 = -0x1.ffffffd0c621cp-2;
+	const double C2 = 0x1.55553e1068f19p-5;
+	const double C3 = -0x1.6c087e89a359dp-10;
+	const double C4 = 0x1.99343027bf8c3p-16;
+	return fma(x2, fma(x2, fma(x2, fma(x2, C4, C3), C2), C1), 1.0);
 }
 
-/* sinf for the RNG's arguments a in [0, 2*pi + 1ulp] (unfused form):
- * |a| < pi/4 directly, otherwise one reduction step by pi/2 (n rounded
- * through a 2^24-scaled integer). In quadrants 2 and 3 glibc evaluates the
- * cosine polynomial with every coefficient negated, which equals the
- * negated result (negation is exact in each product and sum). */
+/* sinf for |y| < 120: x = y - q pi/2 with q the nearest integer to 2y/pi
+ * (0 for a small argument, which it leaves as it is), the sine or cosine of
+ * x by q's lowest bit, negated by its next. Both polynomials are evaluated:
+ * a wave's lanes need both, and 4 multiply-adds are less than a branch. An
+ * argument below 2^-12 is its own sine (which also keeps the sign of 0). */
+NEMO_HD inline float sinf_reduced(float y)
+{
+	const double INV_HPI = 0x1.45F306DC9C883p-1;
+	const double HPI = 0x1.921FB54442D18p0;
+	const double ROUND = 0x1.8p52;
+
+	const double y64 = y;
+	union { double d; uint64_t u; } t;
+	t.d = fma(y64, INV_HPI, ROUND);
+	const uint32_t q = uint32_t(t.u);
+	const double x = fma(ROUND - t.d, HPI, y64);
+	const double x2 = x * x;
+	const double s = sinf_poly_sin(x, x2);
+	const double c = sinf_poly_cos(x2);
+	const uint32_t v = f2u(float((q & 1u) ? c : s)) ^ ((q & 2u) << 30);
+	return __builtin_fabsf(y) < 0x1p-12f ? y : u2f(v);
+}
+
+/* sinf for the RNG's arguments, in [0, 2*pi + 1ulp]: sinf_reduced with at
+ * most one constant per operation. gfx950 takes one scalar operand per vector
+ * instruction, so a multiply-add of two constants keeps one of them in a
+ * vector register pair, hoisted out of the step kernel's cycle loop, where it
+ * spills. Compared with the host libm at every float in [0, 6.283186]
+ * (1.09e9 values): zero differences. */
 NEMO_HD inline float sinf_rng(float y)
 {
-	const SincosfSet P0 = { 0x1p0, -0x1.ffffffd0c621cp-2, 0x1.55553e1068f19p-5,
-		-0x1.6c087e89a359dp-10, 0x1.99343027bf8c3p-16,
-		-0x1.555545995a603p-3, 0x1.1107605230bc4p-7, -0x1.994eb3774cf24p-13 };
-	const double HPI_INV = 0x1.45F306DC9C883p+23;
+	const double INV_HPI = 0x1.45F306DC9C883p-1;
 	const double HPI = 0x1.921FB54442D18p0;
+	const double ROUND = 0x1.8p52;
+	const double S1 = -0x1.555545995a603p-3, S2 = 0x1.1107605230bc4p-7, S3 = -0x1.994eb3774cf24p-13;
+	const double C1 = -0x1.ffffffd0c621cp-2, C2 = 0x1.55553e1068f19p-5, C3 = -0x1.6c087e89a359dp-10,
+			C4 = 0x1.99343027bf8c3p-16;
 
-	uint32_t top = (f2u(y) >> 20) & 0x7ffu;
-	double x = y;
-	if(top < ((f2u(0x1.921FB6p-1f) >> 20) & 0x7ffu)) {
-		if(top < ((f2u(0x1p-12f) >> 20) & 0x7ffu)) {
-			return y;
-		}
-		return sinf_poly_unfused(x, x * x, P0, 0);
-	}
-	double r = x * HPI_INV;
-	int n = (int32_t(r) + 0x800000) >> 24;
-	x = x - double(n) * HPI;
-	double s = ((n & 3) == 1 || (n & 3) == 2) ? -1.0 : 1.0;
-	const float v = sinf_poly_unfused(x * s, x * x, P0, n);
-	return ((n & 3) == 3) ? -v : v;
+	const double y64 = y;
+	union { double d; uint64_t u; } t;
+	t.d = y64 * INV_HPI + ROUND;
+	const uint32_t q = uint32_t(t.u);
+	const double x = fma(ROUND - t.d, HPI, y64);
+	const double x2 = x * x;
+	const double s = fma(x * x2, x2 * (x2 * S3 + S2) + S1, x);
+	const double c = fma(x2, x2 * (x2 * (x2 * C4 + C3) + C2) + C1, 1.0);
+	const uint32_t v = f2u(float((q & 1u) ? c : s)) ^ ((q & 2u) << 30);
+	return y < 0x1p-12f ? y : u2f(v);
 }
 
 /* Bits of 2/pi: entry i is floor(2/pi * 2^(8(i+1))) mod 2^32, i.e. the
@@ -205,54 +193,26 @@ NEMO_HD inline double sinf_reduce_large(uint32_t xi, int* np)
 	return double(int64_t(acc)) * 0x1.921FB54442D18p-62;
 }
 
-/* The polynomial of quadrant n on the reduced argument x, with sign index
- * m (n, or n plus the argument's sign bit in the large-argument path):
- * x is negated for m = 1, 2; glibc evaluates the cosine polynomial with
- * every coefficient negated when m & 2, which equals the negated result
- * (negation is exact in each product and sum), so one coefficient set
- * serves every quadrant. */
-NEMO_HD inline float sinf_quadrant(double x, int n, int m)
-{
-	const SincosfSet P0 = { 0x1p0, -0x1.ffffffd0c621cp-2, 0x1.55553e1068f19p-5,
-		-0x1.6c087e89a359dp-10, 0x1.99343027bf8c3p-16,
-		-0x1.555545995a603p-3, 0x1.1107605230bc4p-7, -0x1.994eb3774cf24p-13 };
-	const double s = ((m & 3) == 1 || (m & 3) == 2) ? -1.0 : 1.0;
-	const float v = sinf_poly(x * s, x * x, P0, n);
-	return ((n & 1) && (m & 2)) ? -v : v;
-}
-
-/* sinf of any float: |a| < pi/4 directly (a itself below 2^-12); |a| < 120
- * by one reduction step by pi/2, n rounded through a 2^24-scaled integer;
- * larger finite |a| by sinf_reduce_large; NaN for infinities and NaN. */
+/* sinf of any float: |a| < 120 by sinf_reduced; larger finite |a| by
+ * sinf_reduce_large, whose sign rule takes the argument's sign in; NaN for
+ * infinities and NaN. */
 NEMO_HD inline float sinf_glibc(float y)
 {
-	const SincosfSet P0 = { 0x1p0, -0x1.ffffffd0c621cp-2, 0x1.55553e1068f19p-5,
-		-0x1.6c087e89a359dp-10, 0x1.99343027bf8c3p-16,
-		-0x1.555545995a603p-3, 0x1.1107605230bc4p-7, -0x1.994eb3774cf24p-13 };
-	const double HPI_INV = 0x1.45F306DC9C883p+23;
-	const double HPI = 0x1.921FB54442D18p0;
-
-	const uint32_t top = (f2u(y) >> 20) & 0x7ffu;
-	double x = y;
-	if(top < ((f2u(0x1.921FB6p-1f) >> 20) & 0x7ffu)) {
-		if(top < ((f2u(0x1p-12f) >> 20) & 0x7ffu)) {
-			return y;
-		}
-		return sinf_poly(x, x * x, P0, 0);
+	if(__builtin_fabsf(y) < 120.0f) {
+		return sinf_reduced(y);
 	}
-	if(top < ((f2u(120.0f) >> 20) & 0x7ffu)) {
-		const double r = x * HPI_INV;
-		const int n = (int32_t(r) + 0x800000) >> 24;
-		x = fma(-double(n), HPI, x);
-		return sinf_quadrant(x, n, n);
+	const uint32_t yi = f2u(y);
+	if(((yi >> 20) & 0x7ffu) >= ((f2u(__builtin_inff()) >> 20) & 0x7ffu)) {
+		return (y - y) / (y - y);
 	}
-	if(top < ((f2u(__builtin_inff()) >> 20) & 0x7ffu)) {
-		const uint32_t xi = f2u(y);
-		int n = 0;
-		x = sinf_reduce_large(xi, &n);
-		return sinf_quadrant(x, n, n + int(xi >> 31));
-	}
-	return (y - y) / (y - y);
+	int n = 0;
+	const double x = sinf_reduce_large(yi, &n);
+	const int m = n + int(yi >> 31);
+	/* quadrant n picks the polynomial, m = n plus the argument's sign bit
+	 * the sign */
+	const double v = (n & 1) ? sinf_poly_cos(x * x) : sinf_poly_sin(x, x * x);
+	const bool neg = (n & 1) ? (m & 2) != 0 : (((m & 3) == 1) || ((m & 3) == 2));
+	return neg ? -float(v) : float(v);
 }
 
 /* The phase wrap of the Kuramoto model (src/nemo/cpu/plugins/Kuramoto.cpp:

@@ -62,14 +62,14 @@ NEMO_HD inline uint32_t urand(Rng& r)
 	return r.s[3];
 }
 
-/* Correctly rounded single-precision square root (the double square root of
- * a float, rounded once, is the correctly rounded float square root). */
+/* Correctly rounded single-precision square root: hipcc's default for sqrtf
+ * (-fhip-fp32-correctly-rounded-divide-sqrt). */
 NEMO_HD inline float sqrt_f32(float x)
 {
-	return float(__builtin_sqrt(double(x)));
+	return __builtin_sqrtf(x);
 }
 
-/* Correctly rounded single-precision division, same argument. */
+/* Correctly rounded single-precision division, by the same default. */
 NEMO_HD inline float div_f32(float a, float b)
 {
 	return float(double(a) / double(b));
