@@ -13,10 +13,10 @@
  * the host C library's sinf restated in csrc/device/libm_f32.h, fmodf exact),
  * so the phases agree bit for bit with the CPU backend.
  *
- * One wave per oscillator: the four stages of a target depend on each other
- * and each is an ordered float sum over its incoming couplings, so the
- * lanes share the loads and the sines of a stage and the sum runs through
- * them in order (through LDS, as 64 dependent register adds). Phase history: plane c mod 32 of the state holds the phase
+ * A workgroup takes a tile of consecutive oscillators, whose rows of the
+ * reverse matrix are contiguous: its threads evaluate the tile's coupling
+ * terms into LDS, then one lane per oscillator adds its row's terms in order.
+ * Phase history: plane c mod 32 of the state holds the phase
  * of cycle c (the descriptor's history=32).
  */
 #include <hip/hip_runtime.h>
@@ -29,130 +29,219 @@ namespace {
 
 constexpr unsigned HISTORY = 32u;   /* history= of Kuramoto.ini */
 
-constexpr unsigned CHUNKS = 4u;     /* chunks of 64 couplings a wave holds in registers */
+constexpr unsigned THREADS = 256u;
+constexpr unsigned TILE_OSC = 64u;            /* oscillators of a tile: one lane each in the sums */
+/* A tile's rows in LDS start at multiples of 4 floats (16-byte reads), and at
+ * least 65 zeros follow each: the sums run in steps of 64 terms, and adding
+ * +0 leaves a sum that started from +0 as it is. */
+constexpr unsigned STEP = 64u;
+constexpr unsigned ROW_GAP = STEP + 4u;
+constexpr unsigned RESIDENT = 1024u;          /* workgroups on the chip at once: 4 per compute unit */
 
-/* s + p(lane 0) + p(lane 1) + ... + p(lane cnt-1), each addition rounded to
- * float, in lane order: the reference's sequential sum over one chunk of 64
- * couplings. The products go through the wave's 64 floats of LDS (`buf`)
- * and every lane reads them all back (broadcast reads, four at a time), so
- * the chain is 64 dependent adds on registers. cnt (1..64) is wave-uniform;
- * every lane ends with the same s. A wave's LDS operations complete in
- * order, so no barrier is needed between the store and the loads. */
-__device__ inline float ordered_sum(float s, float p, unsigned cnt, float* buf, unsigned lane)
+/* couplings of a tile whose threads hold PER each, and its floats in LDS (the
+ * sums read half a step further) */
+template<unsigned PER> struct Tile {
+	static constexpr unsigned couplings = THREADS * PER;
+	static constexpr unsigned half = PER > 9u ? 4u : 8u;   /* 16-byte reads per half step of the sums */
+	static constexpr unsigned lds = couplings + ROW_GAP * TILE_OSC + STEP / 2u;
+};
+
+/* how much further row j starts in LDS than its first coupling's number
+ * within the tile, off */
+__device__ inline unsigned row_shift(unsigned off, unsigned j)
 {
-	buf[lane] = p;
-	__builtin_amdgcn_wave_barrier();
-	const float4* b4 = reinterpret_cast<const float4*>(buf);
-	if(cnt == 64u) {
-#pragma unroll
-		for(int q = 0; q < 16; ++q) {
-			const float4 v = b4[q];
-			s = s + v.x;
-			s = s + v.y;
-			s = s + v.z;
-			s = s + v.w;
-		}
-	} else {
-#pragma unroll
-		for(int q = 0; q < 16; ++q) {
-			if(unsigned(4 * q) < cnt) {
-				const float4 v = b4[q];
-				s = s + v.x;
-				if(unsigned(4 * q + 1) < cnt) s = s + v.y;
-				if(unsigned(4 * q + 2) < cnt) s = s + v.z;
-				if(unsigned(4 * q + 3) < cnt) s = s + v.w;
-			}
-		}
-	}
-	__builtin_amdgcn_wave_barrier();   /* the reads are done before the next chunk's store */
-	return s;
+	return ((off + ROW_GAP * j) & ~3u) - off;
 }
 
-/* weight and source phase of the couplings rb + c*64 + lane, c < CHUNKS
- * (zero past rend); the phase of the source at cycle t - (delay - 1) */
-__device__ inline void load_chunks(float (&sp)[CHUNKS], float (&wt)[CHUNKS], uint32_t rb, uint32_t rend,
-		unsigned lane, const uint32_t* src, const uint32_t* dly, const float* w, const float* state,
-		size_t hstride, unsigned cycle, unsigned start)
-{
-#pragma unroll
-	for(unsigned c = 0; c < CHUNKS; ++c) {
-		const uint32_t r = rb + c * 64u + lane;
-		sp[c] = 0.0f;
-		wt[c] = 0.0f;
-		if(r < rend) {
-			const unsigned plane = (cycle - (dly[r] - 1u)) % HISTORY;
-			sp[c] = state[size_t(plane) * hstride + (src[r] - start)];
-			wt[c] = w[r];
-		}
-	}
-}
+typedef float Quad __attribute__((ext_vector_type(4)));
+#if defined(__HIP_DEVICE_COMPILE__)
+typedef const volatile __attribute__((address_space(3))) Quad* LdsQuads;   /* volatile generic reads are flat ones */
+#else
+typedef const volatile Quad* LdsQuads;
+#endif
 
-/* s plus the couplings held in sp/wt (cnt of them from the first chunk on,
- * at most CHUNKS*64), each w * sin(theta_source - x) rounded to float
- * (src/nemo/cpu/plugins/Kuramoto.cpp:18-29), summed in order */
-__device__ inline float sum_chunks(float s, const float (&sp)[CHUNKS], const float (&wt)[CHUNKS], float x, uint32_t cnt,
-		float* buf, unsigned lane)
+/* s + row[0] + ... + row[len-1], each addition rounded to float, in that
+ * order (the reference's sequential sum); the row is followed by zeros up to
+ * the next multiple of STEP terms. The chain of dependent adds bounds a long
+ * row (4.5 cycles each), so half a step is read while the half before is
+ * added. The reads are volatile and the sum passes through empty asm between
+ * them: left alone, the compiler gathers the reads at their use, and every
+ * step waits for LDS (13 cycles a term). H: 16-byte reads per half step. */
+template<unsigned H>
+__device__ inline float ordered_sum(float s, const float* row, unsigned len)
 {
+	LdsQuads r4 = (LdsQuads) row;
+	Quad a[H], b[H];
 #pragma unroll
-	for(unsigned c = 0; c < CHUNKS; ++c) {
-		if(c * 64u >= cnt) {
-			break;
+	for(unsigned q = 0; q < H; ++q) a[q] = r4[q];
+	for(unsigned i = 0; i < len; i += 8u * H) {
+#pragma unroll
+		for(unsigned q = 0; q < H; ++q) b[q] = r4[H + q];
+		asm volatile("" : "+v"(s));
+#pragma unroll
+		for(unsigned q = 0; q < H; ++q) {
+			s = s + a[q].x;
+			s = s + a[q].y;
+			s = s + a[q].z;
+			s = s + a[q].w;
 		}
-		const float p = wt[c] * nemo_libm::sinf_glibc(sp[c] - x);
-		s = ordered_sum(s, p, min(64u, cnt - c * 64u), buf, lane);
+		asm volatile("" : "+v"(s));
+		r4 += 2u * H;
+#pragma unroll
+		for(unsigned q = 0; q < H; ++q) a[q] = r4[q];
+		asm volatile("" : "+v"(s));
+#pragma unroll
+		for(unsigned q = 0; q < H; ++q) {
+			s = s + b[q].x;
+			s = s + b[q].y;
+			s = s + b[q].z;
+			s = s + b[q].w;
+		}
+		asm volatile("" : "+v"(s));
 	}
 	return s;
 }
 
-/* One wave per oscillator: its lanes load 64 couplings at a time (the row of
- * the reverse matrix is contiguous, so the loads are coalesced) and evaluate
- * their sines together; the sum then runs through the lanes in order. Rows
- * of up to CHUNKS*64 couplings stay in registers over the four stages;
- * longer rows are read again for each stage. */
-__global__ void __launch_bounds__(256) kuramoto_update_kernel(unsigned start, unsigned end, unsigned cycle,
-		const float* freq, float* state, size_t hstride, const uint32_t* rstart,
+/* One workgroup per `per` consecutive oscillators. Tiles of them whose rows
+ * hold at most TILE = 256 PER couplings together are done one after the other (one tile,
+ * unless rows are uneven); a row longer than TILE is a tile of its own and is
+ * read in pieces, again for each stage, where the others stay in registers
+ * over the four stages.
+ *
+ * What bounds it: with few and long rows the chains of dependent adds, 4
+ * stages x row length x 4.5 cycles, so that as many of them as possible run at
+ * once; with many oscillators the reads of the sources' phases (random, 32
+ * planes) and the sines (about 30 instructions each). One cycle, with the
+ * plugin step's other kernels (about 11 us), before (one wave per oscillator,
+ * which evaluated 64 couplings at a time, every lane repeating the sum) and
+ * now: 1000 oscillators x 1000 couplings 65 -> 35 us, 4000 x 1000 101 -> 61,
+ * 2000 x 2500 (rows in pieces) 182 -> 129, 3000 x 300 36 -> 25, 20000 x 100
+ * 48 -> 33, 50000 x 100 99 -> 76. */
+template<unsigned PER>
+__global__ void __launch_bounds__(256, 4) kuramoto_update_kernel(unsigned start, unsigned end, unsigned per,
+		unsigned cycle, const float* freq, float* state, size_t hstride, const uint32_t* rstart,
 		const uint32_t* src, const uint32_t* dly, const float* w)
 {
-	__shared__ __align__(16) float sumBuf[4][64];   /* one row per wave of the 256-thread block */
-	const unsigned lane = threadIdx.x & 63u;
-	float* buf = sumBuf[threadIdx.x >> 6];
-	const unsigned o = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);   /* wave-uniform */
-	if(o >= end - start) {
-		return;
-	}
+	constexpr unsigned TILE = Tile<PER>::couplings;
+	struct Row { float x; uint32_t shift; };  /* the stage's phase; row_shift */
+	__shared__ __align__(16) float term[Tile<PER>::lds];
+	__shared__ uint32_t rs[TILE_OSC + 1u];    /* row starts of the block's remaining oscillators */
+	__shared__ Row rows[TILE_OSC];
+	const unsigned tid = threadIdx.x;
 	const float* phase0 = state + size_t(cycle % HISTORY) * hstride;
 	float* phase1 = state + size_t((cycle + 1u) % HISTORY) * hstride;
-	const float f = freq[o];
-	const float theta = phase0[o];
-	const uint32_t r0 = rstart[start + o], r1 = rstart[start + o + 1u];
-	float k0, k1, k2, k3;
-	if(r1 - r0 <= CHUNKS * 64u) {
-		float sp[CHUNKS], wt[CHUNKS];
-		load_chunks(sp, wt, r0, r1, lane, src, dly, w, state, hstride, cycle, start);
-		const uint32_t cnt = r1 - r0;
-		k0 = f + sum_chunks(0.0f, sp, wt, theta, cnt, buf, lane);
-		k1 = f + sum_chunks(0.0f, sp, wt, theta + k0 * 0.5f, cnt, buf, lane);
-		k2 = f + sum_chunks(0.0f, sp, wt, theta + k1 * 0.5f, cnt, buf, lane);
-		k3 = f + sum_chunks(0.0f, sp, wt, theta + k2, cnt, buf, lane);
-	} else {
-		auto stage = [&](float x) {
+	const unsigned last = min(end - start, (blockIdx.x + 1u) * per);
+	unsigned o = blockIdx.x * per;
+	while(o < last) {   /* block-uniform */
+		const unsigned left = min(last - o, TILE_OSC);
+		if(tid <= left) rs[tid] = rstart[start + o + tid];
+		__syncthreads();
+		const uint32_t r0 = rs[0];
+		unsigned nb = left;                                     /* oscillators of the tile */
+		while(nb > 1u && rs[nb] - r0 > TILE) --nb;
+		const uint32_t total = rs[nb] - r0;                     /* couplings of the tile */
+		const uint32_t pieces = total <= TILE ? 1u : (total + TILE - 1u) / TILE;   /* > 1: one oscillator */
+		const uint32_t used = min(TILE, total) + ROW_GAP * nb + STEP / 2u;   /* of `term` */
+		for(unsigned i = tid; i < used; i += THREADS) term[i] = 0.0f;
+		float f = 0.0f, theta = 0.0f, k0 = 0.0f, k1 = 0.0f, k2 = 0.0f, k3 = 0.0f;
+		const bool owner = tid < nb;
+		if(owner) {
+			f = freq[o + tid];
+			theta = phase0[o + tid];
+			rows[tid] = Row{theta, row_shift(rs[tid] - r0, tid)};
+		}
+		float sp[PER], wt[PER];
+		uint32_t osc[(PER + 3u) / 4u];                          /* oscillators of the couplings, 8 bits each */
+		for(unsigned stage = 0; stage < 4u; ++stage) {
 			float s = 0.0f;
-			for(uint32_t rb = r0; rb < r1; rb += CHUNKS * 64u) {
-				float sp[CHUNKS], wt[CHUNKS];
-				load_chunks(sp, wt, rb, r1, lane, src, dly, w, state, hstride, cycle, start);
-				s = sum_chunks(s, sp, wt, x, r1 - rb, buf, lane);
+			for(uint32_t pc = 0; pc < pieces; ++pc) {
+				const uint32_t base = pc * TILE;
+				const uint32_t cnt = min(TILE, total - base);
+				if(stage == 0u || pieces > 1u) {
+#pragma unroll
+					for(unsigned k = 0; k < PER; ++k) {
+						const uint32_t i = k * THREADS + tid;
+						if(k % 4u == 0u) osc[k / 4u] = 0u;
+						sp[k] = 0.0f;
+						wt[k] = 0.0f;
+						if(i < cnt) {
+							const uint32_t r = r0 + base + i;
+							/* phase of the source at cycle t - (delay - 1) */
+							const unsigned plane = (cycle - (dly[r] - 1u)) % HISTORY;
+							sp[k] = state[size_t(plane) * hstride + (src[r] - start)];
+							wt[k] = w[r];
+							unsigned lo = 0, hi = nb;
+							while(hi - lo > 1u) {
+								const unsigned mid = (lo + hi) >> 1;
+								if(rs[mid] <= r) lo = mid; else hi = mid;
+							}
+							osc[k / 4u] |= lo << (8u * (k % 4u));
+						}
+					}
+				}
+				__syncthreads();   /* the stage's phases are in `rows`; the last sums have read `term` */
+				if(pieces > 1u && tid < STEP) term[cnt + tid] = 0.0f;   /* a shorter piece than the one before */
+#pragma unroll
+				for(unsigned k = 0; k < PER; ++k) {
+					const uint32_t i = k * THREADS + tid;
+					if(k * THREADS >= cnt) break;   /* block-uniform */
+					if(i < cnt) {
+						/* w * sin(theta_source - x), rounded to float (src/nemo/cpu/plugins/Kuramoto.cpp:18-29) */
+						const Row row = rows[(osc[k / 4u] >> (8u * (k % 4u))) & 0xffu];
+						term[i + row.shift] = wt[k] * nemo_libm::sinf_glibc(sp[k] - row.x);
+					}
+				}
+				__syncthreads();
+				if(owner) {
+					const bool whole = pieces == 1u;
+					s = ordered_sum<Tile<PER>::half>(s, term + (whole ? rs[tid] - r0 + rows[tid].shift : 0u),
+							whole ? rs[tid + 1u] - rs[tid] : cnt);
+				}
 			}
-			return s;
-		};
-		k0 = f + stage(theta);
-		k1 = f + stage(theta + k0 * 0.5f);
-		k2 = f + stage(theta + k1 * 0.5f);
-		k3 = f + stage(theta + k2);
+			if(owner) {
+				const float k = f + s;
+				if(stage == 0u) { k0 = k; rows[tid].x = theta + k * 0.5f; }
+				else if(stage == 1u) { k1 = k; rows[tid].x = theta + k * 0.5f; }
+				else if(stage == 2u) { k2 = k; rows[tid].x = theta + k; }
+				else { k3 = k; }
+			}
+		}
+		if(owner) {
+			const float next = theta + (k0 + 2.0f * k1 + 2.0f * k2 + k3) / 6.0f;
+			phase1[o + tid] = nemo_libm::kuramoto_wrap(next);
+		}
+		o += nb;
+		__syncthreads();   /* rs, rows and term are written again by the next tile */
 	}
-	if(lane == 0) {
-		const float next = theta + (k0 + 2.0f * k1 + 2.0f * k2 + k3) / 6.0f;
-		phase1[o] = nemo_libm::kuramoto_wrap(next);
+}
+
+/* Couplings per thread and oscillators per workgroup. A tile holds as many
+ * oscillators as fit on average, with room for three standard deviations of
+ * random rows, and the workgroups are whole rounds of RESIDENT. The smallest
+ * tile with which all of them run at once is taken (fewer instructions and
+ * registers: see the figures at the kernel); where none is large enough, the
+ * middle one, in several rounds. */
+struct Plan { unsigned per, threadCouplings; };
+
+Plan plan(unsigned n, const nemo_hip_rcm* rcm)
+{
+	const double avg = rcm->targets ? double(rcm->synapses) / double(rcm->targets) : 0.0;
+	auto fit = [&](unsigned couplings) {
+		unsigned b = TILE_OSC;
+		while(b > 0u && double(b) * avg + 3.0 * __builtin_sqrt(double(b) * avg) > double(couplings)) --b;
+		return b;
+	};
+	auto spread = [&](unsigned b) {
+		const unsigned rounds = (n + RESIDENT * b - 1u) / (RESIDENT * b);
+		return (n + RESIDENT * rounds - 1u) / (RESIDENT * rounds);
+	};
+	const unsigned sizes[3] = { 3u, 9u, 18u };
+	for(unsigned c : sizes) {
+		const unsigned b = fit(THREADS * c);
+		if(b > 0u && n <= RESIDENT * b) return Plan{spread(b), c};
 	}
+	const unsigned b = fit(THREADS * 9u);
+	return b > 0u ? Plan{spread(b), 9u} : Plan{1u, 18u};
 }
 
 /* src/nemo/cpu/plugins/Kuramoto.cpp:133-152: the planes of cycles -1 .. -31
@@ -187,8 +276,11 @@ int hip_update_neurons(void* stream, unsigned cycle, unsigned start, unsigned en
 		return int(hipErrorInvalidValue);   /* the descriptor asks for sources, delays and weights */
 	}
 	const unsigned n = end - start;
-	hipLaunchKernelGGL(kuramoto_update_kernel, dim3((n + 3u) / 4u), dim3(256), 0,
-			static_cast<hipStream_t>(stream), start, end, cycle, param, state, stateHistoryStride,
+	const Plan pl = plan(n, rcm);
+	auto kernel = pl.threadCouplings == 3u ? &kuramoto_update_kernel<3u>
+		: pl.threadCouplings == 9u ? &kuramoto_update_kernel<9u> : &kuramoto_update_kernel<18u>;
+	hipLaunchKernelGGL(kernel, dim3((n + pl.per - 1u) / pl.per), dim3(THREADS), 0,
+			static_cast<hipStream_t>(stream), start, end, pl.per, cycle, param, state, stateHistoryStride,
 			rcm->start, rcm->source, rcm->delay, rcm->weight);
 	return int(hipGetLastError());
 }
