@@ -1,6 +1,7 @@
 /*
- * plugin_abi.h -- POD descriptor of one network for the modular (plugin)
- * step kernels in plugin_step.hip, shared by host C++ and HIP.
+ * plugin_abi.h -- POD descriptor of one network for the per-cycle step
+ * kernels in plugin_step.hip (plugins, and built-in models beyond the fused
+ * kernel's range), shared by host C++ and HIP.
  */
 #ifndef NEMOSIM_PLUGIN_ABI_H
 #define NEMOSIM_PLUGIN_ABI_H
@@ -14,23 +15,31 @@ extern "C" {
 
 typedef struct PluginStepDev {
 	uint32_t n;            /* neurons */
-	uint32_t D;            /* ring depth = maximum delay */
+	uint32_t D;            /* maximum delay */
 	uint32_t words32;      /* 32-bit raster words per cycle (even: whole 64-bit words) */
-	uint32_t pad;
+	uint32_t R;            /* ring depth: D with plugins; D + 1 for built-in models, whose spikes are
+	                        * delivered while other neurons still read the cycle's slot */
 	uint64_t cycle0;       /* cycle at the start of the run */
 
-	long long* acc;        /* [2][D][n] pending E (plane 0) and I (plane 1) current, Q11.20 */
+	void* acc;             /* [2][R][n] pending E (plane 0) and I (plane 1) current, Q11.20: int64;
+	                        * int32 for built-in models where no sum can leave that range */
 	float* curE;           /* [n] this cycle's input, converted */
 	float* curI;
 	float* curX;           /* [n] external current */
 	uint32_t* fstim;       /* [words32] forced-firing bits */
 	uint32_t* raster;      /* [cycles][words32] fired bits; the plugin's `fired` row */
-	uint32_t* list;        /* [n] fired neurons of the cycle */
-	uint32_t* nfired;      /* their count */
 	const uint32_t* off;   /* [n+1] synapses of source s: syn[off[s] .. off[s+1]) */
 	const uint32_t* syn;   /* records {target | (delay-1) << 26, Q11.20 weight} */
 	uint64_t* recent;      /* [n] firing history */
 	unsigned long long* events;
+	unsigned long long* part;   /* [nemo_dev_pm_parts(n)] delivered synapses by
+	                             * workgroup, summed into *events by pm_finish */
+
+	/* built-in models */
+	const uint8_t* model;  /* [n] */
+	const float* param;    /* [MAX_PARAM][n] */
+	float* state;          /* [MAX_STATE][n] */
+	uint32_t* rng;         /* [4][n] */
 
 	const uint32_t* rcm_start;
 	const uint32_t* rcm_sd;
@@ -46,10 +55,17 @@ typedef struct PluginStepDev {
 
 int nemo_dev_pm_begin(const PluginStepDev* s, uint32_t k, void* stream);
 int nemo_dev_pm_stimulus(const PluginStepDev* s, uint32_t k, uint32_t entries, void* stream);
-int nemo_dev_pm_compact(const PluginStepDev* s, uint32_t k, void* stream);
 int nemo_dev_pm_scatter(const PluginStepDev* s, uint32_t k, void* stream);
 int nemo_dev_pm_stdp(const PluginStepDev* s, void* stream);
-int nemo_dev_pm_replay(const PluginStepDev* s, void* stream);
+/* rebuilds the zeroed ring; narrow: int32 accumulators */
+int nemo_dev_pm_replay(const PluginStepDev* s, int narrow, void* stream);
+/* one cycle of built-in models; stim: the cycle's stimulus is in fstim and
+ * curX, which are cleared */
+int nemo_dev_pm_cycle(const PluginStepDev* s, uint32_t k, int stim, int narrow, int izhikevichOnly, void* stream);
+/* workgroups of the kernels that count events in `part`, and their sum */
+#define NEMO_PM_SCATTER_BLOCKS 1024u
+uint32_t nemo_dev_pm_parts(uint32_t n);
+int nemo_dev_pm_finish(const PluginStepDev* s, void* stream);
 
 #ifdef __cplusplus
 }

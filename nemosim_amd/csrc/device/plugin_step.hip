@@ -1,16 +1,20 @@
 /*
- * plugin_step.hip -- the modular step: one cycle as a sequence of kernels
- * around the neuron-model plugin's hip_update_neurons (the structure of
- * NeMo's CUDA step, src/nemo/cuda/Simulation.cpp:336-430: gather, plugin
- * update, scatter, STDP). It runs any model a plugin provides and any network
- * size that fits in device memory; the fused persistent kernel
- * (step_kernel.hip) is the fast path for the built-in models.
+ * plugin_step.hip -- the step as kernels launched every cycle, for what the
+ * fused persistent kernel (step_kernel.hip) cannot run:
  *
- * Pending current lives in a global ring of int64 accumulators
- * acc[2][D][n] (E, I); spikes are added with 64-bit global atomics at fire
- * time into slot (t + delay) mod D, so sums equal NeMo's int64 sums exactly
+ *   - models that exist as a plugin: gather, the plugin's hip_update_neurons,
+ *     scatter, STDP (the structure of NeMo's CUDA step,
+ *     src/nemo/cuda/Simulation.cpp:336-430);
+ *   - networks of built-in models beyond its range (more neurons or longer
+ *     delays than the chip's LDS holds): one kernel that updates, lists the
+ *     fired neurons and delivers their spikes, and STDP.
+ *
+ * Pending current lives in a global ring of accumulators acc[2][R][n] (E, I);
+ * spikes are added with global atomics at fire time into slot (t + delay) mod
+ * R. They are int64, so that sums equal NeMo's int64 sums exactly
  * (src/nemo/cpu/Simulation.cpp:292-307) and are clamped at conversion
- * (src/nemo/fixedpoint.cpp:41-49).
+ * (src/nemo/fixedpoint.cpp:41-49), or int32 where the host has proven that no
+ * sum can leave that range, which is the same sums.
  *
  * Forward records here carry the absolute target: {target | (delay-1) << 26,
  * Q11.20 weight}; a source's synapses are syn[off[s] .. off[s+1]).
@@ -32,14 +36,25 @@ __device__ inline float sat_to_float(long long v)
 	return float(int32_t(v)) / 1048576.0f;
 }
 
-/* Start of cycle: convert and clear this cycle's ring slot, clear the
+__device__ inline float acc_to_float(long long v) { return sat_to_float(v); }
+__device__ inline float acc_to_float(int32_t v) { return fx20_to_float(v); }
+
+__device__ inline void acc_add(long long* p, int32_t w)
+{
+	atomicAdd(reinterpret_cast<unsigned long long*>(p), (unsigned long long)(long long) w);
+}
+
+__device__ inline void acc_add(int32_t* p, int32_t w) { atomicAdd(p, w); }
+
+/* Start of cycle, plugins: convert and clear this cycle's ring slot, clear the
  * external current, forced-firing bits and the cycle's fired bits. */
 __global__ void pm_begin_kernel(PluginStepDev s, uint32_t k)
 {
 	const uint64_t t = s.cycle0 + k;
-	const uint32_t slot = uint32_t(t % s.D);
-	long long* accE = s.acc + size_t(slot) * s.n;
-	long long* accI = s.acc + size_t(s.D + slot) * s.n;
+	const uint32_t slot = uint32_t(t % s.R);
+	long long* acc = static_cast<long long*>(s.acc);
+	long long* accE = acc + size_t(slot) * s.n;
+	long long* accI = acc + size_t(s.R + slot) * s.n;
 	uint32_t* fired = s.raster + size_t(k) * s.words32;
 	const size_t stride = size_t(gridDim.x) * blockDim.x;
 	for(size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < s.n; i += stride) {
@@ -52,9 +67,6 @@ __global__ void pm_begin_kernel(PluginStepDev s, uint32_t k)
 	for(size_t w = size_t(blockIdx.x) * blockDim.x + threadIdx.x; w < s.words32; w += stride) {
 		s.fstim[w] = 0u;
 		fired[w] = 0u;
-	}
-	if(blockIdx.x == 0 && threadIdx.x == 0) {
-		*s.nfired = 0u;
 	}
 }
 
@@ -76,73 +88,219 @@ __global__ void pm_stimulus_kernel(PluginStepDev s, uint32_t k)
 	}
 }
 
-/* Fired bits of cycle k -> list of fired neurons (any order: delivery is
- * order-independent; the ordered output is the bit raster). */
-__global__ void pm_compact_kernel(PluginStepDev s, uint32_t k)
+/* The synapses of `count` fired sources (in LDS) into ring slots (base + d)
+ * mod R, by the four waves of a workgroup: chunk c of 256 synapses of the j-th
+ * source goes to wave (c + j) mod 4, four records per lane loaded together.
+ * Returns the synapses of the chunks this wave did (wave-uniform). */
+template<typename ACC>
+__device__ inline uint32_t deliver_listed(const PluginStepDev& s, const uint32_t* list, uint32_t count,
+		uint32_t base, uint32_t wave, uint32_t lane)
 {
-	const uint32_t* fired = s.raster + size_t(k) * s.words32;
-	const size_t stride = size_t(gridDim.x) * blockDim.x;
-	for(size_t w = size_t(blockIdx.x) * blockDim.x + threadIdx.x; w < s.words32; w += stride) {
-		uint32_t b = fired[w];
-		if(b) {
-			uint32_t pos = atomicAdd(s.nfired, uint32_t(__popc(b)));
-			while(b) {
-				uint32_t bit = uint32_t(__ffs(b) - 1);
-				b &= b - 1;
-				s.list[pos++] = uint32_t(w * 32u + bit);
+	ACC* acc = static_cast<ACC*>(s.acc);
+	const uint2* syn = reinterpret_cast<const uint2*>(s.syn);
+	uint32_t ev = 0;
+	for(uint32_t j = 0; j < count; ++j) {
+		const uint32_t src = list[j];
+		const uint32_t a = s.off[src], b = s.off[src + 1];
+		for(uint32_t c = a + 256u * ((wave - j) & 3u); c < b; c += 1024u) {
+			uint2 rec[4];
+#pragma unroll
+			for(uint32_t i = 0; i < 4u; ++i) {
+				const uint32_t q = c + 64u * i + lane;
+				rec[i] = (q < b) ? syn[q] : make_uint2(0u, 0u);
 			}
+#pragma unroll
+			for(uint32_t i = 0; i < 4u; ++i) {
+				if(c + 64u * i + lane < b) {
+					const int32_t w = int32_t(rec[i].y);
+					uint32_t sl = base + (rec[i].x >> 26) + 1u;
+					sl = (sl >= s.R) ? sl - s.R : sl;
+					const uint32_t plane = (w >= 0) ? 0u : s.R;
+					acc_add(acc + size_t(plane + sl) * s.n + (rec[i].x & 0x3ffffffu), w);
+				}
+			}
+			ev += min(256u, b - c);
 		}
+	}
+	return ev;
+}
+
+/* part[blockIdx.x] += the waves' ev: the workgroup's own counter, since a
+ * shared one, and a shared list of the fired neurons, serialise the atomics of
+ * all workgroups (compaction and scatter of 150k synapses: 28 us a cycle with
+ * them, 19 without) */
+__device__ inline void count_events(unsigned long long* part, uint32_t ev, uint32_t* wsum, uint32_t wave, uint32_t lane)
+{
+	if(lane == 0) wsum[wave] = ev;
+	__syncthreads();
+	if(threadIdx.x == 0) {
+		const uint32_t sum = wsum[0] + wsum[1] + wsum[2] + wsum[3];
+		if(sum) part[blockIdx.x] += sum;
 	}
 }
 
-/* One wave per fired source: its synapses into ring slots (t + d) mod D. */
-__global__ void pm_scatter_kernel(PluginStepDev s, uint32_t k)
+/* Plugins: the fired bits of cycle k, listed and delivered. Each workgroup
+ * takes 64 words of the raster (2048 neurons) at a time, lists their bits in
+ * LDS and delivers them. */
+__global__ void __launch_bounds__(256) pm_scatter_kernel(PluginStepDev s, uint32_t k)
 {
-	const uint64_t t = s.cycle0 + k;
-	const uint32_t base = uint32_t(t % s.D);
+	__shared__ uint32_t list[2048];
+	__shared__ uint32_t count;
+	__shared__ uint32_t wsum[4];
 	const uint32_t lane = threadIdx.x & 63u;
-	const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-	const uint32_t nwaves = (gridDim.x * blockDim.x) >> 6;
-	const uint32_t nf = *s.nfired;
-	unsigned long long ev = 0;
-	for(uint32_t j = wave; j < nf; j += nwaves) {
-		const uint32_t src = s.list[j];
-		const uint32_t a = s.off[src], b = s.off[src + 1];
-		ev += b - a;
-		for(uint32_t q = a + lane; q < b; q += 64u) {
-			const uint32_t x = s.syn[2 * size_t(q)];
-			const int32_t w = int32_t(s.syn[2 * size_t(q) + 1]);
-			const uint32_t tgt = x & 0x3ffffffu;
-			uint32_t sl = base + (x >> 26) + 1u;
-			sl = (sl >= s.D) ? sl - s.D : sl;
-			const uint32_t plane = (w >= 0) ? 0u : s.D;
-			atomicAdd(reinterpret_cast<unsigned long long*>(&s.acc[size_t(plane + sl) * s.n + tgt]),
-					(unsigned long long)(long long) w);
+	const uint32_t wave = threadIdx.x >> 6;
+	const uint32_t* fired = s.raster + size_t(k) * s.words32;
+	const uint32_t base = uint32_t((s.cycle0 + k) % s.R);
+	uint32_t ev = 0;
+	for(size_t w0 = size_t(blockIdx.x) * 64u; w0 < s.words32; w0 += size_t(gridDim.x) * 64u) {   /* block-uniform */
+		if(wave == 0) {
+			uint32_t b = (w0 + lane < s.words32) ? fired[w0 + lane] : 0u;
+			const uint32_t c = uint32_t(__popc(b));
+			uint32_t x = c;
+			for(uint32_t d = 1; d < 64u; d <<= 1) {
+				const uint32_t y = __shfl_up(x, d, 64);
+				if(lane >= d) x += y;
+			}
+			uint32_t at = x - c;
+			while(b) {
+				list[at++] = uint32_t((w0 + lane) * 32u) + uint32_t(__ffs(b) - 1);
+				b &= b - 1u;
+			}
+			if(lane == 63u) count = x;
+		}
+		__syncthreads();
+		ev += deliver_listed<long long>(s, list, count, base, wave, lane);
+		__syncthreads();   /* the list is written again */
+	}
+	count_events(s.part, ev, wsum, wave, lane);
+}
+
+/* Built-in models: one cycle of 256 neurons per workgroup. Reads and clears
+ * the cycle's ring slot, updates the neurons (models.h), writes their raster
+ * words, lists the fired ones in LDS and delivers them at once into slots t+1
+ * .. t+D, none of which is slot t of a ring of D+1: other workgroups may still
+ * be reading it. So a cycle is one launch where plugins need three.
+ *
+ * What bounds it: the neurons' parameters, state and ring slot (about 90 bytes
+ * each) and the chain slot -> update -> row bounds -> records -> atomics; with
+ * many spikes the atomics. Per cycle, against the plugins' sequence as it was
+ * (begin, update, compact, scatter): 300k x 100 37 -> 14.2 us, 400k x 250 62 ->
+ * 31, 100k x 100 with delays up to 60 20.8 -> 8.9, 70k x 60 IF_curr_exp_noise
+ * at 333 Hz 114 -> 31, 150k x 60 with STDP 35 -> 15.7. */
+template<typename ACC, bool IZO>
+__global__ void __launch_bounds__(256) pm_cycle_kernel(PluginStepDev s, uint32_t k, int stim)
+{
+	constexpr int NP = IZO ? 5 : MAX_PARAM;
+	constexpr int NS = IZO ? 2 : MAX_STATE;
+	__shared__ uint32_t list[256];
+	__shared__ uint32_t wsum[4], wfired[4];
+	const uint32_t lane = threadIdx.x & 63u;
+	const uint32_t wave = threadIdx.x >> 6;
+	const uint32_t n = s.n;
+	const uint32_t l = blockIdx.x * 256u + threadIdx.x;
+	const uint32_t slot = uint32_t((s.cycle0 + k) % s.R);
+	bool fired = false;
+	if(l < n) {
+		ACC* acc = static_cast<ACC*>(s.acc);
+		ACC* pe = acc + size_t(slot) * n + l;
+		ACC* pi = acc + size_t(s.R + slot) * n + l;
+		const ACC e = *pe, i = *pi;
+		float p[NP], st[NS];
+#pragma unroll
+		for(int q = 0; q < NP; ++q) p[q] = s.param[size_t(q) * n + l];
+#pragma unroll
+		for(int q = 0; q < NS; ++q) st[q] = s.state[size_t(q) * n + l];
+		Rng r;
+#pragma unroll
+		for(int q = 0; q < 4; ++q) r.s[q] = s.rng[size_t(q) * n + l];
+		const uint64_t recent = s.recent[l];
+		float x = 0.0f;
+		bool fs = false;
+		if(stim) {
+			x = s.curX[l];
+			fs = ((s.fstim[l >> 5] >> (l & 31u)) & 1u) != 0u;
+			s.curX[l] = 0.0f;
+		}
+		*pe = 0;
+		*pi = 0;
+		if(IZO) {
+			fired = izhikevich(p, st, r, acc_to_float(e), acc_to_float(i), x, fs);
+		} else {
+			fired = update_neuron(s.model[l], p, st, r, acc_to_float(e), acc_to_float(i), x, fs);
+		}
+#pragma unroll
+		for(int q = 0; q < NS; ++q) s.state[size_t(q) * n + l] = st[q];
+#pragma unroll
+		for(int q = 0; q < 4; ++q) s.rng[size_t(q) * n + l] = r.s[q];
+		s.recent[l] = (recent << 1) | (fired ? 1ull : 0ull);
+	}
+	const uint64_t mask = __ballot(fired);
+	if(lane == 0) {
+		wfired[wave] = uint32_t(__popcll(mask));
+		const uint32_t word = l >> 6;
+		if(word < s.words32 / 2u) {
+			reinterpret_cast<uint64_t*>(s.raster)[size_t(k) * (s.words32 / 2u) + word] = mask;
+			/* every lane of the wave has read its bit */
+			if(stim) reinterpret_cast<uint64_t*>(s.fstim)[word] = 0ull;
 		}
 	}
-	if(lane == 0 && ev) {
-		atomicAdd(s.events, ev);
+	__syncthreads();
+	uint32_t before = 0, total = 0;
+#pragma unroll
+	for(uint32_t w = 0; w < 4u; ++w) {
+		before += (w < wave) ? wfired[w] : 0u;
+		total += wfired[w];
+	}
+	if(total == 0u) return;   /* block-uniform */
+	if(fired) {
+		const uint64_t below = lane ? (mask & (~0ull >> (64u - lane))) : 0ull;
+		list[before + uint32_t(__popcll(below))] = l;
+	}
+	__syncthreads();
+	const uint32_t ev = deliver_listed<ACC>(s, list, total, slot, wave, lane);
+	count_events(s.part, ev, wsum, wave, lane);
+}
+
+/* *events += the workgroups' counters (one workgroup) */
+__global__ void __launch_bounds__(256) pm_finish_kernel(PluginStepDev s, uint32_t parts)
+{
+	__shared__ unsigned long long sums[256];
+	unsigned long long e = 0;
+	for(uint32_t i = threadIdx.x; i < parts; i += 256u) {
+		e += s.part[i];
+		s.part[i] = 0ull;
+	}
+	sums[threadIdx.x] = e;
+	__syncthreads();
+	if(threadIdx.x == 0) {
+		for(uint32_t i = 1; i < 256u; ++i) e += sums[i];
+		*s.events += e;
 	}
 }
 
 /* STDP: targets whose history has bit postLen set walk their plastic
- * in-synapses (src/nemo/ConnectivityMatrix.cpp:193-227). One wave per
- * qualifying target. */
+ * in-synapses (src/nemo/ConnectivityMatrix.cpp:193-227). Each wave looks at 64
+ * targets at a time and walks the rows of those that qualify. */
 __global__ void pm_stdp_kernel(PluginStepDev s)
 {
 	const StdpParams& sp = *reinterpret_cast<const StdpParams*>(s.stdp);
 	const uint32_t lane = threadIdx.x & 63u;
 	const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
 	const uint32_t nwaves = (gridDim.x * blockDim.x) >> 6;
-	for(uint32_t tgt = wave; tgt < s.n; tgt += nwaves) {
-		if(!((s.recent[tgt] >> sp.postLen) & 1ull)) continue;
-		const uint32_t r0 = s.rcm_start[tgt], r1 = s.rcm_start[tgt + 1];
-		for(uint32_t r = r0 + lane; r < r1; r += 64u) {
-			const uint32_t sd = s.rcm_sd[r];
-			const uint64_t pre = s.recent[sd & 0x3ffffffu] >> ((sd >> 26) + 1u);
-			const int32_t wd = stdp_weight_change(sp, pre);
-			if(wd != 0) {
-				s.rcm_acc[r] = int32_t(uint32_t(s.rcm_acc[r]) + uint32_t(wd));
+	for(uint32_t t0 = wave * 64u; t0 < s.n; t0 += nwaves * 64u) {
+		const uint32_t tl = t0 + lane;
+		uint64_t todo = __ballot(tl < s.n && ((s.recent[tl] >> sp.postLen) & 1ull));
+		while(todo) {
+			const uint32_t tgt = t0 + uint32_t(__ffsll((unsigned long long) todo) - 1);
+			todo &= todo - 1ull;
+			const uint32_t r0 = s.rcm_start[tgt], r1 = s.rcm_start[tgt + 1];
+			for(uint32_t r = r0 + lane; r < r1; r += 64u) {
+				const uint32_t sd = s.rcm_sd[r];
+				const uint64_t pre = s.recent[sd & 0x3ffffffu] >> ((sd >> 26) + 1u);
+				const int32_t wd = stdp_weight_change(sp, pre);
+				if(wd != 0) {
+					s.rcm_acc[r] = int32_t(uint32_t(s.rcm_acc[r]) + uint32_t(wd));
+				}
 			}
 		}
 	}
@@ -152,14 +310,16 @@ __global__ void pm_stdp_kernel(PluginStepDev s)
  * history, since NeMo reads a weight when the spike arrives
  * (src/nemo/cpu/Simulation.cpp:258-307). The ring has been zeroed; a spike
  * fired at cycle0-1-k with delay d > k is still pending and lands in slot
- * (cycle0-1-k+d) mod D. One wave per source with pending spikes. */
+ * (cycle0-1-k+d) mod R. One wave per source with pending spikes. */
+template<typename ACC>
 __global__ void pm_replay_kernel(PluginStepDev s)
 {
+	ACC* acc = static_cast<ACC*>(s.acc);
 	const uint32_t lane = threadIdx.x & 63u;
 	const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
 	const uint32_t nwaves = (gridDim.x * blockDim.x) >> 6;
 	const uint64_t pend = (s.D >= 64u) ? ~0ull : ((1ull << s.D) - 1ull);
-	const uint32_t last = uint32_t((s.cycle0 + s.D - 1u) % s.D);
+	const uint32_t last = uint32_t((s.cycle0 + s.R - 1u) % s.R);
 	for(uint32_t src = wave; src < s.n; src += nwaves) {
 		const uint64_t h = s.recent[src] & pend;
 		if(!h) continue;
@@ -169,14 +329,13 @@ __global__ void pm_replay_kernel(PluginStepDev s)
 			const int32_t w = int32_t(s.syn[2 * size_t(q) + 1]);
 			const uint32_t tgt = x & 0x3ffffffu;
 			const uint32_t d = (x >> 26) + 1u;
-			const uint32_t plane = (w >= 0) ? 0u : s.D;
+			const uint32_t plane = (w >= 0) ? 0u : s.R;
 			uint64_t hb = h & ((d >= 64u) ? ~0ull : ((1ull << d) - 1ull));
 			while(hb) {
 				const uint32_t kk = uint32_t(__builtin_ctzll(hb));
 				hb &= hb - 1ull;
-				const uint32_t sl = (last + d - kk) % s.D;
-				atomicAdd(reinterpret_cast<unsigned long long*>(&s.acc[size_t(plane + sl) * s.n + tgt]),
-						(unsigned long long)(long long) w);
+				const uint32_t sl = (last + d - kk) % s.R;
+				acc_add(acc + size_t(plane + sl) * s.n + tgt, w);
 			}
 		}
 	}
@@ -209,30 +368,47 @@ int nemo_dev_pm_stimulus(const PluginStepDev* s, uint32_t k, uint32_t entries, v
 	return int(hipGetLastError());
 }
 
-int nemo_dev_pm_compact(const PluginStepDev* s, uint32_t k, void* stream)
-{
-	hipLaunchKernelGGL(pm_compact_kernel, dim3(grid(s->words32, 256, 1024)), dim3(256), 0,
-			static_cast<hipStream_t>(stream), *s, k);
-	return int(hipGetLastError());
-}
-
 int nemo_dev_pm_scatter(const PluginStepDev* s, uint32_t k, void* stream)
 {
-	hipLaunchKernelGGL(pm_scatter_kernel, dim3(2048), dim3(256), 0,
+	hipLaunchKernelGGL(pm_scatter_kernel, dim3(grid(s->words32, 64, NEMO_PM_SCATTER_BLOCKS)), dim3(256), 0,
 			static_cast<hipStream_t>(stream), *s, k);
 	return int(hipGetLastError());
 }
 
-int nemo_dev_pm_replay(const PluginStepDev* s, void* stream)
+int nemo_dev_pm_replay(const PluginStepDev* s, int narrow, void* stream)
 {
-	hipLaunchKernelGGL(pm_replay_kernel, dim3(2048), dim3(256), 0,
-			static_cast<hipStream_t>(stream), *s);
+	if(narrow) {
+		hipLaunchKernelGGL(pm_replay_kernel<int32_t>, dim3(2048), dim3(256), 0, static_cast<hipStream_t>(stream), *s);
+	} else {
+		hipLaunchKernelGGL(pm_replay_kernel<long long>, dim3(2048), dim3(256), 0, static_cast<hipStream_t>(stream), *s);
+	}
+	return int(hipGetLastError());
+}
+
+int nemo_dev_pm_cycle(const PluginStepDev* s, uint32_t k, int stim, int narrow, int izhikevichOnly, void* stream)
+{
+	auto kernel = narrow ? (izhikevichOnly ? &pm_cycle_kernel<int32_t, true> : &pm_cycle_kernel<int32_t, false>)
+		: (izhikevichOnly ? &pm_cycle_kernel<long long, true> : &pm_cycle_kernel<long long, false>);
+	hipLaunchKernelGGL(kernel, dim3((s->n + 255u) / 256u), dim3(256), 0, static_cast<hipStream_t>(stream), *s, k, stim);
+	return int(hipGetLastError());
+}
+
+uint32_t nemo_dev_pm_parts(uint32_t n)
+{
+	const uint32_t blocks = (n + 255u) / 256u;
+	return blocks > NEMO_PM_SCATTER_BLOCKS ? blocks : NEMO_PM_SCATTER_BLOCKS;
+}
+
+int nemo_dev_pm_finish(const PluginStepDev* s, void* stream)
+{
+	hipLaunchKernelGGL(pm_finish_kernel, dim3(1), dim3(256), 0, static_cast<hipStream_t>(stream), *s,
+			nemo_dev_pm_parts(s->n));
 	return int(hipGetLastError());
 }
 
 int nemo_dev_pm_stdp(const PluginStepDev* s, void* stream)
 {
-	hipLaunchKernelGGL(pm_stdp_kernel, dim3(grid(size_t(s->n) * 64, 256, 4096)), dim3(256), 0,
+	hipLaunchKernelGGL(pm_stdp_kernel, dim3(grid(s->n, 256, 4096)), dim3(256), 0,
 			static_cast<hipStream_t>(stream), *s);
 	return int(hipGetLastError());
 }

@@ -458,10 +458,11 @@ Simulation::Simulation(const NetworkImpl& net, const ConfigurationImpl& conf) :
 		}
 		if(conf.stepMode == NEMO_STEP_AUTO) {
 			/* a different kernel sequence with its own speed: say why */
-			fprintf(stderr, "nemosim HIP: %u neurons run on the plugin step (%s)\n", m_n, whyNotFused.c_str());
+			m_builtinStep = allBuiltin;
+			fprintf(stderr, "nemosim HIP: %u neurons run on the %s step (%s)\n", m_n,
+					m_builtinStep ? "per-cycle" : "plugin", whyNotFused.c_str());
 		}
-		/* plugin path: one bucket per source holding all its synapses, with
-		 * absolute targets */
+		/* one bucket per source holding all its synapses, with absolute targets */
 		m_fused = false;
 		m_P = 1;
 		m_T = 0;
@@ -746,15 +747,22 @@ Simulation::Simulation(const NetworkImpl& net, const ConfigurationImpl& conf) :
 		std::vector<WorkItem> work = xcdWorkTable(items);
 		d_work.upload(work.data(), work.size() * sizeof(WorkItem));
 	} else {
-		/* pending current as int64 ring [2][D][n], converted inputs, bits */
-		d_acc.alloc(std::max<size_t>(size_t(2) * m_D * m_n, 1) * 8);
-		d_curE.alloc(std::max<size_t>(m_n, 1) * 4);
-		d_curI.alloc(std::max<size_t>(m_n, 1) * 4);
+		/* the pending-current ring [2][R][n] (see PluginStepDev), the plugins'
+		 * converted inputs, stimulus, event counters */
+		m_ringDepth = m_builtinStep ? m_D + 1 : m_D;
+		const size_t accBytes = m_builtinStep && !m_saturate ? 4 : 8;
+		d_acc.alloc((std::max<size_t>(size_t(2) * m_ringDepth * m_n, 1) * accBytes + 7u) & ~size_t(7));
+		if(!m_builtinStep) {
+			d_curE.alloc(std::max<size_t>(m_n, 1) * 4);
+			d_curI.alloc(std::max<size_t>(m_n, 1) * 4);
+		}
 		d_curX.alloc(std::max<size_t>(m_n, 1) * 4);
 		d_fstim.alloc(std::max<size_t>(m_words32, 2) * 4);
-		d_list.alloc(std::max<size_t>(m_n, 1) * 4 + 4);
+		d_part.alloc(size_t(nemo_dev_pm_parts(m_n)) * 8);
 		hipCheck(nemo_dev_fill_u64(d_acc.as<uint64_t>(), 0, d_acc.bytes / 8, s), "fill");
-		loadPlugins(net);
+		hipCheck(nemo_dev_fill_u32(d_curX.as<uint32_t>(), 0, d_curX.bytes / 4, s), "fill");
+		hipCheck(nemo_dev_fill_u32(d_fstim.as<uint32_t>(), 0, d_fstim.bytes / 4, s), "fill");
+		if(!m_builtinStep) loadPlugins(net);
 	}
 	hipCheck(hipHostMalloc(reinterpret_cast<void**>(&h_step), std::max<size_t>(m_words, 1) * 8), "hipHostMalloc");
 	ensureRaster(8);
@@ -1247,10 +1255,12 @@ Simulation::completeLaunch(unsigned nsteps, const uint32_t ctl[8])
 	}
 }
 
-/* The modular step: per cycle, convert the due ring slot, apply stimulus,
- * run each type's plugin, compact the fired bits, scatter the fired
- * sources' synapses into the int64 ring, accumulate STDP
- * (src/nemo/cuda/Simulation.cpp:336-430 has the same phase structure). */
+/* The per-cycle step (csrc/device/plugin_step.hip). With plugins: convert the
+ * due ring slot, apply stimulus, run each type's plugin, deliver the fired
+ * sources' synapses into the ring, accumulate STDP
+ * (src/nemo/cuda/Simulation.cpp:336-430 has the same phase structure). For
+ * built-in models beyond the fused kernel's range one kernel does all but the
+ * stimulus and STDP. */
 void
 Simulation::launchPlugins(unsigned nsteps, unsigned long long* events)
 {
@@ -1265,19 +1275,28 @@ Simulation::launchPlugins(unsigned nsteps, unsigned long long* events)
 	s.n = m_n;
 	s.D = m_D;
 	s.words32 = m_words32;
+	s.R = m_ringDepth;
 	s.cycle0 = m_cycle;
-	s.acc = d_acc.as<long long>();
+	s.acc = d_acc.ptr;
 	s.curE = d_curE.as<float>();
 	s.curI = d_curI.as<float>();
 	s.curX = d_curX.as<float>();
 	s.fstim = d_fstim.as<uint32_t>();
 	s.raster = d_raster.as<uint32_t>();
-	s.list = d_list.as<uint32_t>();
-	s.nfired = d_list.as<uint32_t>() + m_n;
 	s.off = d_off.as<uint32_t>();
 	s.syn = d_syn.as<uint32_t>();
 	s.recent = d_recent.as<uint64_t>();
 	s.events = reinterpret_cast<unsigned long long*>(d_ctl.as<uint32_t>() + 2);
+	s.part = d_part.as<unsigned long long>();
+	s.model = d_model.as<uint8_t>();
+	s.param = d_param.as<float>();
+	s.state = d_state.as<float>();
+	s.rng = d_rng.as<uint32_t>();
+	const int narrow = m_builtinStep && !m_saturate ? 1 : 0;
+	if(m_partDirty) {
+		hipCheck(nemo_dev_fill_u64(d_part.as<uint64_t>(), 0, d_part.bytes / 8, st), "fill");
+	}
+	m_partDirty = true;
 	s.rcm_start = d_rcmStart.as<uint32_t>();
 	s.rcm_sd = d_rcmSd.as<uint32_t>();
 	s.rcm_acc = d_rcmAcc.as<int32_t>();
@@ -1294,30 +1313,34 @@ Simulation::launchPlugins(unsigned nsteps, unsigned long long* events)
 	if(m_replay) {
 		/* weights changed: rebuild the pending current from the history */
 		hipCheck(nemo_dev_fill_u64(d_acc.as<uint64_t>(), 0, d_acc.bytes / 8, st), "fill");
-		hipCheck(nemo_dev_pm_replay(&s, st), "plugin step: replay");
+		hipCheck(nemo_dev_pm_replay(&s, narrow, st), "plugin step: replay");
 		m_replay = false;
 	}
 	for(unsigned k = 0; k < nsteps; ++k) {
-		hipCheck(nemo_dev_pm_begin(&s, k, st), "plugin step: begin");
-		if(m_hasSchedule) {
-			uint32_t entries = (m_fsPtrHost[k + 1] - m_fsPtrHost[k]) + (m_isPtrHost[k + 1] - m_isPtrHost[k]);
-			hipCheck(nemo_dev_pm_stimulus(&s, k, entries, st), "plugin step: stimulus");
+		const uint32_t entries = m_hasSchedule
+			? (m_fsPtrHost[k + 1] - m_fsPtrHost[k]) + (m_isPtrHost[k + 1] - m_isPtrHost[k]) : 0u;
+		if(!m_builtinStep) hipCheck(nemo_dev_pm_begin(&s, k, st), "plugin step: begin");
+		hipCheck(nemo_dev_pm_stimulus(&s, k, entries, st), "plugin step: stimulus");
+		if(m_builtinStep) {
+			hipCheck(nemo_dev_pm_cycle(&s, k, entries ? 1 : 0, narrow, m_izOnly ? 1 : 0, st), "per-cycle step");
+		} else {
+			uint32_t* firedRow = s.raster + size_t(k) * m_words32;
+			/* the cycle a plugin sees is the timer's (src/nemo/cpu/Simulation.cpp:98) */
+			const unsigned tcycle = unsigned(m_timerCycles + k);
+			for(const PluginGroup& pg : m_plugins) {
+				hipCheck(pg.update(m_stream, tcycle, pg.start, pg.end,
+							d_param.as<float>() + pg.start, m_n, d_state.as<float>() + pg.start, size_t(m_ns) * m_n, m_n,
+							d_rng.as<uint32_t>() + pg.start, m_n, s.fstim, s.curE, s.curI, s.curX,
+							s.recent, firedRow, m_hasRcm ? &m_rcmDesc : nullptr), "hip_update_neurons");
+			}
+			hipCheck(nemo_dev_pm_scatter(&s, k, st), "plugin step: scatter");
 		}
-		uint32_t* firedRow = s.raster + size_t(k) * m_words32;
-		/* the cycle a plugin sees is the timer's (src/nemo/cpu/Simulation.cpp:98) */
-		const unsigned tcycle = unsigned(m_timerCycles + k);
-		for(const PluginGroup& pg : m_plugins) {
-			hipCheck(pg.update(m_stream, tcycle, pg.start, pg.end,
-						d_param.as<float>() + pg.start, m_n, d_state.as<float>() + pg.start, size_t(m_ns) * m_n, m_n,
-						d_rng.as<uint32_t>() + pg.start, m_n, s.fstim, s.curE, s.curI, s.curX,
-						s.recent, firedRow, m_hasRcm ? &m_rcmDesc : nullptr), "hip_update_neurons");
-		}
-		hipCheck(nemo_dev_pm_compact(&s, k, st), "plugin step: compact");
-		hipCheck(nemo_dev_pm_scatter(&s, k, st), "plugin step: scatter");
 		if(m_stdp) {
 			hipCheck(nemo_dev_pm_stdp(&s, st), "plugin step: stdp");
 		}
 	}
+	hipCheck(nemo_dev_pm_finish(&s, st), "plugin step: events");
+	m_partDirty = false;
 	hipCheck(hipEventRecord(e1, st), "hipEventRecord");
 	uint32_t ctl[8];
 	hipCheck(hipMemcpyAsync(h_ctl, d_ctl.ptr, sizeof(ctl), hipMemcpyDeviceToHost, st), "D2H");

@@ -160,7 +160,10 @@ class Simulation
 		nemo_hip_rcm m_rcmDesc = {};
 		bool m_hasRcm = false;
 		uint32_t m_words32 = 0;
-		DevBuf d_acc, d_curE, d_curI, d_curX, d_fstim, d_list;
+		DevBuf d_acc, d_curE, d_curI, d_curX, d_fstim, d_part;
+		bool m_builtinStep = false;    /* per-cycle step of built-in models, no plugins */
+		uint32_t m_ringDepth = 1;      /* PluginStepDev.R */
+		bool m_partDirty = true;       /* d_part holds an unfinished run's counts */
 		std::vector<uint32_t> m_fsPtrHost, m_isPtrHost;
 		void loadPlugins(const NetworkImpl& net);
 		void launchPlugins(unsigned nsteps, unsigned long long* events);
