@@ -66,7 +66,8 @@ typedef struct NetDev {
 	float* state;             /* [MAX_STATE][n] */
 	uint32_t* rng;            /* [4][n] */
 	uint64_t* recent;         /* [n] firing history, bit 0 = last cycle */
-	int32_t* ring;            /* [P][2][D][T] pending current (saved between launches) */
+	int32_t* ring;            /* [P][2][D+1][T] pending current between launches: slot t mod (D+1) for
+	                           * the input of cycle t, the slot of no pending cycle zero */
 
 	/* forward matrix: synapses of source s bucketed by target partition;
 	 * partition p's bucket is syn[off[s*(P+1)+p] .. off[s*(P+1)+p+1]).
@@ -101,6 +102,32 @@ typedef struct NetDev {
 	uint64_t* raster;         /* [nsteps][words] fired bits */
 } NetDev;
 
+/* One cycle by cycle_kernel.hip: its place in the launch and its stimulus,
+ * where the launch's descriptor holds no schedule (one current per neuron). */
+#define NEMO_CYCLE_STIM 64u
+#define NEMO_CYCLE_GROUPS 16u   /* first-level counters of finished workgroups */
+
+/* what the last workgroup of a launch writes to host memory: the device wall
+ * clock at its start and end, then the launch's number */
+typedef struct CycleReport {
+	uint64_t start, end;
+	uint64_t sequence;
+} CycleReport;
+
+typedef struct CycleArgs {
+	uint32_t k;               /* cycle within the launch (raster row, schedule entry) */
+	uint32_t slot;            /* (cycle0 + k) mod (D+1) */
+	uint32_t nf, ni;
+	uint64_t* hostRow;        /* the cycle's raster words in host memory too; NULL: no */
+	unsigned long long* part; /* [nemo_dev_cycle_blocks] delivered synapses by workgroup; NULL: not counted */
+	CycleReport* report;      /* host memory; NULL: none */
+	uint64_t sequence;
+	uint32_t* done;           /* [1 + NEMO_CYCLE_GROUPS][32] counters, zero between launches (with report) */
+	uint32_t fidx[NEMO_CYCLE_STIM];
+	uint32_t iidx[NEMO_CYCLE_STIM];
+	float ival[NEMO_CYCLE_STIM];
+} CycleArgs;
+
 /* blockIdx -> (network, partition) */
 typedef struct WorkItem {
 	uint32_t net;
@@ -122,6 +149,9 @@ int nemo_dev_step_launch(const NetDev* nets_dev, const WorkItem* work_dev, uint3
  * call), the work table maps blocks to its partitions. */
 int nemo_dev_step_launch_one(const NetDev* nd_host, const WorkItem* work_dev, uint32_t nblocks,
 		uint32_t blockDim, uint32_t ldsBytes, uint32_t variant, void* stream);
+/* One cycle of a network without STDP whose sums stay within int32 */
+int nemo_dev_cycle(const NetDev* nd_host, const CycleArgs* ca, void* stream);
+uint32_t nemo_dev_cycle_blocks(uint32_t P, uint32_t T);
 int nemo_dev_step_max_blocks(uint32_t blockDim, uint32_t ldsBytes, uint32_t variant, uint32_t* maxBlocks);
 /* Batched step as an instantiated HIP graph (clear -> persistent step ->
  * collect); collect_dev receives [nnets][16] words: the first 12 words of

@@ -675,6 +675,18 @@ __device__ inline void far_phase(const NetDev& nd, uint32_t Fp, const uint32_t* 
 	}
 }
 
+/* Row r (plane E for r < D, then I; LDS slot r mod D) of the LDS ring as a row
+ * of the ring in memory, whose planes have D+1 slots. s0 and m0 are the slots
+ * of the first pending cycle in each. */
+__device__ inline uint32_t ring_row(uint32_t r, uint32_t D, uint32_t s0, uint32_t m0)
+{
+	const uint32_t plane = r >= D ? 1u : 0u;
+	const uint32_t sl = r - plane * D;
+	uint32_t m = m0 + (sl >= s0 ? sl - s0 : sl + D - s0);
+	m = m >= D + 1u ? m - (D + 1u) : m;
+	return plane * (D + 1u) + m;
+}
+
 /* IZO: every neuron of the network is an Izhikevich neuron, so only its 5
  * parameters and 2 state variables are held in registers. Always inlined
  * into the kernels: as a call, the network descriptor is copied to scratch
@@ -733,11 +745,11 @@ __device__ __forceinline__ void run_partition(const NetDev& nd, uint32_t p)
 		atomicMin(reinterpret_cast<unsigned long long*>(nd.status + 7), (unsigned long long) wall_clock64());
 	}
 
-	/* restore the pending-current ring: 1 KB per wave instruction straight
-	 * into LDS (16 bytes per lane), every load in flight at once; the ring
-	 * is 8 D T bytes, a multiple of 512 since T is a multiple of 64, so at
-	 * most half a KB is left for ordinary loads */
-	const int32_t* gring = nd.ring + size_t(p) * 2u * D * T;
+	/* restore the pending-current ring, slot by slot: LDS slot t mod D of the
+	 * input of cycle t is slot t mod (D+1) in memory (which cycle_kernel.hip
+	 * needs). Up to 1 KB per wave instruction straight into LDS (16 bytes per
+	 * lane), every load in flight at once. */
+	int32_t* gring = nd.ring + size_t(p) * 2u * (D + 1u) * T;
 	const bool replay = (nd.flags & NEMO_NET_REPLAY) != 0u;
 	const uint32_t ringWords = 2u * D * T;
 	if(replay) {
@@ -745,13 +757,15 @@ __device__ __forceinline__ void run_partition(const NetDev& nd, uint32_t p)
 			ringE[i] = 0;
 		}
 	} else {
-		const uint32_t chunks = ringWords / 256u;
-		for(uint32_t c = wave; c < chunks; c += nwaves) {   /* wave-uniform */
-			__builtin_amdgcn_global_load_lds((NEMO_GLOBAL void*)(gring + c * 256u + lane * 4u),
-					(NEMO_LDS void*)(ringE + c * 256u), 16, 0, 0);
-		}
-		for(uint32_t i = chunks * 256u + tid; i < ringWords; i += nthreads) {
-			ringE[i] = gring[i];
+		const uint32_t s0 = uint32_t(nd.cycle0 % D), m0 = uint32_t(nd.cycle0 % (D + 1u));
+		for(uint32_t r = wave; r < 2u * D; r += nwaves) {   /* wave-uniform */
+			const int32_t* src = gring + size_t(ring_row(r, D, s0, m0)) * T;
+			for(uint32_t c = 0; c < T; c += 256u) {
+				if(c + lane * 4u < T) {
+					__builtin_amdgcn_global_load_lds((NEMO_GLOBAL void*)(src + c + lane * 4u),
+							(NEMO_LDS void*)(ringE + r * T + c), 16, 0, 0);
+				}
+			}
 		}
 		__builtin_amdgcn_s_waitcnt(0);
 	}
@@ -1280,24 +1294,31 @@ __device__ __forceinline__ void run_partition(const NetDev& nd, uint32_t p)
 		for(int k = 0; k < 4; ++k) nd.rng[size_t(k) * n_total + n] = rng.s[k];
 		nd.recent[n] = recent;
 	}
-	int32_t* gout = nd.ring + size_t(p) * 2u * D * T;
-	if(SAT) {
-		/* fold sticky overflow into the saved values */
-		for(uint32_t i = tid; i < D * T; i += nthreads) {
-			uint32_t sl = i / T, tl = i % T;
-			uint32_t bit = 1u << (tl & 31u);
-			int32_t e = ringE[i], ii = ringI[i];
-			if(ovf[sl * fwords + (tl >> 5)] & bit) e = INT32_MAX;
-			if(ovf[(D + sl) * fwords + (tl >> 5)] & bit) ii = INT32_MIN;
-			gout[i] = e;
-			gout[D * T + i] = ii;
+	{
+		const uint64_t tend = nd.cycle0 + nd.nsteps;
+		const uint32_t s0 = uint32_t(tend % D), m0 = uint32_t(tend % (D + 1u));
+		for(uint32_t r = wave; r < 2u * D; r += nwaves) {   /* wave-uniform; 16 bytes per lane */
+			NEMO_GLOBAL int4* dst = glb(reinterpret_cast<int4*>(gring + size_t(ring_row(r, D, s0, m0)) * T));
+			const int4* src = reinterpret_cast<const int4*>(ringE + r * T);
+			for(uint32_t c = lane; c < T / 4u; c += 64u) {
+				int4 v = src[c];
+				if(SAT) {
+					/* fold sticky overflow into the saved values */
+					const uint32_t o = ovf[r * fwords + (c >> 3)] >> (4u * (c & 7u));
+					const int32_t lim = r < D ? INT32_MAX : INT32_MIN;
+					if(o & 1u) v.x = lim;
+					if(o & 2u) v.y = lim;
+					if(o & 4u) v.z = lim;
+					if(o & 8u) v.w = lim;
+				}
+				dst[c] = v;
+			}
 		}
-	} else {
-		/* 16 bytes per lane and instruction (both sides 16-byte aligned) */
-		const uint4* src4 = reinterpret_cast<const uint4*>(ringE);
-		NEMO_GLOBAL uint4* dst4 = glb(reinterpret_cast<uint4*>(gout));
-		for(uint32_t i = tid; i < ringWords / 4u; i += nthreads) {
-			dst4[i] = src4[i];
+		/* the slot of no pending cycle, that of cycle tend + D, starts empty */
+		const uint32_t e0 = (m0 + D >= D + 1u) ? m0 - 1u : m0 + D;
+		for(uint32_t c = tid; c < T; c += nthreads) {
+			gring[size_t(e0) * T + c] = 0;
+			gring[size_t(D + 1u + e0) * T + c] = 0;
 		}
 	}
 	/* delivered-synapse count */

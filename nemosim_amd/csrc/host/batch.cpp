@@ -78,19 +78,6 @@ batchStream(int dev)
 	return g_streams[dev];
 }
 
-/* the device wall clock's rate (wall_clock64 in the step kernel), kHz */
-double
-wallClockKHz(int dev)
-{
-	static double g_khz[64] = {};
-	if(g_khz[dev] == 0.0) {
-		int khz = 0;
-		hipCheck(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev), "hipDeviceGetAttribute");
-		g_khz[dev] = khz > 0 ? double(khz) : 100000.0;
-	}
-	return g_khz[dev];
-}
-
 BatchPlan&
 getPlan(int dev, uint32_t variant, uint32_t blockDim, uint32_t lds, uint32_t nnets,
 		const std::vector<WorkItem>& work)

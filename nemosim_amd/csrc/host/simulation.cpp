@@ -1,6 +1,8 @@
 #include "simulation.hpp"
 
 #include <algorithm>
+#include <atomic>
+#include <cstddef>
 #include <cstdio>
 #include <cstring>
 #include <random>
@@ -173,8 +175,8 @@ Simulation::Simulation(const NetworkImpl& net, const ConfigurationImpl& conf) :
 		hipCheck(hipEventCreate(&ev1), "hipEventCreate");
 		m_ev1 = ev1;
 	}
-	hipCheck(hipHostMalloc(reinterpret_cast<void**>(&h_ctl), NEMO_CTL_WORDS * 4), "hipHostMalloc");
-	std::memset(h_ctl, 0, NEMO_CTL_WORDS * 4);
+	hipCheck(hipHostMalloc(reinterpret_cast<void**>(&h_ctl), NEMO_CTL_WORDS * 4 + sizeof(CycleReport)), "hipHostMalloc");
+	std::memset(h_ctl, 0, NEMO_CTL_WORDS * 4 + sizeof(CycleReport));
 
 	/* ---- simulation-local indices: types in order, insertion order within a
 	 * type (src/nemo/cpu/Simulation.cpp:58-73, src/nemo/cpu/Neurons.cpp:26-39) */
@@ -697,7 +699,7 @@ Simulation::Simulation(const NetworkImpl& net, const ConfigurationImpl& conf) :
 	d_state.upload(state.data(), state.size() * sizeof(float));
 	d_rng.upload(rng.data(), rng.size() * sizeof(uint32_t));
 	d_recent.alloc(size_t(m_n) * 8);
-	d_ring.alloc(size_t(m_P) * 2 * m_D * m_T * 4);
+	d_ring.alloc(size_t(m_P) * 2 * (m_D + 1) * m_T * 4);
 	if(!m_deviceBuilt) {
 		d_off.upload(off.data(), off.size() * sizeof(uint32_t));
 		if(syn.size() < 2) {
@@ -715,6 +717,10 @@ Simulation::Simulation(const NetworkImpl& net, const ConfigurationImpl& conf) :
 	d_fl.alloc(size_t(m_flRing) * m_P * m_T * 8);
 	d_fc.alloc(size_t(m_flRing) * m_P * 8 + 8);
 	d_ctl.alloc(64);
+	if(cycleKernelRuns()) {
+		d_done.alloc((1u + NEMO_CYCLE_GROUPS) * 128u);
+		hipCheck(nemo_dev_fill_u32(d_done.as<uint32_t>(), 0, d_done.bytes / 4, static_cast<hipStream_t>(m_stream)), "fill");
+	}
 	if(m_stdp) {
 		d_rfg.alloc(size_t(2) * m_n * 8);
 		if(!m_deviceBuilt) {
@@ -1498,6 +1504,82 @@ Simulation::decodeStep(const uint64_t* words, std::vector<unsigned>& out) const
 	}
 }
 
+/* the device wall clock's rate (wall_clock64 in the kernels), kHz */
+double
+wallClockKHz(int dev)
+{
+	static double khz[64] = {};
+	if(dev < 0 || dev >= 64) throw exception(NEMO_INVALID_INPUT, "device index out of range");
+	if(khz[dev] == 0.0) {
+		int r = 0;
+		hipCheck(hipDeviceGetAttribute(&r, hipDeviceAttributeWallClockRate, dev), "hipDeviceGetAttribute");
+		khz[dev] = r > 0 ? double(r) : 100000.0;
+	}
+	return khz[dev];
+}
+
+/* Synapses delivered in a cycle up to which the cycle kernel takes a step
+ * (call times, cycle kernel against fused: 3k x 1000 IF_curr_exp_noise, 1.0e6
+ * synapses, 106 us against 101; 8k x 300, 0.8e6, 85 against 97; 20k x 300,
+ * 2.0e6, 167 against 145; at 8 Hz 1k x 100 19 against 39, 100k x 300 41
+ * against 86). */
+static const double CYCLE_MAX_EVENTS = 1.0e6;
+
+/* whether csrc/device/cycle_kernel.hip can run a cycle of this network */
+bool
+Simulation::cycleKernelRuns() const
+{
+	return m_fused && !m_stdp && !m_saturate && m_P > 0 && m_n > 0;
+}
+
+/* One cycle by cycle_kernel.hip. Its stimulus travels in the kernel's
+ * arguments and its raster words come back by the kernel's own writes to
+ * pinned memory, so the call is one launch and one wait, without copies. A
+ * stimulus of more than NEMO_CYCLE_STIM entries goes through the fused kernel. */
+void
+Simulation::stepCycle(const nemo_schedule_t& s)
+{
+	CycleArgs ca;
+	std::memset(&ca, 0, offsetof(CycleArgs, fidx));
+	if(s.fstim_ptr) {
+		for(; ca.nf < s.fstim_ptr[1]; ++ca.nf) ca.fidx[ca.nf] = localIdx(s.fstim_idx[ca.nf]);
+	}
+	if(s.istim_ptr) {
+		for(unsigned j = 0; j < s.istim_ptr[1]; ++j) {
+			/* a later assignment replaces an earlier one (src/nemo/cpu/Simulation.cpp:140-163) */
+			const uint32_t l = localIdx(s.istim_idx[j]);
+			const uint32_t e = uint32_t(std::find(ca.iidx, ca.iidx + ca.ni, l) - ca.iidx);
+			ca.iidx[e] = l;
+			ca.ival[e] = s.istim_val[j];
+			if(e == ca.ni) ++ca.ni;
+		}
+	}
+	m_hasSchedule = false;
+	const NetDev nd = prepareLaunch(1);
+	ca.slot = uint32_t(m_cycle % (m_D + 1));
+	ca.hostRow = h_step;
+	CycleReport* rep = reinterpret_cast<CycleReport*>(h_ctl + NEMO_CTL_WORDS);
+	volatile uint64_t* seen = &rep->sequence;
+	ca.report = rep;
+	ca.sequence = ++m_cycleSequence;
+	ca.done = d_done.as<uint32_t>();
+	hipStream_t st = static_cast<hipStream_t>(m_stream);
+	hipCheck(nemo_dev_cycle(&nd, &ca, st), "cycle kernel launch");
+	/* the kernel's own report, which its last workgroup writes; if it does not
+	 * come, the synchronisation says why */
+	const auto patience = std::chrono::steady_clock::now() + std::chrono::milliseconds(100);
+	for(unsigned polls = 0; *seen != ca.sequence; ++polls) {
+		if((polls & 1023u) == 1023u && std::chrono::steady_clock::now() > patience) {
+			hipCheck(hipStreamSynchronize(st), "hipStreamSynchronize");
+			if(*seen != ca.sequence) throw exception(NEMO_CUDA_ERROR, "the cycle kernel ended without its report");
+		}
+	}
+	std::atomic_thread_fence(std::memory_order_acquire);
+	m_kernelMs = float(double(rep->end - rep->start) / wallClockKHz(m_device));
+	const uint32_t ctl[8] = {};
+	completeLaunch(1, ctl);
+}
+
 const std::vector<unsigned>&
 Simulation::step(const std::vector<unsigned>& fstim, const unsigned* istimIdx, const float* istimVal, size_t nistim)
 {
@@ -1512,6 +1594,14 @@ Simulation::step(const std::vector<unsigned>& fstim, const unsigned* istimIdx, c
 	s.istim_val = istimVal;
 	if(fstim.empty()) { s.fstim_ptr = nullptr; }
 	if(nistim == 0) { s.istim_ptr = nullptr; s.istim_idx = nullptr; s.istim_val = nullptr; }
+	/* while the network fires densely the cycle kernel's global atomics cost
+	 * more than the fused kernel's fixed cost; the step before says how dense */
+	const bool dense = double(m_fired.size()) * double(m_nsyn) > CYCLE_MAX_EVENTS * double(m_n);
+	if(cycleKernelRuns() && !dense && fstim.size() <= NEMO_CYCLE_STIM && nistim <= NEMO_CYCLE_STIM) {
+		stepCycle(s);
+		decodeStep(h_step, m_fired);
+		return m_fired;
+	}
 	uploadSchedule(1, &s);
 	if(m_fused && m_P > 0 && m_n > 0) {
 		/* the raster words come back with the control block */

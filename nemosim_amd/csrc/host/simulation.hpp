@@ -235,8 +235,8 @@ class Simulation
 		/* HIP events around each step-kernel launch (created once) */
 		void* m_ev0 = nullptr;
 		void* m_ev1 = nullptr;
-		/* pinned host staging: [0..15] the control block read back after a
-		 * launch, then one cycle's raster words (nemo_step) */
+		/* pinned host staging: the control block read back after a launch and
+		 * the cycle kernel's report; one cycle's raster words (nemo_step) */
 		uint32_t* h_ctl = nullptr;
 		uint64_t* h_step = nullptr;
 		/* control-block words 0 (workgroups started) and 2..3 (delivered
@@ -248,6 +248,10 @@ class Simulation
 		/* the step kernel's launch: descriptor by value, no copies before it */
 		void launchFused(unsigned nsteps, bool stepOut);
 		void launchDescriptor(const NetDev& nd, bool stepOut);
+		bool cycleKernelRuns() const;
+		void stepCycle(const nemo_schedule_t& s);
+		DevBuf d_done;                 /* CycleArgs.done */
+		uint64_t m_cycleSequence = 0;  /* launches of the cycle kernel */
 		void ensureRaster(size_t bytes);
 		NetDev descriptor(unsigned nsteps) const;
 		bool translateSchedule(unsigned nsteps, const nemo_schedule_t* s, std::vector<uint32_t>& fsPtr,
@@ -284,6 +288,9 @@ class Simulation
 				const int32_t* wfx, const uint8_t* dDl, const uint8_t* dPl);
 		bool m_deviceBuilt = false;   /* synapse structures built on the device */
 };
+
+/* the device wall clock's rate, kHz; the caller holds the device lock */
+double wallClockKHz(int dev);
 
 } // namespace hip
 } // namespace nemo

@@ -246,7 +246,7 @@ class Simulation(object):
         n = ctypes.c_size_t()
         _check(self._lib.nemo_step(self._h, _uptr(fs), len(fs), _uptr(ii), _fptr(iv), len(ii),
                                    ctypes.byref(fired), ctypes.byref(n)))
-        return [fired[i] for i in range(n.value)]
+        return fired[:n.value]
 
     # reference binding names
     def step_noinput(self):
