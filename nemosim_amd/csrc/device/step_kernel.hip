@@ -65,6 +65,21 @@ __device__ inline uint32_t lds_prefix_waves(uint32_t* wsum, uint32_t wave, uint3
 	return before;
 }
 
+/* Inclusive sum over the lanes of a wave by DPP moves (a scan by shuffles
+ * waits for LDS six times: four of them took 0.7 us of a cycle's exchange).
+ * Every lane must be active. */
+__device__ inline uint32_t wave_scan(uint32_t x)
+{
+	int v = int(x);
+	v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);   /* row_shr:1 */
+	v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);   /* row_shr:2 */
+	v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);   /* row_shr:4 */
+	v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);   /* row_shr:8 */
+	v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   /* row_bcast:15 into rows 1, 3 */
+	v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);   /* row_bcast:31 into rows 2, 3 */
+	return uint32_t(v);
+}
+
 /* Cross-workgroup data (fired lists, their tagged counts, the STDP firing
  * history) is exchanged with agent-scope relaxed atomic loads and stores.
  * On gfx950 these are sc1 accesses, coherent across the XCDs' L2s, so no L2
@@ -173,15 +188,11 @@ __device__ inline void gather_counts(const NEMO_GLOBAL uint64_t* fc, uint32_t P,
 		}
 #pragma unroll
 		for(uint32_t i = 0; i < GATHER_CH; ++i) {
-			uint32_t x = cnt[i];
-#pragma unroll
-			for(uint32_t d = 1; d < 64u; d <<= 1) {
-				uint32_t y = __shfl_up(x, d, 64);
-				if(lane >= d) x += y;
-			}
+			if(c0 + 64u * i >= P) break;   /* wave-uniform */
+			const uint32_t x = wave_scan(cnt[i]);
 			const uint32_t q = c0 + 64u * i + lane;
 			if(q < P) pref[q + 1] = carry + x;
-			carry += __shfl(x, 63, 64);
+			carry += uint32_t(__builtin_amdgcn_readlane(int(x), 63));
 		}
 	}
 	if(lane == 0) pref[0] = 0u;
