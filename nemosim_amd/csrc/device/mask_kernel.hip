@@ -1,0 +1,476 @@
+/*
+ * mask_kernel.hip -- the persistent step of networks without STDP: the fused
+ * kernel of step_kernel.hip with another exchange between partitions.
+ *
+ * There, a partition publishes a list of its fired neurons and a count, and
+ * the others read the counts, then the entries, then each source's bucket
+ * bounds, then its records: four dependent round trips, behind a barrier for
+ * the list's positions and one for the counts. Here every wave publishes its
+ * 64 fired bits as they are, two words of 32 bits with the cycle's number in
+ * the upper half, as soon as it has them; every wave of every workgroup polls
+ * its share of the network's words and delivers the sources it finds there.
+ * That is one round trip less, two barriers a cycle instead of three, and no
+ * search for a source's partition. Each workgroup reads n/32 words a cycle
+ * whatever fires (50 KB at 200k neurons), which costs a wave up to eight loads
+ * that are in flight together.
+ *
+ * What bounds it: the latency of the chain update -> words -> bounds -> delay-1
+ * records of one cycle; no unit is busy. Per cycle, against the lists on the
+ * same build: 1k x 100 5.2 -> 3.9 us (with stimulus), 10k x 313 5.6 -> 4.4,
+ * 60k x 300 6.3 -> 5.3, 100k x 100 (20 cycles) 9.1 -> 7.5, 200k x 1000 13.8 ->
+ * 12.2, 12k x 550 IF_curr_exp_noise at 333 Hz 57 -> 48; 48 networks of 1k-20k
+ * batched, 200 cycles, 3.96 -> 3.04 ms.
+ *
+ * Two buffers of words are enough: a wave publishes cycle t+1 after its own
+ * reads of cycle t, and a workgroup publishes t+2 only once its waves have
+ * seen every word of t+1.
+ */
+#include <algorithm>
+
+#include "step_device.h"
+
+namespace {
+
+constexpr uint32_t LIST = 128u;      /* sources a wave lists in LDS at a time (16 bits: from its first word on) */
+
+/* WORDS: words a lane polls together. A wave whose share of the words takes
+ * more than 64 WORDS of them goes through the rest of the cycle's chain once
+ * per 64 WORDS, and every word costs instructions whether it is there or not
+ * (10k x 100: 4.0 us a cycle with 4, 4.5 with 8; 200k x 100: 9.0 with 4, 8.4
+ * with 8), so the host picks the smallest of 1, 4 and 8 that covers the share. */
+template<bool SAT, bool IZO, uint32_t WORDS>
+__device__ __forceinline__ void run_masked(const NetDev& nd, uint32_t p)
+{
+	constexpr int NP = IZO ? 5 : MAX_PARAM;
+	constexpr int NS = IZO ? 2 : MAX_STATE;
+	constexpr uint32_t PAIRS = (WORDS + 1u) / 2u;   /* words joined to 64 bits */
+	extern __shared__ __align__(16) uint8_t lds[];
+
+	const uint32_t T = nd.T, D = nd.D, P = nd.P;
+	const uint32_t n_total = nd.n;
+	const uint32_t tid = threadIdx.x;
+	const uint32_t nthreads = blockDim.x;
+	const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);   /* wave-uniform, in a scalar register */
+	const uint32_t lane = tid & 63u;
+	const uint32_t nwaves = nthreads >> 6;
+	const uint32_t nw = T >> 6;                 /* waves that have neurons; the rest (batches) only keep the barriers */
+	const uint32_t n = p * T + tid;
+	const bool active = (tid < T) && (n < n_total);
+	const uint32_t fwords = T >> 5;
+
+	/* LDS: see nemo_mask_lds_bytes */
+	int32_t* ringE = reinterpret_cast<int32_t*>(lds);
+	int32_t* ringI = ringE + D * T;
+	float* ext = reinterpret_cast<float*>(ringI + D * T);
+	uint32_t* fst = reinterpret_cast<uint32_t*>(ext + T);
+	uint32_t* ovf = fst + fwords;                                      /* [2][D][T/32] when SAT */
+	uint16_t* list = reinterpret_cast<uint16_t*>(ovf + (SAT ? 2u * D * fwords : 0u)) + wave * LIST;
+	const bool defer = (nd.flags & NEMO_NET_DEFER) != 0u;
+	const uint32_t offMask = defer ? ((1u << OFF_NEAR_SHIFT) - 1u) : ~0u;
+	const NEMO_GLOBAL uint2* syn = glb(reinterpret_cast<const uint2*>(nd.syn));
+	const NEMO_GLOBAL uint32_t* off = glb(nd.off);
+
+	/* as in step_kernel.hip: workgroups started, first start (diagnostics) */
+	if(tid == 0) {
+		atomicAdd(nd.status - 1, 1u);
+		atomicMin(reinterpret_cast<unsigned long long*>(nd.status + 7), (unsigned long long) wall_clock64());
+	}
+
+	int32_t* gring = nd.ring + size_t(p) * 2u * (D + 1u) * T;
+	ring_restore(gring, ringE, T, D, nd.cycle0, wave, nwaves, lane);
+	if(SAT) {
+		for(uint32_t i = tid; i < 2u * D * fwords; i += nthreads) ovf[i] = 0u;
+	}
+	if(tid < T) ext[tid] = 0.0f;
+	if(tid < fwords) fst[tid] = 0u;
+
+	/* neuron registers */
+	int model = 0;
+	float prm[NP];
+	float st[NS];
+	Rng rng;
+	uint64_t recent = 0;
+#pragma unroll
+	for(int k = 0; k < NP; ++k) prm[k] = 0.0f;
+#pragma unroll
+	for(int k = 0; k < NS; ++k) st[k] = 0.0f;
+	rng.s[0] = rng.s[1] = rng.s[2] = rng.s[3] = 0u;
+	if(active) {
+		model = nd.model[n];
+#pragma unroll
+		for(int k = 0; k < NP; ++k) prm[k] = nd.param[size_t(k) * n_total + n];
+#pragma unroll
+		for(int k = 0; k < NS; ++k) st[k] = nd.state[size_t(k) * n_total + n];
+#pragma unroll
+		for(int k = 0; k < 4; ++k) rng.s[k] = nd.rng[size_t(k) * n_total + n];
+		recent = nd.recent[n];
+	}
+	unsigned long long events = 0;
+	/* deferred delivery: this wave's far ranges (delays >= 2) of the previous
+	 * cycle's sources, one per lane, kn of them (wave-uniform) */
+	uint32_t ka0 = 0, kb0 = 0, ka1 = 0, kb1 = 0, kn = 0;
+	/* Lanes per source: as many as cover a bucket in one pass, fewer (down to
+	 * glog2) where that would take more rounds than are in flight together */
+	auto lanes = [&](uint32_t nsrc) {
+		uint32_t g = nd.glogFew;
+		while(g > nd.glog2 && pass_rounds(nsrc, g) > DeliverRounds<SAT, IZO>::value) --g;
+		return g;
+	};
+	/* the Gaussian input of Izhikevich networks is drawn a cycle ahead */
+	float noise = 0.0f;
+	if(IZO && active && nd.nsteps > 0u && prm[IZ_SIGMA] != 0.0f) {
+		noise = prm[IZ_SIGMA] * nrand(rng);
+	}
+	const uint32_t W = P * fwords;
+	const uint32_t w0 = wave < nw ? W * wave / nw : 0u;     /* this wave's share of the words */
+	const uint32_t w1 = wave < nw ? W * (wave + 1u) / nw : 0u;
+
+	/* Stimulus is put into LDS a cycle ahead: the schedule's bounds of the next
+	 * cycle are in registers, its first entries are loaded after the publish
+	 * and stored before the cycle's last barrier; the update that reads them
+	 * clears them. */
+	const bool sched = nd.fs_ptr != nullptr;
+	uint32_t fb = 0, fe = 0, ib = 0, ie = 0;    /* bounds of the next cycle's entries */
+	const uint32_t lo = p * T;
+	auto force = [&](uint32_t idx) {
+		const uint32_t l = idx - lo;
+		if(l < T) atomicOr(&fst[l >> 5], 1u << (l & 31u));
+	};
+	auto drive = [&](uint32_t idx, float v) {
+		const uint32_t l = idx - lo;
+		if(l < T) ext[l] = v;
+	};
+	__syncthreads();
+	if(sched && nd.nsteps > 0u) {
+		const uint32_t f0 = glb(nd.fs_ptr)[0], i0 = glb(nd.is_ptr)[0];
+		fb = glb(nd.fs_ptr)[1];
+		ib = glb(nd.is_ptr)[1];
+		for(uint32_t e = f0 + tid; e < fb; e += nthreads) force(glb(nd.fs_idx)[e]);
+		for(uint32_t e = i0 + tid; e < ib; e += nthreads) drive(glb(nd.is_idx)[e], glb(nd.is_val)[e]);
+		if(nd.nsteps > 1u) {
+			fe = glb(nd.fs_ptr)[2];
+			ie = glb(nd.is_ptr)[2];
+		}
+	}
+	uint32_t slotK = uint32_t(nd.cycle0 % D);
+	__syncthreads();
+
+	for(uint32_t k = 0; k < nd.nsteps; ++k) {
+		const uint64_t t = nd.cycle0 + k;
+		const uint32_t tag = uint32_t(t);
+		const uint32_t slot = slotK;
+		slotK = (slotK + 1u == D) ? 0u : slotK + 1u;
+		const bool drawn = !(IZO && active && k + 1u < nd.nsteps && prm[IZ_SIGMA] != 0.0f);
+		NEMO_GLOBAL uint64_t* words = glb(nd.mk) + size_t(tag & 1u) * W;
+
+		/* ---- 1. neuron update */
+		bool fired = false;
+		if(active) {
+			const uint32_t r = slot * T + tid;
+			int32_t e = ringE[r];
+			int32_t i = ringI[r];
+			if(SAT) {
+				const uint32_t bit = 1u << (tid & 31u);
+				if(ovf[slot * fwords + (tid >> 5)] & bit) e = INT32_MAX;
+				if(ovf[(D + slot) * fwords + (tid >> 5)] & bit) i = INT32_MIN;
+			}
+			ringE[r] = 0;
+			ringI[r] = 0;
+			float cx = 0.0f;
+			bool fs = false;
+			if(sched) {
+				cx = ext[tid];
+				fs = ((fst[tid >> 5] >> (tid & 31u)) & 1u) != 0u;
+				ext[tid] = 0.0f;
+			}
+			if(IZO) {
+				fired = izhikevich_drawn(prm, st, noise, fx20_to_float(e), fx20_to_float(i), cx, fs);
+			} else {
+				fired = update_neuron(model, prm, st, rng, fx20_to_float(e), fx20_to_float(i), cx, fs);
+			}
+			recent = (recent << 1) | (fired ? 1ull : 0ull);
+		}
+
+		/* ---- 2. publish the wave's fired bits; the raster */
+		const uint64_t mask = __ballot(fired);
+		if(wave < nw) {
+			if(lane < 2u) {
+				st_agent(words + p * fwords + wave * 2u + lane,
+						(uint64_t(tag) << 32) | uint64_t(uint32_t(mask >> (32u * lane))));
+				/* the wave's forced-firing bits have been read */
+				if(sched) fst[wave * 2u + lane] = 0u;
+			}
+			if(lane == 0u) {
+				glb(nd.raster)[size_t(k) * nd.words + p * (T >> 6) + wave] = mask;
+			}
+		}
+		/* every wave has read its slot before records of delay D, or the
+		 * next stimulus, are added */
+		__syncthreads();
+		if(SAT) {
+			/* the slot just consumed starts empty for cycle t + D */
+			for(uint32_t w = tid; w < fwords; w += nthreads) {
+				ovf[slot * fwords + w] = 0u;
+				ovf[(D + slot) * fwords + w] = 0u;
+			}
+			__syncthreads();
+		}
+
+		/* the next cycle's first stimulus entries, and the bounds of the one after */
+		uint32_t fx = ~0u, ix = ~0u, fnext = 0, inext = 0;
+		float iv = 0.0f;
+		if(sched) {
+			if(fb + tid < fe) fx = glb(nd.fs_idx)[fb + tid];
+			if(ib + tid < ie) {
+				ix = glb(nd.is_idx)[ib + tid];
+				iv = glb(nd.is_val)[ib + tid];
+			}
+			if(k + 2u < nd.nsteps) {
+				fnext = glb(nd.fs_ptr)[k + 3u];
+				inext = glb(nd.is_ptr)[k + 3u];
+			}
+		}
+
+		/* the next cycle's Gaussian input, while the words are under way */
+		if(!drawn) {
+			noise = prm[IZ_SIGMA] * nrand(rng);
+		}
+
+		/* ---- deferred records (delays >= 2) of the previous cycle's spikes */
+		if(kn) {
+			deliver_ranges<SAT, IZO>(ka0, kb0, ka1, kb1, kn, lanes(kn), lane, (slot + D - 1u) % D, syn,
+					ringE, ringI, ovf, D, T, fwords);
+			kn = 0;
+		}
+
+		/* ---- 3. this wave's words of every partition; 4. delivery of the
+		 * sources in them */
+		bool first = true;
+		for(uint32_t c0 = w0; c0 < w1; c0 += 64u * WORDS) {   /* wave-uniform */
+			uint64_t m[PAIRS];
+			uint32_t pos[PAIRS];
+			uint32_t pending = 0;
+#pragma unroll
+			for(uint32_t i = 0; i < PAIRS; ++i) m[i] = 0ull;
+#pragma unroll
+			for(uint32_t i = 0; i < WORDS; ++i) {
+				if(c0 + 64u * i + lane < w1) pending |= 1u << i;
+			}
+			uint32_t spins = 0;
+			while(pending) {
+				uint64_t v[WORDS];
+#pragma unroll
+				for(uint32_t i = 0; i < WORDS; ++i) {
+					v[i] = 0ull;
+					if(c0 + 64u * i < w1) {   /* wave-uniform */
+						if((pending >> i) & 1u) v[i] = ld_agent(words + c0 + 64u * i + lane);
+					}
+				}
+#pragma unroll
+				for(uint32_t i = 0; i < WORDS; ++i) {
+					if(((pending >> i) & 1u) && uint32_t(v[i] >> 32) == tag) {
+						m[i / 2u] |= uint64_t(uint32_t(v[i])) << (32u * (i & 1u));
+						pending &= ~(1u << i);
+					}
+				}
+				if(!pending) break;
+				/* bounded, as gather_counts in step_kernel.hip */
+				if((++spins & 15u) == 0u) {
+					if(ld_agent(glb(nd.status)) != 0u) break;
+					if(spins > nd.spinLimit) {
+						report_timeout(nd.status, NEMO_STATUS_BARRIER_TIMEOUT, tag, p,
+								(c0 + 64u * uint32_t(__builtin_ctz(pending)) + lane) / fwords);
+						break;
+					}
+				}
+			}
+			uint32_t total = 0;
+#pragma unroll
+			for(uint32_t i = 0; i < PAIRS; ++i) {
+				pos[i] = 0u;
+				if(c0 + 128u * i < w1) {   /* wave-uniform */
+					const uint32_t c = uint32_t(__popcll(m[i]));
+					const uint32_t x = wave_scan(c);
+					pos[i] = total + x - c;
+					total += uint32_t(__builtin_amdgcn_readlane(int(x), 63));
+				}
+			}
+			/* The sources, up to LIST at a time, in LDS so that one lane takes
+			 * each: every lane writes its own bits. More than one list (dense
+			 * firing): word by word, so that a list's bits are spread over
+			 * more lanes. */
+			const bool dense = total > LIST;
+			uint32_t word = 0, cur = 0, cpos = 0, ctotal = 0, cdone = 0;   /* dense: the word being listed */
+			for(uint32_t left = total; left > 0u; ) {   /* wave-uniform */
+				uint32_t nsrc = total;
+				if(!dense) {
+#pragma unroll
+					for(uint32_t i = 0; i < PAIRS; ++i) {
+						while(m[i]) {
+							const uint32_t x = uint32_t(__builtin_ctzll(m[i]));
+							list[pos[i]++] = uint16_t((128u * i + 64u * (x >> 5) + lane) * 32u + (x & 31u));
+							m[i] &= m[i] - 1ull;
+						}
+					}
+				} else {
+					nsrc = 0u;
+					while(nsrc < LIST && nsrc < left) {
+						while(cdone == ctotal) {   /* the next word that has bits */
+#pragma unroll
+							for(uint32_t i = 0; i < PAIRS; ++i) {
+								if(word >> 1 == i) cur = (word & 1u) ? uint32_t(m[i] >> 32) : uint32_t(m[i]);
+							}
+							word += 1u;
+							const uint32_t c = uint32_t(__popc(cur));
+							const uint32_t x = wave_scan(c);
+							cpos = x - c;
+							ctotal = uint32_t(__builtin_amdgcn_readlane(int(x), 63));
+							cdone = 0u;
+						}
+						const uint32_t take = min(LIST - nsrc, ctotal - cdone);
+						while(cur && cpos < cdone + take) {
+							list[nsrc + cpos - cdone] = uint16_t((64u * (word - 1u) + lane) * 32u + uint32_t(__builtin_ctz(cur)));
+							cur &= cur - 1u;
+							cpos += 1u;
+						}
+						nsrc += take;
+						cdone += take;
+					}
+				}
+				left -= nsrc;
+				__builtin_amdgcn_wave_barrier();   /* a wave's LDS operations complete in order */
+				const bool v0 = lane < nsrc;
+				const bool v1 = 64u + lane < nsrc;
+				uint32_t a0 = 0, b0r = 0, a1 = 0, b1r = 0;
+				if(v0) {
+					const NEMO_GLOBAL uint32_t* o = off + size_t(c0 * 32u + list[lane]) * (P + 1u) + p;
+					a0 = ld_off(o);
+					b0r = ld_off(o + 1) & offMask;
+				}
+				if(v1) {
+					const NEMO_GLOBAL uint32_t* o = off + size_t(c0 * 32u + list[64u + lane]) * (P + 1u) + p;
+					a1 = ld_off(o);
+					b1r = ld_off(o + 1) & offMask;
+				}
+				__builtin_amdgcn_wave_barrier();   /* the list is written again */
+				const uint32_t n0 = a0 >> OFF_NEAR_SHIFT, n1 = a1 >> OFF_NEAR_SHIFT;
+				a0 &= offMask;
+				a1 &= offMask;
+				events += (b0r - a0) + (b1r - a1);
+				if(defer && first) {
+					/* the records of delay 1 (first in each bucket, their count
+					 * in the top bits of its start) now, the rest in the next
+					 * cycle while its words are under way */
+					const uint32_t mx = max(n0, n1);
+					const uint32_t sl = (slot + 1u >= D) ? slot + 1u - D : slot + 1u;
+					for(uint32_t i = 0; i < mx; i += 2u) {
+						const bool ok00 = i < n0, ok01 = i + 1u < n0, ok10 = i < n1, ok11 = i + 1u < n1;
+						const uint2 r00 = ld_rec(syn, ok00 ? a0 + i : 0u);
+						const uint2 r01 = ld_rec(syn, ok01 ? a0 + i + 1u : 0u);
+						const uint2 r10 = ld_rec(syn, ok10 ? a1 + i : 0u);
+						const uint2 r11 = ld_rec(syn, ok11 ? a1 + i + 1u : 0u);
+						if(ok00) ring_add<SAT>(ringE, ringI, ovf, D, T, fwords, sl, r00.x & 0xffffu, int32_t(r00.y));
+						if(ok01) ring_add<SAT>(ringE, ringI, ovf, D, T, fwords, sl, r01.x & 0xffffu, int32_t(r01.y));
+						if(ok10) ring_add<SAT>(ringE, ringI, ovf, D, T, fwords, sl, r10.x & 0xffffu, int32_t(r10.y));
+						if(ok11) ring_add<SAT>(ringE, ringI, ovf, D, T, fwords, sl, r11.x & 0xffffu, int32_t(r11.y));
+					}
+					ka0 = a0 + n0;
+					kb0 = b0r;
+					ka1 = a1 + n1;
+					kb1 = b1r;
+					kn = nsrc;
+					first = false;
+				} else {
+					deliver_ranges<SAT, IZO>(a0, b0r, a1, b1r, nsrc, lanes(nsrc), lane, slot, syn,
+							ringE, ringI, ovf, D, T, fwords);
+				}
+			}
+		}
+
+		if(sched) {
+			if(fx != ~0u) force(fx);
+			if(ix != ~0u) drive(ix, iv);
+			for(uint32_t e = fb + nthreads + tid; e < fe; e += nthreads) force(glb(nd.fs_idx)[e]);
+			for(uint32_t e = ib + nthreads + tid; e < ie; e += nthreads) drive(glb(nd.is_idx)[e], glb(nd.is_val)[e]);
+			fb = fe;
+			ib = ie;
+			fe = k + 2u < nd.nsteps ? fnext : fe;
+			ie = k + 2u < nd.nsteps ? inext : ie;
+		}
+		__syncthreads();
+	}
+
+	/* ---- the last cycle's deferred records */
+	if(kn) {
+		deliver_ranges<SAT, IZO>(ka0, kb0, ka1, kb1, kn, lanes(kn), lane,
+				uint32_t((nd.cycle0 + nd.nsteps - 1u) % D), syn, ringE, ringI, ovf, D, T, fwords);
+	}
+	__syncthreads();
+
+	/* ---- save state and the ring for the next launch */
+	if(active) {
+#pragma unroll
+		for(int k = 0; k < NS; ++k) nd.state[size_t(k) * n_total + n] = st[k];
+#pragma unroll
+		for(int k = 0; k < 4; ++k) nd.rng[size_t(k) * n_total + n] = rng.s[k];
+		nd.recent[n] = recent;
+	}
+	ring_save<SAT>(gring, ringE, ovf, T, D, nd.cycle0 + nd.nsteps, wave, nwaves, lane);
+	for(uint32_t d = 32; d >= 1; d >>= 1) {
+		events += __shfl_down(events, d, 64);
+	}
+	if(lane == 0 && events) {
+		atomicAdd(nd.events, events);
+	}
+	__syncthreads();
+	if(tid == 0) {
+		atomicMax(reinterpret_cast<unsigned long long*>(nd.status + 9), (unsigned long long) wall_clock64());
+	}
+}
+
+} // namespace
+
+template<bool SAT, bool IZO>
+__global__ void __launch_bounds__(1024)
+nemo_mask_kernel(const NetDev* __restrict__ nets, const WorkItem* __restrict__ work)
+{
+	const WorkItem wi = work[blockIdx.x];
+	const NetDev nd = nets[wi.net];
+	run_masked<SAT, IZO, 4u>(nd, wi.part);
+}
+
+/* one network per launch: the descriptor as a kernel argument */
+template<bool SAT, bool IZO, uint32_t WORDS>
+__global__ void __launch_bounds__(1024)
+nemo_mask_kernel_single(const NetDev nd, const WorkItem* __restrict__ work)
+{
+	run_masked<SAT, IZO, WORDS>(nd, work[blockIdx.x].part);
+}
+
+namespace {
+
+template<bool SAT, bool IZO>
+const void* mask_kernel(uint32_t words)
+{
+	if(words == 0u) return reinterpret_cast<const void*>(&nemo_mask_kernel<SAT, IZO>);
+	/* saturating networks, whose atomics take more registers, always 4 */
+	if(!SAT && words <= 64u) return reinterpret_cast<const void*>(&nemo_mask_kernel_single<SAT, IZO, SAT ? 4u : 1u>);
+	if(!SAT && words > 256u) return reinterpret_cast<const void*>(&nemo_mask_kernel_single<SAT, IZO, SAT ? 4u : 8u>);
+	return reinterpret_cast<const void*>(&nemo_mask_kernel_single<SAT, IZO, 4u>);
+}
+
+} // namespace
+
+extern "C" {
+
+const void* nemo_dev_mask_kernel(uint32_t variant, uint32_t words)
+{
+	switch(variant & 3u) {
+	case 0: return mask_kernel<false, false>(words);
+	case 1: return mask_kernel<true, false>(words);
+	case 2: return mask_kernel<false, true>(words);
+	default: return mask_kernel<true, true>(words);
+	}
+}
+
+} // extern "C"

@@ -25,6 +25,8 @@ extern "C" {
 #define NEMO_NET_PREF_RING 32u  /* STDP: prefixes of the fired counts of the last
                                  * postLen cycles kept in LDS */
 
+#define NEMO_NET_MASKS 64u      /* fired bits exchanged as words (mask_kernel.hip) */
+
 /* Bits of the per-network status word */
 #define NEMO_STATUS_BARRIER_TIMEOUT 1u   /* a fired count never arrived */
 #define NEMO_STATUS_ENTRY_TIMEOUT   2u   /* a fired-list entry never arrived */
@@ -52,6 +54,7 @@ typedef struct NetDev {
 	uint32_t nsteps;     /* steps this network runs in the current launch */
 	uint32_t spinLimit;  /* barrier spin bound (iterations) */
 	uint32_t glog2;      /* log2 of the lanes that share one fired source in delivery (0..6) */
+	uint32_t glogFew;    /* the same where a wave has few fired sources (NEMO_NET_MASKS; >= glog2) */
 	uint32_t flRing;     /* fired lists and counts kept for this many cycles (buffer t mod flRing) */
 	uint32_t stdpCache;  /* STDP chunks whose reverse records are staged in LDS (64 words each) */
 	uint32_t exWaves;    /* with NEMO_NET_DEFER: waves of a workgroup that run the exchange and the
@@ -79,6 +82,7 @@ typedef struct NetDev {
 	 * by cycle parity */
 	uint64_t* fl;             /* [flRing][P][T] fired neurons of each partition, (cycle << 32) | neuron */
 	uint64_t* fc;             /* [flRing][P] (cycle << 32) | fired count; starts all-ones */
+	uint64_t* mk;             /* [2][P*T/32] (cycle << 32) | 32 fired bits; starts all-ones (NEMO_NET_MASKS) */
 	uint64_t* rfg;            /* [2][n] firing history (STDP only) */
 	uint32_t* status;         /* NEMO_STATUS_* */
 	unsigned long long* events; /* delivered-synapse counter */
@@ -137,12 +141,17 @@ typedef struct WorkItem {
 /* Kernel launchers (nemosim_amd/csrc/device/step_kernel.hip). They return a
  * hipError_t value as int and take a hipStream_t as void*. */
 /* Step-kernel variants: bit 0 = saturating accumulation (NEMO_NET_SATURATE),
- * bit 1 = Izhikevich-only network (NEMO_NET_IZHIKEVICH_ONLY). All networks
- * of one launch must be of the launch's variant. */
+ * bit 1 = Izhikevich-only network (NEMO_NET_IZHIKEVICH_ONLY), bit 2 = fired
+ * bits exchanged as words (NEMO_NET_MASKS, mask_kernel.hip). All networks of
+ * one launch must be of the launch's variant. */
 static inline uint32_t nemo_step_variant(uint32_t flags)
 {
-	return ((flags & NEMO_NET_SATURATE) ? 1u : 0u) | ((flags & NEMO_NET_IZHIKEVICH_ONLY) ? 2u : 0u);
+	return ((flags & NEMO_NET_SATURATE) ? 1u : 0u) | ((flags & NEMO_NET_IZHIKEVICH_ONLY) ? 2u : 0u)
+		| ((flags & NEMO_NET_MASKS) ? 4u : 0u);
 }
+/* The kernel of mask_kernel.hip for a variant: for one network whose waves
+ * take up to `words` words each, or for batches (words = 0) */
+const void* nemo_dev_mask_kernel(uint32_t variant, uint32_t words);
 int nemo_dev_step_launch(const NetDev* nets_dev, const WorkItem* work_dev, uint32_t nblocks,
 		uint32_t blockDim, uint32_t ldsBytes, uint32_t variant, void* stream);
 /* One network: the descriptor is passed by value (nd_host is read at the
@@ -220,6 +229,13 @@ static inline uint32_t nemo_step_lds_bytes(uint32_t T, uint32_t D, uint32_t P, i
 		b += ((P + 1u + 63u) & ~63u) * 4u;   /* prefix of the counts of the targets' cycle */
 	}
 	return b;
+}
+
+/* LDS bytes of mask_kernel.hip: the ring, external current, forced-firing
+ * bits, overflow bits and 128 16-bit sources per wave */
+static inline uint32_t nemo_mask_lds_bytes(uint32_t T, uint32_t D, int saturate)
+{
+	return 2u * D * T * 4u + T * 4u + (T / 32u) * 4u + (saturate ? 2u * D * (T / 32u) * 4u : 0u) + (T / 64u) * 256u;
 }
 
 #ifdef __cplusplus

@@ -387,31 +387,61 @@ Simulation::Simulation(const NetworkImpl& net, const ConfigurationImpl& conf) :
 		whyNotFused = "a neuron type has no fused implementation";
 	}
 
+	/* Networks without STDP exchange their fired bits as words
+	 * (mask_kernel.hip), unless the configuration asks for exchange waves or
+	 * that kernel's LDS leaves too few neurons per workgroup. Per cycle, lists
+	 * against words: 1k x 100 4.5 -> 3.4 us, 10k x 1000 9.1 -> 6.0, 60k x 300
+	 * 6.3 -> 5.4, 200k x 1000 13.8 -> 12.8, 12k x 550 IF_curr_exp_noise at 333
+	 * Hz 57 -> 47. */
+	m_masks = !m_stdp && conf.exchangeWaves <= 0;
+	auto ldsFor = [&](uint32_t t) {
+		uint32_t p = (m_n + t - 1) / t;
+		if(m_masks) return nemo_mask_lds_bytes(t, m_D, m_saturate ? 1 : 0);
+		return nemo_step_lds_bytes(t, m_D, std::max(1u, p), m_saturate ? 1 : 0, m_stdp ? 1 : 0);
+	};
 	/* T: neurons per partition. The automatic choice takes at most one
 	 * partition per compute unit (256), and for mid-size networks fewer,
 	 * wider partitions: their cycle is bound by the exchange between
-	 * partitions. Measured per cycle: about 40 partitions of up to 512
-	 * neurons (10k x 100: 7.2 -> 6.3 us; 50k x 1000: 10.4 -> 9.7 us), and
-	 * with rows of 500 synapses or more, from 1.5k to 12k neurons, about 13
-	 * partitions (2k x 1000: 8.0 -> 7.2 us; 5k x 1000: 9.6 -> 7.1 us; 10k x
-	 * 1000: 10.2 -> 8.6 us). The LDS ring [D][T] bounds it from above. */
-	uint32_t T;
-	if(conf.partitionSize) {
-		T = std::min(1024u, roundUp64(conf.partitionSize));
-	} else {
-		const uint32_t perCU = roundUp64(std::max<uint32_t>(1u, (m_n + 255u) / 256u));
-		const bool longRows = m_n >= 1500u && m_n <= 12000u && m_nsyn / m_n >= 500u;
-		const uint32_t parts = longRows ? 13u : 40u;
-		const uint32_t wide = std::min(longRows ? 1024u : 512u,
-				roundUp64(std::max<uint32_t>(1u, (m_n + parts - 1u) / parts)));
-		T = std::max(64u, std::min(1024u, std::max(perCU, wide)));
-	}
-	auto ldsFor = [&](uint32_t t) {
-		uint32_t p = (m_n + t - 1) / t;
-		return nemo_step_lds_bytes(t, m_D, std::max(1u, p), m_saturate ? 1 : 0, m_stdp ? 1 : 0);
+	 * partitions. The LDS ring [D][T] bounds it from above.
+	 *   With words: about 27 partitions of up to 512 neurons (3k x 300: 128
+	 * neurons 3.7 us per cycle, 256 4.1; 10k x 100: 384 4.0, 128 4.1, 960 4.9;
+	 * 20k x 1000: 320 6.3, 512 6.9, 960 7.6), rows of 500 synapses from 1.5k to
+	 * 3k neurons about 13 (2k x 1000: 192 4.1, 128 5.3, 512 6.2), from 48k
+	 * neurons on about 160 (100k x 300: 640 6.5, 832 6.9; 200k x 1000: 960
+	 * 12.8, 832 13.7).
+	 *   With lists: about 40 partitions of up to 512 neurons (10k x 100: 7.2 ->
+	 * 6.3 us; 50k x 1000: 10.4 -> 9.7 us), and with rows of 500 synapses or
+	 * more, from 1.5k to 12k neurons, about 13 partitions (2k x 1000: 8.0 ->
+	 * 7.2 us; 5k x 1000: 9.6 -> 7.1 us; 10k x 1000: 10.2 -> 8.6 us). */
+	auto partitionSize = [&]() {
+		uint32_t t;
+		if(conf.partitionSize) {
+			t = std::min(1024u, roundUp64(conf.partitionSize));
+		} else {
+			const uint32_t perCU = roundUp64(std::max<uint32_t>(1u, (m_n + 255u) / 256u));
+			const bool large = m_masks && m_n >= 49152u;
+			const bool longRows = m_n >= 1500u && m_n <= (m_masks ? 3000u : 12000u) && m_nsyn / m_n >= 500u;
+			const uint32_t parts = longRows ? 13u : (large ? 160u : (m_masks ? 27u : 40u));
+			uint32_t wide = roundUp64(std::max<uint32_t>(1u, (m_n + parts - 1u) / parts));
+			wide = std::min(longRows ? 1024u : (large ? 960u : 512u), std::max(wide, large ? 512u : 64u));
+			t = std::max(64u, std::min(1024u, std::max(perCU, wide)));
+		}
+		while(t > 64 && ldsFor(t) > ldsLimit) {
+			t -= 64;
+		}
+		return t;
 	};
-	while(T > 64 && ldsFor(T) > ldsLimit) {
-		T -= 64;
+	uint32_t T = partitionSize();
+	m_izOnly = !m_model.empty() && std::all_of(m_model.begin(), m_model.end(),
+			[](uint8_t m) { return m == uint8_t(nemo_dev::MODEL_IZHIKEVICH); });
+	if(m_masks && m_n > 0 && whyNotFused.empty()) {
+		uint32_t maxBlocks = 0;
+		const uint32_t lds = ldsFor(T);
+		if(lds <= ldsLimit) hipCheck(nemo_dev_step_max_blocks(T, lds, variant(), &maxBlocks), "occupancy query");
+		if((m_n + T - 1) / T > maxBlocks) {
+			m_masks = false;
+			T = partitionSize();
+		}
 	}
 	if(whyNotFused.empty() && ldsFor(T) > ldsLimit) {
 		whyNotFused = "maximum delay too large for the LDS delay ring";
@@ -419,8 +449,6 @@ Simulation::Simulation(const NetworkImpl& net, const ConfigurationImpl& conf) :
 	m_T = T;
 	m_P = (m_n + T - 1) / T;
 	m_lds = ldsFor(T);
-	m_izOnly = !m_model.empty() && std::all_of(m_model.begin(), m_model.end(),
-			[](uint8_t m) { return m == uint8_t(nemo_dev::MODEL_IZHIKEVICH); });
 	if(whyNotFused.empty() && m_P > 0) {
 		uint32_t maxBlocks = 0;
 		hipCheck(nemo_dev_step_max_blocks(m_T, m_lds, variant(), &maxBlocks), "occupancy query");
@@ -477,27 +505,30 @@ Simulation::Simulation(const NetworkImpl& net, const ConfigurationImpl& conf) :
 		 * (synapses of one source into one partition): a power of two about
 		 * 1.5x of it for short buckets, so that one pass (two records per
 		 * lane) covers almost every bucket (200k x 1000, buckets of 4: 8
-		 * lanes beat 4 and 2); for long buckets no more than half of it,
-		 * and at least 8, since every round serves only 64/lanes sources
-		 * and a wave with many fired sources runs as many rounds. Measured
-		 * per cycle, the capped count against 1.5x: 20k x 1000 (buckets of
-		 * 25) 8.6 against 10.9 us; IF_curr_exp_noise at 333 Hz, 3k x 300
-		 * (12.5) 28.1 against 48.8, 12k x 550 (42) 57.8 against 74.1,
-		 * 50k x 1000 (10) 145.5 against 165.8; 3k x 300 at 6 Hz 6.7
-		 * against 6.1. */
+		 * lanes beat 4 and 2), at least 4 (200k x 100, buckets of 0.4: 8.8 us
+		 * per cycle with 2 or 4 lanes, 9.7 with 1); for long buckets no more
+		 * than half of it, and at least 8, since every round serves only
+		 * 64/lanes sources and a wave with many fired sources runs as many
+		 * rounds. Measured per cycle, the capped count against 1.5x: 20k x
+		 * 1000 (buckets of 25) 8.6 against 10.9 us; IF_curr_exp_noise at 333
+		 * Hz, 3k x 300 (12.5) 28.1 against 48.8, 12k x 550 (42) 57.8 against
+		 * 74.1, 50k x 1000 (10) 145.5 against 165.8. The mask kernel takes
+		 * glogFew (about 0.75x) while a wave's sources fit its rounds in
+		 * flight (3k x 300, buckets of 12.5: 16 lanes 3.7 us, 8 lanes 4.5). */
 		const double lavg = m_n ? double(m_nsyn) / (double(m_n) * double(m_P)) : 0.0;
 		m_glog2 = 0;
+		auto log2Of = [](double v) {
+			uint32_t g = 0;
+			while(g < 6 && double(1u << g) < v) ++g;
+			return g;
+		};
 		if(conf.deliveryLanes) {
 			while((1u << m_glog2) < conf.deliveryLanes) ++m_glog2;
+			m_glogFew = m_glog2;
 		} else {
-			while(m_glog2 < 6 && double(1u << m_glog2) < 1.5 * lavg) {
-				++m_glog2;
-			}
-			uint32_t half = 0;
-			while(half < 6 && double(1u << half) < 0.5 * lavg) {
-				++half;
-			}
-			m_glog2 = std::min(m_glog2, std::max(3u, half));
+			m_glogFew = std::max(2u, std::max(log2Of(0.75 * lavg), std::min(3u, log2Of(1.5 * lavg))));
+			m_glog2 = std::max(2u, std::min(log2Of(1.5 * lavg), std::max(3u, log2Of(0.5 * lavg))));
+			m_glogFew = std::max(m_glogFew, m_glog2);
 		}
 	}
 
@@ -716,6 +747,7 @@ Simulation::Simulation(const NetworkImpl& net, const ConfigurationImpl& conf) :
 	m_flRing = m_stdp ? std::max(3u, uint32_t(m_sp.postLen) + 2u) : (m_defer ? 3u : 2u);
 	d_fl.alloc(size_t(m_flRing) * m_P * m_T * 8);
 	d_fc.alloc(size_t(m_flRing) * m_P * 8 + 8);
+	if(m_fused && m_masks) d_mk.alloc(size_t(2) * m_P * (m_T / 32u) * 8);
 	d_ctl.alloc(64);
 	if(cycleKernelRuns()) {
 		d_done.alloc((1u + NEMO_CYCLE_GROUPS) * 128u);
@@ -743,6 +775,7 @@ Simulation::Simulation(const NetworkImpl& net, const ConfigurationImpl& conf) :
 	if(d_rcmAcc.bytes) hipCheck(nemo_dev_fill_u32(d_rcmAcc.as<uint32_t>(), 0, d_rcmAcc.bytes / 4, s), "fill");
 	/* tagged fired counts: all-ones never matches a cycle's tag */
 	if(d_fc.bytes) hipCheck(nemo_dev_fill_u64(d_fc.as<uint64_t>(), ~0ull, d_fc.bytes / 8, s), "fill");
+	if(d_mk.bytes) hipCheck(nemo_dev_fill_u64(d_mk.as<uint64_t>(), ~0ull, d_mk.bytes / 8, s), "fill");
 	/* fired-list entries are tagged with their cycle: no entry is valid yet */
 	if(d_fl.bytes) hipCheck(nemo_dev_fill_u64(d_fl.as<uint64_t>(), ~0ull, d_fl.bytes / 8, s), "fill");
 	hipCheck(nemo_dev_fill_u32(d_ctl.as<uint32_t>(), 0, 16, s), "fill");
@@ -1170,10 +1203,12 @@ Simulation::descriptor(unsigned nsteps) const
 	nd.words = m_words;
 	nd.flags = (m_stdp ? NEMO_NET_STDP : 0u) | (m_saturate ? NEMO_NET_SATURATE : 0u)
 		| (m_replay ? NEMO_NET_REPLAY : 0u) | (m_defer ? NEMO_NET_DEFER : 0u)
-		| (m_izOnly ? NEMO_NET_IZHIKEVICH_ONLY : 0u) | (m_prefRing ? NEMO_NET_PREF_RING : 0u);
+		| (m_izOnly ? NEMO_NET_IZHIKEVICH_ONLY : 0u) | (m_prefRing ? NEMO_NET_PREF_RING : 0u)
+		| (m_masks ? NEMO_NET_MASKS : 0u);
 	nd.nsteps = nsteps;
 	nd.spinLimit = m_spinLimit;
 	nd.glog2 = m_glog2;
+	nd.glogFew = m_glogFew;
 	nd.flRing = m_flRing;
 	nd.stdpCache = m_stdpCache;
 	nd.exWaves = m_exWaves;
@@ -1189,6 +1224,7 @@ Simulation::descriptor(unsigned nsteps) const
 	nd.syn = d_syn.as<uint32_t>();
 	nd.fl = d_fl.as<uint64_t>();
 	nd.fc = d_fc.as<uint64_t>();
+	nd.mk = d_mk.as<uint64_t>();
 	nd.rfg = d_rfg.as<uint64_t>();
 	nd.status = d_ctl.as<uint32_t>() + 1;
 	nd.events = reinterpret_cast<unsigned long long*>(d_ctl.as<uint32_t>() + 2);

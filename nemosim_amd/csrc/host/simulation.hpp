@@ -130,8 +130,8 @@ class Simulation
 		void setControlBase(const uint32_t ctl[8]);
 		unsigned neuronCount() const { return m_n; }
 		int device() const { return m_device; }
-		/* step-kernel variant (nemo_step_variant): saturating, Izhikevich-only */
-		uint32_t variant() const { return (m_saturate ? 1u : 0u) | (m_izOnly ? 2u : 0u); }
+		/* step-kernel variant (nemo_step_variant): saturating, Izhikevich-only, masks */
+		uint32_t variant() const { return (m_saturate ? 1u : 0u) | (m_izOnly ? 2u : 0u) | (m_masks ? 4u : 0u); }
 		/* true: the fused persistent kernel; false: plugin kernels per cycle */
 		bool fused() const { return m_fused; }
 
@@ -180,7 +180,7 @@ class Simulation
 		 * 0.1-0.2 us each, so seconds -- a safety net against workgroups
 		 * that never run, not a bound any legitimate wait approaches */
 		uint32_t m_spinLimit = 1u << 26;
-		uint32_t m_glog2 = 0;
+		uint32_t m_glog2 = 0, m_glogFew = 0;
 		/* fused step delivers delay >= 2 records one cycle late (NEMO_NET_DEFER) */
 		bool m_defer = false;
 		/* cycles of fired lists and counts kept on the device */
@@ -192,6 +192,8 @@ class Simulation
 		uint32_t m_ldsNoFar = 0;     /* m_lds without the far list */
 		uint32_t m_farCap = 0;       /* far-list capacity in sources (NetDev.farCap) */
 		void planExchange(const ConfigurationImpl& conf, uint32_t ldsLimit);
+		bool m_masks = false;          /* fired bits exchanged as words (NEMO_NET_MASKS) */
+		DevBuf d_mk;
 		/* every neuron is an Izhikevich neuron (NEMO_NET_IZHIKEVICH_ONLY) */
 		bool m_izOnly = false;
 
