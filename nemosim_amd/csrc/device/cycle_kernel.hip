@@ -24,6 +24,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "host_report.h"
 #include "models.h"
 #include "step_abi.h"
 
@@ -44,37 +45,13 @@ __host__ __device__ inline uint32_t neurons_per_block(uint32_t neurons)
 	return neurons <= SMALL ? 64u : BLOCK;
 }
 
-/* Stores to the caller's host memory: written through, so that s_waitcnt waits
- * until they are there */
-template<typename V>
-__device__ inline void st_host(V* p, V v)
+/* the end of the launch, and the report */
+__device__ inline void finish_cycle(const CycleArgs& ca)
 {
-	__hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-}
-
-/* Counts the workgroup as finished, once its stores have landed; the last one
- * of the launch reports to the host. Two levels of counters, each in a line of
- * its own: one shared by hundreds of workgroups takes 10 ns for each. They
- * return to zero for the next launch. Called by whole workgroups. */
-__device__ inline void finish_block(const CycleArgs& ca, uint32_t blocks)
-{
-	__builtin_amdgcn_s_waitcnt(0);
-	__syncthreads();
-	if(threadIdx.x == 0) {
-		const uint32_t groups = min(blocks, NEMO_CYCLE_GROUPS);
-		const uint32_t g = blockIdx.x % groups;
-		const uint32_t mine = (blocks - g + groups - 1u) / groups;
-		uint32_t* c = ca.done + 32u * (g + 1u);
-		if(atomicAdd(c, 1u) + 1u == mine) {
-			*c = 0u;
-			__builtin_amdgcn_s_waitcnt(0);
-			if(atomicAdd(ca.done, 1u) + 1u == groups) {
-				*ca.done = 0u;
-				st_host(&ca.report->end, (uint64_t) wall_clock64());
-				__builtin_amdgcn_s_waitcnt(0);
-				st_host(&ca.report->sequence, ca.sequence);
-			}
-		}
+	if(last_block(ca.done, blockIdx.x, gridDim.x)) {
+		st_host(&ca.report->end, (uint64_t) wall_clock64());
+		__builtin_amdgcn_s_waitcnt(0);
+		st_host(&ca.report->sequence, ca.sequence);
 	}
 }
 
@@ -176,7 +153,7 @@ __global__ void __launch_bounds__(BLOCK) nemo_cycle_kernel(const NetDev nd, cons
 		total += wfired[w];
 	}
 	if(total == 0u) {   /* block-uniform */
-		if(ca.report) finish_block(ca, gridDim.x);
+		if(ca.report) finish_cycle(ca);
 		return;
 	}
 	if(fired) {
@@ -261,7 +238,7 @@ __global__ void __launch_bounds__(BLOCK) nemo_cycle_kernel(const NetDev nd, cons
 			ca.part[blockIdx.x] += sum;
 		}
 	}
-	if(ca.report) finish_block(ca, gridDim.x);
+	if(ca.report) finish_cycle(ca);
 }
 
 } // namespace

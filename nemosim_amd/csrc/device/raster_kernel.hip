@@ -3,15 +3,18 @@
  * counts per cycle and lists of user indices (the form nemo_step reports,
  * src/nemo/FiringBuffer.cpp, for every cycle of a run).
  *
- * What bounds it: the raster is read once per call (25 MB for 1000 cycles of
- * 200k neurons, ~10 us), the ids leave over PCIe, and the host copies them
- * into the caller's buffer. Decoded on the host, with the whole raster copied
- * back and walked bit by bit, 200k x 1000 cycles took 26.8 ms per
- * nemosim_amd.Simulation.read_fired(), 50k x 1000 6.7 ms.
+ * What bounds it: for long runs the ids, which leave over PCIe and are copied
+ * into the caller's buffer (6 MB for 1000 cycles of 200k neurons at 8 Hz, 0.45
+ * ms; the raster itself, 25 MB, is read in 10 us); for short ones the launches
+ * and the wait. The kernels report to host memory, where the caller polls, and
+ * the second follows the first without the host. Decoded on the host, with the
+ * whole raster copied back and walked bit by bit, 200k x 1000 cycles took 26.8
+ * ms per nemosim_amd.Simulation.read_fired(), 50k x 1000 6.7 ms.
  */
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "host_report.h"
 #include "step_abi.h"
 
 namespace {
@@ -28,23 +31,56 @@ __device__ inline uint64_t fired_word(const uint64_t* row, uint32_t w, uint32_t 
 	return left >= 64u ? b : b & ((1ull << left) - 1ull);
 }
 
-/* one block per cycle: counts[t] = fired neurons of cycle t (host memory) */
+/* One block per cycle: counts[t] = fired neurons of cycle t (host memory).
+ * With offs the last block to finish also writes the exclusive prefix of the
+ * counts there. */
 __global__ void __launch_bounds__(BLOCK) raster_count_kernel(const uint64_t* raster, uint32_t words, uint32_t n,
-		uint32_t* counts)
+		uint32_t* counts, uint32_t* devCounts, uint64_t* offs, DoneReport report)
 {
-	__shared__ uint32_t wsum[WAVES];
+	__shared__ uint64_t wsum[WAVES];
+	__shared__ bool last;
+	const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
 	const uint64_t* row = raster + size_t(blockIdx.x) * words;
 	uint32_t c = 0;
-	for(uint32_t w = threadIdx.x; w < words; w += BLOCK) {
+	for(uint32_t w = tid; w < words; w += BLOCK) {
 		c += uint32_t(__popcll(fired_word(row, w, words, n)));
 	}
 	for(uint32_t d = 32; d >= 1; d >>= 1) c += __shfl_down(c, d, 64);
-	if((threadIdx.x & 63u) == 0u) wsum[threadIdx.x >> 6] = c;
+	if(lane == 0u) wsum[wave] = c;
 	__syncthreads();
-	if(threadIdx.x == 0) {
-		for(uint32_t k = 1; k < WAVES; ++k) c += wsum[k];
-		counts[blockIdx.x] = c;
+	if(tid == 0) {
+		for(uint32_t k = 1; k < WAVES; ++k) c += uint32_t(wsum[k]);
+		st_host(counts + blockIdx.x, c);
+		if(offs) __hip_atomic_store(devCounts + blockIdx.x, c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 	}
+	const bool l = last_block(report.done, blockIdx.x, gridDim.x);
+	if(tid == 0) last = l;
+	__syncthreads();
+	if(!last) return;   /* block-uniform */
+	if(offs) {
+		/* each thread a contiguous share of the cycles */
+		const uint32_t share = (gridDim.x + BLOCK - 1u) / BLOCK;
+		const uint32_t t0 = min(gridDim.x, tid * share), t1 = min(gridDim.x, t0 + share);
+		auto count = [&](uint32_t t) {
+			return __hip_atomic_load(devCounts + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+		};
+		uint64_t mine = 0;
+		for(uint32_t t = t0; t < t1; ++t) mine += count(t);
+		uint64_t x = mine;
+		for(uint32_t d = 1; d < 64u; d <<= 1) {
+			const uint64_t y = __shfl_up((unsigned long long) x, d, 64);
+			if(lane >= d) x += y;
+		}
+		if(lane == 63u) wsum[wave] = x;
+		__syncthreads();
+		x -= mine;
+		for(uint32_t k = 0; k < wave; ++k) x += wsum[k];
+		for(uint32_t t = t0; t < t1; ++t) {
+			offs[t] = x;
+			x += count(t);
+		}
+	}
+	if(tid == 0) st_host(report.seen, report.sequence);
 }
 
 /* One block per cycle. The cycle's ids have positions offs[t], offs[t]+1, ...
@@ -54,7 +90,8 @@ __global__ void __launch_bounds__(BLOCK) raster_count_kernel(const uint64_t* ras
  * written by the lanes that find them they are 4-byte PCIe writes once words
  * hold several bits. */
 __global__ void __launch_bounds__(BLOCK) raster_ids_kernel(const uint64_t* raster, uint32_t words, uint32_t n,
-		const uint64_t* offs, uint64_t lo, uint64_t hi, const uint32_t* ids, uint32_t first, uint32_t* out)
+		const uint64_t* offs, uint64_t lo, uint64_t hi, const uint32_t* ids, uint32_t first, uint32_t* out,
+		DoneReport report)
 {
 	__shared__ uint16_t list[BLOCK * 64u];
 	__shared__ uint32_t wsum[WAVES];
@@ -87,12 +124,20 @@ __global__ void __launch_bounds__(BLOCK) raster_ids_kernel(const uint64_t* raste
 			const uint64_t p = pos + i;
 			if(p >= lo && p < hi) {
 				const uint32_t l = w0 * 64u + list[i];
-				out[p - lo] = ids ? ids[l] : first + l;
+				st_host(out + (p - lo), ids ? ids[l] : first + l);
 			}
 		}
 		__syncthreads();   /* the list and the sums are written again by the next pass */
 		pos += total;
 	}
+	report_done(report, blockIdx.x, gridDim.x);
+}
+
+__global__ void peek_kernel(const uint32_t* src, uint32_t* out, DoneReport report)
+{
+	st_host(out, *src);
+	__builtin_amdgcn_s_waitcnt(0);
+	st_host(report.seen, report.sequence);
 }
 
 } // namespace
@@ -100,20 +145,25 @@ __global__ void __launch_bounds__(BLOCK) raster_ids_kernel(const uint64_t* raste
 extern "C" {
 
 int nemo_dev_raster_count(const uint64_t* raster, uint32_t words, uint32_t n, uint32_t cycles, uint32_t* counts,
-		void* stream)
+		uint32_t* devCounts, uint64_t* offs, const DoneReport* report, void* stream)
 {
-	if(cycles == 0) return 0;
 	hipLaunchKernelGGL(raster_count_kernel, dim3(cycles), dim3(BLOCK), 0, static_cast<hipStream_t>(stream),
-			raster, words, n, counts);
+			raster, words, n, counts, devCounts, offs, *report);
 	return int(hipGetLastError());
 }
 
 int nemo_dev_raster_ids(const uint64_t* raster, uint32_t words, uint32_t n, uint32_t cycles, const uint64_t* offs,
-		uint64_t lo, uint64_t hi, const uint32_t* ids, uint32_t first, uint32_t* out, void* stream)
+		uint64_t lo, uint64_t hi, const uint32_t* ids, uint32_t first, uint32_t* out, const DoneReport* report,
+		void* stream)
 {
-	if(cycles == 0 || lo >= hi) return 0;
 	hipLaunchKernelGGL(raster_ids_kernel, dim3(cycles), dim3(BLOCK), 0, static_cast<hipStream_t>(stream),
-			raster, words, n, offs, lo, hi, ids, first, out);
+			raster, words, n, offs, lo, hi, ids, first, out, *report);
+	return int(hipGetLastError());
+}
+
+int nemo_dev_peek(const uint32_t* src, uint32_t* out, const DoneReport* report, void* stream)
+{
+	hipLaunchKernelGGL(peek_kernel, dim3(1), dim3(1), 0, static_cast<hipStream_t>(stream), src, out, *report);
 	return int(hipGetLastError());
 }
 

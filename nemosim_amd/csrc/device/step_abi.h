@@ -109,7 +109,7 @@ typedef struct NetDev {
 /* One cycle by cycle_kernel.hip: its place in the launch and its stimulus,
  * where the launch's descriptor holds no schedule (one current per neuron). */
 #define NEMO_CYCLE_STIM 64u
-#define NEMO_CYCLE_GROUPS 16u   /* first-level counters of finished workgroups */
+#define NEMO_DONE_GROUPS 16u   /* first-level counters of finished workgroups */
 
 /* what the last workgroup of a launch writes to host memory: the device wall
  * clock at its start and end, then the launch's number */
@@ -126,7 +126,7 @@ typedef struct CycleArgs {
 	unsigned long long* part; /* [nemo_dev_cycle_blocks] delivered synapses by workgroup; NULL: not counted */
 	CycleReport* report;      /* host memory; NULL: none */
 	uint64_t sequence;
-	uint32_t* done;           /* [1 + NEMO_CYCLE_GROUPS][32] counters, zero between launches (with report) */
+	uint32_t* done;           /* [1 + NEMO_DONE_GROUPS][32] counters, zero between launches (with report) */
 	uint32_t fidx[NEMO_CYCLE_STIM];
 	uint32_t iidx[NEMO_CYCLE_STIM];
 	float ival[NEMO_CYCLE_STIM];
@@ -183,16 +183,29 @@ int nemo_dev_apply_stdp(uint32_t* syn, const uint32_t* rcm_fwd, int32_t* rcm_acc
 		const void* stdp_dev, int32_t fx_reward, void* stream);
 int nemo_dev_fill_u32(uint32_t* p, uint32_t value, size_t n, void* stream);
 int nemo_dev_fill_u64(uint64_t* p, uint64_t value, size_t n, void* stream);
+/* Where a kernel says that it is done: its last workgroup writes `sequence`
+ * to *seen in host memory, which the caller polls. done: counters of finished
+ * workgroups, zero between launches. */
+typedef struct DoneReport {
+	uint64_t* seen;
+	uint64_t sequence;
+	uint32_t* done;           /* [1 + NEMO_DONE_GROUPS][32] */
+} DoneReport;
+
 /* The raster of a run (rows of `words` 64-bit words, one per cycle) as fired
- * counts and ids (csrc/device/raster_kernel.hip). counts, offs and out are
- * host memory the device can reach (pinned). The ids of cycle t take the
- * positions offs[t], offs[t]+1, ... of the run's list; those in [lo, hi) are
- * written to out[position - lo], as ids[local index], or first + local index
- * where ids is NULL. */
+ * counts and ids (csrc/device/raster_kernel.hip). counts and out are host
+ * memory the device can reach (pinned), offs is device memory: its first call
+ * writes counts[t] and, with offs, the positions offs[t] of the cycles' ids in
+ * the run's list. The second writes the ids with positions in [lo, hi) to
+ * out[position - lo], as ids[local index], or first + local index where ids is
+ * NULL. Both report. */
 int nemo_dev_raster_count(const uint64_t* raster, uint32_t words, uint32_t n, uint32_t cycles, uint32_t* counts,
-		void* stream);
+		uint32_t* devCounts, uint64_t* offs, const DoneReport* report, void* stream);
 int nemo_dev_raster_ids(const uint64_t* raster, uint32_t words, uint32_t n, uint32_t cycles, const uint64_t* offs,
-		uint64_t lo, uint64_t hi, const uint32_t* ids, uint32_t first, uint32_t* out, void* stream);
+		uint64_t lo, uint64_t hi, const uint32_t* ids, uint32_t first, uint32_t* out, const DoneReport* report,
+		void* stream);
+/* *out (host memory) = the 4-byte word at src, then the report */
+int nemo_dev_peek(const uint32_t* src, uint32_t* out, const DoneReport* report, void* stream);
 /* Evaluates the device math pieces on inputs in[] (for tests):
  * kind 0 = logf_glibc(in), 1 = sinf_rng(in), 2 = kuramoto_wrap(in), 3 = sinf_glibc(in) */
 int nemo_dev_eval_libm(int kind, const float* in_dev, float* out_dev, size_t n, void* stream);

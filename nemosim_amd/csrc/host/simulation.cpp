@@ -750,7 +750,7 @@ Simulation::Simulation(const NetworkImpl& net, const ConfigurationImpl& conf) :
 	if(m_fused && m_masks) d_mk.alloc(size_t(2) * m_P * (m_T / 32u) * 8);
 	d_ctl.alloc(64);
 	if(cycleKernelRuns()) {
-		d_done.alloc((1u + NEMO_CYCLE_GROUPS) * 128u);
+		d_done.alloc((1u + NEMO_DONE_GROUPS) * 128u);
 		hipCheck(nemo_dev_fill_u32(d_done.as<uint32_t>(), 0, d_done.bytes / 4, static_cast<hipStream_t>(m_stream)), "fill");
 	}
 	if(m_stdp) {
@@ -1540,6 +1540,21 @@ Simulation::decodeStep(const uint64_t* words, std::vector<unsigned>& out) const
 	}
 }
 
+/* Waits until a kernel's own report is there; if it does not come, the
+ * synchronisation says why. */
+static void
+waitReport(const volatile uint64_t* seen, uint64_t sequence, hipStream_t st, const char* what)
+{
+	const auto patience = std::chrono::steady_clock::now() + std::chrono::milliseconds(100);
+	for(unsigned polls = 0; *seen != sequence; ++polls) {
+		if((polls & 1023u) == 1023u && std::chrono::steady_clock::now() > patience) {
+			hipCheck(hipStreamSynchronize(st), "hipStreamSynchronize");
+			if(*seen != sequence) throw exception(NEMO_CUDA_ERROR, fmt(what, ": ended without its report"));
+		}
+	}
+	std::atomic_thread_fence(std::memory_order_acquire);
+}
+
 /* the device wall clock's rate (wall_clock64 in the kernels), kHz */
 double
 wallClockKHz(int dev)
@@ -1595,22 +1610,12 @@ Simulation::stepCycle(const nemo_schedule_t& s)
 	ca.slot = uint32_t(m_cycle % (m_D + 1));
 	ca.hostRow = h_step;
 	CycleReport* rep = reinterpret_cast<CycleReport*>(h_ctl + NEMO_CTL_WORDS);
-	volatile uint64_t* seen = &rep->sequence;
 	ca.report = rep;
 	ca.sequence = ++m_cycleSequence;
 	ca.done = d_done.as<uint32_t>();
 	hipStream_t st = static_cast<hipStream_t>(m_stream);
 	hipCheck(nemo_dev_cycle(&nd, &ca, st), "cycle kernel launch");
-	/* the kernel's own report, which its last workgroup writes; if it does not
-	 * come, the synchronisation says why */
-	const auto patience = std::chrono::steady_clock::now() + std::chrono::milliseconds(100);
-	for(unsigned polls = 0; *seen != ca.sequence; ++polls) {
-		if((polls & 1023u) == 1023u && std::chrono::steady_clock::now() > patience) {
-			hipCheck(hipStreamSynchronize(st), "hipStreamSynchronize");
-			if(*seen != ca.sequence) throw exception(NEMO_CUDA_ERROR, "the cycle kernel ended without its report");
-		}
-	}
-	std::atomic_thread_fence(std::memory_order_acquire);
+	waitReport(&rep->sequence, ca.sequence, st, "cycle kernel");
 	m_kernelMs = float(double(rep->end - rep->start) / wallClockKHz(m_device));
 	const uint32_t ctl[8] = {};
 	completeLaunch(1, ctl);
@@ -1662,67 +1667,72 @@ Simulation::run(unsigned nsteps, const nemo_schedule_t* schedule, unsigned long 
 	launch(nsteps, events);
 }
 
-/* Pinned staging of readFired, one block for the process: it is used only
- * while the device lock is held, and never freed, so no HIP call runs at
- * process exit. Counts and list positions of READ_CYCLES cycles at a time,
- * and two windows of ids, so that the device fills one while the host copies
- * the other into the caller's buffer. */
+/* Staging of the results that kernels write to host memory (readFired,
+ * readScalar), one per device: it is used only while the device lock is held,
+ * and never freed, so no HIP call runs at process exit. Counts and list
+ * positions of READ_CYCLES cycles at a time, and two windows of ids, so that
+ * the device fills one while the host copies the other into the caller's
+ * buffer. */
 namespace {
 const size_t READ_CYCLES = 16384;
 const size_t READ_WINDOW = size_t(1) << 18;   /* ids: 1 MB */
 
 struct ReadStaging {
-	uint64_t offs[READ_CYCLES];
-	uint32_t counts[READ_CYCLES];
-	uint32_t ids[2][READ_WINDOW];
+	struct Host {
+		uint64_t seen;
+		uint32_t word;
+		uint32_t counts[READ_CYCLES];
+		uint32_t ids[2][READ_WINDOW];
+	};
+	struct Device {
+		uint32_t done[1 + NEMO_DONE_GROUPS][32];
+		uint64_t offs[READ_CYCLES];
+		uint32_t counts[READ_CYCLES];
+	};
+	Host* host = nullptr;
+	Device* dev = nullptr;
+	uint64_t sequence = 0;
+
+	DoneReport next()
+	{
+		return DoneReport{&host->seen, ++sequence, dev->done[0]};
+	}
 };
 
-ReadStaging*
-readStaging()
+ReadStaging&
+readStaging(int dev)
 {
-	static ReadStaging* st = nullptr;
-	if(!st) {
-		void* p = nullptr;
-		hipCheck(hipHostMalloc(&p, sizeof(ReadStaging), hipHostMallocPortable), "hipHostMalloc");
-		st = static_cast<ReadStaging*>(p);
+	static ReadStaging* all = new ReadStaging[64];
+	if(dev < 0 || dev >= 64) throw exception(NEMO_INVALID_INPUT, "device index out of range");
+	ReadStaging& rs = all[dev];
+	if(!rs.dev) {
+		void* h = nullptr;
+		void* d = nullptr;
+		hipCheck(hipHostMalloc(&h, sizeof(ReadStaging::Host)), "hipHostMalloc");
+		rs.host = static_cast<ReadStaging::Host*>(h);
+		rs.host->seen = 0;
+		hipCheck(hipMalloc(&d, sizeof(ReadStaging::Device)), "hipMalloc");
+		hipCheck(hipMemset(d, 0, sizeof(ReadStaging::Device)), "hipMemset");
+		rs.dev = static_cast<ReadStaging::Device*>(d);
 	}
-	return st;
+	return rs;
 }
 } // namespace
 
-/* Rasters of up to 96 KB are copied and decoded here (62 KB: 35 us for the
- * count and the list, 47 us by the kernels, whose launches and waits cost
- * that much whatever the size; 125 KB: 50 us either way), larger ones by the
- * kernels of csrc/device/raster_kernel.hip (250 KB: 73 us here, 48 us there;
- * 25 MB: 26.8 against 0.5 ms). An ids buffer that is too small receives the
- * cycles that fit in whole, and counts those and the one that did not. */
-static const size_t READ_HOST_WORDS = 96u * 1024u / 8u;
-
+/* By the kernels of csrc/device/raster_kernel.hip for any size: 18 us for the
+ * smallest raster, 26 for 1 MB. Small ones (up to 96 KB) copied back and
+ * decoded here took 16 to 23 us for a simulation that is read again and again,
+ * but 51 where one after the other is read (the networks of a batch: 23 by the
+ * kernels). An ids buffer that is too small receives the cycles that fit in
+ * whole, and counts those and the one that did not. */
 void
 Simulation::readFired(unsigned counts[], unsigned ids[], size_t cap, size_t* total)
 {
 	std::lock_guard<DeviceMutex> devLock(deviceMutex());
 	requireOwnRaster();
-	const size_t nw = size_t(m_lastRunSteps) * m_words;
-	if(nw <= READ_HOST_WORDS || m_n == 0) {
-		m_rasterHost.resize(nw);
-		if(nw) {
-			hipCheck(hipMemcpy(m_rasterHost.data(), d_raster.ptr, nw * 8, hipMemcpyDeviceToHost), "D2H");
-		}
-		size_t k = 0;
-		std::vector<unsigned> one;
-		for(unsigned t = 0; t < m_lastRunSteps; ++t) {
-			decodeStep(m_rasterHost.data() + size_t(t) * m_words, one);
-			if(counts) counts[t] = unsigned(one.size());
-			if(ids) {
-				if(k + one.size() > cap) {
-					throw exception(NEMO_BUFFER_OVERFLOW, "fired-id buffer too small");
-				}
-				std::copy(one.begin(), one.end(), ids + k);
-			}
-			k += one.size();
-		}
-		if(total) *total = k;
+	if(m_n == 0) {
+		if(counts) std::fill(counts, counts + m_lastRunSteps, 0u);
+		if(total) *total = 0;
 		return;
 	}
 	hipStream_t st = static_cast<hipStream_t>(m_stream);
@@ -1730,42 +1740,55 @@ Simulation::readFired(unsigned counts[], unsigned ids[], size_t cap, size_t* tot
 	if(ids && !m_affineIds && !d_ids.ptr) {
 		d_ids.upload(m_localToGlobal.data(), size_t(m_n) * 4);
 	}
-	ReadStaging* rs = readStaging();
+	ReadStaging& rs = readStaging(m_device);
 	const uint64_t* raster = d_raster.as<uint64_t>();
+	std::vector<uint64_t> offs;
 	size_t done = 0;   /* ids of the earlier cycles */
 	for(size_t t0 = 0; t0 < m_lastRunSteps; t0 += READ_CYCLES) {
 		const size_t nt = std::min<size_t>(READ_CYCLES, m_lastRunSteps - t0);
 		const uint64_t* rows = raster + t0 * m_words;
-		hipCheck(nemo_dev_raster_count(rows, m_words, m_n, uint32_t(nt), rs->counts, st), "raster counts");
-		hipCheck(hipStreamSynchronize(st), "hipStreamSynchronize");
+		/* the ids of positions [lo, lo + window) of these cycles; a launch
+		 * covers the cycles that may have some */
+		DoneReport last;
+		auto list = [&](size_t c0, size_t c1, uint64_t lo, uint64_t hi) {
+			last = rs.next();
+			hipCheck(nemo_dev_raster_ids(rows + c0 * m_words, m_words, m_n, uint32_t(c1 - c0), rs.dev->offs + c0, lo, hi,
+						m_affineIds ? nullptr : d_ids.as<uint32_t>(), m_minG, rs.host->ids[(lo / READ_WINDOW) & 1u], &last,
+						st), "raster ids");
+		};
+		last = rs.next();
+		hipCheck(nemo_dev_raster_count(rows, m_words, m_n, uint32_t(nt), rs.host->counts, rs.dev->counts,
+					ids ? rs.dev->offs : nullptr, &last, st), "raster counts");
+		if(ids) list(0, nt, 0, READ_WINDOW);
+		waitReport(&rs.host->seen, last.sequence, st, "raster kernels");
 		uint64_t here = 0;
 		size_t fit = 0;   /* cycles whose ids fit */
 		bool over = false;
-		for(; fit < nt && !over; ++fit) {
-			if(counts) counts[t0 + fit] = rs->counts[fit];
-			if(ids && done + here + rs->counts[fit] > cap) {
+		offs.resize(nt);
+		for(; fit < nt; ++fit) {
+			const uint32_t c = rs.host->counts[fit];
+			if(counts) counts[t0 + fit] = c;
+			if(ids && done + here + c > cap) {
 				over = true;
 				break;
 			}
-			rs->offs[fit] = here;
-			here += rs->counts[fit];
+			offs[fit] = here;
+			here += c;
 		}
-		if(ids && here > 0) {
-			/* window by window; a window's launch covers the cycles with ids in it */
-			auto list = [&](uint64_t lo) {
-				const uint64_t hi = std::min<uint64_t>(here, lo + READ_WINDOW);
-				const size_t c0 = size_t(std::upper_bound(rs->offs, rs->offs + fit, lo) - rs->offs) - 1;
-				const size_t c1 = size_t(std::lower_bound(rs->offs, rs->offs + fit, hi) - rs->offs);
-				hipCheck(nemo_dev_raster_ids(rows + c0 * m_words, m_words, m_n, uint32_t(c1 - c0), rs->offs + c0, lo, hi,
-							m_affineIds ? nullptr : d_ids.as<uint32_t>(), m_minG, rs->ids[(lo / READ_WINDOW) & 1u], st),
-						"raster ids");
-			};
-			list(0);
+		if(ids) {
 			for(uint64_t lo = 0; lo < here; lo += READ_WINDOW) {
-				hipCheck(hipStreamSynchronize(st), "hipStreamSynchronize");
-				if(lo + READ_WINDOW < here) list(lo + READ_WINDOW);
-				std::memcpy(ids + done + lo, rs->ids[(lo / READ_WINDOW) & 1u],
+				/* this window has been waited for; the next one is listed
+				 * while it is copied */
+				const uint64_t next = lo + READ_WINDOW;
+				if(next < here) {
+					const uint64_t hi = std::min<uint64_t>(here, next + READ_WINDOW);
+					const auto end = offs.begin() + long(fit);
+					list(size_t(std::upper_bound(offs.begin(), end, next) - offs.begin()) - 1,
+							size_t(std::lower_bound(offs.begin(), end, hi) - offs.begin()), next, hi);
+				}
+				std::memcpy(ids + done + lo, rs.host->ids[(lo / READ_WINDOW) & 1u],
 						size_t(std::min<uint64_t>(here - lo, READ_WINDOW)) * 4);
+				if(next < here) waitReport(&rs.host->seen, last.sequence, st, "raster kernels");
 			}
 		}
 		done += size_t(here);
@@ -1857,12 +1880,20 @@ Simulation::applyStdpFinish()
 	m_replay = true;
 }
 
+/* A 4-byte word of device memory, by a kernel that writes it to host memory
+ * (7 us with the call; a synchronous copy takes 13). */
 void
-Simulation::readScalar(const DevBuf& b, size_t offset, void* out, size_t bytes) const
+Simulation::readScalar(const DevBuf& b, size_t offset, void* out) const
 {
 	std::lock_guard<DeviceMutex> devLock(deviceMutex());
 	hipCheck(hipSetDevice(m_device), "hipSetDevice");
-	hipCheck(hipMemcpy(out, static_cast<const char*>(b.ptr) + offset, bytes, hipMemcpyDeviceToHost), "D2H");
+	ReadStaging& rs = readStaging(m_device);
+	const DoneReport report = rs.next();
+	hipStream_t st = static_cast<hipStream_t>(m_stream);
+	hipCheck(nemo_dev_peek(reinterpret_cast<const uint32_t*>(static_cast<const char*>(b.ptr) + offset), &rs.host->word,
+				&report, st), "peek kernel");
+	waitReport(&rs.host->seen, report.sequence, st, "peek kernel");
+	std::memcpy(out, &rs.host->word, 4);
 }
 
 void
@@ -1881,7 +1912,7 @@ Simulation::getNeuronState(unsigned g, unsigned var) const
 		throw exception(NEMO_INVALID_INPUT, fmt("Invalid state variable index ", var));
 	}
 	float v;
-	readScalar(d_state, stateOffset(l, var) * 4, &v, 4);
+	readScalar(d_state, stateOffset(l, var) * 4, &v);
 	return v;
 }
 
@@ -1902,7 +1933,7 @@ Simulation::getNeuronParameter(unsigned g, unsigned param) const
 		throw exception(NEMO_INVALID_INPUT, fmt("Invalid parameter index ", param));
 	}
 	float v;
-	readScalar(d_param, (size_t(param) * m_n + l) * 4, &v, 4);
+	readScalar(d_param, (size_t(param) * m_n + l) * 4, &v);
 	return v;
 }
 
@@ -1996,7 +2027,7 @@ Simulation::getSynapseWeight(synapse_id id) const
 {
 	size_t q = synapseRecord(id);
 	int32_t w;
-	readScalar(d_syn, (size_t(m_qFwd[q]) * 2 + 1) * 4, &w, 4);
+	readScalar(d_syn, (size_t(m_qFwd[q]) * 2 + 1) * 4, &w);
 	return fx_toFloat(w);
 }
 

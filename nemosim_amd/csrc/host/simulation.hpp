@@ -278,7 +278,7 @@ class Simulation
 		unsigned localIdx(unsigned g) const;
 		void uploadSchedule(unsigned nsteps, const nemo_schedule_t* s);
 		void launch(unsigned nsteps, unsigned long long* events);
-		void readScalar(const DevBuf& b, size_t offset, void* out, size_t bytes) const;
+		void readScalar(const DevBuf& b, size_t offset, void* out) const;
 		void writeScalar(DevBuf& b, size_t offset, const void* in, size_t bytes);
 		void decodeStep(const uint64_t* words, std::vector<unsigned>& out) const;
 		size_t synapseRecord(synapse_id id) const;

@@ -1,8 +1,8 @@
 """nemo_hip_read_fired counts and lists the spikes of a run on the device
 (csrc/device/raster_kernel.hip). Checked against the raw raster decoded here,
-at the edges of the rule that leaves small rasters to the host (96 KB), of its
-passes (16384 neurons), of its windows of 2^18 ids and of its groups of 16384
-cycles, with contiguous and scattered user indices."""
+at one cycle, at the edges of its passes (16384 neurons), of its windows of 2^18
+ids and of its groups of 16384 cycles, in one call and in two (from 2^22 bits),
+with contiguous and scattered user indices."""
 import ctypes
 
 import numpy as np
@@ -29,13 +29,16 @@ def decoded(sim, idx):
 
 
 @pytest.mark.parametrize("n,first,step,cycles,rate", [
-    (63, 5, 1, 4, 0.5),           # decoded on the host: up to 12288 words
+    (63, 5, 1, 4, 0.5),
+    (64, 2, 1, 1, 0.5),
     (64, 0, 3, 12288, 0.02),
-    (65, 0, 3, 6145, 0.02),       # two words, one over
+    (65, 0, 3, 6145, 0.02),       # two words
     (16384, 0, 1, 49, 0.01),      # one pass per cycle
     (16385, 7, 1, 60, 1.0),       # one id past a pass; 655k ids: three windows
     (20001, 3, 2, 50, 1.0),       # scattered ids over three windows
     (70, 0, 1, 16390, 0.02),      # two groups of cycles
+    (64, 0, 3, 65536, 0.05),      # the most that one call reads, in four groups
+    (65, 0, 3, 32769, 0.05),      # two calls
 ])
 def test_read_fired_equals_raster(n, first, step, cycles, rate):
     rng = np.random.default_rng(n)
@@ -53,7 +56,7 @@ def test_read_fired_equals_raster(n, first, step, cycles, rate):
 @pytest.mark.parametrize("quiet", [0, 6200])
 def test_read_fired_small_buffer(quiet):
     """a buffer that ends inside a cycle receives the cycles before it (with
-    6200 quiet cycles after them, listed by the device)"""
+    6200 quiet cycles after them, too)"""
     idx = np.arange(100, dtype=np.uint32)
     sim = forced_network(idx)
     sim.run(3 + quiet, fstim=[idx[:10], idx[20:50], idx] + [[]] * quiet)
