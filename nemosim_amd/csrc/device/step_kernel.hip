@@ -525,30 +525,8 @@ __device__ __forceinline__ void run_partition(const NetDev& nd, uint32_t p)
 		}
 	}
 	if(replay) {
-		/* Weights changed (applyStdp) since the ring was filled. NeMo reads a
-		 * weight when the spike arrives (src/nemo/cpu/Simulation.cpp:258-307),
-		 * so rebuild the ring from the firing history: every spike fired at
-		 * cycle0-1-k whose synapse delay d > k has not arrived yet and lands
-		 * in slot (cycle0-1-k+d) mod D, with the current weight. */
 		__syncthreads();
-		const uint64_t pend = (D >= 64u) ? ~0ull : ((1ull << D) - 1ull);
-		const uint32_t last = uint32_t((nd.cycle0 + D - 1u) % D);    /* slot of cycle0-1 */
-		for(uint32_t s = tid; s < n_total; s += nthreads) {
-			const uint64_t h = glb(nd.recent)[s] & pend;
-			if(!h) continue;
-			const NEMO_GLOBAL uint32_t* o = off + size_t(s) * (P + 1u) + p;
-			const uint32_t a = o[0] & offMask, b = o[1] & offMask;
-			for(uint32_t q = a; q < b; ++q) {
-				const uint2 rec = syn[q];
-				const uint32_t d = rec.x >> 16;
-				uint64_t hb = h & ((d >= 64u) ? ~0ull : ((1ull << d) - 1ull));
-				while(hb) {
-					const uint32_t kk = uint32_t(__builtin_ctzll(hb));
-					hb &= hb - 1ull;
-					ring_add<SAT>(ringE, ringI, ovf, D, T, fwords, (last + d - kk) % D, rec.x & 0xffffu, int32_t(rec.y));
-				}
-			}
-		}
+		ring_replay<SAT>(nd, p, syn, off, offMask, ringE, ringI, ovf, fwords, wave, nwaves, lane);
 	}
 
 	/* neuron registers */
