@@ -74,8 +74,9 @@ nemo_status_t nemo_set_device_construction(nemo_configuration_t conf, int enable
  * work lists and accumulate): n > 0 = n waves (at least one other must
  * remain; needs deferred delivery and LDS room for the far list), < 0 =
  * none (every wave does both, one after the other), 0 (default) =
- * automatic: 3 of every 8 waves for networks with STDP and at least 8
- * waves (512 neurons) per workgroup, none otherwise. Same results either
+ * automatic: 3 of every 8 waves for networks with STDP whose workgroups
+ * nemo_set_partition_size makes 8 waves (512 neurons) or more, and for those
+ * that need more than 10 waves; none otherwise. Same results either
  * way. No counterpart in NeMo; a tuning knob of the fused step kernel. */
 nemo_status_t nemo_set_exchange_waves(nemo_configuration_t conf, int waves);
 
@@ -194,7 +195,7 @@ typedef struct nemo_hip_info {
 	unsigned deferred;           /* 1: records of delay >= 2 delivered one cycle late */
 	unsigned lanes_per_source;   /* lanes sharing one fired source in delivery */
 	unsigned stdp_staged_chunks; /* STDP chunks whose reverse records are staged in LDS per cycle */
-	unsigned stdp_prefix_ring;   /* 1: fired-count prefixes of the last postLen cycles kept in LDS */
+	unsigned stdp_prefix_ring;   /* 1: STDP work lists need no fired counts of earlier cycles from memory */
 	unsigned device_built;       /* 1: synapse structures were built on the device */
 	unsigned exchange_waves;     /* waves per workgroup running the exchange and delay-1 delivery */
 	unsigned far_list_sources;   /* fired sources per cycle whose far records wait in the LDS far list */

@@ -1,6 +1,6 @@
 /*
- * mask_kernel.hip -- the persistent step of networks without STDP: the fused
- * kernel of step_kernel.hip with another exchange between partitions.
+ * mask_kernel.hip -- the persistent step: the fused kernel of step_kernel.hip
+ * with another exchange between partitions, and with STDP on waves of its own.
  *
  * There, a partition publishes a list of its fired neurons and a count, and
  * the others read the counts, then the entries, then each source's bucket
@@ -19,9 +19,10 @@
  * same build: 1k x 100 5.2 -> 3.9 us (with stimulus), 10k x 313 5.6 -> 4.4,
  * 60k x 300 6.3 -> 5.3, 100k x 100 (20 cycles) 9.1 -> 7.5, 200k x 1000 13.8 ->
  * 12.2, 12k x 550 IF_curr_exp_noise at 333 Hz 57 -> 48; 48 networks of 1k-20k
- * batched, 200 cycles, 3.96 -> 3.04 ms.
+ * batched, 200 cycles, 3.96 -> 3.04 ms. With STDP, 3k x 300 10.9 -> 3.6 us, 10k
+ * x 300 10.5 -> 4.2, 50k x 1000 17.4 -> 11.9 (see stdp_waves).
  *
- * Two buffers of words are enough: a wave publishes cycle t+1 after its own
+ * Without STDP two buffers of words are enough: a wave publishes cycle t+1 after its own
  * reads of cycle t, and a workgroup publishes t+2 only once its waves have
  * seen every word of t+1.
  */
@@ -33,12 +34,245 @@ namespace {
 
 constexpr uint32_t LIST = 128u;      /* sources a wave lists in LDS at a time (16 bits: from its first word on) */
 
+constexpr uint32_t CHUNK = 64u;      /* synapses per STDP work item (one per lane of a wave) */
+
+/* The neurons that fired in an earlier cycle, whose words are complete, of the
+ * words [w0, w1): f(valid, neuron) for whole waves. */
+template<uint32_t WORDS, typename F>
+__device__ inline void each_fired(const NEMO_GLOBAL uint64_t* words, uint32_t tag, uint32_t w0, uint32_t w1,
+		uint16_t* list, uint32_t lane, F f)
+{
+	for(uint32_t c0 = w0; c0 < w1; c0 += 64u * WORDS) {   /* wave-uniform */
+		uint32_t v[WORDS], pos[WORDS];
+#pragma unroll
+		for(uint32_t i = 0; i < WORDS; ++i) {
+			const uint32_t w = c0 + 64u * i + lane;
+			const uint64_t e = w < w1 ? ld_agent(words + w) : 0ull;
+			v[i] = w < w1 && uint32_t(e >> 32) == tag ? uint32_t(e) : 0u;
+		}
+		uint32_t total = 0;
+#pragma unroll
+		for(uint32_t i = 0; i < WORDS; ++i) {
+			const uint32_t c = uint32_t(__popc(v[i]));
+			const uint32_t x = wave_scan(c);
+			pos[i] = total + x - c;
+			total += uint32_t(__builtin_amdgcn_readlane(int(x), 63));
+		}
+		for(uint32_t l0 = 0; l0 < total; l0 += LIST) {   /* wave-uniform */
+#pragma unroll
+			for(uint32_t i = 0; i < WORDS; ++i) {
+				uint32_t b = v[i];
+				for(uint32_t at = pos[i]; b; ++at) {
+					if(at - l0 < LIST) list[at - l0] = uint16_t((64u * i + lane) * 32u + uint32_t(__builtin_ctz(b)));
+					b &= b - 1u;
+				}
+			}
+			__builtin_amdgcn_wave_barrier();   /* a wave's LDS operations complete in order */
+			const uint32_t n = min(LIST, total - l0);
+			for(uint32_t h = 0; h < n; h += 64u) {   /* wave-uniform */
+				const bool ok = h + lane < n;
+				f(ok, c0 * 32u + (ok ? list[h + lane] : 0u));
+			}
+			__builtin_amdgcn_wave_barrier();   /* the list is written again */
+		}
+	}
+}
+
+/* stdp_weight_change of models.h without branches, so that the chunks that a
+ * wave has in flight overlap (with them a chunk took about 1000 cycles, most of
+ * them waits for LDS). Per region (potentiation, depression) the closest
+ * arrival before and after the target's firing and their distances; the closer
+ * one's table entry, none if there is none or they are equally close. m: the
+ * regions' masks over h >> postLen and over h << (64 - postLen). h: the
+ * source's firing history as it arrived at the target. */
+struct StdpMasks { uint64_t pre[2], post[2]; };
+
+__device__ inline int32_t stdp_change(const StdpMasks& m, uint32_t postLen, const int32_t* fn, uint64_t h)
+{
+	const uint64_t hp = h >> postLen, hq = h << (64u - postLen);   /* postLen: 1..63 */
+	uint32_t w = 0;
+#pragma unroll
+	for(uint32_t i = 0; i < 2u; ++i) {
+		const uint64_t a = hp & m.pre[i], b = hq & m.post[i];
+		const uint32_t da = a ? uint32_t(__builtin_ctzll(a)) : 64u;
+		const uint32_t db = b ? uint32_t(__builtin_clzll(b)) : 64u;
+		const int32_t v = fn[min(da, 63u) < db ? da : 64u + min(db, 63u)];   /* fnPre, then fnPost */
+		w += da == db ? 0u : uint32_t(v);
+	}
+	return int32_t(w);
+}
+
+/* ---- STDP (src/nemo/ConnectivityMatrix.cpp:193-227), on waves of its own that
+ * have no neurons. The targets of cycle t fired in cycle t-postLen; their rows
+ * of plastic in-synapses are cut into chunks of CHUNK, and chunk c of target x
+ * belongs to partition (x + c) mod P, always: no other workgroup of the launch
+ * adds to it, so its XCD's cache can (shares made equal by the targets'
+ * position in the cycle's list had to add at the memory side, 50k x 1000 19.1
+ * us per cycle against 18.2 then). The chunks are listed in cycle t and
+ * accumulated in cycle t+1: then every word of cycle t has been seen, and
+ * behind a wave's word of cycle t are its neurons' histories up to t-1, stored
+ * a cycle earlier, so no wave waits for its stores. The history without cycle
+ * t's spikes is enough: they arrive a cycle later at the earliest; its oldest
+ * bit would have been shifted out. Histories are kept for 4 cycles: a
+ * partition reads those of t-1 in t+1, when another may be storing t+2's.
+ * Words are kept for postLen+3: if there are more chunks than a list holds it
+ * is left, and each wave accumulates the targets that it finds in its words,
+ * in t+1.
+ *
+ * What bounds it: the histories, 8 bytes each from anywhere (400k a cycle at
+ * 50k x 1000 and 8 Hz, 3.6 us), and the latency of the chain records, history,
+ * table, add. On waves of its own it runs beside the exchange and the delivery:
+ * done by the neurons' waves, where those wait for words, a cycle took 17.3 us
+ * (50k x 1000) and 6.3 (3k x 300) instead of 11.9 and 3.6. */
+struct StdpLds {
+	StdpParams* table;
+	uint2* work;          /* [2][NEMO_MASK_STDP_CAP] {row index, length}, by cycle parity */
+	uint32_t* count;      /* [2] */
+	StdpMasks* masks;
+	uint32_t* records;    /* [2][stdpCache][CHUNK] reverse records of the first chunks */
+};
+
+/* K: chunks of a wave whose loads are in flight together */
+template<bool SAT, uint32_t WORDS, uint32_t K>
+__device__ inline void stdp_waves(const NetDev& nd, uint32_t p, uint32_t wave, uint32_t nwaves, uint32_t lane,
+		const StdpLds& l, uint16_t* list)
+{
+	const uint32_t P = nd.P, R = nd.flRing, n_total = nd.n, cache = nd.stdpCache;
+	const uint32_t postLen = uint32_t(l.table->postLen);
+	const uint32_t W = P * (nd.T >> 5);
+	const uint32_t w0 = W * wave / nwaves, w1 = W * (wave + 1u) / nwaves;
+	const NEMO_GLOBAL uint32_t* rsd = glb(nd.rcm_sd);
+	NEMO_GLOBAL int32_t* racc = glb(nd.rcm_acc);
+	const StdpMasks m = *l.masks;
+	/* the first `count` of K chunks, one synapse per lane: the sources'
+	 * histories, the weight changes, the adds */
+	auto chunks = [&](const NEMO_GLOBAL uint64_t* h, const uint32_t* r, const uint32_t* len, const uint32_t* sd,
+			uint32_t count) {
+		uint64_t hh[K];
+		int32_t wd[K];
+#pragma unroll
+		for(uint32_t i = 0; i < K; ++i) {
+			hh[i] = 0ull;
+			if(i < count) hh[i] = ld_agent(h + (sd[i] & 0x3ffffffu));
+		}
+#pragma unroll
+		for(uint32_t i = 0; i < K; ++i) {
+			wd[i] = stdp_change(m, postLen, l.table->fnPre, (hh[i] & (~0ull >> 1)) >> (sd[i] >> 26));
+		}
+#pragma unroll
+		for(uint32_t i = 0; i < K; ++i) {
+			if(i < count && lane < len[i] && wd[i] != 0) {
+				(void) __hip_atomic_fetch_add(racc + r[i] + lane, wd[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+			}
+		}
+	};
+	/* a lane's target: the bounds of its row, and its first chunk (or a number
+	 * beyond the last) of this partition */
+	struct Row { uint32_t begin, len, ch; };
+	auto row_of = [&](bool ok, uint32_t x) {
+		Row r = {0u, 0u, (p + P - x % P) % P};
+		if(ok) {
+			r.begin = glb(nd.rcm_start)[x];
+			r.len = glb(nd.rcm_start)[x + 1u] - r.begin;
+		}
+		return r;
+	};
+	/* the list of cycle tc, whose words are in slot tslot */
+	auto accumulate = [&](uint32_t tc, uint32_t tslot) {
+		const uint32_t par = tc & 1u, total = l.count[par];
+		const NEMO_GLOBAL uint64_t* h = glb(nd.rfg) + size_t((tc - 1u) & 3u) * n_total;
+		const uint2* work = l.work + par * NEMO_MASK_STDP_CAP;
+		const uint32_t* rec = l.records + par * cache * CHUNK;
+		if(total <= NEMO_MASK_STDP_CAP) {
+			for(uint32_t c0 = wave; c0 < total; c0 += K * nwaves) {   /* wave-uniform */
+				uint32_t r[K], len[K], sd[K], count = 0;
+#pragma unroll
+				for(uint32_t i = 0; i < K; ++i) {
+					const uint32_t c = min(c0 + i * nwaves, total - 1u);
+					const uint2 ck = work[c];
+					r[i] = __builtin_amdgcn_readfirstlane(ck.x);
+					len[i] = __builtin_amdgcn_readfirstlane(ck.y);
+					count += c0 + i * nwaves < total ? 1u : 0u;
+					if(c < cache) sd[i] = rec[c * CHUNK + lane];
+					else sd[i] = rsd[r[i] + min(lane, len[i] - 1u)];
+				}
+				chunks(h, r, len, sd, count);
+			}
+			return;
+		}
+		const uint32_t s = tslot >= postLen ? tslot - postLen : tslot + R - postLen;
+		each_fired<WORDS>(glb(nd.mk) + size_t(s) * W, tc - postLen, w0, w1, list, lane, [&](bool ok, uint32_t x) {
+			const Row row = row_of(ok, x);
+			uint32_t ch = row.ch;
+			while(__any(ch * CHUNK < row.len)) {   /* wave-uniform */
+				const uint32_t mr = row.begin + ch * CHUNK;
+				const uint32_t ml = ch * CHUNK < row.len ? min(CHUNK, row.len - ch * CHUNK) : 0u;
+				for(uint64_t b = __ballot(ml != 0u); b; ) {
+					uint32_t r[K], len[K], sd[K], count = 0;
+#pragma unroll
+					for(uint32_t i = 0; i < K; ++i) {
+						const int src = __builtin_ctzll(b | 1ull << 63);
+						r[i] = uint32_t(__builtin_amdgcn_readlane(int(mr), src));
+						len[i] = uint32_t(__builtin_amdgcn_readlane(int(ml), src));
+						sd[i] = 0u;
+						if(b) sd[i] = rsd[r[i] + min(lane, len[i] - 1u)];
+						count += b ? 1u : 0u;
+						b &= b - 1ull;
+					}
+					chunks(h, r, len, sd, count);
+				}
+				ch += P;
+			}
+		});
+	};
+	uint32_t wslot = uint32_t(nd.cycle0 % R);
+	for(uint32_t k = 0; k < nd.nsteps; ++k) {
+		const uint64_t t = nd.cycle0 + k;
+		const uint32_t tag = uint32_t(t), par = tag & 1u;
+		if(wave == 0u && lane == 0u) l.count[par] = 0u;   /* the last list of this parity is done */
+		__syncthreads();
+		if(SAT) __syncthreads();
+		if(k > 0u) accumulate(tag - 1u, wslot ? wslot - 1u : R - 1u);
+		/* this cycle's chunks; the records of the first `cache` go to LDS */
+		if(t >= postLen) {
+			const uint32_t s = wslot >= postLen ? wslot - postLen : wslot + R - postLen;
+			each_fired<WORDS>(glb(nd.mk) + size_t(s) * W, tag - postLen, w0, w1, list, lane, [&](bool ok, uint32_t x) {
+				const Row row = row_of(ok, x);
+				uint32_t ch = row.ch;
+				while(__any(ch * CHUNK < row.len)) {   /* wave-uniform */
+					const bool has = ch * CHUNK < row.len;
+					const uint32_t r = row.begin + ch * CHUNK;
+					const uint32_t len = has ? min(CHUNK, row.len - ch * CHUNK) : 0u;
+					uint32_t at = ~0u;
+					if(has) {
+						at = atomicAdd(l.count + par, 1u);
+						if(at < NEMO_MASK_STDP_CAP) l.work[par * NEMO_MASK_STDP_CAP + at] = make_uint2(r, len);
+					}
+					for(uint64_t b = __ballot(has && at < cache); b; b &= b - 1ull) {
+						const int src = __builtin_ctzll(b);
+						const uint32_t as = uint32_t(__builtin_amdgcn_readlane(int(at), src));
+						const uint32_t rs = uint32_t(__builtin_amdgcn_readlane(int(r), src));
+						const uint32_t ls = uint32_t(__builtin_amdgcn_readlane(int(len), src));   /* >= 1 */
+						__builtin_amdgcn_global_load_lds((NEMO_GLOBAL void*)(rsd + rs + min(lane, ls - 1u)),
+								(NEMO_LDS void*)(l.records + (par * cache + as) * CHUNK), 4, 0, 0);
+					}
+					ch += P;
+				}
+			});
+		}
+		__builtin_amdgcn_s_waitcnt(0);   /* the staged records are in LDS */
+		__syncthreads();
+		wslot = wslot + 1u == R ? 0u : wslot + 1u;
+	}
+	if(nd.nsteps > 0u) accumulate(uint32_t(nd.cycle0) + nd.nsteps - 1u, wslot ? wslot - 1u : R - 1u);
+}
+
 /* WORDS: words a lane polls together. A wave whose share of the words takes
  * more than 64 WORDS of them goes through the rest of the cycle's chain once
  * per 64 WORDS, and every word costs instructions whether it is there or not
  * (10k x 100: 4.0 us a cycle with 4, 4.5 with 8; 200k x 100: 9.0 with 4, 8.4
  * with 8), so the host picks the smallest of 1, 4 and 8 that covers the share. */
-template<bool SAT, bool IZO, uint32_t WORDS>
+template<bool SAT, bool IZO, uint32_t WORDS, bool STDP>
 __device__ __forceinline__ void run_masked(const NetDev& nd, uint32_t p)
 {
 	constexpr int NP = IZO ? 5 : MAX_PARAM;
@@ -65,6 +299,16 @@ __device__ __forceinline__ void run_masked(const NetDev& nd, uint32_t p)
 	uint32_t* fst = reinterpret_cast<uint32_t*>(ext + T);
 	uint32_t* ovf = fst + fwords;                                      /* [2][D][T/32] when SAT */
 	uint16_t* list = reinterpret_cast<uint16_t*>(ovf + (SAT ? 2u * D * fwords : 0u)) + wave * LIST;
+	/* with STDP (nemo_mask_stdp_lds_bytes), lists by cycle parity */
+	const uint32_t R = STDP ? nd.flRing : 2u;          /* cycles of words kept */
+	const uint32_t nsw = STDP ? nd.stdpWaves : 0u;
+	StdpLds stdpLds;
+	uint8_t* area = reinterpret_cast<uint8_t*>(ovf + (SAT ? 2u * D * fwords : 0u)) + (nw + nsw) * LIST * 2u;
+	stdpLds.table = reinterpret_cast<StdpParams*>(area);
+	stdpLds.work = reinterpret_cast<uint2*>(area + NEMO_STDP_LDS_BYTES);
+	stdpLds.count = reinterpret_cast<uint32_t*>(stdpLds.work + 2u * NEMO_MASK_STDP_CAP);
+	stdpLds.masks = reinterpret_cast<StdpMasks*>(stdpLds.count + 4);
+	stdpLds.records = stdpLds.count + 16;
 	const bool defer = (nd.flags & NEMO_NET_DEFER) != 0u;
 	const uint32_t offMask = defer ? ((1u << OFF_NEAR_SHIFT) - 1u) : ~0u;
 	const NEMO_GLOBAL uint2* syn = glb(reinterpret_cast<const uint2*>(nd.syn));
@@ -77,12 +321,21 @@ __device__ __forceinline__ void run_masked(const NetDev& nd, uint32_t p)
 	}
 
 	int32_t* gring = nd.ring + size_t(p) * 2u * (D + 1u) * T;
-	ring_restore(gring, ringE, T, D, nd.cycle0, wave, nwaves, lane);
+	const bool replay = STDP && (nd.flags & NEMO_NET_REPLAY) != 0u;
+	if(replay) {
+		for(uint32_t i = tid; i < 2u * D * T; i += nthreads) ringE[i] = 0;
+	} else {
+		ring_restore(gring, ringE, T, D, nd.cycle0, wave, nwaves, lane);
+	}
 	if(SAT) {
 		for(uint32_t i = tid; i < 2u * D * fwords; i += nthreads) ovf[i] = 0u;
 	}
 	if(tid < T) ext[tid] = 0.0f;
 	if(tid < fwords) fst[tid] = 0u;
+	if(replay) {
+		__syncthreads();
+		ring_replay<SAT>(nd, p, syn, off, offMask, ringE, ringI, ovf, fwords, wave, nwaves, lane);
+	}
 
 	/* neuron registers */
 	int model = 0;
@@ -124,12 +377,28 @@ __device__ __forceinline__ void run_masked(const NetDev& nd, uint32_t p)
 	const uint32_t W = P * fwords;
 	const uint32_t w0 = wave < nw ? W * wave / nw : 0u;     /* this wave's share of the words */
 	const uint32_t w1 = wave < nw ? W * (wave + 1u) / nw : 0u;
+	uint32_t wslot = uint32_t(nd.cycle0 % R);               /* cycle mod R */
+	if(STDP) {
+		/* the tables to LDS: they are read for every plastic synapse */
+		const NEMO_GLOBAL StdpParams* sp = glb(static_cast<const StdpParams*>(nd.stdp));
+		const NEMO_GLOBAL uint32_t* src = glb(static_cast<const uint32_t*>(nd.stdp));
+		uint32_t* dst = reinterpret_cast<uint32_t*>(stdpLds.table);
+		for(uint32_t i = tid; i < uint32_t(sizeof(StdpParams) / 4u); i += nthreads) dst[i] = src[i];
+		if(tid < 2u) {
+			stdpLds.count[tid] = 0u;
+			const uint64_t region = tid ? sp->depression : sp->potentiation;
+			stdpLds.masks->pre[tid] = (region & sp->prePost) >> sp->postLen;
+			stdpLds.masks->post[tid] = (region & sp->postPre) << (64 - sp->postLen);
+		}
+	}
 
 	/* Stimulus is put into LDS a cycle ahead: the schedule's bounds of the next
 	 * cycle are in registers, its first entries are loaded after the publish
 	 * and stored before the cycle's last barrier; the update that reads them
 	 * clears them. */
 	const bool sched = nd.fs_ptr != nullptr;
+	const uint32_t sthreads = STDP ? T : nthreads;   /* threads that take entries */
+	const bool takes = tid < sthreads;
 	uint32_t fb = 0, fe = 0, ib = 0, ie = 0;    /* bounds of the next cycle's entries */
 	const uint32_t lo = p * T;
 	auto force = [&](uint32_t idx) {
@@ -155,13 +424,16 @@ __device__ __forceinline__ void run_masked(const NetDev& nd, uint32_t p)
 	uint32_t slotK = uint32_t(nd.cycle0 % D);
 	__syncthreads();
 
-	for(uint32_t k = 0; k < nd.nsteps; ++k) {
+	const bool learns = STDP && wave >= nw && wave < nw + nsw;   /* its barriers are those of this loop */
+	if(learns) stdp_waves<SAT, WORDS, IZO ? 8u : 4u>(nd, p, wave - nw, nsw, lane, stdpLds, list);
+	const uint32_t nsteps = learns ? 0u : nd.nsteps;
+	for(uint32_t k = 0; k < nsteps; ++k) {
 		const uint64_t t = nd.cycle0 + k;
 		const uint32_t tag = uint32_t(t);
 		const uint32_t slot = slotK;
 		slotK = (slotK + 1u == D) ? 0u : slotK + 1u;
 		const bool drawn = !(IZO && active && k + 1u < nd.nsteps && prm[IZ_SIGMA] != 0.0f);
-		NEMO_GLOBAL uint64_t* words = glb(nd.mk) + size_t(tag & 1u) * W;
+		NEMO_GLOBAL uint64_t* words = glb(nd.mk) + size_t(wslot) * W;
 
 		/* ---- 1. neuron update */
 		bool fired = false;
@@ -189,6 +461,7 @@ __device__ __forceinline__ void run_masked(const NetDev& nd, uint32_t p)
 				fired = update_neuron(model, prm, st, rng, fx20_to_float(e), fx20_to_float(i), cx, fs);
 			}
 			recent = (recent << 1) | (fired ? 1ull : 0ull);
+			if(STDP) st_agent(glb(nd.rfg) + size_t(tag & 3u) * n_total + n, recent);
 		}
 
 		/* ---- 2. publish the wave's fired bits; the raster */
@@ -220,8 +493,8 @@ __device__ __forceinline__ void run_masked(const NetDev& nd, uint32_t p)
 		uint32_t fx = ~0u, ix = ~0u, fnext = 0, inext = 0;
 		float iv = 0.0f;
 		if(sched) {
-			if(fb + tid < fe) fx = glb(nd.fs_idx)[fb + tid];
-			if(ib + tid < ie) {
+			if(takes && fb + tid < fe) fx = glb(nd.fs_idx)[fb + tid];
+			if(takes && ib + tid < ie) {
 				ix = glb(nd.is_idx)[ib + tid];
 				iv = glb(nd.is_val)[ib + tid];
 			}
@@ -390,14 +663,18 @@ __device__ __forceinline__ void run_masked(const NetDev& nd, uint32_t p)
 		if(sched) {
 			if(fx != ~0u) force(fx);
 			if(ix != ~0u) drive(ix, iv);
-			for(uint32_t e = fb + nthreads + tid; e < fe; e += nthreads) force(glb(nd.fs_idx)[e]);
-			for(uint32_t e = ib + nthreads + tid; e < ie; e += nthreads) drive(glb(nd.is_idx)[e], glb(nd.is_val)[e]);
+			if(takes) {
+				for(uint32_t e = fb + sthreads + tid; e < fe; e += sthreads) force(glb(nd.fs_idx)[e]);
+				for(uint32_t e = ib + sthreads + tid; e < ie; e += sthreads) drive(glb(nd.is_idx)[e], glb(nd.is_val)[e]);
+			}
 			fb = fe;
 			ib = ie;
 			fe = k + 2u < nd.nsteps ? fnext : fe;
 			ie = k + 2u < nd.nsteps ? inext : ie;
 		}
+		if(STDP) __builtin_amdgcn_s_waitcnt(0);   /* this cycle's histories are out */
 		__syncthreads();
+		wslot = wslot + 1u == R ? 0u : wslot + 1u;
 	}
 
 	/* ---- the last cycle's deferred records */
@@ -430,33 +707,47 @@ __device__ __forceinline__ void run_masked(const NetDev& nd, uint32_t p)
 
 } // namespace
 
-template<bool SAT, bool IZO>
+template<bool SAT, bool IZO, bool STDP>
 __global__ void __launch_bounds__(1024)
 nemo_mask_kernel(const NetDev* __restrict__ nets, const WorkItem* __restrict__ work)
 {
 	const WorkItem wi = work[blockIdx.x];
 	const NetDev nd = nets[wi.net];
-	run_masked<SAT, IZO, 4u>(nd, wi.part);
+	run_masked<SAT, IZO, 4u, STDP>(nd, wi.part);
 }
 
 /* one network per launch: the descriptor as a kernel argument */
-template<bool SAT, bool IZO, uint32_t WORDS>
+template<bool SAT, bool IZO, uint32_t WORDS, bool STDP>
 __global__ void __launch_bounds__(1024)
 nemo_mask_kernel_single(const NetDev nd, const WorkItem* __restrict__ work)
 {
-	run_masked<SAT, IZO, WORDS>(nd, work[blockIdx.x].part);
+	run_masked<SAT, IZO, WORDS, STDP>(nd, work[blockIdx.x].part);
 }
 
 namespace {
 
-template<bool SAT, bool IZO>
+template<bool SAT, bool IZO, bool STDP>
 const void* mask_kernel(uint32_t words)
 {
-	if(words == 0u) return reinterpret_cast<const void*>(&nemo_mask_kernel<SAT, IZO>);
-	/* saturating networks, whose atomics take more registers, always 4 */
-	if(!SAT && words <= 64u) return reinterpret_cast<const void*>(&nemo_mask_kernel_single<SAT, IZO, SAT ? 4u : 1u>);
-	if(!SAT && words > 256u) return reinterpret_cast<const void*>(&nemo_mask_kernel_single<SAT, IZO, SAT ? 4u : 8u>);
-	return reinterpret_cast<const void*>(&nemo_mask_kernel_single<SAT, IZO, 4u>);
+	if(words == 0u) return reinterpret_cast<const void*>(&nemo_mask_kernel<SAT, IZO, STDP>);
+	/* saturating networks, whose atomics take more registers, always 4; with
+	 * STDP at most 4 */
+	if(!SAT && words <= 64u) return reinterpret_cast<const void*>(&nemo_mask_kernel_single<SAT, IZO, SAT ? 4u : 1u, STDP>);
+	if(!SAT && !STDP && words > 256u) {
+		return reinterpret_cast<const void*>(&nemo_mask_kernel_single<SAT, IZO, SAT || STDP ? 4u : 8u, STDP>);
+	}
+	return reinterpret_cast<const void*>(&nemo_mask_kernel_single<SAT, IZO, 4u, STDP>);
+}
+
+template<bool STDP>
+const void* mask_kernel_variant(uint32_t variant, uint32_t words)
+{
+	switch(variant & 3u) {
+	case 0: return mask_kernel<false, false, STDP>(words);
+	case 1: return mask_kernel<true, false, STDP>(words);
+	case 2: return mask_kernel<false, true, STDP>(words);
+	default: return mask_kernel<true, true, STDP>(words);
+	}
 }
 
 } // namespace
@@ -465,12 +756,7 @@ extern "C" {
 
 const void* nemo_dev_mask_kernel(uint32_t variant, uint32_t words)
 {
-	switch(variant & 3u) {
-	case 0: return mask_kernel<false, false>(words);
-	case 1: return mask_kernel<true, false>(words);
-	case 2: return mask_kernel<false, true>(words);
-	default: return mask_kernel<true, true>(words);
-	}
+	return (variant & 8u) ? mask_kernel_variant<true>(variant, words) : mask_kernel_variant<false>(variant, words);
 }
 
 } // extern "C"

@@ -55,8 +55,9 @@ typedef struct NetDev {
 	uint32_t spinLimit;  /* barrier spin bound (iterations) */
 	uint32_t glog2;      /* log2 of the lanes that share one fired source in delivery (0..6) */
 	uint32_t glogFew;    /* the same where a wave has few fired sources (NEMO_NET_MASKS; >= glog2) */
-	uint32_t flRing;     /* fired lists and counts kept for this many cycles (buffer t mod flRing) */
+	uint32_t flRing;     /* fired lists and counts, or fired words, kept for this many cycles (buffer t mod flRing) */
 	uint32_t stdpCache;  /* STDP chunks whose reverse records are staged in LDS (64 words each) */
+	uint32_t stdpWaves;  /* waves for STDP after those of the neurons (NEMO_NET_MASKS) */
 	uint32_t exWaves;    /* with NEMO_NET_DEFER: waves of a workgroup that run the exchange and the
 	                      * delay-1 delivery while the others deliver the previous cycle's far
 	                      * records (0: every wave does both, one after the other) */
@@ -82,8 +83,8 @@ typedef struct NetDev {
 	 * by cycle parity */
 	uint64_t* fl;             /* [flRing][P][T] fired neurons of each partition, (cycle << 32) | neuron */
 	uint64_t* fc;             /* [flRing][P] (cycle << 32) | fired count; starts all-ones */
-	uint64_t* mk;             /* [2][P*T/32] (cycle << 32) | 32 fired bits; starts all-ones (NEMO_NET_MASKS) */
-	uint64_t* rfg;            /* [2][n] firing history (STDP only) */
+	uint64_t* mk;             /* [flRing][P*T/32] (cycle << 32) | 32 fired bits; starts all-ones (NEMO_NET_MASKS) */
+	uint64_t* rfg;            /* [2][n], with NEMO_NET_MASKS [4][n], firing history by cycle (STDP only) */
 	uint32_t* status;         /* NEMO_STATUS_* */
 	unsigned long long* events; /* delivered-synapse counter */
 
@@ -142,12 +143,13 @@ typedef struct WorkItem {
  * hipError_t value as int and take a hipStream_t as void*. */
 /* Step-kernel variants: bit 0 = saturating accumulation (NEMO_NET_SATURATE),
  * bit 1 = Izhikevich-only network (NEMO_NET_IZHIKEVICH_ONLY), bit 2 = fired
- * bits exchanged as words (NEMO_NET_MASKS, mask_kernel.hip). All networks of
- * one launch must be of the launch's variant. */
+ * bits exchanged as words (NEMO_NET_MASKS, mask_kernel.hip), bit 3 = STDP
+ * there. All networks of one launch must be of the launch's variant. */
 static inline uint32_t nemo_step_variant(uint32_t flags)
 {
 	return ((flags & NEMO_NET_SATURATE) ? 1u : 0u) | ((flags & NEMO_NET_IZHIKEVICH_ONLY) ? 2u : 0u)
-		| ((flags & NEMO_NET_MASKS) ? 4u : 0u);
+		| ((flags & NEMO_NET_MASKS) ? 4u : 0u)
+		| ((flags & (NEMO_NET_MASKS | NEMO_NET_STDP)) == (NEMO_NET_MASKS | NEMO_NET_STDP) ? 8u : 0u);
 }
 /* The kernel of mask_kernel.hip for a variant: for one network whose waves
  * take up to `words` words each, or for batches (words = 0) */
@@ -213,8 +215,10 @@ int nemo_dev_nrand_seq(const uint32_t* state4_dev, float* out_dev, size_t n, voi
 
 /* Bytes of LDS the STDP tables take (the StdpParams of models.h, rounded) */
 #define NEMO_STDP_LDS_BYTES 576u
-/* Entries of a workgroup's per-cycle STDP work list (64-synapse chunks) */
+/* Entries of a workgroup's per-cycle STDP work list (64-synapse chunks), and
+ * of each of mask_kernel.hip's two */
 #define NEMO_STDP_WORK_CAP 1024u
+#define NEMO_MASK_STDP_CAP 512u
 
 /* LDS bytes the step kernel needs for partitions of T neurons, ring depth D,
  * P partitions. Optional STDP areas follow, in this order, when the host
@@ -249,6 +253,13 @@ static inline uint32_t nemo_step_lds_bytes(uint32_t T, uint32_t D, uint32_t P, i
 static inline uint32_t nemo_mask_lds_bytes(uint32_t T, uint32_t D, int saturate)
 {
 	return 2u * D * T * 4u + T * 4u + (T / 32u) * 4u + (saturate ? 2u * D * (T / 32u) * 4u : 0u) + (T / 64u) * 256u;
+}
+
+/* and with STDP: the sources of its waves, the tables, two work lists (by
+ * cycle parity) and their lengths, and the staged reverse records of both */
+static inline uint32_t nemo_mask_stdp_lds_bytes(uint32_t waves, uint32_t cache)
+{
+	return waves * 256u + NEMO_STDP_LDS_BYTES + 2u * NEMO_MASK_STDP_CAP * 8u + 64u + 2u * cache * 256u;
 }
 
 #ifdef __cplusplus

@@ -387,16 +387,33 @@ Simulation::Simulation(const NetworkImpl& net, const ConfigurationImpl& conf) :
 		whyNotFused = "a neuron type has no fused implementation";
 	}
 
-	/* Networks without STDP exchange their fired bits as words
-	 * (mask_kernel.hip), unless the configuration asks for exchange waves or
-	 * that kernel's LDS leaves too few neurons per workgroup. Per cycle, lists
-	 * against words: 1k x 100 4.5 -> 3.4 us, 10k x 1000 9.1 -> 6.0, 60k x 300
-	 * 6.3 -> 5.4, 200k x 1000 13.8 -> 12.8, 12k x 550 IF_curr_exp_noise at 333
-	 * Hz 57 -> 47. */
-	m_masks = !m_stdp && conf.exchangeWaves <= 0;
+	/* Networks exchange their fired bits as words (mask_kernel.hip), unless
+	 * the configuration asks for exchange waves or that kernel's LDS leaves too
+	 * few neurons per workgroup. Per cycle, lists against words: 1k x 100 4.5
+	 * -> 3.4 us, 10k x 1000 9.1 -> 6.0, 60k x 300 6.3 -> 5.4, 200k x 1000 13.8
+	 * -> 12.8, 12k x 550 IF_curr_exp_noise at 333 Hz 57 -> 47; with STDP 3k x
+	 * 300 10.9 -> 3.6, 10k x 300 10.5 -> 4.2, 50k x 1000 17.4 -> 11.9, 12k x
+	 * 550 at 333 Hz 283 -> 98. With STDP lists remain for what words do not
+	 * have: a window without cycles after the spike, work lists that are not to
+	 * be staged, workgroups that leave less than 6 of 16 waves for it, and a
+	 * configured workgroup of 512 neurons or more, which gets exchange waves. */
+	const uint32_t postLen = m_stdp ? uint32_t(m_sp.postLen) : 0u;
+	m_masks = conf.exchangeWaves <= 0;
+	if(m_stdp && (postLen < 1u || !conf.stdpLdsStaging || conf.partitionSize >= 512u)) m_masks = false;
+	/* STDP there: two waves of their own more than a workgroup has for its
+	 * neurons, as far as 16 in all go (5k x 1000, 3 neurons' waves: 12.5 us per
+	 * cycle with 1, 5.9 with 3, 5.5 with 5; 20k x 1000, 4: 7.6 with 4, 7.3 with
+	 * 6; 50k x 1000, 8: 16.2 with 4, 11.8 with 8) */
+	auto stdpWaves = [&](uint32_t t) {
+		const uint32_t nw = t / 64u;
+		return m_masks && m_stdp ? std::min(nw + 2u, 16u - std::min(16u, nw)) : 0u;
+	};
 	auto ldsFor = [&](uint32_t t) {
 		uint32_t p = (m_n + t - 1) / t;
-		if(m_masks) return nemo_mask_lds_bytes(t, m_D, m_saturate ? 1 : 0);
+		if(m_masks) {
+			return nemo_mask_lds_bytes(t, m_D, m_saturate ? 1 : 0)
+				+ (m_stdp ? nemo_mask_stdp_lds_bytes(stdpWaves(t), 0u) : 0u);
+		}
 		return nemo_step_lds_bytes(t, m_D, std::max(1u, p), m_saturate ? 1 : 0, m_stdp ? 1 : 0);
 	};
 	/* T: neurons per partition. The automatic choice takes at most one
@@ -409,6 +426,9 @@ Simulation::Simulation(const NetworkImpl& net, const ConfigurationImpl& conf) :
 	 * 3k neurons about 13 (2k x 1000: 192 4.1, 128 5.3, 512 6.2), from 48k
 	 * neurons on about 160 (100k x 300: 640 6.5, 832 6.9; 200k x 1000: 960
 	 * 12.8, 832 13.7).
+	 *   With words and STDP: about 27 partitions up to 6k neurons, 79 from there
+	 * (10k x 300: 128 neurons 4.5, 384 4.8; 20k x 1000: 256 7.6, 512 9.5; 50k x
+	 * 1000: 448 or 512 11.8, 256 11.9; 100k x 300: 512 10.1, 640 11.8).
 	 *   With lists: about 40 partitions of up to 512 neurons (10k x 100: 7.2 ->
 	 * 6.3 us; 50k x 1000: 10.4 -> 9.7 us), and with rows of 500 synapses or
 	 * more, from 1.5k to 12k neurons, about 13 partitions (2k x 1000: 8.0 ->
@@ -419,9 +439,10 @@ Simulation::Simulation(const NetworkImpl& net, const ConfigurationImpl& conf) :
 			t = std::min(1024u, roundUp64(conf.partitionSize));
 		} else {
 			const uint32_t perCU = roundUp64(std::max<uint32_t>(1u, (m_n + 255u) / 256u));
-			const bool large = m_masks && m_n >= 49152u;
-			const bool longRows = m_n >= 1500u && m_n <= (m_masks ? 3000u : 12000u) && m_nsyn / m_n >= 500u;
-			const uint32_t parts = longRows ? 13u : (large ? 160u : (m_masks ? 27u : 40u));
+			const bool large = m_masks && !m_stdp && m_n >= 49152u;
+			const bool longRows = !(m_masks && m_stdp) && m_n >= 1500u && m_n <= (m_masks ? 3000u : 12000u) && m_nsyn / m_n >= 500u;
+			const uint32_t parts = m_masks && m_stdp ? (m_n < 6144u ? 27u : 79u)
+				: (longRows ? 13u : (large ? 160u : (m_masks ? 27u : 40u)));
 			uint32_t wide = roundUp64(std::max<uint32_t>(1u, (m_n + parts - 1u) / parts));
 			wide = std::min(longRows ? 1024u : (large ? 960u : 512u), std::max(wide, large ? 512u : 64u));
 			t = std::max(64u, std::min(1024u, std::max(perCU, wide)));
@@ -437,8 +458,8 @@ Simulation::Simulation(const NetworkImpl& net, const ConfigurationImpl& conf) :
 	if(m_masks && m_n > 0 && whyNotFused.empty()) {
 		uint32_t maxBlocks = 0;
 		const uint32_t lds = ldsFor(T);
-		if(lds <= ldsLimit) hipCheck(nemo_dev_step_max_blocks(T, lds, variant(), &maxBlocks), "occupancy query");
-		if((m_n + T - 1) / T > maxBlocks) {
+		if(lds <= ldsLimit) hipCheck(nemo_dev_step_max_blocks(T + 64u * stdpWaves(T), lds, variant(), &maxBlocks), "occupancy query");
+		if((m_n + T - 1) / T > maxBlocks || (m_stdp && T > 640u)) {
 			m_masks = false;
 			T = partitionSize();
 		}
@@ -447,27 +468,29 @@ Simulation::Simulation(const NetworkImpl& net, const ConfigurationImpl& conf) :
 		whyNotFused = "maximum delay too large for the LDS delay ring";
 	}
 	m_T = T;
+	m_stdpWaves = stdpWaves(T);
 	m_P = (m_n + T - 1) / T;
 	m_lds = ldsFor(T);
 	if(whyNotFused.empty() && m_P > 0) {
 		uint32_t maxBlocks = 0;
-		hipCheck(nemo_dev_step_max_blocks(m_T, m_lds, variant(), &maxBlocks), "occupancy query");
+		hipCheck(nemo_dev_step_max_blocks(blockThreads(), m_lds, variant(), &maxBlocks), "occupancy query");
 		if(m_P > maxBlocks) {
 			whyNotFused = fmt("network of ", m_n, " neurons needs ", m_P,
 					" co-resident workgroups of ", m_T, " neurons; the device holds ", maxBlocks);
 		}
 		/* STDP, with LDS left over while the workgroups stay co-resident:
-		 * first the prefixes of the fired counts of the last postLen cycles
-		 * (the work lists' targets; otherwise gathered again each cycle),
-		 * then the reverse records of up to 64 chunks (256 bytes each) of
-		 * every cycle's work list */
+		 * with lists first the prefixes of the fired counts of the last
+		 * postLen cycles (the work lists' targets; otherwise gathered again
+		 * each cycle; words need none), then the reverse records of up to 64
+		 * chunks (256 bytes each, twice with words) of every cycle's work list */
 		auto fits = [&](uint32_t lds) {
 			if(lds > ldsLimit) return false;
-			hipCheck(nemo_dev_step_max_blocks(m_T, lds, variant(), &maxBlocks), "occupancy query");
+			hipCheck(nemo_dev_step_max_blocks(blockThreads(), lds, variant(), &maxBlocks), "occupancy query");
 			return m_P <= maxBlocks;
 		};
-		const uint32_t postLen = uint32_t(m_sp.postLen);
-		if(m_stdp && conf.stdpLdsStaging && whyNotFused.empty() && postLen >= 2) {
+		if(m_stdp && m_masks) {
+			m_prefRing = true;
+		} else if(m_stdp && conf.stdpLdsStaging && whyNotFused.empty() && postLen >= 2) {
 			const uint32_t ring = postLen * ((m_P + 1u + 63u) & ~63u) * 4u;
 			if(fits(m_lds + ring)) {
 				m_prefRing = true;
@@ -475,9 +498,10 @@ Simulation::Simulation(const NetworkImpl& net, const ConfigurationImpl& conf) :
 			}
 		}
 		for(uint32_t c = 64; m_stdp && conf.stdpLdsStaging && whyNotFused.empty() && c >= 8; c /= 2) {
-			if(fits(m_lds + c * 256u)) {
+			const uint32_t bytes = (m_masks ? 2u : 1u) * c * 256u;
+			if(fits(m_lds + bytes)) {
 				m_stdpCache = c;
-				m_lds += c * 256u;
+				m_lds += bytes;
 				break;
 			}
 		}
@@ -496,6 +520,7 @@ Simulation::Simulation(const NetworkImpl& net, const ConfigurationImpl& conf) :
 		m_fused = false;
 		m_P = 1;
 		m_T = 0;
+		m_stdpWaves = 0;
 		m_lds = 0;
 		m_words32 = 2 * ((m_n + 63) / 64);
 		m_words = m_words32 / 2;
@@ -743,18 +768,24 @@ Simulation::Simulation(const NetworkImpl& net, const ConfigurationImpl& conf) :
 
 	/* fired lists and counts are kept for flRing cycles: 2 (parity), 3 when
 	 * deferred delivery reads the previous cycle's, postLen + 2 with STDP,
-	 * whose accumulation reads those of cycle t - postLen */
-	m_flRing = m_stdp ? std::max(3u, uint32_t(m_sp.postLen) + 2u) : (m_defer ? 3u : 2u);
-	d_fl.alloc(size_t(m_flRing) * m_P * m_T * 8);
-	d_fc.alloc(size_t(m_flRing) * m_P * 8 + 8);
-	if(m_fused && m_masks) d_mk.alloc(size_t(2) * m_P * (m_T / 32u) * 8);
+	 * whose accumulation reads those of cycle t - postLen; words for 2, or
+	 * postLen + 3, where the accumulation is a cycle behind */
+	const bool words = m_fused && m_masks;
+	if(words) {
+		m_flRing = m_stdp ? postLen + 3u : 2u;
+		d_mk.alloc(size_t(m_flRing) * m_P * (m_T / 32u) * 8);
+	} else {
+		m_flRing = m_stdp ? std::max(3u, postLen + 2u) : (m_defer ? 3u : 2u);
+		d_fl.alloc(size_t(m_flRing) * m_P * m_T * 8);
+		d_fc.alloc(size_t(m_flRing) * m_P * 8 + 8);
+	}
 	d_ctl.alloc(64);
 	if(cycleKernelRuns()) {
 		d_done.alloc((1u + NEMO_DONE_GROUPS) * 128u);
 		hipCheck(nemo_dev_fill_u32(d_done.as<uint32_t>(), 0, d_done.bytes / 4, static_cast<hipStream_t>(m_stream)), "fill");
 	}
 	if(m_stdp) {
-		d_rfg.alloc(size_t(2) * m_n * 8);
+		d_rfg.alloc(size_t(words ? 4 : 2) * m_n * 8);
 		if(!m_deviceBuilt) {
 			d_rcmStart.upload(rcmStart.data(), rcmStart.size() * 4);
 			d_rcmSd.upload(rcmSd.data(), rcmSd.size() * 4);
@@ -762,7 +793,7 @@ Simulation::Simulation(const NetworkImpl& net, const ConfigurationImpl& conf) :
 		}
 		d_rcmAcc.alloc(std::max<size_t>(m_nplastic, 1) * 4);
 		d_stdp.upload(&m_sp, sizeof(m_sp));
-		if(m_fused) {
+		if(m_fused && !words) {
 			/* reverse row {start, length} of each fired neuron, beside its
 			 * fired-list entry (the next STDP work lists are built from it) */
 			d_srow.alloc(size_t(m_flRing) * m_P * m_T * 8);
@@ -771,7 +802,7 @@ Simulation::Simulation(const NetworkImpl& net, const ConfigurationImpl& conf) :
 	hipStream_t s = static_cast<hipStream_t>(m_stream);
 	if(d_recent.bytes) hipCheck(nemo_dev_fill_u64(d_recent.as<uint64_t>(), 0, m_n, s), "fill");
 	if(d_ring.bytes) hipCheck(nemo_dev_fill_u32(d_ring.as<uint32_t>(), 0, d_ring.bytes / 4, s), "fill");
-	if(d_rfg.bytes) hipCheck(nemo_dev_fill_u64(d_rfg.as<uint64_t>(), 0, size_t(2) * m_n, s), "fill");
+	if(d_rfg.bytes) hipCheck(nemo_dev_fill_u64(d_rfg.as<uint64_t>(), 0, d_rfg.bytes / 8, s), "fill");
 	if(d_rcmAcc.bytes) hipCheck(nemo_dev_fill_u32(d_rcmAcc.as<uint32_t>(), 0, d_rcmAcc.bytes / 4, s), "fill");
 	/* tagged fired counts: all-ones never matches a cycle's tag */
 	if(d_fc.bytes) hipCheck(nemo_dev_fill_u64(d_fc.as<uint64_t>(), ~0ull, d_fc.bytes / 8, s), "fill");
@@ -1135,7 +1166,7 @@ Simulation::planExchange(const ConfigurationImpl& conf, uint32_t ldsLimit)
 	m_exAuto = false;
 	m_ldsNoFar = m_lds;
 	const uint32_t nw = m_T / 64u;
-	if(!m_fused || !m_defer || m_P == 0 || conf.exchangeWaves < 0) return;
+	if(!m_fused || !m_defer || m_P == 0 || conf.exchangeWaves < 0 || m_masks) return;
 	uint32_t ex = uint32_t(conf.exchangeWaves);
 	if(conf.exchangeWaves == 0) {
 		if(!m_stdp || nw < 8u) return;
@@ -1147,7 +1178,7 @@ Simulation::planExchange(const ConfigurationImpl& conf, uint32_t ldsLimit)
 		const uint32_t lds = m_lds + NEMO_FAR_LDS_BYTES(cap);
 		if(lds > ldsLimit) continue;
 		uint32_t maxBlocks = 0;
-		hipCheck(nemo_dev_step_max_blocks(m_T, lds, variant(), &maxBlocks), "occupancy query");
+		hipCheck(nemo_dev_step_max_blocks(blockThreads(), lds, variant(), &maxBlocks), "occupancy query");
 		if(m_P <= maxBlocks) {
 			m_exWaves = ex;
 			m_farCap = cap;
@@ -1211,6 +1242,7 @@ Simulation::descriptor(unsigned nsteps) const
 	nd.glogFew = m_glogFew;
 	nd.flRing = m_flRing;
 	nd.stdpCache = m_stdpCache;
+	nd.stdpWaves = m_stdpWaves;
 	nd.exWaves = m_exWaves;
 	nd.farCap = m_farCap;
 	nd.cycle0 = m_cycle;
@@ -1446,7 +1478,7 @@ Simulation::launchDescriptor(const NetDev& nd, bool stepOut)
 	hipStream_t st = static_cast<hipStream_t>(m_stream);
 	hipEvent_t e0 = static_cast<hipEvent_t>(m_ev0), e1 = static_cast<hipEvent_t>(m_ev1);
 	hipCheck(hipEventRecord(e0, st), "hipEventRecord");
-	hipCheck(nemo_dev_step_launch_one(&nd, d_work.as<WorkItem>(), m_P, m_T, m_lds, variant(), st),
+	hipCheck(nemo_dev_step_launch_one(&nd, d_work.as<WorkItem>(), m_P, blockThreads(), m_lds, variant(), st),
 			"step kernel launch");
 	hipCheck(hipEventRecord(e1, st), "hipEventRecord");
 	hipCheck(hipMemcpyAsync(h_ctl, d_ctl.ptr, 32, hipMemcpyDeviceToHost, st), "D2H");
@@ -1834,7 +1866,7 @@ Simulation::info(nemo_hip_info_t* out) const
 	out->plastic_synapses = m_nplastic;
 	out->device_bytes = m_deviceBytes;
 	out->lds_bytes = m_lds;
-	out->block_threads = m_T;
+	out->block_threads = blockThreads();
 	out->last_kernel_ms = m_kernelMs;
 	out->fused = m_fused ? 1u : 0u;
 	out->deferred = m_defer ? 1u : 0u;

@@ -106,7 +106,7 @@ class Simulation
 
 		/* batched launches (nemo_hip_run_batch) */
 		uint32_t partitions() const { return m_P; }
-		uint32_t blockThreads() const { return m_T; }
+		uint32_t blockThreads() const { return m_T + 64u * m_stdpWaves; }
 		uint32_t ldsBytes() const { return m_lds; }
 		/* LDS of a batched launch: without the far list of exchange waves
 		 * the library chose by itself (a batched launch runs every
@@ -131,7 +131,7 @@ class Simulation
 		unsigned neuronCount() const { return m_n; }
 		int device() const { return m_device; }
 		/* step-kernel variant (nemo_step_variant): saturating, Izhikevich-only, masks */
-		uint32_t variant() const { return (m_saturate ? 1u : 0u) | (m_izOnly ? 2u : 0u) | (m_masks ? 4u : 0u); }
+		uint32_t variant() const { return (m_saturate ? 1u : 0u) | (m_izOnly ? 2u : 0u) | (m_masks ? (m_stdp ? 12u : 4u) : 0u); }
 		/* true: the fused persistent kernel; false: plugin kernels per cycle */
 		bool fused() const { return m_fused; }
 
@@ -185,6 +185,7 @@ class Simulation
 		bool m_defer = false;
 		/* cycles of fired lists and counts kept on the device */
 		uint32_t m_flRing = 2;
+		uint32_t m_stdpWaves = 0;    /* of mask_kernel.hip */
 		uint32_t m_stdpCache = 0;    /* STDP chunks staged in LDS per cycle */
 		bool m_prefRing = false;     /* STDP list prefixes of postLen cycles kept in LDS */
 		uint32_t m_exWaves = 0;      /* exchange waves (NetDev.exWaves) */
