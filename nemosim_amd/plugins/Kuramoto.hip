@@ -15,7 +15,8 @@
  *
  * A workgroup takes a tile of consecutive oscillators, whose rows of the
  * reverse matrix are contiguous: its threads evaluate the tile's coupling
- * terms into LDS, then one lane per oscillator adds its row's terms in order.
+ * terms into LDS, then a lane, or a row of 16, per oscillator adds its row's
+ * terms in order.
  * Phase history: plane c mod 32 of the state holds the phase
  * of cycle c (the descriptor's history=32).
  */
@@ -30,7 +31,7 @@ namespace {
 constexpr unsigned HISTORY = 32u;   /* history= of Kuramoto.ini */
 
 constexpr unsigned THREADS = 256u;
-constexpr unsigned TILE_OSC = 64u;            /* oscillators of a tile: one lane each in the sums */
+constexpr unsigned TILE_OSC = 64u;            /* oscillators of a tile: at least a lane each in the sums */
 /* A tile's rows in LDS start at multiples of 4 floats (16-byte reads), and at
  * least 65 zeros follow each: the sums run in steps of 64 terms, and adding
  * +0 leaves a sum that started from +0 as it is. */
@@ -39,11 +40,11 @@ constexpr unsigned ROW_GAP = STEP + 4u;
 constexpr unsigned RESIDENT = 1024u;          /* workgroups on the chip at once: 4 per compute unit */
 
 /* couplings of a tile whose threads hold PER each, and its floats in LDS (the
- * sums read half a step further) */
+ * sums read up to a step further) */
 template<unsigned PER> struct Tile {
 	static constexpr unsigned couplings = THREADS * PER;
 	static constexpr unsigned half = PER > 9u ? 4u : 8u;   /* 16-byte reads per half step of the sums */
-	static constexpr unsigned lds = couplings + ROW_GAP * TILE_OSC + STEP / 2u;
+	static constexpr unsigned lds = couplings + ROW_GAP * TILE_OSC + STEP;
 };
 
 /* how much further row j starts in LDS than its first coupling's number
@@ -102,6 +103,40 @@ __device__ inline float ordered_sum(float s, const float* row, unsigned len)
 	return s;
 }
 
+/* The same by 16 lanes (a DPP row), all of which have the sum: they read a step
+ * of 64 terms at once, 4 each, and every add takes its term from the lane that
+ * has it. So a read of LDS goes with 64 adds instead of 4, and a term takes 6.3
+ * cycles of a 1000-term row instead of 8.9 (4.8 without the loop around it). In assembly since
+ * the compiler waits between DPP adds for the operand that is not moved, too;
+ * the moved ones are not written here, and what may have written them, or the
+ * lanes in use, just before is waited for at the start. */
+#define ADD_LANE(L) \
+	"v_add_f32_dpp %0, %1, %0 row_newbcast:" #L " row_mask:0xf bank_mask:0xf\n" \
+	"v_add_f32_dpp %0, %2, %0 row_newbcast:" #L " row_mask:0xf bank_mask:0xf\n" \
+	"v_add_f32_dpp %0, %3, %0 row_newbcast:" #L " row_mask:0xf bank_mask:0xf\n" \
+	"v_add_f32_dpp %0, %4, %0 row_newbcast:" #L " row_mask:0xf bank_mask:0xf\n"
+
+__device__ inline float ordered_sum_row(float s, const float* row, unsigned len, unsigned lane)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+	LdsQuads r4 = (LdsQuads) row + lane;
+	Quad v = r4[0];
+	for(unsigned i = 0; i < len; i += STEP) {
+		r4 += STEP / 4u;
+		const Quad next = r4[0];
+		asm volatile("s_nop 4\n"
+				ADD_LANE(0) ADD_LANE(1) ADD_LANE(2) ADD_LANE(3) ADD_LANE(4) ADD_LANE(5) ADD_LANE(6) ADD_LANE(7)
+				ADD_LANE(8) ADD_LANE(9) ADD_LANE(10) ADD_LANE(11) ADD_LANE(12) ADD_LANE(13) ADD_LANE(14) ADD_LANE(15)
+				: "+v"(s) : "v"(v.x), "v"(v.y), "v"(v.z), "v"(v.w));
+		v = next;
+	}
+#else
+	(void) row; (void) len; (void) lane;
+#endif
+	return s;
+}
+#undef ADD_LANE
+
 /* One workgroup per `per` consecutive oscillators. Tiles of them whose rows
  * hold at most TILE = 256 PER couplings together are done one after the other (one tile,
  * unless rows are uneven); a row longer than TILE is a tile of its own and is
@@ -112,11 +147,11 @@ __device__ inline float ordered_sum(float s, const float* row, unsigned len)
  * stages x row length x 4.5 cycles, so that as many of them as possible run at
  * once; with many oscillators the reads of the sources' phases (random, 32
  * planes) and the sines (about 30 instructions each). One cycle, with the
- * plugin step's other kernels (about 11 us), before (one wave per oscillator,
+ * plugin step's other kernels (about 10 us), before (one wave per oscillator,
  * which evaluated 64 couplings at a time, every lane repeating the sum) and
- * now: 1000 oscillators x 1000 couplings 65 -> 35 us, 4000 x 1000 101 -> 61,
- * 2000 x 2500 (rows in pieces) 182 -> 129, 3000 x 300 36 -> 25, 20000 x 100
- * 48 -> 33, 50000 x 100 99 -> 76. */
+ * now: 1000 oscillators x 1000 couplings 65 -> 28 us (33 with a lane's sums
+ * alone), 4000 x 1000 101 -> 57, 2000 x 2500 182 -> 113, 3000 x 300 36 -> 21,
+ * 20000 x 100 48 -> 31, 50000 x 100 99 -> 75. */
 template<unsigned PER>
 __global__ void __launch_bounds__(256, 4) kuramoto_update_kernel(unsigned start, unsigned end, unsigned per,
 		unsigned cycle, const float* freq, float* state, size_t hstride, const uint32_t* rstart,
@@ -141,14 +176,17 @@ __global__ void __launch_bounds__(256, 4) kuramoto_update_kernel(unsigned start,
 		while(nb > 1u && rs[nb] - r0 > TILE) --nb;
 		const uint32_t total = rs[nb] - r0;                     /* couplings of the tile */
 		const uint32_t pieces = total <= TILE ? 1u : (total + TILE - 1u) / TILE;   /* > 1: one oscillator */
-		const uint32_t used = min(TILE, total) + ROW_GAP * nb + STEP / 2u;   /* of `term` */
+		const uint32_t used = min(TILE, total) + ROW_GAP * nb + STEP;   /* of `term` */
 		for(unsigned i = tid; i < used; i += THREADS) term[i] = 0.0f;
 		float f = 0.0f, theta = 0.0f, k0 = 0.0f, k1 = 0.0f, k2 = 0.0f, k3 = 0.0f;
-		const bool owner = tid < nb;
+		/* the lane of an oscillator, or with few of them the row of 16 lanes */
+		const bool byRow = nb <= THREADS / 16u;
+		const unsigned own = byRow ? tid / 16u : tid;
+		const bool owner = own < nb;
 		if(owner) {
-			f = freq[o + tid];
-			theta = phase0[o + tid];
-			rows[tid] = Row{theta, row_shift(rs[tid] - r0, tid)};
+			f = freq[o + own];
+			theta = phase0[o + own];
+			rows[own] = Row{theta, row_shift(rs[own] - r0, own)};
 		}
 		float sp[PER], wt[PER];
 		uint32_t osc[(PER + 3u) / 4u];                          /* oscillators of the couplings, 8 bits each */
@@ -194,21 +232,23 @@ __global__ void __launch_bounds__(256, 4) kuramoto_update_kernel(unsigned start,
 				__syncthreads();
 				if(owner) {
 					const bool whole = pieces == 1u;
-					s = ordered_sum<Tile<PER>::half>(s, term + (whole ? rs[tid] - r0 + rows[tid].shift : 0u),
-							whole ? rs[tid + 1u] - rs[tid] : cnt);
+					const float* row = term + (whole ? rs[own] - r0 + rows[own].shift : 0u);
+					const unsigned len = whole ? rs[own + 1u] - rs[own] : cnt;
+					if(byRow) s = ordered_sum_row(s, row, len, tid & 15u);
+					else s = ordered_sum<Tile<PER>::half>(s, row, len);
 				}
 			}
 			if(owner) {
 				const float k = f + s;
-				if(stage == 0u) { k0 = k; rows[tid].x = theta + k * 0.5f; }
-				else if(stage == 1u) { k1 = k; rows[tid].x = theta + k * 0.5f; }
-				else if(stage == 2u) { k2 = k; rows[tid].x = theta + k; }
+				if(stage == 0u) { k0 = k; rows[own].x = theta + k * 0.5f; }
+				else if(stage == 1u) { k1 = k; rows[own].x = theta + k * 0.5f; }
+				else if(stage == 2u) { k2 = k; rows[own].x = theta + k; }
 				else { k3 = k; }
 			}
 		}
 		if(owner) {
 			const float next = theta + (k0 + 2.0f * k1 + 2.0f * k2 + k3) / 6.0f;
-			phase1[o + tid] = nemo_libm::kuramoto_wrap(next);
+			phase1[o + own] = nemo_libm::kuramoto_wrap(next);
 		}
 		o += nb;
 		__syncthreads();   /* rs, rows and term are written again by the next tile */

@@ -1,6 +1,6 @@
 """The Kuramoto kernel's tiles (nemosim_amd/plugins/Kuramoto.hip) at their
 edges, bit for bit against the oracle: workgroups of 768, 2304 and 4608
-couplings, rows that end on them and one past them (read in pieces), several
+couplings, up to 16 oscillators of a workgroup and more, rows that end on them and one past them (read in pieces), several
 tiles in one workgroup where rows are uneven, rows around the sums' steps of
 32 and 64 terms, and empty rows."""
 import numpy as np
@@ -27,10 +27,12 @@ def uneven(n, seed):
     uneven(1024, 1),                                 # one oscillator per workgroup
     uneven(1025, 2),                                 # two
     uneven(5000, 3),                                 # five
+    uneven(16384, 4),                                # 16, a row of lanes each
+    uneven(16385, 5),                                # 17, a lane each
     np.array([2000, 2100, 1900, 2303, 2304, 2305, 2000]),    # tiles of 2304, one row past
     np.array([2400, 4608, 2304, 2305, 4609, 2200]),  # tiles of 4608, one row past
     np.array([4608, 9217, 4600]),                    # every row in pieces or a whole tile
-], ids=["1024", "1025", "5000", "2304", "4608", "pieces"])
+], ids=["1024", "1025", "5000", "16384", "16385", "2304", "4608", "pieces"])
 def test_tiles(nemo_mod, oracle_mod, deg):
     n = len(deg)
     rng = np.random.default_rng(n)
