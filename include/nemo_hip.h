@@ -187,7 +187,7 @@ typedef struct nemo_hip_info {
 	unsigned long long synapses;
 	unsigned long long plastic_synapses;
 	unsigned long long device_bytes;
-	unsigned lds_bytes;
+	unsigned lds_bytes;          /* per workgroup; without the far list of a launch of its own that has far waves */
 	unsigned block_threads;
 	float last_kernel_ms;        /* step-kernel time of the last run: HIP events for its own launches;
 	                              * in a batched run, its workgroups' first start to last end */

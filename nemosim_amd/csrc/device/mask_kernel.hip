@@ -1,6 +1,7 @@
 /*
  * mask_kernel.hip -- the persistent step: the fused kernel of step_kernel.hip
- * with another exchange between partitions, and with STDP on waves of its own.
+ * with another exchange between partitions, and with far waves, which deliver
+ * the previous cycle's records of delays >= 2, and STDP beside the neurons'.
  *
  * There, a partition publishes a list of its fired neurons and a count, and
  * the others read the counts, then the entries, then each source's bucket
@@ -15,12 +16,14 @@
  * that are in flight together.
  *
  * What bounds it: the latency of the chain update -> words -> bounds -> delay-1
- * records of one cycle; no unit is busy. Per cycle, against the lists on the
- * same build: 1k x 100 5.2 -> 3.9 us (with stimulus), 10k x 313 5.6 -> 4.4,
- * 60k x 300 6.3 -> 5.3, 100k x 100 (20 cycles) 9.1 -> 7.5, 200k x 1000 13.8 ->
- * 12.2, 12k x 550 IF_curr_exp_noise at 333 Hz 57 -> 48; 48 networks of 1k-20k
- * batched, 200 cycles, 3.96 -> 3.04 ms. With STDP, 3k x 300 10.9 -> 3.6 us, 10k
- * x 300 10.5 -> 4.2, 50k x 1000 17.4 -> 11.9 (see stdp_waves).
+ * records of one cycle; no unit is busy. From 200k neurons on, with few waves
+ * left over, the requests for bounds and records. Per cycle, lists, words with
+ * the far records on the neurons' waves, and on far waves: 1k x 100 4.5, 3.5,
+ * 2.6 us; 10k x 313 5.6, 4.6, 3.5; 60k x 300 6.3, 5.7, 4.6; 100k x 100 7.6, 6.3,
+ * 5.3; 200k x 1000 13.8, 12.9, 12.9; 12k x 550 IF_curr_exp_noise at 333 Hz 57,
+ * 49, 38. 48 networks of 1k-20k batched (no far waves), 200 cycles, 3.96 ->
+ * 3.04 ms. With STDP, 3k x 300 10.9 -> 3.5 us, 10k
+ * x 300 10.5 -> 4.3, 50k x 1000 17.4 -> 10.7 (see stdp_waves).
  *
  * Without STDP two buffers of words are enough: a wave publishes cycle t+1 after its own
  * reads of cycle t, and a workgroup publishes t+2 only once its waves have
@@ -100,6 +103,16 @@ __device__ inline int32_t stdp_change(const StdpMasks& m, uint32_t postLen, cons
 		w += da == db ? 0u : uint32_t(v);
 	}
 	return int32_t(w);
+}
+
+/* Lanes per source: as many as cover a bucket in one pass, fewer (down to
+ * glog2) where that would take more rounds than are in flight together */
+template<bool SAT, bool IZO>
+__device__ inline uint32_t lanes_for(const NetDev& nd, uint32_t nsrc)
+{
+	uint32_t g = nd.glogFew;
+	while(g > nd.glog2 && pass_rounds(nsrc, g) > DeliverRounds<SAT, IZO>::value) --g;
+	return g;
 }
 
 /* ---- STDP (src/nemo/ConnectivityMatrix.cpp:193-227), on waves of its own that
@@ -267,6 +280,23 @@ __device__ inline void stdp_waves(const NetDev& nd, uint32_t p, uint32_t wave, u
 	if(nd.nsteps > 0u) accumulate(uint32_t(nd.cycle0) + nd.nsteps - 1u, wslot ? wslot - 1u : R - 1u);
 }
 
+/* The far list of a cycle (ranges [x, y) of records, relative to ring slot
+ * base) by nw waves, wave w taking a contiguous share */
+template<bool SAT, bool IZO>
+__device__ inline void deliver_far(const NetDev& nd, const uint2* far, uint32_t count, uint32_t w, uint32_t nw,
+		uint32_t lane, uint32_t base, const NEMO_GLOBAL uint2* syn, int32_t* ringE, int32_t* ringI, uint32_t* ovf)
+{
+	const uint32_t share = (count + nw - 1u) / nw;
+	const uint32_t j0 = min(count, w * share), j1 = min(count, j0 + share);
+	for(uint32_t jb = j0; jb < j1; jb += 128u) {   /* wave-uniform */
+		const uint32_t nsrc = min(128u, j1 - jb);
+		const uint2 e0 = lane < nsrc ? far[jb + lane] : make_uint2(0u, 0u);
+		const uint2 e1 = 64u + lane < nsrc ? far[jb + 64u + lane] : make_uint2(0u, 0u);
+		deliver_ranges<SAT, IZO>(e0.x, e0.y, e1.x, e1.y, nsrc, lanes_for<SAT, IZO>(nd, nsrc), lane, base, syn,
+				ringE, ringI, ovf, nd.D, nd.T, nd.T >> 5);
+	}
+}
+
 /* WORDS: words a lane polls together. A wave whose share of the words takes
  * more than 64 WORDS of them goes through the rest of the cycle's chain once
  * per 64 WORDS, and every word costs instructions whether it is there or not
@@ -309,6 +339,14 @@ __device__ __forceinline__ void run_masked(const NetDev& nd, uint32_t p)
 	stdpLds.count = reinterpret_cast<uint32_t*>(stdpLds.work + 2u * NEMO_MASK_STDP_CAP);
 	stdpLds.masks = reinterpret_cast<StdpMasks*>(stdpLds.count + 4);
 	stdpLds.records = stdpLds.count + 16;
+	/* With far waves: two far lists, by cycle parity. The neurons' waves of
+	 * cycle t leave the ranges of delays >= 2 there, which the far waves
+	 * deliver in cycle t+1, none of them into slot t+1. */
+	const uint32_t nfw = nd.farWaves, fcap = nd.farCap;
+	uint2* far = reinterpret_cast<uint2*>(STDP ? reinterpret_cast<uint8_t*>(stdpLds.records + 2u * nd.stdpCache * CHUNK) : area);
+	uint32_t* farAsked = reinterpret_cast<uint32_t*>(far + 2u * fcap);   /* [2] */
+	uint32_t* farLen = farAsked + 2;                                     /* [2] */
+	if(nfw && tid < 2u) farAsked[tid] = farLen[tid] = 0u;
 	const bool defer = (nd.flags & NEMO_NET_DEFER) != 0u;
 	const uint32_t offMask = defer ? ((1u << OFF_NEAR_SHIFT) - 1u) : ~0u;
 	const NEMO_GLOBAL uint2* syn = glb(reinterpret_cast<const uint2*>(nd.syn));
@@ -362,13 +400,7 @@ __device__ __forceinline__ void run_masked(const NetDev& nd, uint32_t p)
 	/* deferred delivery: this wave's far ranges (delays >= 2) of the previous
 	 * cycle's sources, one per lane, kn of them (wave-uniform) */
 	uint32_t ka0 = 0, kb0 = 0, ka1 = 0, kb1 = 0, kn = 0;
-	/* Lanes per source: as many as cover a bucket in one pass, fewer (down to
-	 * glog2) where that would take more rounds than are in flight together */
-	auto lanes = [&](uint32_t nsrc) {
-		uint32_t g = nd.glogFew;
-		while(g > nd.glog2 && pass_rounds(nsrc, g) > DeliverRounds<SAT, IZO>::value) --g;
-		return g;
-	};
+	auto lanes = [&](uint32_t nsrc) { return lanes_for<SAT, IZO>(nd, nsrc); };
 	/* the Gaussian input of Izhikevich networks is drawn a cycle ahead */
 	float noise = 0.0f;
 	if(IZO && active && nd.nsteps > 0u && prm[IZ_SIGMA] != 0.0f) {
@@ -397,7 +429,7 @@ __device__ __forceinline__ void run_masked(const NetDev& nd, uint32_t p)
 	 * and stored before the cycle's last barrier; the update that reads them
 	 * clears them. */
 	const bool sched = nd.fs_ptr != nullptr;
-	const uint32_t sthreads = STDP ? T : nthreads;   /* threads that take entries */
+	const uint32_t sthreads = STDP || nfw ? T : nthreads;   /* threads that take entries */
 	const bool takes = tid < sthreads;
 	uint32_t fb = 0, fe = 0, ib = 0, ie = 0;    /* bounds of the next cycle's entries */
 	const uint32_t lo = p * T;
@@ -426,7 +458,23 @@ __device__ __forceinline__ void run_masked(const NetDev& nd, uint32_t p)
 
 	const bool learns = STDP && wave >= nw && wave < nw + nsw;   /* its barriers are those of this loop */
 	if(learns) stdp_waves<SAT, WORDS, IZO ? 8u : 4u>(nd, p, wave - nw, nsw, lane, stdpLds, list);
-	const uint32_t nsteps = learns ? 0u : nd.nsteps;
+	const bool carries = nfw && wave >= nw + nsw && wave < nw + nsw + nfw;
+	if(carries) {
+		uint32_t prev = slotK;   /* slot of the cycle before */
+		for(uint32_t k = 0; k < nd.nsteps; ++k) {
+			const uint32_t par = uint32_t(nd.cycle0 + k) & 1u;
+			prev = prev ? prev - 1u : D - 1u;
+			__syncthreads();
+			if(SAT) __syncthreads();
+			if(k > 0u) {
+				deliver_far<SAT, IZO>(nd, far + (par ^ 1u) * fcap, farLen[par ^ 1u], wave - nw - nsw, nfw, lane, prev, syn,
+						ringE, ringI, ovf);
+			}
+			__syncthreads();
+			prev = prev + 2u >= D ? prev + 2u - D : prev + 2u;
+		}
+	}
+	const uint32_t nsteps = learns || carries ? 0u : nd.nsteps;
 	for(uint32_t k = 0; k < nsteps; ++k) {
 		const uint64_t t = nd.cycle0 + k;
 		const uint32_t tag = uint32_t(t);
@@ -463,6 +511,8 @@ __device__ __forceinline__ void run_masked(const NetDev& nd, uint32_t p)
 			recent = (recent << 1) | (fired ? 1ull : 0ull);
 			if(STDP) st_agent(glb(nd.rfg) + size_t(tag & 3u) * n_total + n, recent);
 		}
+
+		if(nfw && tid == 0u) farAsked[tag & 1u] = farLen[tag & 1u] = 0u;   /* the last list of this parity is done */
 
 		/* ---- 2. publish the wave's fired bits; the raster */
 		const uint64_t mask = __ballot(fired);
@@ -630,7 +680,19 @@ __device__ __forceinline__ void run_masked(const NetDev& nd, uint32_t p)
 				a0 &= offMask;
 				a1 &= offMask;
 				events += (b0r - a0) + (b1r - a1);
-				if(defer && first) {
+				/* places in the far list. Once a wave asks for more than are
+				 * left, no wave gets any more in this cycle, so the places
+				 * given are the first farLen of the list, without gaps. */
+				uint32_t at = ~0u;
+				if(defer && nfw) {
+					if(lane == 0u) {
+						at = atomicAdd(farAsked + (tag & 1u), nsrc);
+						if(at + nsrc > fcap) at = ~0u;
+						else atomicAdd(farLen + (tag & 1u), nsrc);
+					}
+					at = uint32_t(__builtin_amdgcn_readfirstlane(int(at)));
+				}
+				if(defer && (nfw ? at != ~0u : first)) {
 					/* the records of delay 1 (first in each bucket, their count
 					 * in the top bits of its start) now, the rest in the next
 					 * cycle while its words are under way */
@@ -647,12 +709,18 @@ __device__ __forceinline__ void run_masked(const NetDev& nd, uint32_t p)
 						if(ok10) ring_add<SAT>(ringE, ringI, ovf, D, T, fwords, sl, r10.x & 0xffffu, int32_t(r10.y));
 						if(ok11) ring_add<SAT>(ringE, ringI, ovf, D, T, fwords, sl, r11.x & 0xffffu, int32_t(r11.y));
 					}
-					ka0 = a0 + n0;
-					kb0 = b0r;
-					ka1 = a1 + n1;
-					kb1 = b1r;
-					kn = nsrc;
-					first = false;
+					if(nfw) {
+						uint2* f = far + (tag & 1u) * fcap + at;
+						if(v0) f[lane] = make_uint2(a0 + n0, b0r);
+						if(v1) f[64u + lane] = make_uint2(a1 + n1, b1r);
+					} else {
+						ka0 = a0 + n0;
+						kb0 = b0r;
+						ka1 = a1 + n1;
+						kb1 = b1r;
+						kn = nsrc;
+						first = false;
+					}
 				} else {
 					deliver_ranges<SAT, IZO>(a0, b0r, a1, b1r, nsrc, lanes(nsrc), lane, slot, syn,
 							ringE, ringI, ovf, D, T, fwords);
@@ -678,6 +746,11 @@ __device__ __forceinline__ void run_masked(const NetDev& nd, uint32_t p)
 	}
 
 	/* ---- the last cycle's deferred records */
+	if(nfw && nd.nsteps > 0u) {
+		const uint64_t tc = nd.cycle0 + nd.nsteps - 1u;
+		deliver_far<SAT, IZO>(nd, far + (uint32_t(tc) & 1u) * fcap, farLen[uint32_t(tc) & 1u], wave, nwaves, lane,
+				uint32_t(tc % D), syn, ringE, ringI, ovf);
+	}
 	if(kn) {
 		deliver_ranges<SAT, IZO>(ka0, kb0, ka1, kb1, kn, lanes(kn), lane,
 				uint32_t((nd.cycle0 + nd.nsteps - 1u) % D), syn, ringE, ringI, ovf, D, T, fwords);

@@ -58,11 +58,13 @@ typedef struct NetDev {
 	uint32_t flRing;     /* fired lists and counts, or fired words, kept for this many cycles (buffer t mod flRing) */
 	uint32_t stdpCache;  /* STDP chunks whose reverse records are staged in LDS (64 words each) */
 	uint32_t stdpWaves;  /* waves for STDP after those of the neurons (NEMO_NET_MASKS) */
+	uint32_t farWaves;   /* with NEMO_NET_MASKS and NEMO_NET_DEFER: waves after those that deliver the previous
+	                      * cycle's far records (0: the neurons' waves do) */
 	uint32_t exWaves;    /* with NEMO_NET_DEFER: waves of a workgroup that run the exchange and the
 	                      * delay-1 delivery while the others deliver the previous cycle's far
 	                      * records (0: every wave does both, one after the other) */
 	uint32_t farCap;     /* fired sources per cycle whose far ranges fit the LDS far list (multiple
-	                      * of 64; with exWaves > 0) */
+	                      * of 64; with exWaves or farWaves) */
 	uint64_t cycle0;     /* cycle count at the start of the launch */
 
 	const uint8_t* model;     /* [n] model id */
@@ -255,7 +257,11 @@ static inline uint32_t nemo_mask_lds_bytes(uint32_t T, uint32_t D, int saturate)
 	return 2u * D * T * 4u + T * 4u + (T / 32u) * 4u + (saturate ? 2u * D * (T / 32u) * 4u : 0u) + (T / 64u) * 256u;
 }
 
-/* and with STDP: the sources of its waves, the tables, two work lists (by
+/* and with farWaves: two far lists (by cycle parity) of cap ranges, and their
+ * lengths, at the end */
+#define NEMO_MASK_FAR_LDS_BYTES(cap) (16u * (cap) + 16u)
+
+/* with STDP: the sources of its waves, the tables, two work lists (by
  * cycle parity) and their lengths, and the staged reverse records of both */
 static inline uint32_t nemo_mask_stdp_lds_bytes(uint32_t waves, uint32_t cache)
 {

@@ -141,7 +141,7 @@ runBatch(Simulation* const sims[], size_t n, const unsigned nsteps[], unsigned l
 		const Simulation* b = sims[y];
 		if(a->device() != b->device()) return a->device() < b->device();
 		if(a->variant() != b->variant()) return a->variant() < b->variant();
-		return a->blockThreads() < b->blockThreads();
+		return a->batchThreads() < b->batchThreads();
 	});
 	size_t i = 0;
 	while(i < order.size()) {
@@ -155,7 +155,7 @@ runBatch(Simulation* const sims[], size_t n, const unsigned nsteps[], unsigned l
 		while(j < order.size()) {
 			Simulation* sim = sims[order[j]];
 			if(sim->device() != dev || sim->variant() != variant) break;
-			const uint32_t bd = std::max(blockDim, sim->blockThreads());
+			const uint32_t bd = std::max(blockDim, sim->batchThreads());
 			const uint32_t ld = std::max(lds, sim->batchLdsBytes());
 			uint32_t maxB = 0;
 			hipCheck(nemo_dev_step_max_blocks(bd, ld, variant, &maxB), "occupancy query");

@@ -392,8 +392,8 @@ Simulation::Simulation(const NetworkImpl& net, const ConfigurationImpl& conf) :
 	 * few neurons per workgroup. Per cycle, lists against words: 1k x 100 4.5
 	 * -> 3.4 us, 10k x 1000 9.1 -> 6.0, 60k x 300 6.3 -> 5.4, 200k x 1000 13.8
 	 * -> 12.8, 12k x 550 IF_curr_exp_noise at 333 Hz 57 -> 47; with STDP 3k x
-	 * 300 10.9 -> 3.6, 10k x 300 10.5 -> 4.2, 50k x 1000 17.4 -> 11.9, 12k x
-	 * 550 at 333 Hz 283 -> 98. With STDP lists remain for what words do not
+	 * 300 10.9 -> 3.5, 10k x 300 10.5 -> 4.3, 50k x 1000 17.4 -> 10.7, 12k x
+	 * 550 at 333 Hz 283 -> 70. With STDP lists remain for what words do not
 	 * have: a window without cycles after the spike, work lists that are not to
 	 * be staged, workgroups that leave less than 6 of 16 waves for it, and a
 	 * configured workgroup of 512 neurons or more, which gets exchange waves. */
@@ -416,19 +416,26 @@ Simulation::Simulation(const NetworkImpl& net, const ConfigurationImpl& conf) :
 		}
 		return nemo_step_lds_bytes(t, m_D, std::max(1u, p), m_saturate ? 1 : 0, m_stdp ? 1 : 0);
 	};
+	m_izOnly = !m_model.empty() && std::all_of(m_model.begin(), m_model.end(),
+			[](uint8_t m) { return m == uint8_t(nemo_dev::MODEL_IZHIKEVICH); });
 	/* T: neurons per partition. The automatic choice takes at most one
-	 * partition per compute unit (256), and for mid-size networks fewer,
-	 * wider partitions: their cycle is bound by the exchange between
-	 * partitions. The LDS ring [D][T] bounds it from above.
-	 *   With words: about 27 partitions of up to 512 neurons (3k x 300: 128
-	 * neurons 3.7 us per cycle, 256 4.1; 10k x 100: 384 4.0, 128 4.1, 960 4.9;
-	 * 20k x 1000: 320 6.3, 512 6.9, 960 7.6), rows of 500 synapses from 1.5k to
-	 * 3k neurons about 13 (2k x 1000: 192 4.1, 128 5.3, 512 6.2), from 48k
-	 * neurons on about 160 (100k x 300: 640 6.5, 832 6.9; 200k x 1000: 960
-	 * 12.8, 832 13.7).
-	 *   With words and STDP: about 27 partitions up to 6k neurons, 79 from there
-	 * (10k x 300: 128 neurons 4.5, 384 4.8; 20k x 1000: 256 7.6, 512 9.5; 50k x
-	 * 1000: 448 or 512 11.8, 256 11.9; 100k x 300: 512 10.1, 640 11.8).
+	 * partition per compute unit (256), and for small and mid-size networks
+	 * fewer, wider partitions: their cycle is bound by the exchange between
+	 * partitions. The LDS ring [D][T] bounds it from above. Times per cycle:
+	 *   With words: about 27 partitions (2k x 1000: 64 neurons 3.1 us, 192 4.2;
+	 * 3k x 300: 128 2.9, 256 3.3; 10k x 100: 384 3.1, 128 3.4, 640 3.3;
+	 * IF_curr_exp_noise at 333 Hz, 12k x 550: 448 38, 256 49), from 16k
+	 * Izhikevich neurons on about 79 (20k x 1000: 256 4.1, 512 4.8; 40k x 300:
+	 * 512 4.2, 256 4.6), up to 512 (60k x 300: 512 4.5, 768 4.8; 100k x 1000:
+	 * 512 7.9, 640 9.2) or what 256 partitions need (150k x 1000: 640 11.0, 960
+	 * 11.5), but 960 where few waves would be left for far records (200k x
+	 * 1000: 960 12.9, 832 14.1; 180k x 300: 960 8.2, 768 8.6).
+	 *   With STDP there: Izhikevich neurons in about 100 partitions below 16k
+	 * (5k x 1000: 64 4.2, 192 5.1; 10k x 300: 128 4.3, 64 4.9, 384 5.0) and 160
+	 * from there, up to 448 (20k x 1000: 128 6.5, 256 7.2; 50k x 1000: 320 10.7,
+	 * 512 11.9; 100k x 300: 448 9.8, 512 10.2); other models in 27 below 6k and
+	 * 79 from there (5k x 100 at 333 Hz: 192 12.3, 128 15.8; 12k x 550: 192 69,
+	 * 128 85, 448 106).
 	 *   With lists: about 40 partitions of up to 512 neurons (10k x 100: 7.2 ->
 	 * 6.3 us; 50k x 1000: 10.4 -> 9.7 us), and with rows of 500 synapses or
 	 * more, from 1.5k to 12k neurons, about 13 partitions (2k x 1000: 8.0 ->
@@ -439,13 +446,21 @@ Simulation::Simulation(const NetworkImpl& net, const ConfigurationImpl& conf) :
 			t = std::min(1024u, roundUp64(conf.partitionSize));
 		} else {
 			const uint32_t perCU = roundUp64(std::max<uint32_t>(1u, (m_n + 255u) / 256u));
-			const bool large = m_masks && !m_stdp && m_n >= 49152u;
-			const bool longRows = !(m_masks && m_stdp) && m_n >= 1500u && m_n <= (m_masks ? 3000u : 12000u) && m_nsyn / m_n >= 500u;
-			const uint32_t parts = m_masks && m_stdp ? (m_n < 6144u ? 27u : 79u)
-				: (longRows ? 13u : (large ? 160u : (m_masks ? 27u : 40u)));
-			uint32_t wide = roundUp64(std::max<uint32_t>(1u, (m_n + parts - 1u) / parts));
-			wide = std::min(longRows ? 1024u : (large ? 960u : 512u), std::max(wide, large ? 512u : 64u));
-			t = std::max(64u, std::min(1024u, std::max(perCU, wide)));
+			uint32_t parts = 40u, most = 512u, round = 63u;
+			if(m_masks && m_stdp) {
+				parts = m_izOnly ? (m_n < 16384u ? 100u : 160u) : (m_n < 6144u ? 27u : 79u);
+				most = m_izOnly ? 448u : 512u;
+			} else if(m_masks) {
+				parts = m_izOnly && m_n >= 16384u ? 79u : 27u;
+				round = 32u;   /* to the nearest multiple of 64 */
+			} else if(m_n >= 1500u && m_n <= 12000u && m_nsyn / m_n >= 500u) {
+				parts = 13u;
+				most = 1024u;
+			}
+			const uint32_t wide = ((m_n + parts - 1u) / parts + round) / 64u * 64u;
+			t = std::max(perCU, std::min(most, std::max(64u, wide)));
+			if(m_masks && !m_stdp && perCU > 704u) t = 960u;
+			t = std::min(1024u, t);
 		}
 		while(t > 64 && ldsFor(t) > ldsLimit) {
 			t -= 64;
@@ -453,8 +468,6 @@ Simulation::Simulation(const NetworkImpl& net, const ConfigurationImpl& conf) :
 		return t;
 	};
 	uint32_t T = partitionSize();
-	m_izOnly = !m_model.empty() && std::all_of(m_model.begin(), m_model.end(),
-			[](uint8_t m) { return m == uint8_t(nemo_dev::MODEL_IZHIKEVICH); });
 	if(m_masks && m_n > 0 && whyNotFused.empty()) {
 		uint32_t maxBlocks = 0;
 		const uint32_t lds = ldsFor(T);
@@ -1166,7 +1179,32 @@ Simulation::planExchange(const ConfigurationImpl& conf, uint32_t ldsLimit)
 	m_exAuto = false;
 	m_ldsNoFar = m_lds;
 	const uint32_t nw = m_T / 64u;
-	if(!m_fused || !m_defer || m_P == 0 || conf.exchangeWaves < 0 || m_masks) return;
+	m_farWaves = 0;
+	if(!m_fused || !m_defer || m_P == 0) return;
+	if(m_masks) {
+		/* Far waves: as many as the neurons' waves, at least 2, as far as 16 in
+		 * all go, unless the device cannot hold the larger workgroups or their
+		 * far list (256 sources per neurons' wave, or fewer, down to 64). Per
+		 * cycle without them, with 2, 4 and 8: 1k x 100 3.5, 2.6, 2.6, 2.6 us;
+		 * 20k x 1000 (512 neurons) 7.1, 7.6, 5.7, 4.9; 60k x 300 5.7, 6.4, 4.4,
+		 * 4.5; 12k x 550 at 333 Hz 49, 61, 38, 38. */
+		const uint32_t used = nw + m_stdpWaves;
+		const uint32_t n = used < 16u ? std::min(std::max(2u, nw), 16u - used) : 0u;
+		for(uint32_t cap = 256u * nw; n && cap >= 64u * nw; cap /= 2) {
+			const uint32_t lds = m_lds + NEMO_MASK_FAR_LDS_BYTES(cap);
+			uint32_t maxBlocks = 0;
+			if(lds > ldsLimit) continue;
+			hipCheck(nemo_dev_step_max_blocks(m_T + 64u * (used - nw + n), lds, variant(), &maxBlocks), "occupancy query");
+			if(m_P <= maxBlocks) {
+				m_farWaves = n;
+				m_farCap = cap;
+				m_lds = lds;
+				return;
+			}
+		}
+		return;
+	}
+	if(conf.exchangeWaves < 0) return;
 	uint32_t ex = uint32_t(conf.exchangeWaves);
 	if(conf.exchangeWaves == 0) {
 		if(!m_stdp || nw < 8u) return;
@@ -1195,7 +1233,10 @@ Simulation::prepareLaunch(unsigned nsteps, bool batched)
 	ensureRaster(size_t(nsteps) * m_words * 8);
 	m_rasterExternal = false;
 	NetDev nd = descriptor(nsteps);
-	if(batched && m_exAuto) {
+	if(batched && m_farWaves) {
+		nd.farWaves = 0;
+		nd.farCap = 0;
+	} else if(batched && m_exAuto) {
 		/* every launch delivers its last cycle's far records before it
 		 * ends, so launches with and without exchange waves can follow
 		 * each other */
@@ -1243,6 +1284,7 @@ Simulation::descriptor(unsigned nsteps) const
 	nd.flRing = m_flRing;
 	nd.stdpCache = m_stdpCache;
 	nd.stdpWaves = m_stdpWaves;
+	nd.farWaves = m_farWaves;
 	nd.exWaves = m_exWaves;
 	nd.farCap = m_farCap;
 	nd.cycle0 = m_cycle;
@@ -1865,7 +1907,7 @@ Simulation::info(nemo_hip_info_t* out) const
 	out->synapses = m_nsyn;
 	out->plastic_synapses = m_nplastic;
 	out->device_bytes = m_deviceBytes;
-	out->lds_bytes = m_lds;
+	out->lds_bytes = m_farWaves ? m_ldsNoFar : m_lds;
 	out->block_threads = blockThreads();
 	out->last_kernel_ms = m_kernelMs;
 	out->fused = m_fused ? 1u : 0u;

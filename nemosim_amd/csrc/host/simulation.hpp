@@ -106,13 +106,14 @@ class Simulation
 
 		/* batched launches (nemo_hip_run_batch) */
 		uint32_t partitions() const { return m_P; }
-		uint32_t blockThreads() const { return m_T + 64u * m_stdpWaves; }
+		uint32_t blockThreads() const { return m_T + 64u * (m_stdpWaves + m_farWaves); }
+		uint32_t batchThreads() const { return m_T + 64u * m_stdpWaves; }
 		uint32_t ldsBytes() const { return m_lds; }
 		/* LDS of a batched launch: without the far list of exchange waves
 		 * the library chose by itself (a batched launch runs every
 		 * workgroup at its largest member's LDS, so one network's far list
 		 * would take co-residency from all the others) */
-		uint32_t batchLdsBytes() const { return m_exAuto ? m_ldsNoFar : m_lds; }
+		uint32_t batchLdsBytes() const { return m_exAuto || m_farWaves ? m_ldsNoFar : m_lds; }
 		/* the step-kernel time of the last run, for a batched one: from the
 		 * first start to the last end of this network's workgroups */
 		void setKernelMs(float ms) { m_kernelMs = ms; }
@@ -186,6 +187,7 @@ class Simulation
 		/* cycles of fired lists and counts kept on the device */
 		uint32_t m_flRing = 2;
 		uint32_t m_stdpWaves = 0;    /* of mask_kernel.hip */
+		uint32_t m_farWaves = 0;
 		uint32_t m_stdpCache = 0;    /* STDP chunks staged in LDS per cycle */
 		bool m_prefRing = false;     /* STDP list prefixes of postLen cycles kept in LDS */
 		uint32_t m_exWaves = 0;      /* exchange waves (NetDev.exWaves) */

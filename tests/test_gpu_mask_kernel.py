@@ -65,6 +65,8 @@ def check(sim, orc, cycles, fstim=None, istim=None):
     (1500, 200, (1, 5, 20), False, 900.0, 128),        # saturating
     (1300, 200, (3, 20), True, 900.0, 320),
     (513, 600, (1, 2, 3), False, 1.0, 0),              # buckets longer than a pass
+    (6000, 40, (1, 2, 20), True, 1.0, 320),            # five waves, more sources than the far list holds (1280)
+    (6000, 40, (1, 2, 20), True, 1.0, 640),            # ten waves and six for far records
 ])
 def test_mask_kernel(nemo_mod, oracle_mod, n, m, delays, mixed, gain, T):
     sim, orc = build(nemo_mod, oracle_mod, n, m, delays, mixed, gain, T)
