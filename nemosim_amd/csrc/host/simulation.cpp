@@ -1227,13 +1227,13 @@ Simulation::planExchange(const ConfigurationImpl& conf, uint32_t ldsLimit)
 }
 
 NetDev
-Simulation::prepareLaunch(unsigned nsteps, bool batched)
+Simulation::prepareLaunch(unsigned nsteps, bool batched, bool far)
 {
 	hipCheck(hipSetDevice(m_device), "hipSetDevice");
 	ensureRaster(size_t(nsteps) * m_words * 8);
 	m_rasterExternal = false;
 	NetDev nd = descriptor(nsteps);
-	if(batched && m_farWaves) {
+	if(batched && m_farWaves && !far) {
 		nd.farWaves = 0;
 		nd.farCap = 0;
 	} else if(batched && m_exAuto) {

@@ -110,17 +110,20 @@ class Simulation
 		uint32_t batchThreads() const { return m_T + 64u * m_stdpWaves; }
 		uint32_t ldsBytes() const { return m_lds; }
 		/* LDS of a batched launch: without the far list of exchange waves
-		 * the library chose by itself (a batched launch runs every
-		 * workgroup at its largest member's LDS, so one network's far list
-		 * would take co-residency from all the others) */
+		 * or far waves the library chose by itself (a batched launch runs
+		 * every workgroup at its largest member's LDS, so one network's far
+		 * list would take co-residency from all the others), or, where all
+		 * members fit with them, with that of far waves */
 		uint32_t batchLdsBytes() const { return m_exAuto || m_farWaves ? m_ldsNoFar : m_lds; }
+		uint32_t farLdsBytes() const { return m_farWaves ? m_lds : batchLdsBytes(); }
 		/* the step-kernel time of the last run, for a batched one: from the
 		 * first start to the last end of this network's workgroups */
 		void setKernelMs(float ms) { m_kernelMs = ms; }
 		/* prepare a launch of nsteps cycles: fills and returns the device
 		 * descriptor (host copy) with per-launch fields set; batched: as
-		 * one member of a batched launch (see batchLdsBytes) */
-		NetDev prepareLaunch(unsigned nsteps, bool batched = false);
+		 * one member of a batched launch (see batchLdsBytes), far: with far
+		 * waves */
+		NetDev prepareLaunch(unsigned nsteps, bool batched = false, bool far = false);
 		/* advance the cycle count by a finished launch; throws on a status
 		 * error. ctl holds the first 8 words of the control block as the
 		 * launch left them, counted from zero at the launch's start (a
