@@ -189,8 +189,8 @@ typedef struct nemo_hip_info {
 	unsigned long long device_bytes;
 	unsigned lds_bytes;          /* per workgroup; without the far list of a launch of its own that has far waves */
 	unsigned block_threads;
-	float last_kernel_ms;        /* step-kernel time of the last run: HIP events for its own launches;
-	                              * in a batched run, its workgroups' first start to last end */
+	float last_kernel_ms;        /* step-kernel time of the last run, from the first start to the last end of its
+	                              * workgroups (plugin and per-cycle step: HIP events around its launches) */
 	unsigned fused;              /* 1: fused persistent step kernel; 0: plugin step */
 	unsigned deferred;           /* 1: records of delay >= 2 delivered one cycle late */
 	unsigned lanes_per_source;   /* lanes sharing one fired source in delivery */

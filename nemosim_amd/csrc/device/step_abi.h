@@ -35,8 +35,8 @@ extern "C" {
  * status, [2..3] delivered-synapse count, and, for the first timeout,
  * [4] cycle, [5] waiting partition, [6] awaited partition, [7] workgroups
  * started by then; [8..9] the earliest start and [10..11] the latest end
- * of its workgroups on the device wall clock (read after batched
- * launches, whose graph initialises them). */
+ * of its workgroups on the device wall clock, all-ones and zero before a
+ * launch. */
 #define NEMO_CTL_WORDS 16u
 
 /*
@@ -118,6 +118,7 @@ typedef struct NetDev {
  * clock at its start and end, then the launch's number */
 typedef struct CycleReport {
 	uint64_t start, end;
+	uint32_t ctl[8];          /* the control block's first words (nemo_dev_step_report) */
 	uint64_t sequence;
 } CycleReport;
 
@@ -165,6 +166,9 @@ int nemo_dev_step_launch_one(const NetDev* nd_host, const WorkItem* work_dev, ui
 /* One cycle of a network without STDP whose sums stay within int32 */
 int nemo_dev_cycle(const NetDev* nd_host, const CycleArgs* ca, void* stream);
 uint32_t nemo_dev_cycle_blocks(uint32_t P, uint32_t T);
+/* The end of a launch of one network, after its step kernel on the stream: its
+ * control block to host memory, then the report; the clock words start anew. */
+int nemo_dev_step_report(uint32_t* ctl, CycleReport* report, uint64_t sequence, void* stream);
 int nemo_dev_step_max_blocks(uint32_t blockDim, uint32_t ldsBytes, uint32_t variant, uint32_t* maxBlocks);
 /* Batched step as an instantiated HIP graph (clear -> persistent step ->
  * collect); collect_dev receives [nnets][16] words: the first 12 words of

@@ -44,6 +44,7 @@
 #include <algorithm>
 #include <stdint.h>
 
+#include "host_report.h"
 #include "step_device.h"
 
 static_assert(sizeof(StdpParams) <= NEMO_STDP_LDS_BYTES, "STDP tables must fit their LDS area");
@@ -1130,9 +1131,25 @@ __global__ void nemo_batch_clear_kernel(const NetDev* __restrict__ nets, uint32_
 __global__ void nemo_batch_collect_kernel(const NetDev* __restrict__ nets, uint32_t count, uint32_t* __restrict__ out)
 {
 	for(uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < count; i += gridDim.x * blockDim.x) {
-		const uint32_t* ctl = nets[i].status - 1;
+		uint32_t* ctl = nets[i].status - 1;
 		for(uint32_t w = 0; w < 12u; ++w) out[16 * i + w] = ctl[w];
+		ctl[8] = ctl[9] = ~0u;   /* for a launch of its own */
+		ctl[10] = ctl[11] = 0u;
 	}
+}
+
+/* After the step kernel of one network: what the host needs, polled there. In
+ * the step kernel itself, as the last workgroup's end, it costs registers that
+ * the cycles need (1k x 100 with stimulus 70 ns each). */
+__global__ void nemo_report_kernel(uint32_t* ctl, CycleReport* r, uint64_t sequence)
+{
+	for(uint32_t w = 0; w < 8u; ++w) st_host(r->ctl + w, ctl[w]);
+	st_host(&r->start, uint64_t(ctl[8]) | (uint64_t(ctl[9]) << 32));
+	st_host(&r->end, uint64_t(ctl[10]) | (uint64_t(ctl[11]) << 32));
+	ctl[8] = ctl[9] = ~0u;
+	ctl[10] = ctl[11] = 0u;
+	__builtin_amdgcn_s_waitcnt(0);
+	st_host(&r->sequence, sequence);
 }
 
 /* applyStdp: src/nemo/ConnectivityMatrix.cpp:241-294. With reward 0 every
@@ -1222,6 +1239,12 @@ int nemo_dev_step_launch_one(const NetDev* nd_host, const WorkItem* work_dev, ui
 	void* args[] = { const_cast<NetDev*>(nd_host), const_cast<WorkItem**>(&work_dev) };
 	e = hipLaunchKernel(kern, dim3(nblocks), dim3(blockDim), args, ldsBytes, static_cast<hipStream_t>(stream));
 	return int(e);
+}
+
+int nemo_dev_step_report(uint32_t* ctl, CycleReport* report, uint64_t sequence, void* stream)
+{
+	hipLaunchKernelGGL(nemo_report_kernel, dim3(1), dim3(1), 0, static_cast<hipStream_t>(stream), ctl, report, sequence);
+	return int(hipGetLastError());
 }
 
 /* The batched step as a HIP graph: clear -> step -> collect.

