@@ -42,6 +42,7 @@
  */
 #include <hip/hip_runtime.h>
 #include <algorithm>
+#include <stddef.h>
 #include <stdint.h>
 
 #include "host_report.h"
@@ -1141,15 +1142,19 @@ __global__ void nemo_batch_collect_kernel(const NetDev* __restrict__ nets, uint3
 /* After the step kernel of one network: what the host needs, polled there. In
  * the step kernel itself, as the last workgroup's end, it costs registers that
  * the cycles need (1k x 100 with stimulus 70 ns each). */
-__global__ void nemo_report_kernel(uint32_t* ctl, CycleReport* r, uint64_t sequence)
+__global__ void __launch_bounds__(64) nemo_report_kernel(uint32_t* ctl, CycleReport* r, uint64_t sequence)
 {
-	for(uint32_t w = 0; w < 8u; ++w) st_host(r->ctl + w, ctl[w]);
-	st_host(&r->start, uint64_t(ctl[8]) | (uint64_t(ctl[9]) << 32));
-	st_host(&r->end, uint64_t(ctl[10]) | (uint64_t(ctl[11]) << 32));
-	ctl[8] = ctl[9] = ~0u;
-	ctl[10] = ctl[11] = 0u;
+	/* a word of the report per lane: start and end (words 8..11 of the control
+	 * block), then its first 8 */
+	static_assert(offsetof(CycleReport, end) == 8u && offsetof(CycleReport, ctl) == 16u, "words of the report");
+	const uint32_t lane = threadIdx.x;
+	if(lane < 12u) {
+		uint32_t* w = ctl + (lane < 4u ? 8u + lane : lane - 4u);
+		st_host(reinterpret_cast<uint32_t*>(r) + lane, *w);
+		if(lane < 4u) *w = lane < 2u ? ~0u : 0u;
+	}
 	__builtin_amdgcn_s_waitcnt(0);
-	st_host(&r->sequence, sequence);
+	if(lane == 0u) st_host(&r->sequence, sequence);
 }
 
 /* applyStdp: src/nemo/ConnectivityMatrix.cpp:241-294. With reward 0 every
@@ -1243,7 +1248,7 @@ int nemo_dev_step_launch_one(const NetDev* nd_host, const WorkItem* work_dev, ui
 
 int nemo_dev_step_report(uint32_t* ctl, CycleReport* report, uint64_t sequence, void* stream)
 {
-	hipLaunchKernelGGL(nemo_report_kernel, dim3(1), dim3(1), 0, static_cast<hipStream_t>(stream), ctl, report, sequence);
+	hipLaunchKernelGGL(nemo_report_kernel, dim3(1), dim3(64), 0, static_cast<hipStream_t>(stream), ctl, report, sequence);
 	return int(hipGetLastError());
 }
 

@@ -1536,7 +1536,7 @@ Simulation::launchDescriptor(const NetDev& nd, bool stepOut)
 {
 	/* the control block comes by a kernel that reports to pinned memory, where
 	 * this polls: with two timing events, a copy and a stream synchronisation
-	 * in its place a run takes 8 us more (20 cycles of 1k x 100 83 us, now 75) */
+	 * in its place a run takes 13 us more (20 cycles of 1k x 100 83 us, now 69) */
 	hipStream_t st = static_cast<hipStream_t>(m_stream);
 	CycleReport* rep = reinterpret_cast<CycleReport*>(h_ctl + NEMO_CTL_WORDS);
 	hipCheck(nemo_dev_step_launch_one(&nd, d_work.as<WorkItem>(), m_P, blockThreads(), m_lds, variant(), st),
