@@ -261,7 +261,7 @@ def bench_plain(args, stdp=False):
         },
         "roofline": {
             "bound": "hbm",
-            "kernel": "nemo_step_kernel",
+            "kernel": "nemo_mask_kernel",
             "achieved": achieved,
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",
@@ -422,7 +422,7 @@ def bench_batch(args):
         "rasters_identical": "%d/%d" % (exact, count),
         "roofline": {
             "bound": "hbm",
-            "kernel": "nemo_step_kernel (batched launches)",
+            "kernel": "nemo_mask_kernel (batched launches)",
             # the algorithmic bytes of every network (8 B per delivered
             # record, 8 B per delivered row, 68 B per neuron and cycle) over
             # the wall time of the whole batched run: launches of several
