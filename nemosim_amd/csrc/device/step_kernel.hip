@@ -1,5 +1,9 @@
 /*
- * step_kernel.hip -- the simulation step on gfx950.
+ * step_kernel.hip -- the simulation step on gfx950, in the form that exchanges
+ * lists of fired neurons. Most networks run on mask_kernel.hip, which exchanges
+ * their fired bits; this one has what that has not: exchange waves, and STDP
+ * with unstaged work lists, without cycles after the spike or in workgroups that
+ * leave it no waves.
  *
  * One persistent kernel runs many 1 ms cycles of one or more independent
  * networks. Each workgroup owns one partition of T target neurons of one
