@@ -1155,7 +1155,9 @@ __global__ void __launch_bounds__(64) nemo_report_kernel(uint32_t* ctl, CycleRep
 	if(lane < 12u) {
 		uint32_t* w = ctl + (lane < 4u ? 8u + lane : lane - 4u);
 		st_host(reinterpret_cast<uint32_t*>(r) + lane, *w);
-		if(lane < 4u) *w = lane < 2u ? ~0u : 0u;
+		/* there before the report: a batched launch, on a stream of its own,
+		 * may be next to write them */
+		if(lane < 4u) st_agent(glb(w), lane < 2u ? ~0u : 0u);
 	}
 	__builtin_amdgcn_s_waitcnt(0);
 	if(lane == 0u) st_host(&r->sequence, sequence);

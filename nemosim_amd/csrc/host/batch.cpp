@@ -196,6 +196,7 @@ runBatch(Simulation* const sims[], size_t n, const unsigned nsteps[], unsigned l
 		for(size_t k : members) {
 			Simulation* sim = sims[k];
 			const uint32_t idx = uint32_t(nets.size());
+			sim->orderBefore(st);
 			nets.push_back(sim->prepareLaunch(nsteps[k], true, far));
 			for(uint32_t p = 0; p < sim->partitions(); ++p) items.push_back(std::make_pair(idx, p));
 		}

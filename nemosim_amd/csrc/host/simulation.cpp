@@ -1547,6 +1547,7 @@ Simulation::launchDescriptor(const NetDev& nd, bool stepOut)
 		hipCheck(hipStreamSynchronize(st), "hipStreamSynchronize");
 	}
 	waitReport(&rep->sequence, m_cycleSequence, st, "step kernel");
+	m_tail = false;
 	std::memcpy(h_ctl, rep->ctl, sizeof(rep->ctl));
 	m_kernelMs = float(double(rep->end - rep->start) / wallClockKHz(m_device));
 }
@@ -1692,10 +1693,25 @@ Simulation::stepCycle(const nemo_schedule_t& s)
 	ca.done = d_done.as<uint32_t>();
 	hipStream_t st = static_cast<hipStream_t>(m_stream);
 	hipCheck(nemo_dev_cycle(&nd, &ca, st), "cycle kernel launch");
+	m_tail = true;
 	waitReport(&rep->sequence, ca.sequence, st, "cycle kernel");
 	m_kernelMs = float(double(rep->end - rep->start) / wallClockKHz(m_device));
 	const uint32_t ctl[8] = {};
 	completeLaunch(1, ctl);
+}
+
+/* The cycle kernel reports from within: its ordinary stores (state, ring,
+ * history) may still be in an XCD's L2 then, and are written back at its end,
+ * which work on its own stream and on the null stream waits for, but no other
+ * does. Kernels that a kernel of their own reports for have ended by then. */
+void
+Simulation::orderBefore(void* stream)
+{
+	if(!m_tail) return;
+	hipEvent_t ev = static_cast<hipEvent_t>(m_ev1);
+	hipCheck(hipEventRecord(ev, static_cast<hipStream_t>(m_stream)), "hipEventRecord");
+	hipCheck(hipStreamWaitEvent(static_cast<hipStream_t>(stream), ev, 0), "hipStreamWaitEvent");
+	m_tail = false;
 }
 
 const std::vector<unsigned>&

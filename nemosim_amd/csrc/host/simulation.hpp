@@ -132,6 +132,9 @@ class Simulation
 		/* the control block's words as a batched launch left them on the
 		 * device: the base from which the next single launch counts */
 		void setControlBase(const uint32_t ctl[8]);
+		/* what this simulation's stream still runs comes before what `stream`
+		 * is given next (a batched launch has a stream of its own) */
+		void orderBefore(void* stream);
 		unsigned neuronCount() const { return m_n; }
 		int device() const { return m_device; }
 		/* step-kernel variant (nemo_step_variant): saturating, Izhikevich-only, masks */
@@ -259,7 +262,8 @@ class Simulation
 		bool cycleKernelRuns() const;
 		void stepCycle(const nemo_schedule_t& s);
 		DevBuf d_done;                 /* CycleArgs.done */
-		uint64_t m_cycleSequence = 0;  /* launches of the cycle kernel */
+		uint64_t m_cycleSequence = 0;  /* launches that report to h_ctl */
+		bool m_tail = false;           /* the cycle kernel has reported, its end was not waited for (orderBefore) */
 		void ensureRaster(size_t bytes);
 		NetDev descriptor(unsigned nsteps) const;
 		bool translateSchedule(unsigned nsteps, const nemo_schedule_t* s, std::vector<uint32_t>& fsPtr,
