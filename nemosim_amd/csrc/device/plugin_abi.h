@@ -63,7 +63,7 @@ int nemo_dev_pm_replay(const PluginStepDev* s, int narrow, void* stream);
  * curX, which are cleared */
 int nemo_dev_pm_cycle(const PluginStepDev* s, uint32_t k, int stim, int narrow, int izhikevichOnly, void* stream);
 /* workgroups of the kernels that count events in `part`, and their sum */
-#define NEMO_PM_SCATTER_BLOCKS 1024u
+#define NEMO_PM_SCATTER_BLOCKS 2048u
 uint32_t nemo_dev_pm_parts(uint32_t n);
 int nemo_dev_pm_finish(const PluginStepDev* s, void* stream);
 

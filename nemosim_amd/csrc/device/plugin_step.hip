@@ -88,39 +88,57 @@ __global__ void pm_stimulus_kernel(PluginStepDev s, uint32_t k)
 	}
 }
 
-/* The synapses of `count` fired sources (in LDS) into ring slots (base + d)
- * mod R, by the four waves of a workgroup: chunk c of 256 synapses of the j-th
- * source goes to wave (c + j) mod 4, four records per lane loaded together.
- * Returns the synapses of the chunks this wave did (wave-uniform). */
+/* The rows of up to 64 fired sources into ring slots (base + d) mod R, by the
+ * four waves of a workgroup. Lane l has the bounds ra, rb of a row if bit l of
+ * `rows` is set (the same in all four waves); chunk c of 256 synapses of the
+ * j-th row goes to wave (c + j) mod 4, four records per lane. The records of
+ * the wave's next chunk are loaded before this one's are added: a load waits
+ * for the atomics issued before it. Returns the synapses of the chunks this
+ * wave did (wave-uniform). */
 template<typename ACC>
-__device__ inline uint32_t deliver_listed(const PluginStepDev& s, const uint32_t* list, uint32_t count,
+__device__ inline uint32_t deliver_rows(const PluginStepDev& s, uint32_t ra, uint32_t rb, uint64_t rows,
 		uint32_t base, uint32_t wave, uint32_t lane)
 {
 	ACC* acc = static_cast<ACC*>(s.acc);
 	const uint2* syn = reinterpret_cast<const uint2*>(s.syn);
-	uint32_t ev = 0;
-	for(uint32_t j = 0; j < count; ++j) {
-		const uint32_t src = list[j];
-		const uint32_t a = s.off[src], b = s.off[src + 1];
-		for(uint32_t c = a + 256u * ((wave - j) & 3u); c < b; c += 1024u) {
-			uint2 rec[4];
-#pragma unroll
-			for(uint32_t i = 0; i < 4u; ++i) {
-				const uint32_t q = c + 64u * i + lane;
-				rec[i] = (q < b) ? syn[q] : make_uint2(0u, 0u);
-			}
-#pragma unroll
-			for(uint32_t i = 0; i < 4u; ++i) {
-				if(c + 64u * i + lane < b) {
-					const int32_t w = int32_t(rec[i].y);
-					uint32_t sl = base + (rec[i].x >> 26) + 1u;
-					sl = (sl >= s.R) ? sl - s.R : sl;
-					const uint32_t plane = (w >= 0) ? 0u : s.R;
-					acc_add(acc + size_t(plane + sl) * s.n + (rec[i].x & 0x3ffffffu), w);
-				}
-			}
-			ev += min(256u, b - c);
+	uint32_t ev = 0, j = 0, c = 0, b = 0;   /* the chunk and its row's end */
+	auto next = [&]() {   /* c >= b: none left */
+		c += 1024u;
+		while(c >= b && rows) {   /* wave-uniform */
+			const int l = __builtin_ctzll(rows);
+			rows &= rows - 1ull;
+			b = uint32_t(__builtin_amdgcn_readlane(int(rb), l));
+			c = uint32_t(__builtin_amdgcn_readlane(int(ra), l)) + 256u * ((wave - j) & 3u);
+			++j;
 		}
+	};
+	auto load = [&](uint2 (&rec)[4]) {
+#pragma unroll
+		for(uint32_t i = 0; i < 4u; ++i) {
+			const uint32_t q = c + 64u * i + lane;
+			rec[i] = (q < b) ? syn[q] : make_uint2(0u, 0u);
+		}
+	};
+	next();
+	uint2 rec[4];
+	load(rec);
+	while(c < b) {   /* wave-uniform */
+		const uint32_t c0 = c, b0 = b;
+		next();
+		uint2 ahead[4];
+		load(ahead);
+#pragma unroll
+		for(uint32_t i = 0; i < 4u; ++i) {
+			if(c0 + 64u * i + lane < b0) {
+				const int32_t w = int32_t(rec[i].y);
+				uint32_t sl = base + (rec[i].x >> 26) + 1u;
+				sl = (sl >= s.R) ? sl - s.R : sl;
+				const uint32_t plane = (w >= 0) ? 0u : s.R;
+				acc_add(acc + size_t(plane + sl) * s.n + (rec[i].x & 0x3ffffffu), w);
+			}
+			rec[i] = ahead[i];
+		}
+		ev += min(256u, b0 - c0);
 	}
 	return ev;
 }
@@ -139,38 +157,31 @@ __device__ inline void count_events(unsigned long long* part, uint32_t ev, uint3
 	}
 }
 
-/* Plugins: the fired bits of cycle k, listed and delivered. Each workgroup
- * takes 64 words of the raster (2048 neurons) at a time, lists their bits in
- * LDS and delivers them. */
+/* Plugins: the spikes of cycle k. Workgroup g of G takes the neurons g, g + G,
+ * g + 2G, ..., a lane each, so that all workgroups have sources whatever fires:
+ * neurons that fire together are often neighbours. Every wave reads the fired
+ * bits and the rows' bounds for itself, so nothing is listed and nothing
+ * waited for.
+ *
+ * What bounds it: with few spikes the launch; with many the atomics. Per cycle
+ * of the plugin step, with a wave per fired source of a list in memory, with a
+ * workgroup per 2048 neurons, and now: 2000 x 1000 IF_curr_exp_noise at 333 Hz
+ * 48, 1504, 44 us; 12000 x 550 140, 1062, 111; Izhikevich at 8 Hz 2000 x 1000
+ * 20, 41, 13, 20000 x 1000 24, 57, 18, 200000 x 100 28, 25, 19. */
 __global__ void __launch_bounds__(256) pm_scatter_kernel(PluginStepDev s, uint32_t k)
 {
-	__shared__ uint32_t list[2048];
-	__shared__ uint32_t count;
 	__shared__ uint32_t wsum[4];
 	const uint32_t lane = threadIdx.x & 63u;
 	const uint32_t wave = threadIdx.x >> 6;
+	const uint32_t G = gridDim.x;
 	const uint32_t* fired = s.raster + size_t(k) * s.words32;
 	const uint32_t base = uint32_t((s.cycle0 + k) % s.R);
 	uint32_t ev = 0;
-	for(size_t w0 = size_t(blockIdx.x) * 64u; w0 < s.words32; w0 += size_t(gridDim.x) * 64u) {   /* block-uniform */
-		if(wave == 0) {
-			uint32_t b = (w0 + lane < s.words32) ? fired[w0 + lane] : 0u;
-			const uint32_t c = uint32_t(__popc(b));
-			uint32_t x = c;
-			for(uint32_t d = 1; d < 64u; d <<= 1) {
-				const uint32_t y = __shfl_up(x, d, 64);
-				if(lane >= d) x += y;
-			}
-			uint32_t at = x - c;
-			while(b) {
-				list[at++] = uint32_t((w0 + lane) * 32u) + uint32_t(__ffs(b) - 1);
-				b &= b - 1u;
-			}
-			if(lane == 63u) count = x;
-		}
-		__syncthreads();
-		ev += deliver_listed<long long>(s, list, count, base, wave, lane);
-		__syncthreads();   /* the list is written again */
+	for(uint32_t i0 = blockIdx.x; i0 < s.n; i0 += 64u * G) {   /* block-uniform */
+		const uint32_t i = i0 + lane * G;
+		const bool f = i < s.n && ((fired[i >> 5] >> (i & 31u)) & 1u) != 0u;
+		const uint32_t ra = f ? s.off[i] : 0u, rb = f ? s.off[i + 1u] : 0u;
+		ev += deliver_rows<long long>(s, ra, rb, __ballot(f), base, wave, lane);
 	}
 	count_events(s.part, ev, wsum, wave, lane);
 }
@@ -257,7 +268,16 @@ __global__ void __launch_bounds__(256) pm_cycle_kernel(PluginStepDev s, uint32_t
 		list[before + uint32_t(__popcll(below))] = l;
 	}
 	__syncthreads();
-	const uint32_t ev = deliver_listed<ACC>(s, list, total, slot, wave, lane);
+	uint32_t ev = 0;
+	for(uint32_t j = 0; j < total; j += 64u) {   /* block-uniform */
+		const uint32_t cnt = min(64u, total - j);
+		uint32_t ra = 0, rb = 0;
+		if(lane < cnt) {
+			ra = s.off[list[j + lane]];
+			rb = s.off[list[j + lane] + 1u];
+		}
+		ev += deliver_rows<ACC>(s, ra, rb, ~0ull >> (64u - cnt), slot, wave, lane);
+	}
 	count_events(s.part, ev, wsum, wave, lane);
 }
 
@@ -370,7 +390,9 @@ int nemo_dev_pm_stimulus(const PluginStepDev* s, uint32_t k, uint32_t entries, v
 
 int nemo_dev_pm_scatter(const PluginStepDev* s, uint32_t k, void* stream)
 {
-	hipLaunchKernelGGL(pm_scatter_kernel, dim3(grid(s->words32, 64, NEMO_PM_SCATTER_BLOCKS)), dim3(256), 0,
+	/* 8 neurons per workgroup while that leaves the chip room; a workgroup each
+	 * costs networks that fire little or not at all */
+	hipLaunchKernelGGL(pm_scatter_kernel, dim3(grid(s->n, 8, NEMO_PM_SCATTER_BLOCKS)), dim3(256), 0,
 			static_cast<hipStream_t>(stream), *s, k);
 	return int(hipGetLastError());
 }

@@ -1,0 +1,50 @@
+"""Spikes of neighbours cost what spikes spread over the network cost. Neurons
+that fire together are often next to each other (a stimulated population, a
+layer), so no path may leave their delivery to the few workgroups or waves that
+hold them. Each case times the same network and the same number of forced
+neurons in every cycle, adjacent and spread, the best of several runs each:
+adjacent ones may take at most twice as long."""
+import time
+
+import numpy as np
+import pytest
+
+from parity import hip_sim
+from nemosim_amd import examples
+
+pytestmark = pytest.mark.gpu
+
+CYCLES = 20
+
+
+def best(f, reps=7):
+    f()
+    times = []
+    for _ in range(reps):
+        t = time.perf_counter()
+        f()
+        times.append(time.perf_counter() - t)
+    return min(times)
+
+
+def simulation(nemo_mod, n, m, mode="auto", stdp=False):
+    spec = examples.izhikevich_80_20(n, m, seed=n, stdp=stdp)
+    net = spec.to_nemo(nemo_mod)
+    conf = nemo_mod.Configuration()
+    conf.set_write_only_synapses()
+    conf.set_step_mode(mode)
+    if stdp:
+        pre, post = examples.stdp_window()
+        conf.set_stdp_function(pre, post, min_e=0.0, max_e=1.0, min_i=0.0, max_i=-1.0)
+    return nemo_mod.Simulation(net, conf)
+
+
+def populations(n, pop):
+    return list(range(pop)), (np.arange(pop, dtype=np.int64) * n // pop).tolist()
+
+
+@pytest.mark.parametrize("n,m,pop", [(20000, 300, 600)])
+def test_plugin_step(nemo_mod, n, m, pop):
+    sim = simulation(nemo_mod, n, m, mode="plugins")
+    adjacent, spread = [best(lambda: sim.run(CYCLES, fstim=[p] * CYCLES)) for p in populations(n, pop)]
+    assert adjacent < 2.0 * spread, (adjacent, spread)
