@@ -43,8 +43,8 @@ def populations(n, pop):
     return list(range(pop)), (np.arange(pop, dtype=np.int64) * n // pop).tolist()
 
 
-@pytest.mark.parametrize("n,m,pop", [(20000, 300, 600)])
-def test_plugin_step(nemo_mod, n, m, pop):
-    sim = simulation(nemo_mod, n, m, mode="plugins")
+@pytest.mark.parametrize("n,m,pop,stdp", [(20000, 300, 600, False), (20000, 300, 128, True)])
+def test_plugin_step(nemo_mod, n, m, pop, stdp):
+    sim = simulation(nemo_mod, n, m, mode="plugins", stdp=stdp)
     adjacent, spread = [best(lambda: sim.run(CYCLES, fstim=[p] * CYCLES)) for p in populations(n, pop)]
     assert adjacent < 2.0 * spread, (adjacent, spread)

@@ -36,6 +36,7 @@ def network(n, rows, stdp):
     (2049, (0, 300, 700), True),
     (17001, (20, 60), False),        # more than 8 neurons for each of 2048 workgroups
     (140000, (3, 7), True),          # more than 64 for each
+    (270001, (2, 5), True),          # STDP's targets in pieces of 8
 ])
 def test_plugin_step_dense(nemo_mod, oracle_mod, n, rows, learns):
     stdp = examples.stdp_window() + (0.0, 1.0, 0.0, -1.0) if learns else None
