@@ -31,9 +31,7 @@ typedef struct PluginStepDev {
 	const uint32_t* off;   /* [n+1] synapses of source s: syn[off[s] .. off[s+1]) */
 	const uint32_t* syn;   /* records {target | (delay-1) << 26, Q11.20 weight} */
 	uint64_t* recent;      /* [n] firing history */
-	unsigned long long* events;
-	unsigned long long* part;   /* [nemo_dev_pm_parts(n)] delivered synapses by
-	                             * workgroup, summed into *events by pm_finish */
+	unsigned long long* part;   /* [NEMO_PM_PARTS][16] delivered synapses, in the first word of each line */
 
 	/* built-in models */
 	const uint8_t* model;  /* [n] */
@@ -62,10 +60,8 @@ int nemo_dev_pm_replay(const PluginStepDev* s, int narrow, void* stream);
 /* one cycle of built-in models; stim: the cycle's stimulus is in fstim and
  * curX, which are cleared */
 int nemo_dev_pm_cycle(const PluginStepDev* s, uint32_t k, int stim, int narrow, int izhikevichOnly, void* stream);
-/* workgroups of the kernels that count events in `part`, and their sum */
 #define NEMO_PM_SCATTER_BLOCKS 2048u
-uint32_t nemo_dev_pm_parts(uint32_t n);
-int nemo_dev_pm_finish(const PluginStepDev* s, void* stream);
+#define NEMO_PM_PARTS 64u
 
 #ifdef __cplusplus
 }

@@ -143,17 +143,14 @@ __device__ inline uint32_t deliver_rows(const PluginStepDev& s, uint32_t ra, uin
 	return ev;
 }
 
-/* part[blockIdx.x] += the waves' ev: the workgroup's own counter, since a
- * shared one, and a shared list of the fired neurons, serialise the atomics of
+/* The wave's ev into one of NEMO_PM_PARTS counters, which the host adds up. A
+ * single one, and a shared list of the fired neurons, serialise the atomics of
  * all workgroups (compaction and scatter of 150k synapses: 28 us a cycle with
- * them, 19 without) */
-__device__ inline void count_events(unsigned long long* part, uint32_t ev, uint32_t* wsum, uint32_t wave, uint32_t lane)
+ * them, 19 without). */
+__device__ inline void count_events(unsigned long long* part, uint32_t ev, uint32_t wave, uint32_t lane)
 {
-	if(lane == 0) wsum[wave] = ev;
-	__syncthreads();
-	if(threadIdx.x == 0) {
-		const uint32_t sum = wsum[0] + wsum[1] + wsum[2] + wsum[3];
-		if(sum) part[blockIdx.x] += sum;
+	if(lane == 0 && ev) {
+		atomicAdd(part + size_t((blockIdx.x * 4u + wave) % NEMO_PM_PARTS) * 16u, (unsigned long long) ev);
 	}
 }
 
@@ -170,7 +167,6 @@ __device__ inline void count_events(unsigned long long* part, uint32_t ev, uint3
  * 20, 41, 13, 20000 x 1000 24, 57, 18, 200000 x 100 28, 25, 19. */
 __global__ void __launch_bounds__(256) pm_scatter_kernel(PluginStepDev s, uint32_t k)
 {
-	__shared__ uint32_t wsum[4];
 	const uint32_t lane = threadIdx.x & 63u;
 	const uint32_t wave = threadIdx.x >> 6;
 	const uint32_t G = gridDim.x;
@@ -183,7 +179,7 @@ __global__ void __launch_bounds__(256) pm_scatter_kernel(PluginStepDev s, uint32
 		const uint32_t ra = f ? s.off[i] : 0u, rb = f ? s.off[i + 1u] : 0u;
 		ev += deliver_rows<long long>(s, ra, rb, __ballot(f), base, wave, lane);
 	}
-	count_events(s.part, ev, wsum, wave, lane);
+	count_events(s.part, ev, wave, lane);
 }
 
 /* Built-in models: one cycle of 256 neurons per workgroup. Reads and clears
@@ -204,7 +200,7 @@ __global__ void __launch_bounds__(256) pm_cycle_kernel(PluginStepDev s, uint32_t
 	constexpr int NP = IZO ? 5 : MAX_PARAM;
 	constexpr int NS = IZO ? 2 : MAX_STATE;
 	__shared__ uint32_t list[256];
-	__shared__ uint32_t wsum[4], wfired[4];
+	__shared__ uint32_t wfired[4];
 	const uint32_t lane = threadIdx.x & 63u;
 	const uint32_t wave = threadIdx.x >> 6;
 	const uint32_t n = s.n;
@@ -278,24 +274,7 @@ __global__ void __launch_bounds__(256) pm_cycle_kernel(PluginStepDev s, uint32_t
 		}
 		ev += deliver_rows<ACC>(s, ra, rb, ~0ull >> (64u - cnt), slot, wave, lane);
 	}
-	count_events(s.part, ev, wsum, wave, lane);
-}
-
-/* *events += the workgroups' counters (one workgroup) */
-__global__ void __launch_bounds__(256) pm_finish_kernel(PluginStepDev s, uint32_t parts)
-{
-	__shared__ unsigned long long sums[256];
-	unsigned long long e = 0;
-	for(uint32_t i = threadIdx.x; i < parts; i += 256u) {
-		e += s.part[i];
-		s.part[i] = 0ull;
-	}
-	sums[threadIdx.x] = e;
-	__syncthreads();
-	if(threadIdx.x == 0) {
-		for(uint32_t i = 1; i < 256u; ++i) e += sums[i];
-		*s.events += e;
-	}
+	count_events(s.part, ev, wave, lane);
 }
 
 /* STDP: targets whose history has bit postLen set walk their plastic
@@ -420,19 +399,6 @@ int nemo_dev_pm_cycle(const PluginStepDev* s, uint32_t k, int stim, int narrow, 
 	auto kernel = narrow ? (izhikevichOnly ? &pm_cycle_kernel<int32_t, true> : &pm_cycle_kernel<int32_t, false>)
 		: (izhikevichOnly ? &pm_cycle_kernel<long long, true> : &pm_cycle_kernel<long long, false>);
 	hipLaunchKernelGGL(kernel, dim3((s->n + 255u) / 256u), dim3(256), 0, static_cast<hipStream_t>(stream), *s, k, stim);
-	return int(hipGetLastError());
-}
-
-uint32_t nemo_dev_pm_parts(uint32_t n)
-{
-	const uint32_t blocks = (n + 255u) / 256u;
-	return blocks > NEMO_PM_SCATTER_BLOCKS ? blocks : NEMO_PM_SCATTER_BLOCKS;
-}
-
-int nemo_dev_pm_finish(const PluginStepDev* s, void* stream)
-{
-	hipLaunchKernelGGL(pm_finish_kernel, dim3(1), dim3(256), 0, static_cast<hipStream_t>(stream), *s,
-			nemo_dev_pm_parts(s->n));
 	return int(hipGetLastError());
 }
 

@@ -842,7 +842,8 @@ Simulation::Simulation(const NetworkImpl& net, const ConfigurationImpl& conf) :
 		}
 		d_curX.alloc(std::max<size_t>(m_n, 1) * 4);
 		d_fstim.alloc(std::max<size_t>(m_words32, 2) * 4);
-		d_part.alloc(size_t(nemo_dev_pm_parts(m_n)) * 8);
+		d_part.alloc(size_t(NEMO_PM_PARTS) * 128);
+		hipCheck(hipHostMalloc(reinterpret_cast<void**>(&h_part), d_part.bytes), "hipHostMalloc");
 		hipCheck(nemo_dev_fill_u64(d_acc.as<uint64_t>(), 0, d_acc.bytes / 8, s), "fill");
 		hipCheck(nemo_dev_fill_u32(d_curX.as<uint32_t>(), 0, d_curX.bytes / 4, s), "fill");
 		hipCheck(nemo_dev_fill_u32(d_fstim.as<uint32_t>(), 0, d_fstim.bytes / 4, s), "fill");
@@ -1056,6 +1057,7 @@ Simulation::~Simulation()
 	}
 	if(h_ctl) (void) hipHostFree(h_ctl);
 	if(h_step) (void) hipHostFree(h_step);
+	if(h_part) (void) hipHostFree(h_part);
 	if(h_sched) (void) hipHostFree(h_sched);
 	for(PluginGroup& pg : m_plugins) {
 		if(pg.handle) dlclose(pg.handle);
@@ -1386,7 +1388,7 @@ Simulation::launchPlugins(unsigned nsteps, unsigned long long* events)
 	hipStream_t st = static_cast<hipStream_t>(m_stream);
 	hipCheck(hipSetDevice(m_device), "hipSetDevice");
 	ensureRaster(size_t(nsteps) * m_words32 * 4);
-	hipCheck(nemo_dev_fill_u32(d_ctl.as<uint32_t>(), 0, 16, st), "fill");
+	hipCheck(nemo_dev_fill_u64(d_part.as<uint64_t>(), 0, d_part.bytes / 8, st), "fill");
 	m_rasterExternal = false;
 	PluginStepDev s;
 	std::memset(&s, 0, sizeof(s));
@@ -1404,17 +1406,12 @@ Simulation::launchPlugins(unsigned nsteps, unsigned long long* events)
 	s.off = d_off.as<uint32_t>();
 	s.syn = d_syn.as<uint32_t>();
 	s.recent = d_recent.as<uint64_t>();
-	s.events = reinterpret_cast<unsigned long long*>(d_ctl.as<uint32_t>() + 2);
 	s.part = d_part.as<unsigned long long>();
 	s.model = d_model.as<uint8_t>();
 	s.param = d_param.as<float>();
 	s.state = d_state.as<float>();
 	s.rng = d_rng.as<uint32_t>();
 	const int narrow = m_builtinStep && !m_saturate ? 1 : 0;
-	if(m_partDirty) {
-		hipCheck(nemo_dev_fill_u64(d_part.as<uint64_t>(), 0, d_part.bytes / 8, st), "fill");
-	}
-	m_partDirty = true;
 	s.rcm_start = d_rcmStart.as<uint32_t>();
 	s.rcm_sd = d_rcmSd.as<uint32_t>();
 	s.rcm_acc = d_rcmAcc.as<int32_t>();
@@ -1457,14 +1454,9 @@ Simulation::launchPlugins(unsigned nsteps, unsigned long long* events)
 			hipCheck(nemo_dev_pm_stdp(&s, st), "plugin step: stdp");
 		}
 	}
-	hipCheck(nemo_dev_pm_finish(&s, st), "plugin step: events");
-	m_partDirty = false;
 	hipCheck(hipEventRecord(e1, st), "hipEventRecord");
-	uint32_t ctl[8];
-	hipCheck(hipMemcpyAsync(h_ctl, d_ctl.ptr, sizeof(ctl), hipMemcpyDeviceToHost, st), "D2H");
+	hipCheck(hipMemcpyAsync(h_part, d_part.ptr, d_part.bytes, hipMemcpyDeviceToHost, st), "D2H");
 	hipCheck(hipStreamSynchronize(st), "hipStreamSynchronize");
-	std::memcpy(ctl, h_ctl, sizeof(ctl));
-	setControlBase(ctl);
 	float ms = 0.0f;
 	hipCheck(hipEventElapsedTime(&ms, e0, e1), "hipEventElapsedTime");
 	m_kernelMs = ms;
@@ -1480,9 +1472,8 @@ Simulation::launchPlugins(unsigned nsteps, unsigned long long* events)
 	m_lastRunSteps = nsteps;
 	m_hasSchedule = false;
 	if(events) {
-		unsigned long long e;
-		std::memcpy(&e, &ctl[2], sizeof(e));
-		*events = e;
+		*events = 0;
+		for(uint32_t i = 0; i < NEMO_PM_PARTS; ++i) *events += h_part[16 * i];
 	}
 }
 

@@ -170,7 +170,7 @@ class Simulation
 		DevBuf d_acc, d_curE, d_curI, d_curX, d_fstim, d_part;
 		bool m_builtinStep = false;    /* per-cycle step of built-in models, no plugins */
 		uint32_t m_ringDepth = 1;      /* PluginStepDev.R */
-		bool m_partDirty = true;       /* d_part holds an unfinished run's counts */
+		uint64_t* h_part = nullptr;    /* d_part, pinned */
 		std::vector<uint32_t> m_fsPtrHost, m_isPtrHost;
 		void loadPlugins(const NetworkImpl& net);
 		void launchPlugins(unsigned nsteps, unsigned long long* events);
