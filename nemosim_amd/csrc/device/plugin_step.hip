@@ -154,9 +154,10 @@ __device__ inline void count_events(unsigned long long* part, uint32_t ev, uint3
 	}
 }
 
-/* Plugins: the spikes of cycle k. Workgroup g of G takes the neurons g, g + G,
- * g + 2G, ..., a lane each, so that all workgroups have sources whatever fires:
- * neurons that fire together are often neighbours. Every wave reads the fired
+/* Plugins: the spikes of cycle k. Workgroup g of G takes the pieces g, g + G,
+ * g + 2G, ... of 1 << plog neighbouring neurons, a neuron per lane, so that all
+ * workgroups have sources whatever fires: neurons that fire together are often
+ * neighbours. Every wave reads the fired
  * bits and the rows' bounds for itself, so nothing is listed and nothing
  * waited for.
  *
@@ -165,7 +166,7 @@ __device__ inline void count_events(unsigned long long* part, uint32_t ev, uint3
  * workgroup per 2048 neurons, and now: 2000 x 1000 IF_curr_exp_noise at 333 Hz
  * 48, 1504, 44 us; 12000 x 550 140, 1062, 111; Izhikevich at 8 Hz 2000 x 1000
  * 20, 41, 13, 20000 x 1000 24, 57, 18, 200000 x 100 28, 25, 19. */
-__global__ void __launch_bounds__(256) pm_scatter_kernel(PluginStepDev s, uint32_t k)
+__global__ void __launch_bounds__(256) pm_scatter_kernel(PluginStepDev s, uint32_t k, uint32_t plog)
 {
 	const uint32_t lane = threadIdx.x & 63u;
 	const uint32_t wave = threadIdx.x >> 6;
@@ -173,8 +174,8 @@ __global__ void __launch_bounds__(256) pm_scatter_kernel(PluginStepDev s, uint32
 	const uint32_t* fired = s.raster + size_t(k) * s.words32;
 	const uint32_t base = uint32_t((s.cycle0 + k) % s.R);
 	uint32_t ev = 0;
-	for(uint32_t i0 = blockIdx.x; i0 < s.n; i0 += 64u * G) {   /* block-uniform */
-		const uint32_t i = i0 + lane * G;
+	for(uint32_t p0 = blockIdx.x; (p0 << plog) < s.n; p0 += G * (64u >> plog)) {   /* block-uniform */
+		const uint32_t i = ((p0 + (lane >> plog) * G) << plog) + (lane & ((1u << plog) - 1u));
 		const bool f = i < s.n && ((fired[i >> 5] >> (i & 31u)) & 1u) != 0u;
 		const uint32_t ra = f ? s.off[i] : 0u, rb = f ? s.off[i + 1u] : 0u;
 		ev += deliver_rows<long long>(s, ra, rb, __ballot(f), base, wave, lane);
@@ -378,9 +379,12 @@ int nemo_dev_pm_stimulus(const PluginStepDev* s, uint32_t k, uint32_t entries, v
 int nemo_dev_pm_scatter(const PluginStepDev* s, uint32_t k, void* stream)
 {
 	/* 8 neurons per workgroup while that leaves the chip room; a workgroup each
-	 * costs networks that fire little or not at all */
+	 * costs networks that fire little or not at all. Where all lanes have one in
+	 * pieces of 8, which read one word of fired bits (500k oscillators x 10, per
+	 * cycle 122 -> 120 us; 200k x 100 at 8 Hz 19 -> 17) */
+	const bool large = s->n > 64u * NEMO_PM_SCATTER_BLOCKS;
 	hipLaunchKernelGGL(pm_scatter_kernel, dim3(grid(s->n, 8, NEMO_PM_SCATTER_BLOCKS)), dim3(256), 0,
-			static_cast<hipStream_t>(stream), *s, k);
+			static_cast<hipStream_t>(stream), *s, k, large ? 3u : 0u);
 	return int(hipGetLastError());
 }
 
