@@ -53,7 +53,7 @@ extern "C" {
  * CPU plugins (src/nemo/cpu/plugins/neuron_model.h:38). */
 typedef struct nemo_hip_rcm {
 	uint32_t targets;          /* simulation-local neurons (start has targets+1 entries) */
-	uint32_t pad;
+	uint32_t longest;          /* the most incoming synapses of a target */
 	size_t synapses;
 	const uint32_t* start;
 	const uint32_t* source;    /* simulation-local source neuron */

@@ -707,6 +707,7 @@ Simulation::Simulation(const NetworkImpl& net, const ConfigurationImpl& conf) :
 			std::lock_guard<DeviceMutex> uploadLock(deviceMutex());
 			std::memset(&m_rcmDesc, 0, sizeof(m_rcmDesc));
 			m_rcmDesc.targets = m_n;
+			for(uint32_t l = 0; l < m_n; ++l) m_rcmDesc.longest = std::max(m_rcmDesc.longest, kStart[l + 1] - kStart[l]);
 			m_rcmDesc.synapses = m_nsyn;
 			d_kStart.upload(kStart.data(), kStart.size() * 4);
 			m_rcmDesc.start = d_kStart.as<uint32_t>();

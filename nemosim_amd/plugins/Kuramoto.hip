@@ -137,7 +137,29 @@ __device__ inline float ordered_sum_row(float s, const float* row, unsigned len,
 }
 #undef ADD_LANE
 
-/* One workgroup per `per` consecutive oscillators. Tiles of them whose rows
+/* Where a workgroup's share starts if work is shared by couplings: the first of
+ * the n oscillators whose rows, counted with OSC_COST couplings for each
+ * oscillator, start at `target` or later. By one wave, in rounds of 64 probes. */
+constexpr unsigned OSC_COST = 16u;
+
+__device__ inline unsigned share_start(const uint32_t* rstart, unsigned n, uint64_t target, unsigned lane)
+{
+	const uint32_t first = rstart[0];
+	unsigned lo = 0, hi = n;
+	while(lo < hi) {   /* wave-uniform; the answer is in lo .. hi */
+		const unsigned step = (hi - lo + 63u) / 64u;
+		const unsigned o = lo + (lane + 1u) * step - 1u;
+		const bool before = o < hi && uint64_t(rstart[o] - first) + uint64_t(OSC_COST) * o < target;
+		const unsigned cnt = unsigned(__popcll(__ballot(before)));
+		hi = min(hi, lo + (cnt + 1u) * step - 1u);
+		lo += cnt * step;
+	}
+	return lo;
+}
+
+/* One workgroup per `per` consecutive oscillators, or, SHARED, per `quota`
+ * couplings: with rows of very different lengths next to each other (hubs)
+ * a workgroup of `per` would have many long rows, one after the other. Tiles of them whose rows
  * hold at most TILE = 256 PER couplings together are done one after the other (one tile,
  * unless rows are uneven); a row longer than TILE is a tile of its own and is
  * read in pieces, again for each stage, where the others stay in registers
@@ -152,9 +174,9 @@ __device__ inline float ordered_sum_row(float s, const float* row, unsigned len,
  * now: 1000 oscillators x 1000 couplings 65 -> 28 us (33 with a lane's sums
  * alone), 4000 x 1000 101 -> 57, 2000 x 2500 182 -> 113, 3000 x 300 36 -> 21,
  * 20000 x 100 48 -> 31, 50000 x 100 99 -> 75. */
-template<unsigned PER>
+template<unsigned PER, bool SHARED = false>
 __global__ void __launch_bounds__(256, 4) kuramoto_update_kernel(unsigned start, unsigned end, unsigned per,
-		unsigned cycle, const float* freq, float* state, size_t hstride, const uint32_t* rstart,
+		uint64_t quota, unsigned cycle, const float* freq, float* state, size_t hstride, const uint32_t* rstart,
 		const uint32_t* src, const uint32_t* dly, const float* w)
 {
 	constexpr unsigned TILE = Tile<PER>::couplings;
@@ -165,8 +187,19 @@ __global__ void __launch_bounds__(256, 4) kuramoto_update_kernel(unsigned start,
 	const unsigned tid = threadIdx.x;
 	const float* phase0 = state + size_t(cycle % HISTORY) * hstride;
 	float* phase1 = state + size_t((cycle + 1u) % HISTORY) * hstride;
-	const unsigned last = min(end - start, (blockIdx.x + 1u) * per);
+	unsigned last = min(end - start, (blockIdx.x + 1u) * per);
 	unsigned o = blockIdx.x * per;
+	if(SHARED) {
+		__shared__ unsigned share[2];
+		const unsigned wave = tid >> 6;
+		if(wave < 2u) {
+			const unsigned at = share_start(rstart + start, end - start, quota * (blockIdx.x + wave), tid & 63u);
+			if((tid & 63u) == 0u) share[wave] = at;
+		}
+		__syncthreads();
+		o = share[0];
+		last = share[1];
+	}
 	while(o < last) {   /* block-uniform */
 		const unsigned left = min(last - o, TILE_OSC);
 		if(tid <= left) rs[tid] = rstart[start + o + tid];
@@ -261,7 +294,11 @@ __global__ void __launch_bounds__(256, 4) kuramoto_update_kernel(unsigned start,
  * tile with which all of them run at once is taken (fewer instructions and
  * registers: see the figures at the kernel); where none is large enough, the
  * middle one, in several rounds. */
-struct Plan { unsigned per, threadCouplings; };
+struct Plan {
+	unsigned per, threadCouplings;
+	uint64_t quota;     /* couplings per workgroup; 0: `per` oscillators each */
+	unsigned blocks;
+};
 
 Plan plan(unsigned n, const nemo_hip_rcm* rcm)
 {
@@ -275,13 +312,33 @@ Plan plan(unsigned n, const nemo_hip_rcm* rcm)
 		const unsigned rounds = (n + RESIDENT * b - 1u) / (RESIDENT * b);
 		return (n + RESIDENT * rounds - 1u) / (RESIDENT * rounds);
 	};
+	Plan p = { 1u, 18u, 0u, 0u };
+	const unsigned mid = fit(THREADS * 9u);
+	if(mid > 0u) p = Plan{ spread(mid), 9u, 0u, 0u };
 	const unsigned sizes[3] = { 3u, 9u, 18u };
 	for(unsigned c : sizes) {
 		const unsigned b = fit(THREADS * c);
-		if(b > 0u && n <= RESIDENT * b) return Plan{spread(b), c};
+		if(b > 0u && n <= RESIDENT * b) {
+			p = Plan{ spread(b), c, 0u, 0u };
+			break;
+		}
 	}
-	const unsigned b = fit(THREADS * 9u);
-	return b > 0u ? Plan{spread(b), 9u} : Plan{1u, 18u};
+	p.blocks = (n + p.per - 1u) / p.per;
+	/* Shared by couplings where the longest rows, next to each other, could make
+	 * a workgroup's share several tiles, and are several times the average, as
+	 * those of random networks are not: two or three rounds of reads more before the
+	 * first tile, two thirds of a tile per workgroup on average. 20000 x 30 with 20
+	 * neighbours of 15000 couplings each: 4311 us per cycle in shares of 20
+	 * oscillators, 223 so. */
+	const uint64_t longest = rcm->longest;
+	if(p.per > 1u && double(longest) > 4.0 * avg && longest * p.per > 2u * THREADS * p.threadCouplings) {
+		const uint64_t work = uint64_t(rcm->synapses) + uint64_t(OSC_COST) * n + 1u;
+		const uint64_t most = THREADS * 9u * 2u / 3u;
+		p.threadCouplings = 9u;
+		p.blocks = unsigned(RESIDENT * ((work + RESIDENT * most - 1u) / (RESIDENT * most)));
+		p.quota = (work + p.blocks - 1u) / p.blocks;
+	}
+	return p;
 }
 
 /* src/nemo/cpu/plugins/Kuramoto.cpp:133-152: the planes of cycles -1 .. -31
@@ -317,10 +374,10 @@ int hip_update_neurons(void* stream, unsigned cycle, unsigned start, unsigned en
 	}
 	const unsigned n = end - start;
 	const Plan pl = plan(n, rcm);
-	auto kernel = pl.threadCouplings == 3u ? &kuramoto_update_kernel<3u>
+	auto kernel = pl.quota ? &kuramoto_update_kernel<9u, true> : pl.threadCouplings == 3u ? &kuramoto_update_kernel<3u>
 		: pl.threadCouplings == 9u ? &kuramoto_update_kernel<9u> : &kuramoto_update_kernel<18u>;
-	hipLaunchKernelGGL(kernel, dim3((n + pl.per - 1u) / pl.per), dim3(THREADS), 0,
-			static_cast<hipStream_t>(stream), start, end, pl.per, cycle, param, state, stateHistoryStride,
+	hipLaunchKernelGGL(kernel, dim3(pl.blocks), dim3(THREADS), 0,
+			static_cast<hipStream_t>(stream), start, end, pl.per, pl.quota, cycle, param, state, stateHistoryStride,
 			rcm->start, rcm->source, rcm->delay, rcm->weight);
 	return int(hipGetLastError());
 }
