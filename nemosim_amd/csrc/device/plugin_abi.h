@@ -53,13 +53,15 @@ typedef struct PluginStepDev {
 
 int nemo_dev_pm_begin(const PluginStepDev* s, uint32_t k, void* stream);
 int nemo_dev_pm_stimulus(const PluginStepDev* s, uint32_t k, uint32_t entries, void* stream);
-int nemo_dev_pm_scatter(const PluginStepDev* s, uint32_t k, void* stream);
+/* narrow: int32 accumulators; longRows: neighbours with long rows */
+int nemo_dev_pm_scatter(const PluginStepDev* s, uint32_t k, int narrow, int longRows, void* stream);
 int nemo_dev_pm_stdp(const PluginStepDev* s, void* stream);
-/* rebuilds the zeroed ring; narrow: int32 accumulators */
+/* rebuilds the zeroed ring */
 int nemo_dev_pm_replay(const PluginStepDev* s, int narrow, void* stream);
 /* one cycle of built-in models; stim: the cycle's stimulus is in fstim and
- * curX, which are cleared */
-int nemo_dev_pm_cycle(const PluginStepDev* s, uint32_t k, int stim, int narrow, int izhikevichOnly, void* stream);
+ * curX, which are cleared; deliver: with its spikes, otherwise nemo_dev_pm_scatter follows */
+int nemo_dev_pm_cycle(const PluginStepDev* s, uint32_t k, int stim, int narrow, int izhikevichOnly, int deliver,
+		void* stream);
 #define NEMO_PM_SCATTER_BLOCKS 2048u
 #define NEMO_PM_PARTS 64u
 

@@ -154,7 +154,7 @@ __device__ inline void count_events(unsigned long long* part, uint32_t ev, uint3
 	}
 }
 
-/* Plugins: the spikes of cycle k. Workgroup g of G takes the pieces g, g + G,
+/* Plugins, and built-in networks with long rows: the spikes of cycle k. Workgroup g of G takes the pieces g, g + G,
  * g + 2G, ... of 1 << plog neighbouring neurons, a neuron per lane, so that all
  * workgroups have sources whatever fires: neurons that fire together are often
  * neighbours. Every wave reads the fired
@@ -166,6 +166,7 @@ __device__ inline void count_events(unsigned long long* part, uint32_t ev, uint3
  * workgroup per 2048 neurons, and now: 2000 x 1000 IF_curr_exp_noise at 333 Hz
  * 48, 1504, 44 us; 12000 x 550 140, 1062, 111; Izhikevich at 8 Hz 2000 x 1000
  * 20, 41, 13, 20000 x 1000 24, 57, 18, 200000 x 100 28, 25, 19. */
+template<typename ACC>
 __global__ void __launch_bounds__(256) pm_scatter_kernel(PluginStepDev s, uint32_t k, uint32_t plog)
 {
 	const uint32_t lane = threadIdx.x & 63u;
@@ -178,16 +179,26 @@ __global__ void __launch_bounds__(256) pm_scatter_kernel(PluginStepDev s, uint32
 		const uint32_t i = ((p0 + (lane >> plog) * G) << plog) + (lane & ((1u << plog) - 1u));
 		const bool f = i < s.n && ((fired[i >> 5] >> (i & 31u)) & 1u) != 0u;
 		const uint32_t ra = f ? s.off[i] : 0u, rb = f ? s.off[i + 1u] : 0u;
-		ev += deliver_rows<long long>(s, ra, rb, __ballot(f), base, wave, lane);
+		ev += deliver_rows<ACC>(s, ra, rb, __ballot(f), base, wave, lane);
 	}
 	count_events(s.part, ev, wave, lane);
 }
 
-/* Built-in models: one cycle of 256 neurons per workgroup. Reads and clears
+/* Built-in models: one cycle of 256 neurons per workgroup, 16 pieces of 16
+ * neighbours that lie a grid apart: neurons that fire together are often
+ * neighbours, and a compute unit adds about 0.4 synapses per ns. The two pieces
+ * of 32 neurons, whose values are one line of memory in each array, go to
+ * workgroups b and b + 8, which run on one XCD: its L2 reads the line once. With
+ * 256 forced neighbours, 270k x 300, a cycle takes 50 us so, 60 with pieces of
+ * 32, 46 with pieces of 8 (but 9 % more without them), and 230 with 256
+ * neighbours in a workgroup; 270k x 300 on the plugins' sequence as it was 66.
+ * Reads and clears
  * the cycle's ring slot, updates the neurons (models.h), writes their raster
  * words, lists the fired ones in LDS and delivers them at once into slots t+1
  * .. t+D, none of which is slot t of a ring of D+1: other workgroups may still
- * be reading it. So a cycle is one launch where plugins need three.
+ * be reading it. So a cycle is one launch where plugins need three. Without
+ * DELIVER the delivery is left to pm_scatter_kernel: for networks with long rows
+ * next to each other.
  *
  * What bounds it: the neurons' parameters, state and ring slot (about 90 bytes
  * each) and the chain slot -> update -> row bounds -> records -> atomics; with
@@ -195,7 +206,7 @@ __global__ void __launch_bounds__(256) pm_scatter_kernel(PluginStepDev s, uint32
  * (begin, update, compact, scatter): 300k x 100 37 -> 14.2 us, 400k x 250 62 ->
  * 31, 100k x 100 with delays up to 60 20.8 -> 8.9, 70k x 60 IF_curr_exp_noise
  * at 333 Hz 114 -> 31, 150k x 60 with STDP 35 -> 15.7. */
-template<typename ACC, bool IZO>
+template<typename ACC, bool IZO, bool DELIVER>
 __global__ void __launch_bounds__(256) pm_cycle_kernel(PluginStepDev s, uint32_t k, int stim)
 {
 	constexpr int NP = IZO ? 5 : MAX_PARAM;
@@ -205,7 +216,10 @@ __global__ void __launch_bounds__(256) pm_cycle_kernel(PluginStepDev s, uint32_t
 	const uint32_t lane = threadIdx.x & 63u;
 	const uint32_t wave = threadIdx.x >> 6;
 	const uint32_t n = s.n;
-	const uint32_t l = blockIdx.x * 256u + threadIdx.x;
+	/* line of 32 neurons, and its half: see above */
+	const uint32_t line = ((threadIdx.x >> 4) * (gridDim.x >> 4) + (blockIdx.x >> 4)) * 8u + (blockIdx.x & 7u);
+	const uint32_t piece = line * 2u + ((blockIdx.x >> 3) & 1u);
+	const uint32_t l = piece * 16u + (lane & 15u);
 	const uint32_t slot = uint32_t((s.cycle0 + k) % s.R);
 	bool fired = false;
 	if(l < n) {
@@ -243,15 +257,13 @@ __global__ void __launch_bounds__(256) pm_cycle_kernel(PluginStepDev s, uint32_t
 		s.recent[l] = (recent << 1) | (fired ? 1ull : 0ull);
 	}
 	const uint64_t mask = __ballot(fired);
-	if(lane == 0) {
-		wfired[wave] = uint32_t(__popcll(mask));
-		const uint32_t word = l >> 6;
-		if(word < s.words32 / 2u) {
-			reinterpret_cast<uint64_t*>(s.raster)[size_t(k) * (s.words32 / 2u) + word] = mask;
-			/* every lane of the wave has read its bit */
-			if(stim) reinterpret_cast<uint64_t*>(s.fstim)[word] = 0ull;
-		}
+	if(lane == 0) wfired[wave] = uint32_t(__popcll(mask));
+	if((lane & 15u) == 0u && line < s.words32) {
+		reinterpret_cast<uint16_t*>(s.raster + size_t(k) * s.words32)[piece] = uint16_t(mask >> lane);
+		/* every lane of the wave has read its bit */
+		if(stim) reinterpret_cast<uint16_t*>(s.fstim)[piece] = 0u;
 	}
+	if(!DELIVER) return;
 	__syncthreads();
 	uint32_t before = 0, total = 0;
 #pragma unroll
@@ -349,6 +361,13 @@ __global__ void pm_replay_kernel(PluginStepDev s)
 	}
 }
 
+template<typename ACC, bool IZO>
+void launch_cycle(const PluginStepDev* s, uint32_t k, int stim, int deliver, hipStream_t stream)
+{
+	auto kernel = deliver ? &pm_cycle_kernel<ACC, IZO, true> : &pm_cycle_kernel<ACC, IZO, false>;
+	hipLaunchKernelGGL(kernel, dim3((s->words32 + 127u) / 128u * 16u), dim3(256), 0, stream, *s, k, stim);
+}
+
 unsigned grid(size_t n, unsigned block, unsigned cap)
 {
 	size_t g = (n + block - 1) / block;
@@ -376,14 +395,15 @@ int nemo_dev_pm_stimulus(const PluginStepDev* s, uint32_t k, uint32_t entries, v
 	return int(hipGetLastError());
 }
 
-int nemo_dev_pm_scatter(const PluginStepDev* s, uint32_t k, void* stream)
+int nemo_dev_pm_scatter(const PluginStepDev* s, uint32_t k, int narrow, int longRows, void* stream)
 {
 	/* 8 neurons per workgroup while that leaves the chip room; a workgroup each
 	 * costs networks that fire little or not at all. Where all lanes have one in
 	 * pieces of 8, which read one word of fired bits (500k oscillators x 10, per
 	 * cycle 122 -> 120 us; 200k x 100 at 8 Hz 19 -> 17) */
-	const bool large = s->n > 64u * NEMO_PM_SCATTER_BLOCKS;
-	hipLaunchKernelGGL(pm_scatter_kernel, dim3(grid(s->n, 8, NEMO_PM_SCATTER_BLOCKS)), dim3(256), 0,
+	const bool large = s->n > 64u * NEMO_PM_SCATTER_BLOCKS && !longRows;
+	auto kernel = narrow ? &pm_scatter_kernel<int32_t> : &pm_scatter_kernel<long long>;
+	hipLaunchKernelGGL(kernel, dim3(grid(s->n, 8, NEMO_PM_SCATTER_BLOCKS)), dim3(256), 0,
 			static_cast<hipStream_t>(stream), *s, k, large ? 3u : 0u);
 	return int(hipGetLastError());
 }
@@ -398,11 +418,17 @@ int nemo_dev_pm_replay(const PluginStepDev* s, int narrow, void* stream)
 	return int(hipGetLastError());
 }
 
-int nemo_dev_pm_cycle(const PluginStepDev* s, uint32_t k, int stim, int narrow, int izhikevichOnly, void* stream)
+int nemo_dev_pm_cycle(const PluginStepDev* s, uint32_t k, int stim, int narrow, int izhikevichOnly, int deliver,
+		void* stream)
 {
-	auto kernel = narrow ? (izhikevichOnly ? &pm_cycle_kernel<int32_t, true> : &pm_cycle_kernel<int32_t, false>)
-		: (izhikevichOnly ? &pm_cycle_kernel<long long, true> : &pm_cycle_kernel<long long, false>);
-	hipLaunchKernelGGL(kernel, dim3((s->n + 255u) / 256u), dim3(256), 0, static_cast<hipStream_t>(stream), *s, k, stim);
+	hipStream_t st = static_cast<hipStream_t>(stream);
+	if(narrow) {
+		if(izhikevichOnly) launch_cycle<int32_t, true>(s, k, stim, deliver, st);
+		else launch_cycle<int32_t, false>(s, k, stim, deliver, st);
+	} else {
+		if(izhikevichOnly) launch_cycle<long long, true>(s, k, stim, deliver, st);
+		else launch_cycle<long long, false>(s, k, stim, deliver, st);
+	}
 	return int(hipGetLastError());
 }
 

@@ -651,6 +651,19 @@ Simulation::Simulation(const NetworkImpl& net, const ConfigurationImpl& conf) :
 			std::vector<uint32_t> rows(size_t(m_n) + 1, 0u);
 			for(uint32_t s = 0; s <= m_n; ++s) rows[s] = off[size_t(s) * 2];
 			off.swap(rows);
+			/* Long rows next to each other (hubs), whose spikes one workgroup of
+			 * the per-cycle step would deliver (it takes neighbours in pieces of
+			 * 16, see plugin_step.hip): a launch more per cycle, about 2.5 us,
+			 * against 391 -> 42 us per cycle for 20 neighbours of 10000 synapses
+			 * that all fire (270k x 20). A piece whose rows hold more than a
+			 * uniform network's, and more than its compute unit does in the time
+			 * that the longest row alone takes. */
+			uint64_t longest = 0, most = 0;
+			for(uint32_t s = 0; s < m_n; s += 16u) {
+				most = std::max<uint64_t>(most, off[std::min(s + 16u, m_n)] - off[s]);
+			}
+			for(uint32_t s = 0; s < m_n; ++s) longest = std::max<uint64_t>(longest, off[s + 1] - off[s]);
+			m_longRows = most > 16384u && most > 3u * longest && double(most) * double(m_n) > 64.0 * double(m_nsyn);
 		}
 		std::vector<uint32_t>().swap(cursor);
 		std::vector<int32_t>().swap(wfx);
@@ -1438,7 +1451,9 @@ Simulation::launchPlugins(unsigned nsteps, unsigned long long* events)
 		if(!m_builtinStep) hipCheck(nemo_dev_pm_begin(&s, k, st), "plugin step: begin");
 		hipCheck(nemo_dev_pm_stimulus(&s, k, entries, st), "plugin step: stimulus");
 		if(m_builtinStep) {
-			hipCheck(nemo_dev_pm_cycle(&s, k, entries ? 1 : 0, narrow, m_izOnly ? 1 : 0, st), "per-cycle step");
+			hipCheck(nemo_dev_pm_cycle(&s, k, entries ? 1 : 0, narrow, m_izOnly ? 1 : 0, m_longRows ? 0 : 1, st),
+					"per-cycle step");
+			if(m_longRows) hipCheck(nemo_dev_pm_scatter(&s, k, narrow, 1, st), "per-cycle step: scatter");
 		} else {
 			uint32_t* firedRow = s.raster + size_t(k) * m_words32;
 			/* the cycle a plugin sees is the timer's (src/nemo/cpu/Simulation.cpp:98) */
@@ -1449,7 +1464,7 @@ Simulation::launchPlugins(unsigned nsteps, unsigned long long* events)
 							d_rng.as<uint32_t>() + pg.start, m_n, s.fstim, s.curE, s.curI, s.curX,
 							s.recent, firedRow, m_hasRcm ? &m_rcmDesc : nullptr), "hip_update_neurons");
 			}
-			hipCheck(nemo_dev_pm_scatter(&s, k, st), "plugin step: scatter");
+			hipCheck(nemo_dev_pm_scatter(&s, k, 0, 0, st), "plugin step: scatter");
 		}
 		if(m_stdp) {
 			hipCheck(nemo_dev_pm_stdp(&s, st), "plugin step: stdp");

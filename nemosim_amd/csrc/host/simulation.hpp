@@ -169,6 +169,7 @@ class Simulation
 		uint32_t m_words32 = 0;
 		DevBuf d_acc, d_curE, d_curI, d_curX, d_fstim, d_part;
 		bool m_builtinStep = false;    /* per-cycle step of built-in models, no plugins */
+		bool m_longRows = false;       /* its spikes delivered by a launch of their own */
 		uint32_t m_ringDepth = 1;      /* PluginStepDev.R */
 		uint64_t* h_part = nullptr;    /* d_part, pinned */
 		std::vector<uint32_t> m_fsPtrHost, m_isPtrHost;

@@ -43,6 +43,37 @@ def populations(n, pop):
     return list(range(pop)), (np.arange(pop, dtype=np.int64) * n // pop).tolist()
 
 
+@pytest.mark.parametrize("stdp", [False, True])
+def test_per_cycle_step(nemo_mod, stdp):
+    n = 300000
+    sim = simulation(nemo_mod, n, 60, stdp=stdp)
+    assert sim.info()["fused"] == 0
+    adjacent, spread = [best(lambda: sim.run(CYCLES, fstim=[p] * CYCLES)) for p in populations(n, 256)]
+    assert adjacent < 2.0 * spread, (adjacent, spread)
+
+
+def test_per_cycle_step_long_rows(nemo_mod):
+    """neurons with rows of 10000 synapses, next to each other and far apart"""
+    n, hubs = 270000, 20
+
+    def run(which):
+        spec = examples.izhikevich_80_20(n, 20, seed=3)
+        length = np.full(n, 20, np.int64)
+        length[which] = 10000
+        spec.rowptr = np.concatenate([[0], np.cumsum(length)]).astype(np.uint64)
+        rng, count = np.random.default_rng(4), int(length.sum())
+        spec.targets = rng.integers(0, n, count).astype(np.uint32)
+        spec.delays = rng.integers(1, 21, count).astype(np.uint8)
+        spec.weights = rng.uniform(-0.1, 0.1, count).astype(np.float32)
+        spec.plastic = np.zeros(count, np.uint8)
+        sim = hip_sim(nemo_mod, spec)
+        assert sim.info()["fused"] == 0
+        return best(lambda: sim.run(CYCLES, fstim=[which] * CYCLES))
+
+    adjacent, spread = [run(p) for p in populations(n, hubs)]
+    assert adjacent < 2.0 * spread, (adjacent, spread)
+
+
 @pytest.mark.parametrize("n,m,pop,stdp", [(20000, 300, 600, False), (20000, 300, 128, True)])
 def test_plugin_step(nemo_mod, n, m, pop, stdp):
     sim = simulation(nemo_mod, n, m, mode="plugins", stdp=stdp)
