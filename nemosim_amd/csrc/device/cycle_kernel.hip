@@ -256,6 +256,11 @@ uint32_t nemo_dev_cycle_blocks(uint32_t P, uint32_t T)
 	return (P * T + nb - 1u) / nb;
 }
 
+uint32_t nemo_dev_cycle_block_neurons(uint32_t P, uint32_t T)
+{
+	return neurons_per_block(P * T);
+}
+
 int nemo_dev_cycle(const NetDev* nd, const CycleArgs* ca, void* stream)
 {
 	const uint32_t blocks = nemo_dev_cycle_blocks(nd->P, nd->T);

@@ -2,6 +2,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <cstddef>
 #include <cstdio>
 #include <cstring>
@@ -1661,6 +1662,47 @@ wallClockKHz(int dev)
  * against 86). */
 static const double CYCLE_MAX_EVENTS = 1.0e6;
 
+/* Whether a workgroup of the cycle kernel would have so many spikes to deliver
+ * that the fused kernel, whose workgroups share all spikes, is faster: 3 us per
+ * four chunks of 256 synapses, 2 where rows are short. Neurons that fire
+ * together are often neighbours. They are counted from this step's forced ones
+ * and from the steps before: the most of a workgroup, beyond twice its share if
+ * all had the same (of uniformly dense firing the fused kernel has as much to
+ * do), less a sixteenth per step. Calls with 4, 16 and 64 forced neighbours,
+ * cycle kernel (fused kernel 36 to 44 us): 1k x 100 20, 26, 49; 5k x 1000 31, 69,
+ * 216; 20k x 300 25, 44, 118; 100k x 300 (fused 72) 41, 58, 138; 200k x 300 (115)
+ * 56, 73, 152. */
+bool
+Simulation::stepCrowded(const std::vector<unsigned>& fstim) const
+{
+	const uint32_t block = nemo_dev_cycle_block_neurons(m_P, m_T);
+	unsigned forced[NEMO_CYCLE_STIM], most = 0;
+	for(size_t i = 0; i < fstim.size(); ++i) forced[i] = localIdx(fstim[i]) / block;
+	std::sort(forced, forced + fstim.size());
+	for(size_t i = 0, same = 0; i < fstim.size(); ++i) {
+		same = i && forced[i] == forced[i - 1] ? same + 1 : 1;
+		most = std::max(most, unsigned(same));
+	}
+	const double row = double(m_nsyn) / double(m_n);
+	const double chunks = row <= 128.0 ? 0.65 : std::ceil(row / 256.0);
+	return std::max(double(most), m_crowd) * chunks > 30.0 + double(m_n) / 4000.0;
+}
+
+/* the fullest workgroup of the cycle kernel in the step whose words are in
+ * h_step, for stepCrowded */
+void
+Simulation::countCrowd()
+{
+	const uint32_t block = nemo_dev_cycle_block_neurons(m_P, m_T);
+	unsigned most = 0;
+	for(uint32_t w = 0; w < m_words; w += block / 64u) {
+		unsigned c = 0;
+		for(uint32_t k = w; k < std::min(m_words, w + block / 64u); ++k) c += unsigned(__builtin_popcountll(h_step[k]));
+		most = std::max(most, c);
+	}
+	m_crowd = std::max(m_crowd * (15.0 / 16.0), double(most) - 2.0 * double(m_fired.size()) * block / m_n);
+}
+
 /* whether csrc/device/cycle_kernel.hip can run a cycle of this network */
 bool
 Simulation::cycleKernelRuns() const
@@ -1738,9 +1780,11 @@ Simulation::step(const std::vector<unsigned>& fstim, const unsigned* istimIdx, c
 	/* while the network fires densely the cycle kernel's global atomics cost
 	 * more than the fused kernel's fixed cost; the step before says how dense */
 	const bool dense = double(m_fired.size()) * double(m_nsyn) > CYCLE_MAX_EVENTS * double(m_n);
-	if(cycleKernelRuns() && !dense && fstim.size() <= NEMO_CYCLE_STIM && nistim <= NEMO_CYCLE_STIM) {
+	if(cycleKernelRuns() && !dense && fstim.size() <= NEMO_CYCLE_STIM && nistim <= NEMO_CYCLE_STIM
+			&& !stepCrowded(fstim)) {
 		stepCycle(s);
 		decodeStep(h_step, m_fired);
+		countCrowd();
 		return m_fired;
 	}
 	uploadSchedule(1, &s);
@@ -1749,6 +1793,7 @@ Simulation::step(const std::vector<unsigned>& fstim, const unsigned* istimIdx, c
 		launchFused(1, true);
 		readControl(1, nullptr);
 		decodeStep(h_step, m_fired);
+		if(cycleKernelRuns()) countCrowd();
 		return m_fired;
 	}
 	launch(1, nullptr);

@@ -262,6 +262,9 @@ class Simulation
 		void launchDescriptor(const NetDev& nd, bool stepOut);
 		bool cycleKernelRuns() const;
 		void stepCycle(const nemo_schedule_t& s);
+		bool stepCrowded(const std::vector<unsigned>& fstim) const;
+		void countCrowd();
+		double m_crowd = 0.0;          /* fired neurons of a workgroup of the cycle kernel beyond its share */
 		DevBuf d_done;                 /* CycleArgs.done */
 		uint64_t m_cycleSequence = 0;  /* launches that report to h_ctl */
 		bool m_tail = false;           /* the cycle kernel has reported, its end was not waited for (orderBefore) */

@@ -52,6 +52,19 @@ def test_per_cycle_step(nemo_mod, stdp):
     assert adjacent < 2.0 * spread, (adjacent, spread)
 
 
+@pytest.mark.parametrize("n,m", [(5000, 1000), (100000, 300)])
+def test_step(nemo_mod, n, m):
+    """steps with 60 forced neurons, more of which at once take another path"""
+    sim = simulation(nemo_mod, n, m)
+
+    def steps(pop):
+        for _ in range(CYCLES):
+            sim.step(pop)
+
+    adjacent, spread = [best(lambda: steps(p)) for p in populations(n, 60)]
+    assert adjacent < 2.0 * spread, (adjacent, spread)
+
+
 def test_per_cycle_step_long_rows(nemo_mod):
     """neurons with rows of 10000 synapses, next to each other and far apart"""
     n, hubs = 270000, 20
