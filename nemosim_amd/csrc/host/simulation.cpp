@@ -1627,18 +1627,25 @@ Simulation::runStatic(unsigned nsteps, const nemo_schedule_t* schedule, uint64_t
 	m_rasterExternal = true;
 }
 
-void
-Simulation::decodeStep(const uint64_t* words, std::vector<unsigned>& out) const
+/* the step's fired neurons; returns the most of `per` words */
+unsigned
+Simulation::decodeStep(const uint64_t* words, std::vector<unsigned>& out, uint32_t per) const
 {
 	out.clear();
-	for(uint32_t w = 0; w < m_words; ++w) {
-		uint64_t b = words[w];
-		while(b) {
-			uint32_t l = w * 64u + uint32_t(__builtin_ctzll(b));
-			b &= b - 1;
-			if(l < m_n) out.push_back(m_localToGlobal[l]);
+	size_t most = 0;
+	for(uint32_t first = 0; first < m_words; first += per) {
+		const size_t before = out.size();
+		for(uint32_t w = first; w < std::min(m_words, first + per); ++w) {
+			uint64_t b = words[w];
+			while(b) {
+				uint32_t l = w * 64u + uint32_t(__builtin_ctzll(b));
+				b &= b - 1;
+				if(l < m_n) out.push_back(m_localToGlobal[l]);
+			}
 		}
+		most = std::max(most, out.size() - before);
 	}
+	return unsigned(most);
 }
 
 /* the device wall clock's rate (wall_clock64 in the kernels), kHz */
@@ -1688,18 +1695,12 @@ Simulation::stepCrowded(const std::vector<unsigned>& fstim) const
 	return std::max(double(most), m_crowd) * chunks > 30.0 + double(m_n) / 4000.0;
 }
 
-/* the fullest workgroup of the cycle kernel in the step whose words are in
- * h_step, for stepCrowded */
+/* decodes the step whose words are in h_step, and counts for stepCrowded */
 void
-Simulation::countCrowd()
+Simulation::decodeCrowd()
 {
 	const uint32_t block = nemo_dev_cycle_block_neurons(m_P, m_T);
-	unsigned most = 0;
-	for(uint32_t w = 0; w < m_words; w += block / 64u) {
-		unsigned c = 0;
-		for(uint32_t k = w; k < std::min(m_words, w + block / 64u); ++k) c += unsigned(__builtin_popcountll(h_step[k]));
-		most = std::max(most, c);
-	}
+	const unsigned most = decodeStep(h_step, m_fired, block / 64u);
 	m_crowd = std::max(m_crowd * (15.0 / 16.0), double(most) - 2.0 * double(m_fired.size()) * block / m_n);
 }
 
@@ -1783,8 +1784,7 @@ Simulation::step(const std::vector<unsigned>& fstim, const unsigned* istimIdx, c
 	if(cycleKernelRuns() && !dense && fstim.size() <= NEMO_CYCLE_STIM && nistim <= NEMO_CYCLE_STIM
 			&& !stepCrowded(fstim)) {
 		stepCycle(s);
-		decodeStep(h_step, m_fired);
-		countCrowd();
+		decodeCrowd();
 		return m_fired;
 	}
 	uploadSchedule(1, &s);
@@ -1792,8 +1792,7 @@ Simulation::step(const std::vector<unsigned>& fstim, const unsigned* istimIdx, c
 		/* the raster words come back with the control block */
 		launchFused(1, true);
 		readControl(1, nullptr);
-		decodeStep(h_step, m_fired);
-		if(cycleKernelRuns()) countCrowd();
+		decodeCrowd();
 		return m_fired;
 	}
 	launch(1, nullptr);
@@ -1801,7 +1800,7 @@ Simulation::step(const std::vector<unsigned>& fstim, const unsigned* istimIdx, c
 	if(m_words) {
 		hipCheck(hipMemcpy(m_rasterHost.data(), d_raster.ptr, size_t(m_words) * 8, hipMemcpyDeviceToHost), "D2H");
 	}
-	decodeStep(m_rasterHost.data(), m_fired);
+	decodeStep(m_rasterHost.data(), m_fired, std::max(1u, m_words));
 	return m_fired;
 }
 
