@@ -85,7 +85,7 @@ typedef struct NetDev {
 	 * by cycle parity */
 	uint64_t* fl;             /* [flRing][P][T] fired neurons of each partition, (cycle << 32) | neuron */
 	uint64_t* fc;             /* [flRing][P] (cycle << 32) | fired count; starts all-ones */
-	uint64_t* mk;             /* [flRing][P*T/32] (cycle << 32) | 32 fired bits; starts all-ones (NEMO_NET_MASKS) */
+	uint64_t* mk;             /* [flRing][nemo_mask_words(P*T/32)] (cycle << 32) | 32 fired bits; starts all-ones (NEMO_NET_MASKS) */
 	uint64_t* rfg;            /* [2][n], with NEMO_NET_MASKS [4][n], firing history by cycle (STDP only) */
 	uint32_t* status;         /* NEMO_STATUS_* */
 	unsigned long long* events; /* delivered-synapse counter */
@@ -255,6 +255,12 @@ static inline uint32_t nemo_step_lds_bytes(uint32_t T, uint32_t D, uint32_t P, i
 	}
 	return b;
 }
+
+/* words between cycles in NetDev.mk: whole lines of memory */
+#ifdef __HIPCC__
+__host__ __device__
+#endif
+static inline uint32_t nemo_mask_words(uint32_t words) { return (words + 15u) & ~15u; }
 
 /* LDS bytes of mask_kernel.hip: the ring, external current, forced-firing
  * bits, overflow bits and 128 16-bit sources per wave */

@@ -801,7 +801,7 @@ Simulation::Simulation(const NetworkImpl& net, const ConfigurationImpl& conf) :
 	const bool words = m_fused && m_masks;
 	if(words) {
 		m_flRing = m_stdp ? postLen + 3u : 2u;
-		d_mk.alloc(size_t(m_flRing) * m_P * (m_T / 32u) * 8);
+		d_mk.alloc(size_t(m_flRing) * nemo_mask_words(m_P * (m_T / 32u)) * 8);
 	} else {
 		m_flRing = m_stdp ? std::max(3u, postLen + 2u) : (m_defer ? 3u : 2u);
 		d_fl.alloc(size_t(m_flRing) * m_P * m_T * 8);

@@ -3,7 +3,8 @@ that fire together are often next to each other (a stimulated population, a
 layer), so no path may leave their delivery to the few workgroups or waves that
 hold them. Each case times the same network and the same number of forced
 neurons in every cycle, adjacent and spread, the best of several runs each:
-adjacent ones may take at most twice as long."""
+adjacent ones may take at most twice as long, half as long again on the fused
+kernel."""
 import time
 
 import numpy as np
@@ -50,6 +51,19 @@ def test_per_cycle_step(nemo_mod, stdp):
     assert sim.info()["fused"] == 0
     adjacent, spread = [best(lambda: sim.run(CYCLES, fstim=[p] * CYCLES)) for p in populations(n, 256)]
     assert adjacent < 2.0 * spread, (adjacent, spread)
+
+
+@pytest.mark.parametrize("n,m,pop,stdp", [
+    (5000, 1000, 1000, False),       # up to 64 words per wave
+    (50000, 300, 2000, False),       # up to 256
+    (200000, 100, 2000, False),      # more
+    (20000, 300, 1000, True),
+])
+def test_fused(nemo_mod, n, m, pop, stdp):
+    sim = simulation(nemo_mod, n, m, stdp=stdp)
+    assert sim.info()["fused"] == 1
+    adjacent, spread = [best(lambda: sim.run(CYCLES, fstim=[p] * CYCLES)) for p in populations(n, pop)]
+    assert adjacent < 1.5 * spread, (adjacent, spread)
 
 
 @pytest.mark.parametrize("n,m", [(5000, 1000), (100000, 300)])
