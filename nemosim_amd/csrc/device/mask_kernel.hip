@@ -58,7 +58,7 @@ struct Deal {
 	{
 		const uint32_t g0 = wave - wave % GROUP, g1 = min(g0 + GROUP, nwaves);
 		waves = g1 - g0;
-		end = g1 == nwaves ? W : (W * g1 / nwaves) & ~15u;
+		end = wave >= nwaves ? 0u : g1 == nwaves ? W : (W * g1 / nwaves) & ~15u;   /* waves beyond: no words */
 		begin = ((W * g0 / nwaves) & ~15u) + ((wave - g0) << PIECE);
 	}
 	/* the j-th of the wave's words; the first of those from the j-th on, j a
@@ -442,8 +442,7 @@ __device__ __forceinline__ void run_masked(const NetDev& nd, uint32_t p)
 	}
 	const uint32_t W = P * fwords;
 	const Deal<WORDS> deal(wave, nw, W);
-	const uint32_t mine = deal.further(lane);
-	const uint32_t wend = wave < nw ? deal.end : 0u;   /* waves beyond the neurons' have none */
+	const uint32_t myFurther = deal.further(lane);
 	uint32_t wslot = uint32_t(nd.cycle0 % R);               /* cycle mod R */
 	if(STDP) {
 		/* the tables to LDS: they are read for every plastic synapse */
@@ -604,7 +603,13 @@ __device__ __forceinline__ void run_masked(const NetDev& nd, uint32_t p)
 		/* ---- 3. this wave's words of every partition; 4. delivery of the
 		 * sources in them */
 		bool first = true;
-		for(uint32_t c0 = 0; deal.first(c0) < wend; c0 += 64u * WORDS) {   /* wave-uniform */
+		for(uint32_t c0 = 0; deal.first(c0) < deal.end; c0 += 64u * WORDS) {   /* wave-uniform */
+			uint32_t mine = myFurther;
+			if(SAT) {   /* found again each time: no register left to keep it in over the cycle */
+				mine = lane;
+				asm volatile("" : "+v"(mine));
+				mine = deal.further(mine);
+			}
 			uint64_t m[PAIRS];
 			uint32_t pos[PAIRS];
 			uint32_t pending = 0;
@@ -612,7 +617,7 @@ __device__ __forceinline__ void run_masked(const NetDev& nd, uint32_t p)
 			for(uint32_t i = 0; i < PAIRS; ++i) m[i] = 0ull;
 #pragma unroll
 			for(uint32_t i = 0; i < WORDS; ++i) {
-				if(deal.first(c0 + 64u * i) + mine < wend) pending |= 1u << i;
+				if(deal.first(c0 + 64u * i) + mine < deal.end) pending |= 1u << i;
 			}
 			uint32_t spins = 0;
 			while(pending) {
@@ -620,7 +625,7 @@ __device__ __forceinline__ void run_masked(const NetDev& nd, uint32_t p)
 #pragma unroll
 				for(uint32_t i = 0; i < WORDS; ++i) {
 					v[i] = 0ull;
-					if(deal.first(c0 + 64u * i) < wend) {   /* wave-uniform */
+					if(deal.first(c0 + 64u * i) < deal.end) {   /* wave-uniform */
 						/* a byte offset from a scalar address */
 						if((pending >> i) & 1u) v[i] = ld_agent(reinterpret_cast<const NEMO_GLOBAL uint64_t*>(
 								reinterpret_cast<const NEMO_GLOBAL uint8_t*>(words + deal.first(c0 + 64u * i)) + mine * 8u));
@@ -648,7 +653,7 @@ __device__ __forceinline__ void run_masked(const NetDev& nd, uint32_t p)
 #pragma unroll
 			for(uint32_t i = 0; i < PAIRS; ++i) {
 				pos[i] = 0u;
-				if(deal.first(c0 + 128u * i) < wend) {   /* wave-uniform */
+				if(deal.first(c0 + 128u * i) < deal.end) {   /* wave-uniform */
 					const uint32_t c = uint32_t(__popcll(m[i]));
 					const uint32_t x = wave_scan(c);
 					pos[i] = total + x - c;
