@@ -171,7 +171,11 @@ uint32_t nemo_dev_cycle_block_neurons(uint32_t P, uint32_t T);
 /* The end of a launch of one network, after its step kernel on the stream: its
  * control block to host memory, then the report; the clock words start anew. */
 int nemo_dev_step_report(uint32_t* ctl, CycleReport* report, uint64_t sequence, void* stream);
-int nemo_dev_step_max_blocks(uint32_t blockDim, uint32_t ldsBytes, uint32_t variant, uint32_t* maxBlocks);
+/* Workgroups that the device holds at once: of the batched launch's kernel, or
+ * with P partitions of T neurons (P > 0) of that and of the one that a launch of
+ * such a network alone takes, whichever are fewer. */
+int nemo_dev_step_max_blocks(uint32_t blockDim, uint32_t ldsBytes, uint32_t variant, uint32_t P, uint32_t T,
+		uint32_t* maxBlocks);
 /* Batched step as an instantiated HIP graph (clear -> persistent step ->
  * collect); collect_dev receives [nnets][16] words: the first 12 words of
  * each network's control block, the last four of them the first start and

@@ -1078,11 +1078,11 @@ static const void* step_kernel_variant(uint32_t variant)
 	}
 }
 
-static const void* step_kernel_one_variant(uint32_t variant, const NetDev* nd)
+static const void* step_kernel_one_variant(uint32_t variant, uint32_t P, uint32_t T)
 {
 	if(variant & 4u) {
-		const uint32_t nw = nd->T / 64u;
-		return nemo_dev_mask_kernel(variant, (nd->P * (nd->T / 32u) + nw - 1u) / nw);
+		const uint32_t nw = T / 64u;
+		return nemo_dev_mask_kernel(variant, (P * (T / 32u) + nw - 1u) / nw);
 	}
 	switch(variant & 3u) {
 	case 0: return reinterpret_cast<const void*>(&nemo_step_kernel_one<false, false>);
@@ -1244,7 +1244,7 @@ int nemo_dev_step_launch(const NetDev* nets_dev, const WorkItem* work_dev, uint3
 int nemo_dev_step_launch_one(const NetDev* nd_host, const WorkItem* work_dev, uint32_t nblocks,
 		uint32_t blockDim, uint32_t ldsBytes, uint32_t variant, void* stream)
 {
-	const void* kern = step_kernel_one_variant(variant, nd_host);
+	const void* kern = step_kernel_one_variant(variant, nd_host->P, nd_host->T);
 	hipError_t e = ensure_lds_limit(kern, ldsBytes);
 	if(e != hipSuccess) return int(e);
 	void* args[] = { const_cast<NetDev*>(nd_host), const_cast<WorkItem**>(&work_dev) };
@@ -1323,16 +1323,21 @@ int nemo_dev_graph_destroy(void* exec)
 	return exec ? int(hipGraphExecDestroy(static_cast<hipGraphExec_t>(exec))) : 0;
 }
 
-int nemo_dev_step_max_blocks(uint32_t blockDim, uint32_t ldsBytes, uint32_t variant, uint32_t* maxBlocks)
+int nemo_dev_step_max_blocks(uint32_t blockDim, uint32_t ldsBytes, uint32_t variant, uint32_t P, uint32_t T,
+		uint32_t* maxBlocks)
 {
-	const void* kern = step_kernel_variant(variant);
-	hipError_t e = ensure_lds_limit(kern, ldsBytes);
-	if(e != hipSuccess) return int(e);
 	int perCU = 0;
-	e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, kern, int(blockDim), size_t(ldsBytes));
-	if(e != hipSuccess) return int(e);
+	for(int single = 0; single < (P ? 2 : 1); ++single) {
+		const void* kern = single ? step_kernel_one_variant(variant, P, T) : step_kernel_variant(variant);
+		hipError_t e = ensure_lds_limit(kern, ldsBytes);
+		if(e != hipSuccess) return int(e);
+		int n = 0;
+		e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kern, int(blockDim), size_t(ldsBytes));
+		if(e != hipSuccess) return int(e);
+		perCU = single ? std::min(perCU, n) : n;
+	}
 	int dev = 0;
-	e = hipGetDevice(&dev);
+	hipError_t e = hipGetDevice(&dev);
 	if(e != hipSuccess) return int(e);
 	int cus = 0;
 	e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);

@@ -158,7 +158,7 @@ runBatch(Simulation* const sims[], size_t n, const unsigned nsteps[], unsigned l
 			const uint32_t bd = std::max(blockDim, sim->batchThreads());
 			const uint32_t ld = std::max(lds, sim->batchLdsBytes());
 			uint32_t maxB = 0;
-			hipCheck(nemo_dev_step_max_blocks(bd, ld, variant, &maxB), "occupancy query");
+			hipCheck(nemo_dev_step_max_blocks(bd, ld, variant, 0, 0, &maxB), "occupancy query");
 			if(blocks + sim->partitions() > maxB) {
 				if(members.empty()) {
 					throw exception(NEMO_API_UNSUPPORTED, "simulation does not fit the device");
@@ -183,7 +183,7 @@ runBatch(Simulation* const sims[], size_t n, const unsigned nsteps[], unsigned l
 		}
 		bool far = false;
 		if(farDim > blockDim) {
-			hipCheck(nemo_dev_step_max_blocks(farDim, farLds, variant, &maxB), "occupancy query");
+			hipCheck(nemo_dev_step_max_blocks(farDim, farLds, variant, 0, 0, &maxB), "occupancy query");
 			far = blocks <= maxB;
 		}
 		if(far) {

@@ -472,7 +472,10 @@ Simulation::Simulation(const NetworkImpl& net, const ConfigurationImpl& conf) :
 	if(m_masks && m_n > 0 && whyNotFused.empty()) {
 		uint32_t maxBlocks = 0;
 		const uint32_t lds = ldsFor(T);
-		if(lds <= ldsLimit) hipCheck(nemo_dev_step_max_blocks(T + 64u * stdpWaves(T), lds, variant(), &maxBlocks), "occupancy query");
+		if(lds <= ldsLimit) {
+			hipCheck(nemo_dev_step_max_blocks(T + 64u * stdpWaves(T), lds, variant(), (m_n + T - 1) / T, T, &maxBlocks),
+					"occupancy query");
+		}
 		if((m_n + T - 1) / T > maxBlocks || (m_stdp && T > 640u)) {
 			m_masks = false;
 			T = partitionSize();
@@ -487,7 +490,7 @@ Simulation::Simulation(const NetworkImpl& net, const ConfigurationImpl& conf) :
 	m_lds = ldsFor(T);
 	if(whyNotFused.empty() && m_P > 0) {
 		uint32_t maxBlocks = 0;
-		hipCheck(nemo_dev_step_max_blocks(blockThreads(), m_lds, variant(), &maxBlocks), "occupancy query");
+		hipCheck(nemo_dev_step_max_blocks(blockThreads(), m_lds, variant(), m_P, m_T, &maxBlocks), "occupancy query");
 		if(m_P > maxBlocks) {
 			whyNotFused = fmt("network of ", m_n, " neurons needs ", m_P,
 					" co-resident workgroups of ", m_T, " neurons; the device holds ", maxBlocks);
@@ -499,7 +502,7 @@ Simulation::Simulation(const NetworkImpl& net, const ConfigurationImpl& conf) :
 		 * chunks (256 bytes each, twice with words) of every cycle's work list */
 		auto fits = [&](uint32_t lds) {
 			if(lds > ldsLimit) return false;
-			hipCheck(nemo_dev_step_max_blocks(blockThreads(), lds, variant(), &maxBlocks), "occupancy query");
+			hipCheck(nemo_dev_step_max_blocks(blockThreads(), lds, variant(), m_P, m_T, &maxBlocks), "occupancy query");
 			return m_P <= maxBlocks;
 		};
 		if(m_stdp && m_masks) {
@@ -1212,7 +1215,8 @@ Simulation::planExchange(const ConfigurationImpl& conf, uint32_t ldsLimit)
 			const uint32_t lds = m_lds + NEMO_MASK_FAR_LDS_BYTES(cap);
 			uint32_t maxBlocks = 0;
 			if(lds > ldsLimit) continue;
-			hipCheck(nemo_dev_step_max_blocks(m_T + 64u * (used - nw + n), lds, variant(), &maxBlocks), "occupancy query");
+			hipCheck(nemo_dev_step_max_blocks(m_T + 64u * (used - nw + n), lds, variant(), m_P, m_T, &maxBlocks),
+					"occupancy query");
 			if(m_P <= maxBlocks) {
 				m_farWaves = n;
 				m_farCap = cap;
@@ -1234,7 +1238,7 @@ Simulation::planExchange(const ConfigurationImpl& conf, uint32_t ldsLimit)
 		const uint32_t lds = m_lds + NEMO_FAR_LDS_BYTES(cap);
 		if(lds > ldsLimit) continue;
 		uint32_t maxBlocks = 0;
-		hipCheck(nemo_dev_step_max_blocks(blockThreads(), lds, variant(), &maxBlocks), "occupancy query");
+		hipCheck(nemo_dev_step_max_blocks(blockThreads(), lds, variant(), m_P, m_T, &maxBlocks), "occupancy query");
 		if(m_P <= maxBlocks) {
 			m_exWaves = ex;
 			m_farCap = cap;
