@@ -46,6 +46,7 @@
  */
 #include <hip/hip_runtime.h>
 #include <algorithm>
+#include <mutex>
 #include <stddef.h>
 #include <stdint.h>
 
@@ -1094,9 +1095,12 @@ static const void* step_kernel_one_variant(uint32_t variant, uint32_t P, uint32_
 
 /* The dynamic LDS limit of a kernel is raised once to the largest size
  * asked for (the attribute call is a host-side round trip per launch
- * otherwise). Launches are serialised by the host library's device lock. */
+ * otherwise). Simulations under construction ask without the host library's
+ * device lock, from several threads. */
 static hipError_t ensure_lds_limit(const void* kern, uint32_t ldsBytes)
 {
+	static std::mutex mutex;
+	std::lock_guard<std::mutex> lock(mutex);
 	static const void* kerns[32] = {};
 	static uint32_t limits[32] = {};
 	for(int i = 0; i < 32; ++i) {
