@@ -45,6 +45,15 @@ __host__ __device__ inline uint32_t neurons_per_block(uint32_t neurons)
 	return neurons <= SMALL ? 64u : BLOCK;
 }
 
+/* Dynamic LDS: a source's bucket bounds for each wave. 64 KB is what a launch
+ * takes without asking for more; 4 KB are for the kernel's own variables. */
+constexpr uint32_t LDS_DYNAMIC = 60u * 1024u;
+
+__host__ inline uint64_t dynamic_lds(uint32_t P)
+{
+	return uint64_t(WAVES) * (uint64_t(P) + 1u) * 4u;
+}
+
 /* the end of the launch, and the report */
 __device__ inline void finish_cycle(const CycleArgs& ca)
 {
@@ -261,10 +270,16 @@ uint32_t nemo_dev_cycle_block_neurons(uint32_t P, uint32_t T)
 	return neurons_per_block(P * T);
 }
 
+int nemo_dev_cycle_fits(uint32_t P)
+{
+	return dynamic_lds(P) <= LDS_DYNAMIC ? 1 : 0;
+}
+
 int nemo_dev_cycle(const NetDev* nd, const CycleArgs* ca, void* stream)
 {
+	if(!nemo_dev_cycle_fits(nd->P)) return int(hipErrorInvalidValue);
 	const uint32_t blocks = nemo_dev_cycle_blocks(nd->P, nd->T);
-	const uint32_t lds = WAVES * (nd->P + 1u) * 4u;
+	const uint32_t lds = uint32_t(dynamic_lds(nd->P));
 	auto kernel = (nd->flags & NEMO_NET_IZHIKEVICH_ONLY) ? &nemo_cycle_kernel<true> : &nemo_cycle_kernel<false>;
 	hipLaunchKernelGGL(kernel, dim3(blocks), dim3(BLOCK), lds, static_cast<hipStream_t>(stream), *nd, *ca);
 	return int(hipGetLastError());

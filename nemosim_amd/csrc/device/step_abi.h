@@ -166,6 +166,8 @@ int nemo_dev_step_launch_one(const NetDev* nd_host, const WorkItem* work_dev, ui
 /* One cycle of a network without STDP whose sums stay within int32 */
 int nemo_dev_cycle(const NetDev* nd_host, const CycleArgs* ca, void* stream);
 uint32_t nemo_dev_cycle_blocks(uint32_t P, uint32_t T);
+/* whether the bucket bounds of P partitions fit its LDS */
+int nemo_dev_cycle_fits(uint32_t P);
 /* neurons of one of its workgroups */
 uint32_t nemo_dev_cycle_block_neurons(uint32_t P, uint32_t T);
 /* The end of a launch of one network, after its step kernel on the stream: its

@@ -1712,7 +1712,7 @@ Simulation::decodeCrowd()
 bool
 Simulation::cycleKernelRuns() const
 {
-	return m_fused && !m_stdp && !m_saturate && m_P > 0 && m_n > 0;
+	return m_fused && !m_stdp && !m_saturate && m_P > 0 && m_n > 0 && nemo_dev_cycle_fits(m_P);
 }
 
 /* One cycle by cycle_kernel.hip. Its stimulus travels in the kernel's
