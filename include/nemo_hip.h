@@ -68,16 +68,20 @@ nemo_status_t nemo_set_stdp_lds_staging(nemo_configuration_t conf, int enable);
  * host (src/nemo/ConnectivityMatrix.cpp:98-161). */
 nemo_status_t nemo_set_device_construction(nemo_configuration_t conf, int enable);
 
-/* Waves of each step-kernel workgroup that run the exchange between
- * partitions and the delivery of delay-1 records, while the others deliver
- * the previous cycle's records of longer delays (and, with STDP, build the
- * work lists and accumulate): n > 0 = n waves (at least one other must
- * remain; needs deferred delivery and LDS room for the far list), < 0 =
- * none (every wave does both, one after the other), 0 (default) =
- * automatic: 3 of every 8 waves for networks with STDP whose workgroups
- * nemo_set_partition_size makes 8 waves (512 neurons) or more, and for those
- * that need more than 10 waves; none otherwise. Same results either
- * way. No counterpart in NeMo; a tuning knob of the fused step kernel. */
+/* Which waves of a step-kernel workgroup run the exchange between partitions
+ * and the delivery of delay-1 records, and which deliver the previous cycle's
+ * records of longer delays. n > 0: n of the neurons' waves run the exchange,
+ * the others the rest, with STDP its work lists and accumulation too (at least
+ * one other must remain; needs deferred delivery and LDS room for the far
+ * list); partitions exchange lists of fired neurons. < 0: no waves of their
+ * own for either, every wave does both, one after the other. 0 (default):
+ * automatic. Networks exchange their fired bits as words, and workgroups get
+ * waves beyond the neurons' for the longer delays (block_threads of
+ * nemo_hip_info counts them), except those with STDP that
+ * nemo_set_partition_size makes 8 waves (512 neurons) or more, and those with
+ * STDP that need more than 10: they exchange lists, by 3 of every 8 waves. Same
+ * results either way. No counterpart in NeMo; a tuning knob of the fused step
+ * kernel. */
 nemo_status_t nemo_set_exchange_waves(nemo_configuration_t conf, int waves);
 
 /* Which step implementation runs a simulation:

@@ -1201,7 +1201,7 @@ Simulation::planExchange(const ConfigurationImpl& conf, uint32_t ldsLimit)
 	m_ldsNoFar = m_lds;
 	const uint32_t nw = m_T / 64u;
 	m_farWaves = 0;
-	if(!m_fused || !m_defer || m_P == 0) return;
+	if(!m_fused || !m_defer || m_P == 0 || conf.exchangeWaves < 0) return;
 	if(m_masks) {
 		/* Far waves: as many as the neurons' waves, at least 2, as far as 16 in
 		 * all go, unless the device cannot hold the larger workgroups or their
@@ -1226,7 +1226,6 @@ Simulation::planExchange(const ConfigurationImpl& conf, uint32_t ldsLimit)
 		}
 		return;
 	}
-	if(conf.exchangeWaves < 0) return;
 	uint32_t ex = uint32_t(conf.exchangeWaves);
 	if(conf.exchangeWaves == 0) {
 		if(!m_stdp || nw < 8u) return;
