@@ -191,18 +191,22 @@ typedef struct nemo_hip_info {
 	unsigned long long synapses;
 	unsigned long long plastic_synapses;
 	unsigned long long device_bytes;
-	unsigned lds_bytes;          /* per workgroup; without the far list of a launch of its own that has far waves */
-	unsigned block_threads;
+	unsigned lds_bytes;          /* LDS of a workgroup as a batched launch packs it: without the far list that a
+	                              * launch of its own has beside its far waves (16 bytes per far_list_sources) */
+	unsigned block_threads;      /* of a workgroup in a launch of its own: a thread per neuron, and 64 for each wave
+	                              * beyond them (far records, STDP) */
 	float last_kernel_ms;        /* step-kernel time of the last run, from the first start to the last end of its
 	                              * workgroups (plugin and per-cycle step: HIP events around its launches) */
 	unsigned fused;              /* 1: fused persistent step kernel; 0: plugin step */
 	unsigned deferred;           /* 1: records of delay >= 2 delivered one cycle late */
 	unsigned lanes_per_source;   /* lanes sharing one fired source in delivery */
 	unsigned stdp_staged_chunks; /* STDP chunks whose reverse records are staged in LDS per cycle */
-	unsigned stdp_prefix_ring;   /* 1: STDP work lists need no fired counts of earlier cycles from memory */
+	unsigned stdp_prefix_ring;   /* 1: fired-count prefixes of the last postLen cycles are kept in LDS, or, where
+	                              * words are exchanged, not needed */
 	unsigned device_built;       /* 1: synapse structures were built on the device */
 	unsigned exchange_waves;     /* waves per workgroup running the exchange and delay-1 delivery */
-	unsigned far_list_sources;   /* fired sources per cycle whose far records wait in the LDS far list */
+	unsigned far_list_sources;   /* fired sources per cycle whose far records (delays of 2 and more) wait in LDS, for
+	                              * the waves beside the exchange waves or for the far waves */
 } nemo_hip_info_t;
 
 nemo_status_t nemo_hip_get_info(nemo_simulation_t sim, nemo_hip_info_t* info);
