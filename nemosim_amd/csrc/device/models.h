@@ -62,14 +62,16 @@ NEMO_HD inline uint32_t urand(Rng& r)
 	return r.s[3];
 }
 
-/* Correctly rounded single-precision square root: hipcc's default for sqrtf
- * (-fhip-fp32-correctly-rounded-divide-sqrt). */
+/* Correctly rounded single-precision square root: the build asks for it
+ * (-fhip-fp32-correctly-rounded-divide-sqrt), hipcc's default too. */
 NEMO_HD inline float sqrt_f32(float x)
 {
 	return __builtin_sqrtf(x);
 }
 
-/* Correctly rounded single-precision division, by the same default. */
+/* Correctly rounded single-precision division: the double quotient of two
+ * floats, rounded once more, is the correctly rounded float quotient. (In
+ * single precision the variants for any model spill.) */
 NEMO_HD inline float div_f32(float a, float b)
 {
 	return float(double(a) / double(b));
