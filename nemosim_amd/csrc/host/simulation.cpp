@@ -1630,25 +1630,18 @@ Simulation::runStatic(unsigned nsteps, const nemo_schedule_t* schedule, uint64_t
 	m_rasterExternal = true;
 }
 
-/* the step's fired neurons; returns the most of `per` words */
-unsigned
-Simulation::decodeStep(const uint64_t* words, std::vector<unsigned>& out, uint32_t per) const
+void
+Simulation::decodeStep(const uint64_t* words, std::vector<unsigned>& out) const
 {
 	out.clear();
-	size_t most = 0;
-	for(uint32_t first = 0; first < m_words; first += per) {
-		const size_t before = out.size();
-		for(uint32_t w = first; w < std::min(m_words, first + per); ++w) {
-			uint64_t b = words[w];
-			while(b) {
-				uint32_t l = w * 64u + uint32_t(__builtin_ctzll(b));
-				b &= b - 1;
-				if(l < m_n) out.push_back(m_localToGlobal[l]);
-			}
+	for(uint32_t w = 0; w < m_words; ++w) {
+		uint64_t b = words[w];
+		while(b) {
+			uint32_t l = w * 64u + uint32_t(__builtin_ctzll(b));
+			b &= b - 1;
+			if(l < m_n) out.push_back(m_localToGlobal[l]);
 		}
-		most = std::max(most, out.size() - before);
 	}
-	return unsigned(most);
 }
 
 /* the device wall clock's rate (wall_clock64 in the kernels), kHz */
@@ -1685,25 +1678,42 @@ static const double CYCLE_MAX_EVENTS = 1.0e6;
 bool
 Simulation::stepCrowded(const std::vector<unsigned>& fstim) const
 {
-	const uint32_t block = nemo_dev_cycle_block_neurons(m_P, m_T);
+	const double row = double(m_nsyn) / double(m_n);
+	const double chunks = row <= 128.0 ? 0.65 : std::ceil(row / 256.0);
+	const double limit = (30.0 + double(m_n) / 4000.0) / chunks;
+	if(m_crowd > limit) return true;
+	if(double(fstim.size()) <= limit) return false;
+	const int shift = __builtin_ctz(nemo_dev_cycle_block_neurons(m_P, m_T));
 	unsigned forced[NEMO_CYCLE_STIM], most = 0;
-	for(size_t i = 0; i < fstim.size(); ++i) forced[i] = localIdx(fstim[i]) / block;
+	unsigned char count[256] = {};   /* by the low bits of the workgroup: no fewer than are in one */
+	for(size_t i = 0; i < fstim.size(); ++i) {
+		forced[i] = localIdx(fstim[i]) >> shift;
+		most = std::max<unsigned>(most, ++count[forced[i] & 255u]);
+	}
+	if(double(most) <= limit) return false;
 	std::sort(forced, forced + fstim.size());
+	most = 0;
 	for(size_t i = 0, same = 0; i < fstim.size(); ++i) {
 		same = i && forced[i] == forced[i - 1] ? same + 1 : 1;
 		most = std::max(most, unsigned(same));
 	}
-	const double row = double(m_nsyn) / double(m_n);
-	const double chunks = row <= 128.0 ? 0.65 : std::ceil(row / 256.0);
-	return std::max(double(most), m_crowd) * chunks > 30.0 + double(m_n) / 4000.0;
+	return double(most) > limit;
 }
 
-/* decodes the step whose words are in h_step, and counts for stepCrowded */
+/* the last step's fired neurons counted for stepCrowded, while the next step's
+ * kernel runs (before its launch it took 0.9 us of a step of 100k neurons) */
 void
-Simulation::decodeCrowd()
+Simulation::countCrowd()
 {
 	const uint32_t block = nemo_dev_cycle_block_neurons(m_P, m_T);
-	const unsigned most = decodeStep(h_step, m_fired, block / 64u);
+	const int shift = __builtin_ctz(block);
+	uint32_t most = 0, same = 0, last = ~0u;
+	for(unsigned g : m_fired) {   /* ascending local index */
+		const uint32_t b = (m_dense[g - m_minG] - 1u) >> shift;
+		same = b == last ? same + 1u : 1u;
+		last = b;
+		most = std::max(most, same);
+	}
 	m_crowd = std::max(m_crowd * (15.0 / 16.0), double(most) - 2.0 * double(m_fired.size()) * block / m_n);
 }
 
@@ -1747,6 +1757,7 @@ Simulation::stepCycle(const nemo_schedule_t& s)
 	hipStream_t st = static_cast<hipStream_t>(m_stream);
 	hipCheck(nemo_dev_cycle(&nd, &ca, st), "cycle kernel launch");
 	m_tail = true;
+	countCrowd();
 	waitReport(&rep->sequence, ca.sequence, st, "cycle kernel");
 	m_kernelMs = float(double(rep->end - rep->start) / wallClockKHz(m_device));
 	const uint32_t ctl[8] = {};
@@ -1787,15 +1798,16 @@ Simulation::step(const std::vector<unsigned>& fstim, const unsigned* istimIdx, c
 	if(cycleKernelRuns() && !dense && fstim.size() <= NEMO_CYCLE_STIM && nistim <= NEMO_CYCLE_STIM
 			&& !stepCrowded(fstim)) {
 		stepCycle(s);
-		decodeCrowd();
+		decodeStep(h_step, m_fired);
 		return m_fired;
 	}
 	uploadSchedule(1, &s);
+	if(cycleKernelRuns()) countCrowd();
 	if(m_fused && m_P > 0 && m_n > 0) {
 		/* the raster words come back with the control block */
 		launchFused(1, true);
 		readControl(1, nullptr);
-		decodeCrowd();
+		decodeStep(h_step, m_fired);
 		return m_fired;
 	}
 	launch(1, nullptr);
@@ -1803,7 +1815,7 @@ Simulation::step(const std::vector<unsigned>& fstim, const unsigned* istimIdx, c
 	if(m_words) {
 		hipCheck(hipMemcpy(m_rasterHost.data(), d_raster.ptr, size_t(m_words) * 8, hipMemcpyDeviceToHost), "D2H");
 	}
-	decodeStep(m_rasterHost.data(), m_fired, std::max(1u, m_words));
+	decodeStep(m_rasterHost.data(), m_fired);
 	return m_fired;
 }
 

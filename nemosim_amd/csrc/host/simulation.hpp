@@ -263,7 +263,7 @@ class Simulation
 		bool cycleKernelRuns() const;
 		void stepCycle(const nemo_schedule_t& s);
 		bool stepCrowded(const std::vector<unsigned>& fstim) const;
-		void decodeCrowd();
+		void countCrowd();
 		double m_crowd = 0.0;          /* fired neurons of a workgroup of the cycle kernel beyond its share */
 		DevBuf d_done;                 /* CycleArgs.done */
 		uint64_t m_cycleSequence = 0;  /* launches that report to h_ctl */
@@ -294,7 +294,7 @@ class Simulation
 		void launch(unsigned nsteps, unsigned long long* events);
 		void readScalar(const DevBuf& b, size_t offset, void* out) const;
 		void writeScalar(DevBuf& b, size_t offset, const void* in, size_t bytes);
-		unsigned decodeStep(const uint64_t* words, std::vector<unsigned>& out, uint32_t per) const;
+		void decodeStep(const uint64_t* words, std::vector<unsigned>& out) const;
 		size_t synapseRecord(synapse_id id) const;
 		/* the forward matrix (d_off, d_syn, m_defer), the synapse query
 		 * tables and, with STDP, the reverse matrix, built on the device from
