@@ -73,7 +73,7 @@ __global__ void __launch_bounds__(BLOCK) nemo_cycle_kernel(const NetDev nd, cons
 	__shared__ float ext[BLOCK];
 	__shared__ uint32_t fst[BLOCK / 32u];
 	__shared__ uint32_t list[BLOCK];
-	__shared__ uint32_t wfired[WAVES], wsum[WAVES];
+	__shared__ uint32_t wfired[WAVES];
 	__shared__ uint64_t wmask[WAVES];
 	const uint32_t tid = threadIdx.x;
 	const uint32_t lane = tid & 63u;
@@ -84,34 +84,22 @@ __global__ void __launch_bounds__(BLOCK) nemo_cycle_kernel(const NetDev nd, cons
 	const uint32_t l = tid < nb ? first + tid : ~0u;
 	const uint32_t p = (first + wave * 64u) / T;   /* T is a multiple of 64: one partition per wave */
 	const uint32_t tl = l - p * T;
-	if(ca.report && l == 0) st_host(&ca.report->start, (uint64_t) wall_clock64());
+	if(l == 0) st_host(&ca.report->start, (uint64_t) wall_clock64());
 
-	/* the cycle's stimulus: in the arguments, or in the launch's lists */
-	uint32_t f0 = 0, f1 = ca.nf, i0 = 0, i1 = ca.ni;
-	const uint32_t* fidx = ca.fidx;
-	const uint32_t* iidx = ca.iidx;
-	const float* ival = ca.ival;
-	if(nd.fs_ptr) {
-		f0 = nd.fs_ptr[ca.k];
-		f1 = nd.fs_ptr[ca.k + 1u];
-		fidx = nd.fs_idx;
-		i0 = nd.is_ptr[ca.k];
-		i1 = nd.is_ptr[ca.k + 1u];
-		iidx = nd.is_idx;
-		ival = nd.is_val;
-	}
-	const bool stim = f1 > f0 || i1 > i0;
+	/* the cycle's stimulus */
+	const bool stim = ca.nf > 0u || ca.ni > 0u;
 	if(stim) {
 		ext[tid] = 0.0f;
 		if(tid < BLOCK / 32u) fst[tid] = 0u;
 		__syncthreads();
-		for(uint32_t e = f0 + tid; e < f1; e += BLOCK) {
-			const uint32_t x = fidx[e] - first;
+		static_assert(NEMO_CYCLE_STIM <= BLOCK, "a thread per entry");
+		if(tid < ca.nf) {
+			const uint32_t x = ca.fidx[tid] - first;
 			if(x < nb) atomicOr(&fst[x >> 5], 1u << (x & 31u));
 		}
-		for(uint32_t e = i0 + tid; e < i1; e += BLOCK) {   /* one entry per neuron */
-			const uint32_t x = iidx[e] - first;
-			if(x < nb) ext[x] = ival[e];
+		if(tid < ca.ni) {   /* one entry per neuron */
+			const uint32_t x = ca.iidx[tid] - first;
+			if(x < nb) ext[x] = ca.ival[tid];
 		}
 		__syncthreads();
 	}
@@ -150,7 +138,7 @@ __global__ void __launch_bounds__(BLOCK) nemo_cycle_kernel(const NetDev nd, cons
 	if(lane == 0) {
 		const uint32_t word = l >> 6;
 		if(word < nd.words) {
-			nd.raster[size_t(ca.k) * nd.words + word] = mask;
+			nd.raster[word] = mask;
 		}
 		wmask[wave] = mask;
 		wfired[wave] = uint32_t(__popcll(mask));
@@ -159,7 +147,7 @@ __global__ void __launch_bounds__(BLOCK) nemo_cycle_kernel(const NetDev nd, cons
 	/* the workgroup's words to the host in one write: over PCIe, and for the
 	 * host's cache, four of 8 bytes cost four times as much (step() of 100k x 100
 	 * 38 -> 33 us, 200k x 100 56 -> 43) */
-	if(ca.hostRow && tid < nb / 64u && first / 64u + tid < nd.words) st_host(ca.hostRow + first / 64u + tid, wmask[tid]);
+	if(tid < nb / 64u && first / 64u + tid < nd.words) st_host(ca.hostRow + first / 64u + tid, wmask[tid]);
 	uint32_t before = 0, total = 0;
 #pragma unroll
 	for(uint32_t w = 0; w < WAVES; ++w) {
@@ -167,7 +155,7 @@ __global__ void __launch_bounds__(BLOCK) nemo_cycle_kernel(const NetDev nd, cons
 		total += wfired[w];
 	}
 	if(total == 0u) {   /* block-uniform */
-		if(ca.report) finish_cycle(ca);
+		finish_cycle(ca);
 		return;
 	}
 	if(fired) {
@@ -184,7 +172,6 @@ __global__ void __launch_bounds__(BLOCK) nemo_cycle_kernel(const NetDev nd, cons
 	const uint2* syn = reinterpret_cast<const uint2*>(nd.syn);
 	uint32_t* row = rows + wave * (P + 1u);
 	const uint32_t top = P > 1u ? 1u << (31u - uint32_t(__builtin_clz(P - 1u))) : 0u;
-	uint32_t ev = 0;
 	uint32_t turn = 0;
 	for(uint32_t j0 = 0; j0 < total; j0 += 64u) {
 		uint32_t ra = 0, rb = 0;     /* rows of 64 sources, one per lane */
@@ -239,31 +226,15 @@ __global__ void __launch_bounds__(BLOCK) nemo_cycle_kernel(const NetDev nd, cons
 						atomicAdd(nd.ring + (size_t(q[u]) * 2u * R + plane + sl) * T + (rec[u].x & 0xffffu), w);
 					}
 				}
-				ev += min(256u, b - c);
 			}
 		}
 	}
-	if(ca.part) {
-		if(lane == 0) wsum[wave] = ev;
-		__syncthreads();
-		if(tid == 0) {
-			uint32_t sum = 0;
-			for(uint32_t w = 0; w < WAVES; ++w) sum += wsum[w];
-			ca.part[blockIdx.x] += sum;
-		}
-	}
-	if(ca.report) finish_cycle(ca);
+	finish_cycle(ca);
 }
 
 } // namespace
 
 extern "C" {
-
-uint32_t nemo_dev_cycle_blocks(uint32_t P, uint32_t T)
-{
-	const uint32_t nb = neurons_per_block(P * T);
-	return (P * T + nb - 1u) / nb;
-}
 
 uint32_t nemo_dev_cycle_block_neurons(uint32_t P, uint32_t T)
 {
@@ -278,7 +249,8 @@ int nemo_dev_cycle_fits(uint32_t P)
 int nemo_dev_cycle(const NetDev* nd, const CycleArgs* ca, void* stream)
 {
 	if(!nemo_dev_cycle_fits(nd->P)) return int(hipErrorInvalidValue);
-	const uint32_t blocks = nemo_dev_cycle_blocks(nd->P, nd->T);
+	const uint32_t nb = neurons_per_block(nd->P * nd->T);
+	const uint32_t blocks = (nd->P * nd->T + nb - 1u) / nb;
 	const uint32_t lds = uint32_t(dynamic_lds(nd->P));
 	auto kernel = (nd->flags & NEMO_NET_IZHIKEVICH_ONLY) ? &nemo_cycle_kernel<true> : &nemo_cycle_kernel<false>;
 	hipLaunchKernelGGL(kernel, dim3(blocks), dim3(BLOCK), lds, static_cast<hipStream_t>(stream), *nd, *ca);

@@ -109,8 +109,8 @@ typedef struct NetDev {
 	uint64_t* raster;         /* [nsteps][words] fired bits */
 } NetDev;
 
-/* One cycle by cycle_kernel.hip: its place in the launch and its stimulus,
- * where the launch's descriptor holds no schedule (one current per neuron). */
+/* One cycle by cycle_kernel.hip: its stimulus (one current per neuron) and its
+ * report */
 #define NEMO_CYCLE_STIM 64u
 #define NEMO_DONE_GROUPS 16u   /* first-level counters of finished workgroups */
 
@@ -123,14 +123,12 @@ typedef struct CycleReport {
 } CycleReport;
 
 typedef struct CycleArgs {
-	uint32_t k;               /* cycle within the launch (raster row, schedule entry) */
-	uint32_t slot;            /* (cycle0 + k) mod (D+1) */
+	uint32_t slot;            /* cycle0 mod (D+1) */
 	uint32_t nf, ni;
-	uint64_t* hostRow;        /* the cycle's raster words in host memory too; NULL: no */
-	unsigned long long* part; /* [nemo_dev_cycle_blocks] delivered synapses by workgroup; NULL: not counted */
-	CycleReport* report;      /* host memory; NULL: none */
+	uint64_t* hostRow;        /* the cycle's raster words in host memory too */
+	CycleReport* report;      /* host memory */
 	uint64_t sequence;
-	uint32_t* done;           /* [1 + NEMO_DONE_GROUPS][32] counters, zero between launches (with report) */
+	uint32_t* done;           /* [1 + NEMO_DONE_GROUPS][32] counters, zero between launches */
 	uint32_t fidx[NEMO_CYCLE_STIM];
 	uint32_t iidx[NEMO_CYCLE_STIM];
 	float ival[NEMO_CYCLE_STIM];
@@ -165,10 +163,9 @@ int nemo_dev_step_launch_one(const NetDev* nd_host, const WorkItem* work_dev, ui
 		uint32_t blockDim, uint32_t ldsBytes, uint32_t variant, void* stream);
 /* One cycle of a network without STDP whose sums stay within int32 */
 int nemo_dev_cycle(const NetDev* nd_host, const CycleArgs* ca, void* stream);
-uint32_t nemo_dev_cycle_blocks(uint32_t P, uint32_t T);
 /* whether the bucket bounds of P partitions fit its LDS */
 int nemo_dev_cycle_fits(uint32_t P);
-/* neurons of one of its workgroups */
+/* neurons of one of its workgroups, a power of two */
 uint32_t nemo_dev_cycle_block_neurons(uint32_t P, uint32_t T);
 /* The end of a launch of one network, after its step kernel on the stream: its
  * control block to host memory, then the report; the clock words start anew. */
