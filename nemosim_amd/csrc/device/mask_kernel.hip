@@ -42,39 +42,52 @@ constexpr uint32_t CHUNK = 64u;      /* synapses per STDP work item (one per lan
 /* The words that a wave polls. Neurons that fire together are often neighbours,
  * and with contiguous shares one wave delivers all of them. So the words are
  * dealt to the waves in turn, one at a time while a wave has up to 64, in pieces
- * of 8 (64 bytes) beyond; there among GROUP waves, since a wave delivers once all
+ * of 8 (64 bytes) beyond; there among four waves, since a wave delivers once all
  * its words have come, and with words from all partitions it waits for the last
- * of them. Per cycle with 1000 forced neighbours, contiguous and dealt: 5k x 1000
- * 97, 51 us (lists 66), 50k x 300 43, 29 (32), 200k x 100 59, 35 (37), with STDP
- * 20k x 300 58, 42 (48); without them 1k x 100 2.61, 2.45, 10k x 313 3.6, 3.4, 60k x
- * 300 4.5, 4.4, 200k x 300 8.5, 8.7 (8.9 dealt to all waves), 200k x 1000 and 50k x
- * 1000 with STDP 1 and 3 % less. */
-template<uint32_t WORDS>
+ * of them. The kernels for batches and for saturating networks (ANY) decide so
+ * for each network, and deal to more than 8 waves by pieces, too (32 networks in
+ * partitions of 512 to 960, 200 cycles: 2.64 ms one at a time, 2.39). Per cycle
+ * with 1000 forced neighbours, contiguous and dealt: 5k x 1000 97, 51 us (lists
+ * 66), 50k x 300 43, 29 (32), 200k x 100 59, 35 (37), with STDP 20k x 300 58, 42
+ * (48); without them 1k x 100 2.7, 2.5, 10k x 313 3.6, 3.4, 60k x 300 4.5, 4.4,
+ * 200k x 300 8.6, 8.8 (9.0 dealt to all waves), 200k x 1000 and 50k x 1000 with
+ * STDP 1 and 3 % less, 1k x 100 IF_curr_exp_noise at 333 Hz 2 % more. */
+template<uint32_t WORDS, bool ANY, bool IZO>
 struct Deal {
-	static constexpr uint32_t PIECE = WORDS == 1u ? 0u : 3u;
-	static constexpr uint32_t GROUP = WORDS == 1u ? 16u : 4u;
 	uint32_t waves, begin, end;   /* of the wave's group; begin: its own first word */
+	uint32_t plog;                /* ANY: of either kind */
+	__device__ inline uint32_t piece() const { return ANY ? plog : WORDS == 1u ? 0u : 3u; }
 	__device__ inline Deal(uint32_t wave, uint32_t nwaves, uint32_t W)
 	{
-		const uint32_t g0 = wave - wave % GROUP, g1 = min(g0 + GROUP, nwaves);
+		const bool few = ANY ? W <= 64u * nwaves && nwaves <= 8u : WORDS == 1u;
+		plog = few ? 0u : 3u;
+		const uint32_t group = few ? 16u : 4u;
+		const uint32_t g0 = wave & ~(group - 1u), g1 = min(g0 + group, nwaves);
 		waves = g1 - g0;
 		end = wave >= nwaves ? 0u : g1 == nwaves ? W : (W * g1 / nwaves) & ~15u;   /* waves beyond: no words */
-		begin = ((W * g0 / nwaves) & ~15u) + ((wave - g0) << PIECE);
+		begin = ((W * g0 / nwaves) & ~15u) + ((wave - g0) << piece());
 	}
-	/* the j-th of the wave's words; the first of those from the j-th on, j a
-	 * multiple of 64, and how much further a lane's own is */
-	__device__ inline uint32_t word(uint32_t j) const { return first(j & ~63u) + further(j & 63u); }
+	/* the first of the wave's words from the j-th on, j a multiple of 64; how much
+	 * further a lane's own is, and the (j+k)-th, k < 64 WORDS */
 	__device__ inline uint32_t first(uint32_t j) const { return begin + j * waves; }
 	__device__ inline uint32_t further(uint32_t lane) const
 	{
-		return (__umul24(lane >> PIECE, waves) << PIECE) | (lane & ((1u << PIECE) - 1u));
+		return (__umul24(lane >> piece(), waves) << piece()) | (lane & ((1u << piece()) - 1u));
+	}
+	__device__ inline uint32_t word(uint32_t j, uint32_t k) const
+	{
+		/* the Izhikevich kernels are slower with the shorter product (60k x 300
+		 * 4.4 -> 4.6 us), the others 3 % faster */
+		if(IZO) return first((j + k) & ~63u) + further(k & 63u);
+		if(WORDS == 1u) return first(j) + further(k);
+		return first(j) + __umul24(k & ~63u, waves) + further(k & 63u);
 	}
 };
 
 /* The neurons that fired in an earlier cycle, whose words are complete, of the
  * words dealt to a wave: f(valid, neuron) for whole waves. */
-template<uint32_t WORDS, typename F>
-__device__ inline void each_fired(const NEMO_GLOBAL uint64_t* words, uint32_t tag, const Deal<WORDS>& deal,
+template<uint32_t WORDS, bool ANY, bool IZO, typename F>
+__device__ inline void each_fired(const NEMO_GLOBAL uint64_t* words, uint32_t tag, const Deal<WORDS, ANY, IZO>& deal,
 		uint16_t* list, uint32_t lane, F f)
 {
 	const uint32_t mine = deal.further(lane);
@@ -108,7 +121,7 @@ __device__ inline void each_fired(const NEMO_GLOBAL uint64_t* words, uint32_t ta
 			for(uint32_t h = 0; h < n; h += 64u) {   /* wave-uniform */
 				const bool ok = h + lane < n;
 				const uint32_t e = ok ? list[h + lane] : 0u;
-				f(ok, deal.word(c0 + (e >> 5)) * 32u + (e & 31u));
+				f(ok, deal.word(c0, e >> 5) * 32u + (e & 31u));
 			}
 			__builtin_amdgcn_wave_barrier();   /* the list is written again */
 		}
@@ -180,14 +193,14 @@ struct StdpLds {
 };
 
 /* K: chunks of a wave whose loads are in flight together */
-template<bool SAT, uint32_t WORDS, uint32_t K>
+template<bool SAT, bool IZO, uint32_t WORDS, bool ANY, uint32_t K>
 __device__ inline void stdp_waves(const NetDev& nd, uint32_t p, uint32_t wave, uint32_t nwaves, uint32_t lane,
 		const StdpLds& l, uint16_t* list)
 {
 	const uint32_t P = nd.P, R = nd.flRing, n_total = nd.n, cache = nd.stdpCache;
 	const uint32_t postLen = uint32_t(l.table->postLen);
 	const uint32_t W = P * (nd.T >> 5);
-	const Deal<WORDS> deal(wave, nwaves, W);
+	const Deal<WORDS, ANY, IZO> deal(wave, nwaves, W);
 	const NEMO_GLOBAL uint32_t* rsd = glb(nd.rcm_sd);
 	NEMO_GLOBAL int32_t* racc = glb(nd.rcm_acc);
 	const StdpMasks m = *l.masks;
@@ -248,7 +261,7 @@ __device__ inline void stdp_waves(const NetDev& nd, uint32_t p, uint32_t wave, u
 			return;
 		}
 		const uint32_t s = tslot >= postLen ? tslot - postLen : tslot + R - postLen;
-		each_fired<WORDS>(glb(nd.mk) + size_t(s) * nemo_mask_words(W), tc - postLen, deal, list, lane, [&](bool ok, uint32_t x) {
+		each_fired<WORDS, ANY, IZO>(glb(nd.mk) + size_t(s) * nemo_mask_words(W), tc - postLen, deal, list, lane, [&](bool ok, uint32_t x) {
 			const Row row = row_of(ok, x);
 			uint32_t ch = row.ch;
 			while(__any(ch * CHUNK < row.len)) {   /* wave-uniform */
@@ -283,7 +296,7 @@ __device__ inline void stdp_waves(const NetDev& nd, uint32_t p, uint32_t wave, u
 		/* this cycle's chunks; the records of the first `cache` go to LDS */
 		if(t >= postLen) {
 			const uint32_t s = wslot >= postLen ? wslot - postLen : wslot + R - postLen;
-			each_fired<WORDS>(glb(nd.mk) + size_t(s) * nemo_mask_words(W), tag - postLen, deal, list, lane, [&](bool ok, uint32_t x) {
+			each_fired<WORDS, ANY, IZO>(glb(nd.mk) + size_t(s) * nemo_mask_words(W), tag - postLen, deal, list, lane, [&](bool ok, uint32_t x) {
 				const Row row = row_of(ok, x);
 				uint32_t ch = row.ch;
 				while(__any(ch * CHUNK < row.len)) {   /* wave-uniform */
@@ -336,7 +349,7 @@ __device__ inline void deliver_far(const NetDev& nd, const uint2* far, uint32_t 
  * per 64 WORDS, and every word costs instructions whether it is there or not
  * (10k x 100: 4.0 us a cycle with 4, 4.5 with 8; 200k x 100: 9.0 with 4, 8.4
  * with 8), so the host picks the smallest of 1, 4 and 8 that covers the share. */
-template<bool SAT, bool IZO, uint32_t WORDS, bool STDP>
+template<bool SAT, bool IZO, uint32_t WORDS, bool STDP, bool ANY>
 __device__ __forceinline__ void run_masked(const NetDev& nd, uint32_t p)
 {
 	constexpr int NP = IZO ? 5 : MAX_PARAM;
@@ -441,7 +454,7 @@ __device__ __forceinline__ void run_masked(const NetDev& nd, uint32_t p)
 		noise = prm[IZ_SIGMA] * nrand(rng);
 	}
 	const uint32_t W = P * fwords;
-	const Deal<WORDS> deal(wave, nw, W);
+	const Deal<WORDS, ANY, IZO> deal(wave, nw, W);
 	const uint32_t myFurther = deal.further(lane);
 	uint32_t wslot = uint32_t(nd.cycle0 % R);               /* cycle mod R */
 	if(STDP) {
@@ -491,7 +504,7 @@ __device__ __forceinline__ void run_masked(const NetDev& nd, uint32_t p)
 	__syncthreads();
 
 	const bool learns = STDP && wave >= nw && wave < nw + nsw;   /* its barriers are those of this loop */
-	if(learns) stdp_waves<SAT, WORDS, IZO ? 8u : 4u>(nd, p, wave - nw, nsw, lane, stdpLds, list);
+	if(learns) stdp_waves<SAT, IZO, WORDS, ANY, IZO ? 8u : 4u>(nd, p, wave - nw, nsw, lane, stdpLds, list);
 	const bool carries = nfw && wave >= nw + nsw && wave < nw + nsw + nfw;
 	if(carries) {
 		uint32_t prev = slotK;   /* slot of the cycle before */
@@ -644,7 +657,7 @@ __device__ __forceinline__ void run_masked(const NetDev& nd, uint32_t p)
 					if(ld_agent(glb(nd.status)) != 0u) break;
 					if(spins > nd.spinLimit) {
 						report_timeout(nd.status, NEMO_STATUS_BARRIER_TIMEOUT, tag, p,
-								deal.word(c0 + 64u * uint32_t(__builtin_ctz(pending)) + lane) / fwords);
+								deal.word(c0, 64u * uint32_t(__builtin_ctz(pending)) + lane) / fwords);
 						break;
 					}
 				}
@@ -709,13 +722,13 @@ __device__ __forceinline__ void run_masked(const NetDev& nd, uint32_t p)
 				uint32_t a0 = 0, b0r = 0, a1 = 0, b1r = 0;
 				if(v0) {
 					const uint32_t e = list[lane];
-					const NEMO_GLOBAL uint32_t* o = off + size_t(deal.word(c0 + (e >> 5)) * 32u + (e & 31u)) * (P + 1u) + p;
+					const NEMO_GLOBAL uint32_t* o = off + size_t(deal.word(c0, e >> 5) * 32u + (e & 31u)) * (P + 1u) + p;
 					a0 = ld_off(o);
 					b0r = ld_off(o + 1) & offMask;
 				}
 				if(v1) {
 					const uint32_t e = list[64u + lane];
-					const NEMO_GLOBAL uint32_t* o = off + size_t(deal.word(c0 + (e >> 5)) * 32u + (e & 31u)) * (P + 1u) + p;
+					const NEMO_GLOBAL uint32_t* o = off + size_t(deal.word(c0, e >> 5) * 32u + (e & 31u)) * (P + 1u) + p;
 					a1 = ld_off(o);
 					b1r = ld_off(o + 1) & offMask;
 				}
@@ -830,7 +843,7 @@ nemo_mask_kernel(const NetDev* __restrict__ nets, const WorkItem* __restrict__ w
 {
 	const WorkItem wi = work[blockIdx.x];
 	const NetDev nd = nets[wi.net];
-	run_masked<SAT, IZO, 4u, STDP>(nd, wi.part);
+	run_masked<SAT, IZO, 4u, STDP, true>(nd, wi.part);
 }
 
 /* one network per launch: the descriptor as a kernel argument */
@@ -838,7 +851,7 @@ template<bool SAT, bool IZO, uint32_t WORDS, bool STDP>
 __global__ void __launch_bounds__(1024)
 nemo_mask_kernel_single(const NetDev nd, const WorkItem* __restrict__ work)
 {
-	run_masked<SAT, IZO, WORDS, STDP>(nd, work[blockIdx.x].part);
+	run_masked<SAT, IZO, WORDS, STDP, SAT>(nd, work[blockIdx.x].part);
 }
 
 namespace {
