@@ -869,8 +869,27 @@ Simulation::Simulation(const NetworkImpl& net, const ConfigurationImpl& conf) :
 	}
 	hipCheck(hipHostMalloc(reinterpret_cast<void**>(&h_step), std::max<size_t>(m_words, 1) * 8), "hipHostMalloc");
 	ensureRaster(8);
+	std::vector<uint32_t> rows;
+	if(cycleKernelRuns() && m_nsyn > 0 && (size_t(m_n) + 1) * 4 <= d_raster.bytes) {
+		/* where the sources' rows start, by way of the raster's buffer */
+		rows.resize(size_t(m_n) + 1);
+		hipCheck(nemo_dev_build_gather(d_off.as<uint32_t>(), m_P + 1, m_n, d_raster.as<uint32_t>(), s), "construction kernel");
+		hipCheck(hipMemcpyAsync(rows.data(), d_raster.ptr, rows.size() * 4, hipMemcpyDeviceToHost, s), "hipMemcpyAsync D2H");
+	}
 	hipCheck(hipStreamSynchronize(s), "hipStreamSynchronize");
 	devLock.unlock();
+	if(!rows.empty()) {
+		const uint32_t mask = m_defer ? (1u << NEAR_SHIFT) - 1u : ~0u;
+		uint32_t longest = 0;
+		for(uint32_t l = 0; l < m_n; ++l) {
+			rows[l] = (rows[l + 1] & mask) - (rows[l] & mask);
+			longest = std::max(longest, rows[l]);
+		}
+		if(longest > 2048u && double(longest) * m_n > 4.0 * double(m_nsyn)) {
+			rows.pop_back();
+			m_rows.swap(rows);
+		}
+	}
 
 	m_deviceBytes = d_model.bytes + d_param.bytes + d_state.bytes + d_rng.bytes + d_recent.bytes
 		+ d_ring.bytes + d_off.bytes + d_syn.bytes + d_fl.bytes + d_fc.bytes + d_mk.bytes + d_rfg.bytes + d_srow.bytes
@@ -1674,7 +1693,8 @@ static const double CYCLE_MAX_EVENTS = 1.0e6;
  * do), less a sixteenth per step. Calls with 4, 16 and 64 forced neighbours,
  * cycle kernel (fused kernel 36 to 44 us): 1k x 100 20, 26, 49; 5k x 1000 31, 69,
  * 216; 20k x 300 25, 44, 118; 100k x 300 (fused 72) 41, 58, 138; 200k x 300 (115)
- * 56, 73, 152. */
+ * 56, 73, 152. With one and four neighbours of 10000 synapses, 100k x 20, 65 and
+ * 165 (74, 74); of 30000 134 and 416 (83, 85). */
 bool
 Simulation::stepCrowded(const std::vector<unsigned>& fstim) const
 {
@@ -1682,8 +1702,23 @@ Simulation::stepCrowded(const std::vector<unsigned>& fstim) const
 	const double chunks = row <= 128.0 ? 0.65 : std::ceil(row / 256.0);
 	const double limit = (30.0 + double(m_n) / 4000.0) / chunks;
 	if(m_crowd > limit) return true;
-	if(double(fstim.size()) <= limit) return false;
 	const int shift = __builtin_ctz(nemo_dev_cycle_block_neurons(m_P, m_T));
+	if(!m_rows.empty()) {
+		/* rows of very different lengths: the forced ones' own */
+		std::pair<unsigned, unsigned> chunksOf[NEMO_CYCLE_STIM];
+		for(size_t i = 0; i < fstim.size(); ++i) {
+			const unsigned l = localIdx(fstim[i]);
+			chunksOf[i] = std::make_pair(l >> shift, (m_rows[l] + 255u) / 256u);
+		}
+		std::sort(chunksOf, chunksOf + fstim.size());
+		uint64_t sum = 0;
+		for(size_t i = 0; i < fstim.size(); ++i) {
+			sum = chunksOf[i].second + (i && chunksOf[i].first == chunksOf[i - 1].first ? sum : 0u);
+			if(double(sum) > limit * chunks) return true;
+		}
+		return false;
+	}
+	if(double(fstim.size()) <= limit) return false;
 	unsigned forced[NEMO_CYCLE_STIM], most = 0;
 	unsigned char count[256] = {};   /* by the low bits of the workgroup: no fewer than are in one */
 	for(size_t i = 0; i < fstim.size(); ++i) {

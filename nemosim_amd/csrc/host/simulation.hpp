@@ -264,6 +264,7 @@ class Simulation
 		void stepCycle(const nemo_schedule_t& s);
 		bool stepCrowded(const std::vector<unsigned>& fstim) const;
 		void countCrowd();
+		std::vector<uint32_t> m_rows;  /* synapses of each source, where some have many times the average */
 		double m_crowd = 0.0;          /* fired neurons of a workgroup of the cycle kernel beyond its share */
 		DevBuf d_done;                 /* CycleArgs.done */
 		uint64_t m_cycleSequence = 0;  /* launches that report to h_ctl */

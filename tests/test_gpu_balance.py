@@ -79,6 +79,32 @@ def test_step(nemo_mod, n, m):
     assert adjacent < 2.0 * spread, (adjacent, spread)
 
 
+def test_step_long_rows(nemo_mod):
+    """steps with four forced neurons with rows of 30000 synapses"""
+    n = 100000
+
+    def run(which):
+        spec = examples.izhikevich_80_20(n, 20, seed=3)
+        length = np.full(n, 20, np.int64)
+        length[which] = 30000
+        spec.rowptr = np.concatenate([[0], np.cumsum(length)]).astype(np.uint64)
+        rng, count = np.random.default_rng(4), int(length.sum())
+        spec.targets = rng.integers(0, n, count).astype(np.uint32)
+        spec.delays = rng.integers(1, 21, count).astype(np.uint8)
+        spec.weights = rng.uniform(-0.1, 0.1, count).astype(np.float32)
+        spec.plastic = np.zeros(count, np.uint8)
+        sim = hip_sim(nemo_mod, spec)
+
+        def steps():
+            for _ in range(CYCLES):
+                sim.step(which)
+
+        return best(steps)
+
+    adjacent, spread = [run(p) for p in populations(n, 4)]
+    assert adjacent < 2.0 * spread, (adjacent, spread)
+
+
 def test_per_cycle_step_long_rows(nemo_mod):
     """neurons with rows of 10000 synapses, next to each other and far apart"""
     n, hubs = 270000, 20
