@@ -12,8 +12,8 @@ ms of wall time per simulated second. Timing follows NeMo's benchmark()
 cycles; the network and its state are resident on the GPU before timing.
 
 The default prints one JSON line with the roofline of the step kernel
-(algorithmic bytes per launch / kernel time from HIP events on the kernel's
-stream) and a CPU baseline: the oracle (a restatement of NeMo's OpenMP CPU
+(algorithmic bytes per launch / kernel time, from the first start to the last
+end of its workgroups on the device clock) and a CPU baseline: the oracle (a restatement of NeMo's OpenMP CPU
 backend) timed on a bounded sample of the same workload on this host.
 
 Other workloads (--workload): "stdp" (50k x 1000, STDP, applyStdp every

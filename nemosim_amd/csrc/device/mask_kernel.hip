@@ -13,7 +13,7 @@
  * That is one round trip less, two barriers a cycle instead of three, and no
  * search for a source's partition. Each workgroup reads n/32 words a cycle
  * whatever fires (50 KB at 200k neurons), which costs a wave up to eight loads
- * that are in flight together.
+ * that are in flight together; how the words are shared is at Deal.
  *
  * What bounds it: the latency of the chain update -> words -> bounds -> delay-1
  * records of one cycle; no unit is busy. From 200k neurons on, with few waves

@@ -388,16 +388,15 @@ Simulation::Simulation(const NetworkImpl& net, const ConfigurationImpl& conf) :
 		whyNotFused = "a neuron type has no fused implementation";
 	}
 
-	/* Networks exchange their fired bits as words (mask_kernel.hip), unless
-	 * the configuration asks for exchange waves or that kernel's LDS leaves too
-	 * few neurons per workgroup. Per cycle, lists against words: 1k x 100 4.5
-	 * -> 3.4 us, 10k x 1000 9.1 -> 6.0, 60k x 300 6.3 -> 5.4, 200k x 1000 13.8
-	 * -> 12.8, 12k x 550 IF_curr_exp_noise at 333 Hz 57 -> 47; with STDP 3k x
-	 * 300 10.9 -> 3.5, 10k x 300 10.5 -> 4.3, 50k x 1000 17.4 -> 10.7, 12k x
-	 * 550 at 333 Hz 283 -> 70. With STDP lists remain for what words do not
-	 * have: a window without cycles after the spike, work lists that are not to
-	 * be staged, workgroups that leave less than 6 of 16 waves for it, and a
-	 * configured workgroup of 512 neurons or more, which gets exchange waves. */
+	/* Networks exchange their fired bits as words (mask_kernel.hip, which has
+	 * the figures), unless the configuration asks for exchange waves or that
+	 * kernel's LDS leaves too few neurons per workgroup. With STDP lists remain
+	 * for what words do not have: a window without cycles after the spike, work
+	 * lists that are not to be staged, workgroups that leave less than 6 of 16
+	 * waves for it; and for a configured workgroup of 512 neurons or more, which
+	 * nemo_set_exchange_waves promises exchange waves. Words would be faster
+	 * there, too: 10k x 300 in partitions of 512 10.8 us per cycle with lists,
+	 * of 448 5.5 with words. */
 	const uint32_t postLen = m_stdp ? uint32_t(m_sp.postLen) : 0u;
 	m_masks = conf.exchangeWaves <= 0;
 	if(m_stdp && (postLen < 1u || !conf.stdpLdsStaging || conf.partitionSize >= 512u)) m_masks = false;
