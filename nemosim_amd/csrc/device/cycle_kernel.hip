@@ -232,9 +232,36 @@ __global__ void __launch_bounds__(BLOCK) nemo_cycle_kernel(const NetDev nd, cons
 	finish_cycle(ca);
 }
 
+__global__ void __launch_bounds__(BLOCK) longest_row_kernel(const uint32_t* off, uint32_t stride, uint32_t n, uint32_t mask,
+		uint32_t* max, uint32_t* done, uint32_t* out)
+{
+	uint32_t most = 0;
+	for(uint32_t i = blockIdx.x * BLOCK + threadIdx.x; i < n; i += gridDim.x * BLOCK) {
+		const uint32_t a = off[size_t(i) * stride] & mask, b = off[(size_t(i) + 1u) * stride] & mask;
+		most = b - a > most ? b - a : most;
+	}
+	for(uint32_t d = 32; d >= 1; d >>= 1) {
+		const uint32_t x = __shfl_down(most, d, 64);
+		most = x > most ? x : most;
+	}
+	if((threadIdx.x & 63u) == 0u) atomicMax(max, most);
+	if(last_block(done, blockIdx.x, gridDim.x)) {
+		st_host(out, __hip_atomic_load(max, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+	}
+}
+
 } // namespace
 
 extern "C" {
+
+int nemo_dev_longest_row(const uint32_t* off, uint32_t stride, uint32_t n, uint32_t mask, uint32_t* max, uint32_t* done,
+		uint32_t* out, void* stream)
+{
+	const uint32_t blocks = n > 256u * BLOCK ? 256u : (n + BLOCK - 1u) / BLOCK;
+	hipLaunchKernelGGL(longest_row_kernel, dim3(blocks), dim3(BLOCK), 0, static_cast<hipStream_t>(stream),
+			off, stride, n, mask, max, done, out);
+	return int(hipGetLastError());
+}
 
 uint32_t nemo_dev_cycle_block_neurons(uint32_t P, uint32_t T)
 {

@@ -18,12 +18,13 @@
  * What bounds it: the latency of the chain update -> words -> bounds -> delay-1
  * records of one cycle; no unit is busy. From 200k neurons on, with few waves
  * left over, the requests for bounds and records. Per cycle, lists, words with
- * the far records on the neurons' waves, and on far waves: 1k x 100 4.5, 3.5,
- * 2.6 us; 10k x 313 5.6, 4.6, 3.5; 60k x 300 6.3, 5.7, 4.6; 100k x 100 7.6, 6.3,
- * 5.3; 200k x 1000 13.8, 12.9, 12.9; 12k x 550 IF_curr_exp_noise at 333 Hz 57,
- * 49, 38. 48 networks of 1k-20k batched (no far waves), 200 cycles, 3.96 ->
- * 3.04 ms. With STDP, 3k x 300 10.9 -> 3.5 us, 10k
- * x 300 10.5 -> 4.3, 50k x 1000 17.4 -> 10.7 (see stdp_waves).
+ * the far records on the neurons' waves, on far waves, and dealt: 1k x 100 4.5,
+ * 3.5, 2.6, 2.5 us; 10k x 313 5.6, 4.6, 3.5, 3.4; 60k x 300 6.3, 5.7, 4.6, 4.4;
+ * 100k x 100 7.6, 6.3, 5.4, 5.3; 200k x 1000 13.8, 12.9, 12.6, 12.7; 12k x 550
+ * IF_curr_exp_noise at 333 Hz 57, 49, 37, 37. 48 networks of 1k-20k batched, 200
+ * cycles, 3.96 -> 3.1 ms (3 launches, with far waves where all of one's networks
+ * fit with them). With STDP, 3k x 300 10.9 -> 3.4 us, 10k x 300 10.5 -> 4.3, 50k x
+ * 1000 17.4 -> 10.2 (see stdp_waves).
  *
  * Without STDP two buffers of words are enough: a wave publishes cycle t+1 after its own
  * reads of cycle t, and a workgroup publishes t+2 only once its waves have

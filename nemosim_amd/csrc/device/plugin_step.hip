@@ -203,9 +203,8 @@ __global__ void __launch_bounds__(256) pm_scatter_kernel(PluginStepDev s, uint32
  * What bounds it: the neurons' parameters, state and ring slot (about 90 bytes
  * each) and the chain slot -> update -> row bounds -> records -> atomics; with
  * many spikes the atomics. Per cycle, against the plugins' sequence as it was
- * (begin, update, compact, scatter): 300k x 100 37 -> 14.2 us, 400k x 250 62 ->
- * 31, 100k x 100 with delays up to 60 20.8 -> 8.9, 70k x 60 IF_curr_exp_noise
- * at 333 Hz 114 -> 31, 150k x 60 with STDP 35 -> 15.7. */
+ * (begin, update, compact, scatter): 300k x 100 37 -> 13.4 us, 300k x 50 35 ->
+ * 9.9, 300k x 30 IF_curr_exp_noise 67 -> 13, 300k x 50 with STDP 56 -> 18. */
 template<typename ACC, bool IZO, bool DELIVER>
 __global__ void __launch_bounds__(256) pm_cycle_kernel(PluginStepDev s, uint32_t k, int stim)
 {

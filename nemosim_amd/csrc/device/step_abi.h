@@ -165,6 +165,10 @@ int nemo_dev_step_launch_one(const NetDev* nd_host, const WorkItem* work_dev, ui
 int nemo_dev_cycle(const NetDev* nd_host, const CycleArgs* ca, void* stream);
 /* whether the bucket bounds of P partitions fit its LDS */
 int nemo_dev_cycle_fits(uint32_t P);
+/* *out (host memory) = the most synapses of a source, whose rows start at
+ * off[i * stride] & mask; max: a zero word, done: counters as in CycleArgs */
+int nemo_dev_longest_row(const uint32_t* off, uint32_t stride, uint32_t n, uint32_t mask, uint32_t* max, uint32_t* done,
+		uint32_t* out, void* stream);
 /* neurons of one of its workgroups, a power of two */
 uint32_t nemo_dev_cycle_block_neurons(uint32_t P, uint32_t T);
 /* The end of a launch of one network, after its step kernel on the stream: its

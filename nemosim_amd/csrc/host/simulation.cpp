@@ -868,27 +868,26 @@ Simulation::Simulation(const NetworkImpl& net, const ConfigurationImpl& conf) :
 	}
 	hipCheck(hipHostMalloc(reinterpret_cast<void**>(&h_step), std::max<size_t>(m_words, 1) * 8), "hipHostMalloc");
 	ensureRaster(8);
-	std::vector<uint32_t> rows;
-	if(cycleKernelRuns() && m_nsyn > 0 && (size_t(m_n) + 1) * 4 <= d_raster.bytes) {
-		/* where the sources' rows start, by way of the raster's buffer */
-		rows.resize(size_t(m_n) + 1);
-		hipCheck(nemo_dev_build_gather(d_off.as<uint32_t>(), m_P + 1, m_n, d_raster.as<uint32_t>(), s), "construction kernel");
-		hipCheck(hipMemcpyAsync(rows.data(), d_raster.ptr, rows.size() * 4, hipMemcpyDeviceToHost, s), "hipMemcpyAsync D2H");
+	/* the longest row of a source, for stepCrowded */
+	const bool longest = cycleKernelRuns() && m_nsyn > 0;
+	if(longest) {
+		hipCheck(nemo_dev_longest_row(d_off.as<uint32_t>(), m_P + 1, m_n, m_defer ? (1u << NEAR_SHIFT) - 1u : ~0u,
+					d_ctl.as<uint32_t>() + 12, d_done.as<uint32_t>(), h_ctl + 12, s), "construction kernel");
 	}
 	hipCheck(hipStreamSynchronize(s), "hipStreamSynchronize");
-	devLock.unlock();
-	if(!rows.empty()) {
+	if(longest && h_ctl[12] > 2048u && double(h_ctl[12]) * m_n > 4.0 * double(m_nsyn)) {
+		/* rows of very different lengths */
+		DevBuf d;
+		d.alloc((size_t(m_n) + 1) * 4);
+		hipCheck(nemo_dev_build_gather(d_off.as<uint32_t>(), m_P + 1, m_n, d.as<uint32_t>(), s), "construction kernel");
+		hipCheck(hipStreamSynchronize(s), "hipStreamSynchronize");
+		m_rows.resize(size_t(m_n) + 1);
+		hipCheck(hipMemcpy(m_rows.data(), d.ptr, m_rows.size() * 4, hipMemcpyDeviceToHost), "hipMemcpy D2H");
 		const uint32_t mask = m_defer ? (1u << NEAR_SHIFT) - 1u : ~0u;
-		uint32_t longest = 0;
-		for(uint32_t l = 0; l < m_n; ++l) {
-			rows[l] = (rows[l + 1] & mask) - (rows[l] & mask);
-			longest = std::max(longest, rows[l]);
-		}
-		if(longest > 2048u && double(longest) * m_n > 4.0 * double(m_nsyn)) {
-			rows.pop_back();
-			m_rows.swap(rows);
-		}
+		for(uint32_t l = 0; l < m_n; ++l) m_rows[l] = (m_rows[l + 1] & mask) - (m_rows[l] & mask);
+		m_rows.pop_back();
 	}
+	devLock.unlock();
 
 	m_deviceBytes = d_model.bytes + d_param.bytes + d_state.bytes + d_rng.bytes + d_recent.bytes
 		+ d_ring.bytes + d_off.bytes + d_syn.bytes + d_fl.bytes + d_fc.bytes + d_mk.bytes + d_rfg.bytes + d_srow.bytes
@@ -1743,7 +1742,7 @@ Simulation::countCrowd()
 	const int shift = __builtin_ctz(block);
 	uint32_t most = 0, same = 0, last = ~0u;
 	for(unsigned g : m_fired) {   /* ascending local index */
-		const uint32_t b = (m_dense[g - m_minG] - 1u) >> shift;
+		const uint32_t b = (m_affineIds ? g - m_minG : m_dense[g - m_minG] - 1u) >> shift;
 		same = b == last ? same + 1u : 1u;
 		last = b;
 		most = std::max(most, same);

@@ -329,7 +329,7 @@ Plan plan(unsigned n, const nemo_hip_rcm* rcm)
 	 * those of random networks are not: two or three rounds of reads more before the
 	 * first tile, two thirds of a tile per workgroup on average. 20000 x 30 with 20
 	 * neighbours of 15000 couplings each: 4311 us per cycle in shares of 20
-	 * oscillators, 223 so. */
+	 * oscillators, 240 so. */
 	const uint64_t longest = rcm->longest;
 	if(p.per > 1u && double(longest) > 4.0 * avg && longest * p.per > 2u * THREADS * p.threadCouplings) {
 		const uint64_t work = uint64_t(rcm->synapses) + uint64_t(OSC_COST) * n + 1u;
