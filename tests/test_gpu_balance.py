@@ -66,7 +66,7 @@ def test_fused(nemo_mod, n, m, pop, stdp):
     assert adjacent < 1.5 * spread, (adjacent, spread)
 
 
-@pytest.mark.parametrize("n,m", [(5000, 1000), (100000, 300)])
+@pytest.mark.parametrize("n,m", [(5000, 1000), (50000, 1000)])
 def test_step(nemo_mod, n, m):
     """steps with 60 forced neurons, more of which at once take another path"""
     sim = simulation(nemo_mod, n, m)
