@@ -154,12 +154,12 @@ __device__ inline void count_events(unsigned long long* part, uint32_t ev, uint3
 	}
 }
 
-/* Plugins, and built-in networks with long rows: the spikes of cycle k. Workgroup g of G takes the pieces g, g + G,
- * g + 2G, ... of 1 << plog neighbouring neurons, a neuron per lane, so that all
- * workgroups have sources whatever fires: neurons that fire together are often
- * neighbours. Every wave reads the fired
- * bits and the rows' bounds for itself, so nothing is listed and nothing
- * waited for.
+/* Plugins, and built-in networks with long rows: the spikes of cycle k.
+ * Workgroup g of G takes the pieces g, g + G, g + 2G, ... of 1 << plog
+ * neighbouring neurons, a neuron per lane, so that all workgroups have sources
+ * whatever fires: neurons that fire together are often neighbours. Every wave
+ * reads the fired bits and the rows' bounds for itself, so nothing is listed and
+ * nothing waited for.
  *
  * What bounds it: with few spikes the launch; with many the atomics. Per cycle
  * of the plugin step, with a wave per fired source of a list in memory, with a
